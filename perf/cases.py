@@ -42,7 +42,7 @@ def listed():
              init_p=10, init_s=10, pct=1.0, asymp=0.0, vaccination=0.0, closure=0),
         # The batcher's sweep also scales locations ten times the people
         # (10, 100): 23.5M agents over ten times as many, emptier locations.
-        dict(name="sim 24M, 10x locations", kind="sim", people=10.0, locations=100.0, days=60, r_p=1.8, r_s=1.3,
+        dict(name="sim 24M 10x locations", kind="sim", people=10.0, locations=100.0, days=60, r_p=1.8, r_s=1.3,
              init_p=60, init_s=60, pct=1.0, asymp=0.0, vaccination=0.0, closure=0),
         # Day by day with interventions and the state read back: 235k agents
         # in a 10x location grid (the sweep's 0.1, 1), asymptomatic cases.
@@ -57,15 +57,15 @@ def listed():
         # 3 scenarios x 8 seeds at 1M agents, 120 days, with interventions.
         dict(name="ensemble 3 x 8 at 1M", kind="ensemble", rows=3, replicates=8, agents=1000000, days=120),
         # The surrogate as it is trained: 5 members, batch 1024.
-        dict(name="train 5 x 1024, 100 steps", kind="train", members=5, batch=1024, steps=100, lr=1e-3, rows=7936),
+        dict(name="train 5 x 1024", kind="train", members=5, batch=1024, steps=100, lr=1e-3, rows=7936),
         # Screening predictions of an odd number of vectors.
         dict(name="predict 5 x 3001", kind="predict", members=5, batch=1024, rows=3001),
         # A handful of scenarios asked of a small ensemble.
         dict(name="predict 2 x 7", kind="predict", members=2, batch=64, rows=7),
         # A large location table: as many buckets as the 50M-agent weekday.
-        dict(name="table 20M, 61597 buckets", kind="table", pairs=20000000, buckets=61597, noalloc=False),
+        dict(name="table 20M to 61597", kind="table", pairs=20000000, buckets=61597, noalloc=False),
         # A small one, allocation-free, as a captured or tight loop calls it.
-        dict(name="table 29919, 545 buckets", kind="table", pairs=29919, buckets=545, noalloc=True),
+        dict(name="table 29919 to 545", kind="table", pairs=29919, buckets=545, noalloc=True),
     ]
 
 
