@@ -381,6 +381,7 @@ __device__ __forceinline__ bool select_block(const Model& M, uint64_t eoff, cons
     uint32_t key[NK];
     uint32_t sel = 0;
     bool bad = false;
+    const ErrandWalk wk = pinned(WEEKEND ? M.we_walk : M.wd_walk);
     if (WEEKEND) {
         const int base = M.we_base, E = M.we_E;
 #pragma unroll
@@ -389,7 +390,7 @@ __device__ __forceinline__ bool select_block(const Model& M, uint64_t eoff, cons
             key[3 * q] = key[3 * q + 1] = key[3 * q + 2] = 0;
             if (p < N) {
                 int32_t hour[3], loc[3];
-                weekend_errands(M, eoff + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
+                weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
 #pragma unroll
                 for (int e = 0; e < 3; ++e) {
                     int32_t l = loc[e] - base;
@@ -425,7 +426,7 @@ __device__ __forceinline__ bool select_block(const Model& M, uint64_t eoff, cons
                     const int64_t p = 2 * g + k;
                     if (p < N) {
                         int32_t d1, d2;
-                        weekday_dests(M, u.w[2 * k], u.w[2 * k + 1], ag[2 * q + k] == kAgeAdult, d1, d2);
+                        weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], ag[2 * q + k] == kAgeAdult, d1, d2);
                         const int i = 4 * q + 2 * k;
                         bad |= !weekday_keys(M, d1, d2, key[i], key[i + 1]);
                         key[i] += kbias;
@@ -736,8 +737,9 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
     // errands (device_recalc_weekdayErrandDests_assignProfile :3667-3705)
     const U4 ue = draw4(eoff + (uint64_t)(idx / 2), M.key0, M.key1);
     const int rs = 2 * (idx % 2);
+    const ErrandWalk wk = pinned(M.wd_walk);
     int32_t d1, d2;
-    weekday_dests(M, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
+    weekday_dests(M, wk, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
     const int prof = adult ? (int)((word(ue, rs) ^ word(ue, rs + 1)) % 3u) : 3;
     const int h0 = M.wd_assign[prof][0], h1 = M.wd_assign[prof][1];
     uint32_t k0, k1;
@@ -826,8 +828,9 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
     const int prof = (int)(u.w[3] % 6u);
     uint32_t v32[2];
     draw2x32((uint32_t)(Mc + 1), (uint32_t)M.key0, (uint32_t)M.key1, v32);
+    const ErrandWalk wk = pinned(M.we_walk);
     int32_t hour[3], loc[3];
-    weekend_errands(M, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
+    weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
     int32_t where[5] = {hh, hh, hh, -1, -1};  // the contact's location (trace only)
     int32_t eo[2], ec[2];
 #pragma unroll
@@ -892,8 +895,9 @@ __device__ __forceinline__ void mark_weekday(const Model& M, const AgentArrays& 
     const bool adult = A.age[idx] == kAgeAdult;
     const U4 ue = draw4(eoff + (uint64_t)(idx / 2), M.key0, M.key1);
     const int rs = 2 * (idx % 2);
+    const ErrandWalk wk = pinned(M.wd_walk);
     int32_t d1, d2;
-    weekday_dests(M, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
+    weekday_dests(M, wk, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
     uint32_t k0, k1;
     weekday_keys(M, d1, d2, k0, k1);
     const int prof = adult ? (int)((word(ue, rs) ^ word(ue, rs + 1)) % 3u) : 3;
@@ -909,8 +913,9 @@ __device__ __forceinline__ void mark_weekend(const Model& M, const AgentArrays& 
     if (!can_infect(M, f) && !A.trace_victim) return;  // as mark_weekday
     const U4 u = draw4(cbase + (uint64_t)(6 * pos), M.key0, M.key1);
     const int prof = (int)(u.w[3] % 6u);
+    const ErrandWalk wk = pinned(M.we_walk);
     int32_t hour[3], loc[3];
-    weekend_errands(M, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
+    weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int slot = M.we_assign[prof][k];

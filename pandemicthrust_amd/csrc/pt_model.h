@@ -27,8 +27,9 @@ enum ContactType : int { CT_NONE = 0, CT_WORKPLACE, CT_SCHOOL, CT_ERRAND, CT_AFT
 constexpr uint8_t kRecovered = 0, kSusceptible = 1, kInfected = 2;
 constexpr uint8_t kDayNone = 255, kGenNone = 255;
 
-// Model tables resident in device memory, one copy per simulation handle.
-struct Model {
+// Model tables of one simulation (also stored in checkpoints: the layout is
+// part of their format).
+struct ModelData {
     float hh_cdf[kHhRows];
     int32_t hh_adults[kHhRows];
     int32_t hh_children[kHhRows];
@@ -69,6 +70,23 @@ struct Model {
     uint64_t ikey0, ikey1;
 };
 
+// An errand walk (walk_errand_rows) prepared for evaluation without division
+// or loop: the rows kFirstErrandRow..kTypes-1 with a non-zero pdf, the pdfs
+// scaled by 2^32 so that the walk starts from (float)u itself.
+constexpr int kWalkRows = 4;
+struct ErrandWalk {
+    float pdf[kWalkRows];    // row pdf * 2^32
+    float rcp[kWalkRows];    // 1 / pdf, rounded to nearest
+    float count[kWalkRows];  // locations of the row
+    int32_t offset[kWalkRows];
+};
+
+// The model with its prepared walks: resident in device memory, one copy per
+// simulation.
+struct Model : ModelData {
+    ErrandWalk wd_walk, we_walk;
+};
+
 // ---------------- Threefry (Salmon et al., SC'11) ----------------
 __host__ __device__ __forceinline__ uint64_t rotl64(uint64_t x, unsigned n) {
     return (x << n) | (x >> (64 - n));
@@ -98,11 +116,23 @@ __device__ __forceinline__ uint64_t rotl64c(uint64_t x) {
     return ((uint64_t)__builtin_amdgcn_alignbit(a, b, s) << 32) | __builtin_amdgcn_alignbit(b, a, s);
 }
 
+// 64-bit add as a 32-bit add with carry out and one with carry in: the
+// v_lshl_add_u64 the compiler picks takes longer than the two (50M draws:
+// 243 us with it, 198 us with these).
+__device__ __forceinline__ uint64_t add64(uint64_t a, uint64_t b) {
+    uint32_t lo, hi;
+    asm("v_add_co_u32 %0, vcc, %2, %4\n\tv_addc_co_u32 %1, vcc, %3, %5, vcc"
+        : "=&v"(lo), "=v"(hi)
+        : "v"((uint32_t)a), "v"((uint32_t)(a >> 32)), "v"((uint32_t)b), "v"((uint32_t)(b >> 32))
+        : "vcc");
+    return ((uint64_t)hi << 32) | lo;
+}
+
 __device__ __forceinline__ U4 draw4(uint64_t c, uint64_t k0, uint64_t k1) {
     const uint64_t k2 = 0x1BD11BDAA9FC1A22ull ^ k0 ^ k1;
     uint64_t x0 = c + k0, x1 = c + k1;
-#define PT_R(n) x0 += x1; x1 = rotl64c<n>(x1); x1 ^= x0;
-#define PT_INJ(a, b, s) x0 += a; x1 += b + (uint64_t)(s);
+#define PT_R(n) x0 = add64(x0, x1); x1 = rotl64c<n>(x1); x1 ^= x0;
+#define PT_INJ(a, b, s) x0 = add64(x0, a); x1 = add64(x1, b + (uint64_t)(s));
     PT_R(16) PT_R(42) PT_R(12) PT_R(31) PT_INJ(k1, k2, 1)
     PT_R(16) PT_R(32) PT_R(24) PT_R(21) PT_INJ(k2, k0, 2)
     PT_R(16) PT_R(42) PT_R(12) PT_R(31) PT_INJ(k0, k1, 3)
@@ -193,71 +223,89 @@ __device__ __forceinline__ int32_t assign_workplace(const Model& M, uint32_t r, 
 }
 
 // ---------------- errand draws ----------------
-// The errand walks below run over rows kFirstErrandRow..kTypes-1 with every
-// step unrolled and predicated: each step subtracts the row's pdf only where
-// the reference's loop would continue, so the float operations and their
-// order are exactly the loop's, while the table reads are uniform (constant
-// row indices) instead of per-lane gathers inside a divergent loop.
-static_assert(kTypes - kFirstErrandRow == 5, "errand walks are unrolled over 5 rows");
+// The reference's errand walks go through the type rows from kFirstErrandRow,
+//     while (frac > pdf[row] && row < kTypes - 1) { frac -= pdf[row]; row++; }
+//     bn = (int)(frac / pdf[row] * count[row])   (at most count[row] - 1)
+// from frac = (float)u / 2^32.  Here the same floats are reached with 30
+// instructions instead of 41 (VALU bound: 50M agents' weekday keys 236 ->
+// 184 us, weekend keys 623 -> 511 us, with the adds of draw4):
+// - Everything is scaled by 2^32, a power of two, so no rounding changes.
+// - A row with pdf 0 is never where the walk stops (frac > 0 behind it), so
+//   it is left out; the 4 remaining rows are three compares and selects.  A
+//   remainder exceeds its row's pdf only if the rows before were passed, so
+//   the compares need no chaining.
+// - frac / pdf: with rcp = RN(1 / pdf), q0 = RN(frac rcp) is within one ulp of
+//   the quotient, its remainder is exact in one fma and q = RN(q0 + rem rcp)
+//   is the correctly rounded quotient (Markstein, 1990); no step over- or
+//   underflows here (2^0 <= frac <= 2^32, or frac = 0).
+// - The result is clamped below count as a float (counts here are below
+//   2^24, so exact): the largest float below count truncates to count - 1.
+static_assert(kTypes - kFirstErrandRow == 5, "errand rows");
+
+// The walk's constants in vector registers: the selects below cannot read
+// them from scalar ones (their condition already takes the one scalar operand
+// an instruction may have), and left to itself the compiler branches around
+// the loads.  Take it outside the loop over agents.
+__device__ __forceinline__ ErrandWalk pinned(const ErrandWalk& m) {
+    ErrandWalk k = m;
+#pragma unroll
+    for (int r = 0; r < kWalkRows; ++r)
+        asm volatile("" : "+v"(k.pdf[r]), "+v"(k.rcp[r]), "+v"(k.count[r]), "+v"(k.offset[r]));
+    return k;
+}
 
 struct RowPick {
-    float frac;   // the walk's remaining uniform
-    float pdf;    // pdf of the row it stopped at
-    int count;    // locations of that row
-    int offset;   // first location of that row
+    float frac, pdf, rcp, count;
+    int32_t offset;
 };
 
-// while (frac > pdf[row] && row < kTypes - 1) { frac -= pdf[row]; row++; }
-// from row kFirstErrandRow, over the pdf row table `pdf`.
-__device__ __forceinline__ RowPick walk_errand_rows(const Model& M, const float* pdf, float frac) {
-    RowPick r{frac, pdf[kFirstErrandRow], M.wp_count[kFirstErrandRow], M.wp_offset[kFirstErrandRow]};
-    bool go = true;
-#pragma unroll
-    for (int row = kFirstErrandRow; row < kTypes - 1; ++row) {
-        go = go && r.frac > pdf[row];
-        const float rest = r.frac - pdf[row];
-        r.frac = go ? rest : r.frac;
-        r.pdf = go ? pdf[row + 1] : r.pdf;
-        r.count = go ? M.wp_count[row + 1] : r.count;
-        r.offset = go ? M.wp_offset[row + 1] : r.offset;
-    }
-    return r;
+__device__ __forceinline__ RowPick walk_errand_rows(const ErrandWalk& k, uint32_t u) {
+    const float y = (float)u;
+    const float r1 = y - k.pdf[0], r2 = r1 - k.pdf[1], r3 = r2 - k.pdf[2];
+    const bool c1 = y > k.pdf[0], c2 = r1 > k.pdf[1], c3 = r2 > k.pdf[2];
+    auto sel = [&](auto a, auto b, auto c, auto d) {
+        a = c1 ? b : a;
+        a = c2 ? c : a;
+        return c3 ? d : a;
+    };
+    return RowPick{sel(y, r1, r2, r3), sel(k.pdf[0], k.pdf[1], k.pdf[2], k.pdf[3]),
+                   sel(k.rcp[0], k.rcp[1], k.rcp[2], k.rcp[3]), sel(k.count[0], k.count[1], k.count[2], k.count[3]),
+                   sel(k.offset[0], k.offset[1], k.offset[2], k.offset[3])};
 }
 
-// device_fishAfterschoolOrErrandDestination_weekday (PandemicSim.cu:2909-2947)
-// Every lane walks the rows and divides, and the child's after-school pick
-// is selected afterwards: a wave holds adults and children alike, so a
-// branch would run both sides anyway, plus its mask handling.
-__device__ __forceinline__ int32_t fish_weekday_dest(const Model& M, uint32_t r, bool adult) {
-    const float u = unit_float(r);
-    const RowPick p = walk_errand_rows(M, M.wd_pdf, u);
-    const float q = p.frac / p.pdf;
-    const float frac = adult ? q : u;
-    const int type_count = adult ? p.count : M.wp_count[kTypeAfterschool];
-    const int type_offset = adult ? p.offset : M.wp_offset[kTypeAfterschool];
-    uint32_t bn = (uint32_t)(frac * (float)type_count);
-    if (bn >= (uint32_t)type_count) bn = (uint32_t)(type_count - 1);
-    bn += (uint32_t)type_offset;
-    return (int32_t)bn;
+// (int)(q * count), at most count - 1.
+__device__ __forceinline__ int32_t location_in_row(float q, float count) {
+    // (min of the bits: both are >= 0, and fminf would first quiet NaNs)
+    return (int32_t)(uint32_t)__uint_as_float(min(__float_as_uint(q * count), __float_as_uint(count) - 1u));
 }
 
-// device_fishWeekendErrandDestination (PandemicSim.cu:1017-1044)
-__device__ __forceinline__ int32_t fish_weekend_dest(const Model& M, uint32_t r) {
-    const RowPick p = walk_errand_rows(M, M.we_pdf, unit_float(r));
-    const float frac = p.frac / p.pdf;
-    int bn = (int)(frac * (float)p.count);
-    if (bn >= p.count) bn = p.count - 1;
-    return bn + p.offset;
+__device__ __forceinline__ int32_t walk_location(const RowPick& p) {
+    const float q0 = p.frac * p.rcp;
+    const float q = __builtin_fmaf(__builtin_fmaf(-q0, p.pdf, p.frac), p.rcp, q0);
+    return location_in_row(q, p.count) + p.offset;
+}
+
+// An adult's weekday errand (device_fishAfterschoolOrErrandDestination_weekday,
+// PandemicSim.cu:2909-2947) or a weekend errand
+// (device_fishWeekendErrandDestination, :1017-1044); a child's weekday
+// destination is its after-school site.
+__device__ __forceinline__ int32_t fish_errand_dest(const ErrandWalk& k, uint32_t r) {
+    return walk_location(walk_errand_rows(k, r));
+}
+__device__ __forceinline__ int32_t fish_afterschool(const Model& M, uint32_t r) {
+    return location_in_row(unit_float(r), (float)M.wp_count[kTypeAfterschool]) + M.wp_offset[kTypeAfterschool];
 }
 
 // Weekday errand destinations of one person from its two draws
 // (device_assignAfterschoolOrErrandDests_weekday, PandemicSim.cu:2950-2969),
 // returned as locations (hour 1's W offset is not added).
-__device__ __forceinline__ void weekday_dests(const Model& M, uint32_t r1, uint32_t r2, bool adult, int32_t& d1,
-                                              int32_t& d2) {
-    d1 = fish_weekday_dest(M, r1, adult);
-    const int32_t e2 = fish_weekday_dest(M, r2, true);
-    d2 = adult ? e2 : d1;
+__device__ __forceinline__ void weekday_dests(const Model& M, const ErrandWalk& k, uint32_t r1, uint32_t r2,
+                                              bool adult, int32_t& d1, int32_t& d2) {
+    // A wave holds adults and children alike, so every lane does both and
+    // selects.
+    const int32_t e1 = fish_errand_dest(k, r1), e2 = fish_errand_dest(k, r2), a = fish_afterschool(M, r1);
+    d1 = adult ? e1 : a;
+    d2 = adult ? e2 : a;
 }
 
 // ---------------- interventions ----------------
@@ -323,25 +371,38 @@ __device__ __forceinline__ bool weekday_keys(const Model& M, int32_t d1, int32_t
     return ok;
 }
 
+// u % kWeHours without the quarter-rate 32-bit multiplies: 65536 = 6 (mod
+// 10), so u = 6 hi + lo (mod 10) < 458,746, whose quotient by 10 is exact in
+// single precision (t / 10 + 0.05 is at least 0.05 from a whole number, the
+// rounding errors are below 0.01).
+__device__ __forceinline__ int mod_hours(uint32_t u) {
+    static_assert(kWeHours == 10, "65536 = 6 (mod 10)");
+    const uint32_t hi = u >> 16, t = (hi << 2) + ((hi << 1) + (u & 0xFFFFu));
+    const uint32_t q = (uint32_t)__builtin_fmaf((float)t, 0.1f, 0.05f);
+    return (int)(t - ((q << 3) + (q << 1)));
+}
+__device__ __forceinline__ int next_hour(int h) { return h == kWeHours - 1 ? 0 : h + 1; }
+
 // device_generateWeekendErrands (PandemicSim.cu:980-1014): three distinct
 // hours and their destinations.
-__device__ __forceinline__ void weekend_errands(const Model& M, uint64_t off, int32_t hour[3], int32_t loc[3]) {
+__device__ __forceinline__ void weekend_errands(const Model& M, const ErrandWalk& k, uint64_t off, int32_t hour[3],
+                                                int32_t loc[3]) {
     const U4 a = draw4(off, M.key0, M.key1);
     const U4 b = draw4(off + 1, M.key0, M.key1);
-    const int h1 = (int)(a.w[0] % kWeHours);
-    int h2 = (int)(a.w[1] % kWeHours);
-    if (h2 == h1) h2 = (h2 + 1) % kWeHours;
-    int h3 = (int)(a.w[2] % kWeHours);
+    const int h1 = mod_hours(a.w[0]);
+    int h2 = mod_hours(a.w[1]);
+    h2 = h2 == h1 ? next_hour(h2) : h2;
+    int h3 = mod_hours(a.w[2]);
     // while (h3 == h1 || h3 == h2) h3 = (h3 + 1) % kWeHours, unrolled: two
     // forbidden hours end it within two steps.
-    h3 = (h3 == h1 || h3 == h2) ? (h3 + 1) % kWeHours : h3;
-    h3 = (h3 == h1 || h3 == h2) ? (h3 + 1) % kWeHours : h3;
+    h3 = ((h3 == h1) | (h3 == h2)) ? next_hour(h3) : h3;
+    h3 = ((h3 == h1) | (h3 == h2)) ? next_hour(h3) : h3;
     hour[0] = h1;
     hour[1] = h2;
     hour[2] = h3;
-    loc[0] = fish_weekend_dest(M, a.w[3]);
-    loc[1] = fish_weekend_dest(M, b.w[0]);
-    loc[2] = fish_weekend_dest(M, b.w[1]);
+    loc[0] = fish_errand_dest(k, a.w[3]);
+    loc[1] = fish_errand_dest(k, b.w[0]);
+    loc[2] = fish_errand_dest(k, b.w[1]);
 }
 
 // device_getWorkplaceMaxContacts (PandemicSim.cu:3492-3511)

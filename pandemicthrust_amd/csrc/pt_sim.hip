@@ -318,6 +318,7 @@ __global__ __launch_bounds__(256) void k_gen_weekday(const Model* __restrict__ M
     const Model& M = *Mp;
     const int N = M.N;
     const uint64_t off = st->errand_off;
+    const ErrandWalk wk = pinned(M.wd_walk);
     bool bad = false;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; 2 * g < N; g += stride) {
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(256) void k_gen_weekday(const Model* __restrict__ M
             if (p < N) {
                 const bool adult = age[p] == kAgeAdult;
                 int32_t d1, d2;
-                weekday_dests(M, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
+                weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
                 uint32_t k0, k1;
                 bad |= !weekday_keys(M, d1, d2, k0, k1);
                 keys[p] = k0;
@@ -348,11 +349,12 @@ __global__ __launch_bounds__(256) void k_gen_weekend(const Model* __restrict__ M
     const int N = M.N;
     const uint64_t off = st->errand_off;
     const int base = M.we_base, E = M.we_E;
+    const ErrandWalk wk = pinned(M.we_walk);
     bool bad = false;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < N; p += stride) {
         int32_t hour[3], loc[3];
-        weekend_errands(M, off + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
+        weekend_errands(M, wk, off + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
             int32_t l = loc[e] - base;
@@ -532,16 +534,17 @@ __global__ void k_errands_of(const Model* __restrict__ Mp, const DayState* __res
                              const uint8_t* __restrict__ age, int64_t N, int32_t* __restrict__ out) {
     const Model& M = *Mp;
     const uint64_t eoff = st->errand_off;
+    const ErrandWalk wk = pinned(weekend ? M.we_walk : M.wd_walk);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (int64_t)gridDim.x * blockDim.x) {
         if (weekend) {
             int32_t hour[3], loc[3];
-            weekend_errands(M, eoff + (uint64_t)(2 * i), hour, loc);
+            weekend_errands(M, wk, eoff + (uint64_t)(2 * i), hour, loc);
             for (int j = 0; j < 3; ++j) out[3 * i + j] = hour[j] * M.W + loc[j];
         } else {
             const U4 ue = draw4(eoff + (uint64_t)(i / 2), M.key0, M.key1);
             const int rs = 2 * (int)(i % 2);
             int32_t d1, d2;
-            weekday_dests(M, word(ue, rs), word(ue, rs + 1), age[i] == kAgeAdult, d1, d2);
+            weekday_dests(M, wk, word(ue, rs), word(ue, rs + 1), age[i] == kAgeAdult, d1, d2);
             out[i] = d1;
             out[N + i] = M.W + d2;
         }
@@ -595,6 +598,21 @@ void base_tables(Model& m) {
 }
 
 const int kBaseCounts[kTypes] = {1000, 7000, 2400, 300, 100, 200, 100, 100, 300, 500, 0, 300, 400, 100};
+
+// The rows of an errand walk with a non-zero pdf (ErrandWalk).
+ErrandWalk prepare_walk(const Model& m, const float* pdf) {
+    ErrandWalk w{};
+    int r = 0;
+    for (int t = kFirstErrandRow; t < kTypes; ++t) {
+        if (!(pdf[t] > 0.f) || r == kWalkRows) continue;
+        w.pdf[r] = pdf[t] * 4294967296.0f;
+        w.rcp[r] = 1.0f / w.pdf[r];
+        w.count[r] = (float)m.wp_count[t];
+        w.offset[r] = m.wp_offset[t];
+        ++r;
+    }
+    return w;
+}
 
 int round_half_up(double d) { return (int)floor(d + 0.5); }  // roundHalfUp_toInt, PandemicSim.cu:1662
 
@@ -697,6 +715,8 @@ int build_model(const pt_params* p, const int32_t seed_key[2], Model& m) {
         m.wp_offset[t] = acc;
         acc += m.wp_count[t];
     }
+    m.wd_walk = prepare_walk(m, m.wd_pdf);
+    m.we_walk = prepare_walk(m, m.we_pdf);
     // setup_calculateInfectionData (PandemicSim.cu:2828-2840)
     for (int i = 3; i < 6; ++i)
         for (int j = 0; j < 10; ++j) m.shed[i][j] = m.shed[i][j] * p->asymp_factor;
@@ -1553,7 +1573,7 @@ int pt_sim_restore(pt_sim* s) {
 //
 // Buffer layout (host byte order, little-endian on every supported host):
 //   CkptHeader
-//   Model          the handle's model after setup (scales, tables, seed
+//   ModelData      the handle's model after setup (scales, tables, seed
 //                  key, interventions, N): a checkpoint loads only into a
 //                  handle built from the same inputs
 //   DayState       the loop's device counters at a day boundary
@@ -1578,7 +1598,7 @@ constexpr uint32_t kCkptVersion = 1;
 constexpr int kCkptRows = 256;
 constexpr int64_t kCkptLogBytes = (int64_t)kCkptRows * (16 + 1 + 1 + 1) * 4;
 
-int64_t ckpt_fixed_bytes() { return (int64_t)sizeof(CkptHeader) + sizeof(Model) + sizeof(DayState) + kCkptLogBytes; }
+int64_t ckpt_fixed_bytes() { return (int64_t)sizeof(CkptHeader) + sizeof(ModelData) + sizeof(DayState) + kCkptLogBytes; }
 
 // FNV-1a over 64-bit words (then the tail bytes).
 uint64_t ckpt_hash(const uint8_t* p, int64_t n) {
@@ -1612,13 +1632,13 @@ int pt_sim_checkpoint_save(pt_sim* s, void* buf, int64_t bytes) {
     CkptHeader hd{};
     memcpy(hd.magic, kCkptMagic, 8);
     hd.version = kCkptVersion;
-    hd.model_bytes = sizeof(Model);
+    hd.model_bytes = sizeof(ModelData);
     hd.state_bytes = sizeof(DayState);
     hd.rows_capacity = kCkptRows;
     hd.n_people = s->N;
     uint8_t* p = out + sizeof hd;
-    memcpy(p, &s->model, sizeof(Model));
-    p += sizeof(Model);
+    memcpy(p, static_cast<const ModelData*>(&s->model), sizeof(ModelData));
+    p += sizeof(ModelData);
     HIP_TRY(hipMemcpy(p, s->d_state, sizeof(DayState), hipMemcpyDeviceToHost));
     p += sizeof(DayState);
     HIP_TRY(hipMemcpy(p, s->d_counts, 4 * kCkptRows * 16, hipMemcpyDeviceToHost));
@@ -1647,7 +1667,7 @@ int pt_sim_checkpoint_load(pt_sim* s, const void* buf, int64_t bytes) {
     CkptHeader hd;
     memcpy(&hd, in, sizeof hd);
     if (memcmp(hd.magic, kCkptMagic, 8) != 0) return fail(PT_EINVAL, "not a checkpoint (bad magic)");
-    if (hd.version != kCkptVersion || hd.model_bytes != sizeof(Model) || hd.state_bytes != sizeof(DayState) ||
+    if (hd.version != kCkptVersion || hd.model_bytes != sizeof(ModelData) || hd.state_bytes != sizeof(DayState) ||
         hd.rows_capacity != (uint32_t)kCkptRows)
         return fail(PT_EINVAL, "checkpoint written by an incompatible library version");
     if (hd.n_people != s->N)
@@ -1659,9 +1679,9 @@ int pt_sim_checkpoint_load(pt_sim* s, const void* buf, int64_t bytes) {
     if (ckpt_hash(in + sizeof hd, need - (int64_t)sizeof hd) != hd.checksum)
         return fail(PT_EINVAL, "checkpoint checksum mismatch (corrupt file)");
     const uint8_t* p = in + sizeof hd;
-    if (memcmp(p, &s->model, sizeof(Model)) != 0)
+    if (memcmp(p, static_cast<const ModelData*>(&s->model), sizeof(ModelData)) != 0)
         return fail(PT_EINVAL, "checkpoint was written for other constants, seed or interventions");
-    p += sizeof(Model);
+    p += sizeof(ModelData);
     DayState st;
     memcpy(&st, p, sizeof st);
     p += sizeof(DayState);
