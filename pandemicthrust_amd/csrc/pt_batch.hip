@@ -90,12 +90,7 @@ __device__ __forceinline__ AgentArrays view(const BatchArrays& B, const RepInfo&
     A.gn_s = B.gn_s + ri.abase;
     A.claim_p = B.claim_p + ri.abase;
     A.claim_s = B.claim_s + ri.abase;
-    A.trace_victim = nullptr;
-    A.trace_type = nullptr;
-    A.trace_loc = nullptr;
-    A.trace_attempt = nullptr;
-    A.trace_draw = nullptr;
-    A.trace_prof = nullptr;
+    A.clear_trace();
     return A;
 }
 
@@ -467,30 +462,38 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts(DayState* __restr
     if (g->done) return;
     const int64_t I = g->n_infected;
     const int lane = threadIdx.x & 63;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x; b0 < I; b0 += stride) {
-        const int64_t pos = b0 + threadIdx.x;
-        int32_t vic[8];
-        int typ[8];
-        bool newp[8], news[8];
-        clear_contacts(vic, typ, newp, news);
-        int32_t bias = 0;
-        if (pos < I) {
+    filtered_contacts<kContactThreads>(
+        I,
+        [&](int64_t pos, QueuedInfector& q) {
             const int r = rep_of(inf_start, R, pos);
             const DayState& st = sts[r];
             const RepInfo ri = reps[r];
             const AgentArrays A = view(B, ri, WEEKEND ? ri.kb_we : ri.kb_wd);
-            const int32_t idx = infected[pos] - (int32_t)ri.abase;
-            const int64_t lpos = pos - inf_start[r];
-            bias = (int32_t)ri.abase;
-            if (WEEKEND)
-                weekend_contacts(models[r], A, st.day, st.contact_base, st.errand_off, idx, lpos, vic, typ, newp, news);
-            else
-                weekday_contacts(models[r], A, st.day, st.contact_base, st.errand_off, ri.workplace_off, idx, lpos, vic,
-                                 typ, newp, news);
-        }
-        append_claims(g->n_claimed, list_p, list_s, bias, vic, newp, news, lane);
-    }
+            q = QueuedInfector{infected[pos] - (int32_t)ri.abase, (int32_t)(pos - inf_start[r]), r};
+            const Infectivity f = infectivity(models[r], A, q.idx, st.day);
+            return can_infect(models[r], f) &&
+                   may_infect<WEEKEND ? 5 : 8>(models[r], f, st.contact_base + (uint64_t)(6 * (int64_t)q.pos) + 2);
+        },
+        [&](bool active, const QueuedInfector& q) {
+            int32_t vic[8];
+            int typ[8];
+            bool newp[8], news[8];
+            clear_contacts(vic, typ, newp, news);
+            int32_t bias = 0;
+            if (active) {
+                const DayState& st = sts[q.r];
+                const RepInfo ri = reps[q.r];
+                const AgentArrays A = view(B, ri, WEEKEND ? ri.kb_we : ri.kb_wd);
+                bias = (int32_t)ri.abase;
+                if (WEEKEND)
+                    weekend_contacts(models[q.r], A, st.day, st.contact_base, st.errand_off, q.idx, q.pos, vic, typ,
+                                     newp, news);
+                else
+                    weekday_contacts(models[q.r], A, st.day, st.contact_base, st.errand_off, ri.workplace_off, q.idx,
+                                     q.pos, vic, typ, newp, news);
+            }
+            append_claims(g->n_claimed, list_p, list_s, bias, vic, newp, news, lane);
+        });
 }
 
 __global__ void kb_end_day(DayState* __restrict__ g, DayState* __restrict__ sts, int R) {

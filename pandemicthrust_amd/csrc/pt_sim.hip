@@ -448,7 +448,8 @@ __global__ __launch_bounds__(256) void k_mark_weekend(const Model* __restrict__ 
 
 // D6w/D6e + D7 over the day's infected list (weekday_contacts,
 // weekend_contacts); claims go to the per-strain claim lists.
-template <bool WEEKEND>
+// TRACE: every infector's contacts are made and recorded (A's trace arrays).
+template <bool WEEKEND, bool TRACE>
 __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __restrict__ Mp, DayState* __restrict__ st,
                                                               const int32_t* __restrict__ infected, AgentArrays A,
                                                               int32_t* __restrict__ list_p,
@@ -460,20 +461,35 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
     const uint64_t cbase = st->contact_base;
     const uint64_t eoff = st->errand_off;
     const int lane = threadIdx.x & 63;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x; b0 < I; b0 += stride) {
-        const int64_t pos = b0 + threadIdx.x;
+    if constexpr (!TRACE) A.clear_trace();  // known to the compiler
+    auto run = [&](bool active, const QueuedInfector& q) {
         int32_t vic[8];
         int typ[8];
         bool newp[8], news[8];
         clear_contacts(vic, typ, newp, news);
-        if (pos < I) {
+        if (active) {
             if (WEEKEND)
-                weekend_contacts(M, A, day, cbase, eoff, infected[pos], pos, vic, typ, newp, news);
+                weekend_contacts(M, A, day, cbase, eoff, q.idx, q.pos, vic, typ, newp, news);
             else
-                weekday_contacts(M, A, day, cbase, eoff, workplace_off, infected[pos], pos, vic, typ, newp, news);
+                weekday_contacts(M, A, day, cbase, eoff, workplace_off, q.idx, q.pos, vic, typ, newp, news);
         }
         append_claims(st->n_claimed, list_p, list_s, 0, vic, newp, news, lane);
+    };
+    if constexpr (TRACE) {
+        const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+        for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x; b0 < I; b0 += stride) {
+            const int64_t pos = b0 + threadIdx.x;
+            run(pos < I, QueuedInfector{pos < I ? infected[pos] : 0, (int32_t)pos, 0});
+        }
+    } else {
+        filtered_contacts<kContactThreads>(
+            I,
+            [&](int64_t pos, QueuedInfector& q) {
+                q = QueuedInfector{infected[pos], (int32_t)pos, 0};
+                const Infectivity f = infectivity(M, A, q.idx, day);
+                return can_infect(M, f) && may_infect<WEEKEND ? 5 : 8>(M, f, cbase + (uint64_t)(6 * pos) + 2);
+            },
+            run);
     }
 }
 
@@ -1037,10 +1053,10 @@ int enqueue_day(pt_sim* s, int d) {
                     weekend ? kNoDrop : (uint32_t)(K - 1), &sel);
     if (e != hipSuccess) return fail(PT_EDEVICE, "table build: %s", hipGetErrorString(e));
     if (weekend)
-        launch(tm, KC_CONTACTS_WEEKEND, k_contacts<true>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
+        launch(tm, KC_CONTACTS_WEEKEND, s->trace_on ? k_contacts<true, true> : k_contacts<true, false>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
                infected, A, s->list_p, s->list_s, s->workplace_off);
     else
-        launch(tm, KC_CONTACTS_WEEKDAY, k_contacts<false>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
+        launch(tm, KC_CONTACTS_WEEKDAY, s->trace_on ? k_contacts<false, true> : k_contacts<false, false>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
                infected, A, s->list_p, s->list_s, s->workplace_off);
     if (s->trace_on)
         k_trace_actions<<<s->grid_contacts, 256, 0, stc>>>((const DayState*)st, weekend ? 5 : 8,
