@@ -146,15 +146,18 @@ int pt_sim_get_scalars(pt_sim* sim, int64_t out[8]);
  * The PT_ERRAND_* hooks always return the reference's layout. */
 int pt_sim_get_layout(pt_sim* sim, int64_t out[8]);
 
-/* Errand-table strategy: 0 automatic (default), 1 build every bucket each
- * day, 2 build only the buckets that day's infectors draw contacts from.
- * Simulation results are identical in all modes; the PT_ERRAND_* parity
- * hooks show complete tables only in mode 1. */
+/* Errand-table strategy: 0 automatic (default), 1 sort every bucket each
+ * day, 2 sort only the buckets that day's infectors draw contacts from.
+ * Automatic counts the buckets without sorting them where the layout allows,
+ * and otherwise sorts either all of them or the queried ones.  Simulation
+ * results are identical in all modes; the PT_ERRAND_* parity hooks show
+ * complete tables in mode 1 and after counted days (built when asked for). */
 int pt_sim_set_table_mode(pt_sim* sim, int32_t mode);
 
 /* Measurement hook: the errand table of each day run since setup / restore.
- * full_out[d] = 1 if day d built every bucket, 0 if only the queried ones;
- * pairs_out[d] = pairs sorted that day.  Fills min(len, days run) entries
+ * full_out[d] = 1 if day d sorted or counted every bucket, 0 if only the
+ * queried ones; pairs_out[d] = pairs sorted that day (counted days: the
+ * E * N pairs that a sort would have taken).  Fills min(len, days run) entries
  * and returns their number (either pointer may be NULL). */
 int pt_sim_table_log(pt_sim* sim, int32_t* full_out, int32_t* pairs_out, int32_t len);
 

@@ -66,6 +66,7 @@ struct BatchArrays {
     const int32_t* hh_off;
     const int32_t* wp_off;
     const int32_t* wp_people;
+    const uint32_t* wp_of;
     const int32_t* er_off;
     const int32_t* er_people;
     const uint8_t *st_p, *st_s, *dy_p, *dy_s, *gn_p, *gn_s;
@@ -82,6 +83,10 @@ __device__ __forceinline__ AgentArrays view(const BatchArrays& B, const RepInfo&
     A.wp_people = B.wp_people + ri.abase;
     A.er_off = B.er_off + kb;
     A.er_people = B.er_people;
+    A.wp_of = B.wp_of + ri.abase;
+    A.er_cnt = nullptr;
+    A.er_keys = nullptr;
+    A.er_slots = 0;
     A.st_p = B.st_p + ri.abase;
     A.st_s = B.st_s + ri.abase;
     A.dy_p = B.dy_p + ri.abase;
@@ -462,19 +467,20 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts(DayState* __restr
     if (g->done) return;
     const int64_t I = g->n_infected;
     const int lane = threadIdx.x & 63;
-    filtered_contacts<kContactThreads>(
+    constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
+    filtered_contacts<kContactThreads, C>(
         I,
-        [&](int64_t pos, QueuedInfector& q) {
+        [&](int64_t pos, QueuedInfector& q, SuccessDraws& draws) {
             const int r = rep_of(inf_start, R, pos);
             const DayState& st = sts[r];
             const RepInfo ri = reps[r];
             const AgentArrays A = view(B, ri, WEEKEND ? ri.kb_we : ri.kb_wd);
             q = QueuedInfector{infected[pos] - (int32_t)ri.abase, (int32_t)(pos - inf_start[r]), r};
+            success_draws<C>(models[r], st.contact_base + (uint64_t)(6 * (int64_t)q.pos) + 2, draws);
             const Infectivity f = infectivity(models[r], A, q.idx, st.day);
-            return can_infect(models[r], f) &&
-                   may_infect<WEEKEND ? 5 : 8>(models[r], f, st.contact_base + (uint64_t)(6 * (int64_t)q.pos) + 2);
+            return can_infect(models[r], f) && may_infect<C>(models[r], f, draws);
         },
-        [&](bool active, const QueuedInfector& q) {
+        [&](bool active, const QueuedInfector& q, const SuccessDraws& draws) {
             int32_t vic[8];
             int typ[8];
             bool newp[8], news[8];
@@ -485,12 +491,13 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts(DayState* __restr
                 const RepInfo ri = reps[q.r];
                 const AgentArrays A = view(B, ri, WEEKEND ? ri.kb_we : ri.kb_wd);
                 bias = (int32_t)ri.abase;
+                const Infectivity f = infectivity(models[q.r], A, q.idx, st.day);
                 if (WEEKEND)
-                    weekend_contacts(models[q.r], A, st.day, st.contact_base, st.errand_off, q.idx, q.pos, vic, typ,
-                                     newp, news);
+                    weekend_contacts(models[q.r], A, true, f, st.day, st.contact_base, st.errand_off, q.idx, q.pos, vic, typ,
+                                     newp, news, draws, NoQueue{});
                 else
-                    weekday_contacts(models[q.r], A, st.day, st.contact_base, st.errand_off, ri.workplace_off, q.idx,
-                                     q.pos, vic, typ, newp, news);
+                    weekday_contacts(models[q.r], A, true, f, st.day, st.contact_base, st.errand_off, q.idx,
+                                     q.pos, vic, typ, newp, news, draws, NoQueue{});
             }
             append_claims(g->n_claimed, list_p, list_s, bias, vic, newp, news, lane);
         });
@@ -541,6 +548,7 @@ struct pt_batch {
     uint8_t *st_p = nullptr, *st_s = nullptr, *dy_p = nullptr, *dy_s = nullptr, *gn_p = nullptr, *gn_s = nullptr;
     uint8_t *age = nullptr, *hh_types = nullptr, *snap = nullptr;
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
+    uint32_t* wp_of = nullptr;
     uint64_t *claim_p = nullptr, *claim_s = nullptr;
     int32_t *list_p = nullptr, *list_s = nullptr, *infected = nullptr, *staging = nullptr;
     uint32_t *blk_counts = nullptr, *blk_ninf = nullptr, *blk_off = nullptr;
@@ -596,6 +604,7 @@ void free_batch_population(pt_batch* b) {
     dev_free(b->hh_off);
     dev_free(b->wp_off);
     dev_free(b->wp_people);
+    dev_free(b->wp_of);
     dev_free(b->claim_p);
     dev_free(b->claim_s);
     dev_free(b->list_p);
@@ -656,6 +665,7 @@ BatchArrays batch_arrays(pt_batch* b) {
     B.hh_off = b->hh_off;
     B.wp_off = b->wp_off;
     B.wp_people = b->wp_people;
+    B.wp_of = b->wp_of;
     B.er_off = b->er_off;
     B.er_people = b->er_people;
     B.st_p = b->st_p;
@@ -923,7 +933,7 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
     if (dev_alloc(&b->tile_rep, tiles) || dev_alloc(&b->st_p, P) || dev_alloc(&b->st_s, P) ||
         dev_alloc(&b->dy_p, P) || dev_alloc(&b->dy_s, P) || dev_alloc(&b->gn_p, P) || dev_alloc(&b->gn_s, P) ||
         dev_alloc(&b->age, P) || dev_alloc(&b->snap, 6 * P) || dev_alloc(&b->household, P) ||
-        dev_alloc(&b->hh_off, HH) || dev_alloc(&b->wp_off, WW) || dev_alloc(&b->wp_people, P) ||
+        dev_alloc(&b->hh_off, HH) || dev_alloc(&b->wp_off, WW) || dev_alloc(&b->wp_people, P) || dev_alloc(&b->wp_of, P) ||
         dev_alloc(&b->claim_p, P) || dev_alloc(&b->claim_s, P) || dev_alloc(&b->list_p, P) ||
         dev_alloc(&b->list_s, P) || dev_alloc(&b->infected, P) || dev_alloc(&b->staging, P) ||
         dev_alloc(&b->blk_counts, (int64_t)tiles * 16) || dev_alloc(&b->blk_ninf, tiles) ||
@@ -1006,7 +1016,7 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
         const RepInfo& ri = b->reps[r];
         const int64_t a = ri.abase;
         const PopArrays Pa{b->hh_types + ri.hbase, b->hh_off + ri.hbase, b->household + a, b->age + a,
-                           b->wp_off + ri.wbase, b->wp_people + a, b->st_p + a, b->st_s + a, b->dy_p + a, b->dy_s + a,
+                           b->wp_off + ri.wbase, b->wp_people + a, b->wp_of + a, b->st_p + a, b->st_s + a, b->dy_p + a, b->dy_s + a,
                            b->gn_p + a, b->gn_s + a, b->claim_p + a, b->claim_s + a};
         hipError_t e = build_population(b->d_models + r, ri.N, ri.H, ri.W, Pa, b->sel_keys, b->tables,
                                         ri.workplace_off, st);

@@ -82,6 +82,10 @@ int build_model(const pt_params* p, const int32_t seed_key[2], Model& m);
 // PT_EINVAL).
 int apply_interventions(const pt_interventions* iv, Model& m);
 
+// Locations number below 2^28 (location_scaling <= 1e4); 0..3 contacts a day.
+constexpr int kWorkplaceBits = 28;
+constexpr uint32_t kWorkplaceMask = (1u << kWorkplaceBits) - 1u;
+
 // Population arrays of one simulation (local numbering).
 struct PopArrays {
     uint8_t* hh_types;   // H + 1
@@ -90,6 +94,7 @@ struct PopArrays {
     uint8_t* age;        // N
     int32_t* wp_off;     // W + 1
     int32_t* wp_people;  // N
+    uint32_t* wp_of;     // N, workplace or school | its contacts per day << kWorkplaceBits
     uint8_t *st_p, *st_s, *dy_p, *dy_s, *gn_p, *gn_s;  // N
     uint64_t *claim_p, *claim_s;                        // N
 };
@@ -200,17 +205,6 @@ __device__ __forceinline__ void wave_sum_bins8(uint64_t v, uint32_t (&out)[8]) {
     out[6] = w[2] >> 16;
     out[5] = w[3] & 0xFFFFu;
     out[7] = w[3] >> 16;
-}
-
-// All 64 lanes must call: reserves n_mine slots per lane in a list whose
-// length lives at *counter; returns the lane's first slot.
-__device__ __forceinline__ uint32_t wave_append(uint32_t* counter, uint32_t n_mine, int lane) {
-    const uint32_t inc = wave_incl_scan(n_mine, lane);
-    const uint32_t total = __shfl(inc, 63, 64);
-    uint32_t base = 0;
-    if (lane == 0 && total) base = atomicAdd(counter, total);
-    base = __shfl(base, 0, 64);
-    return base + inc - n_mine;
 }
 
 // ---------------- D1 + D2: sweep ----------------
@@ -502,6 +496,7 @@ __device__ __forceinline__ int select_person(int32_t infector, int32_t loc_off, 
 // gathering one from a location table for every slot: the contact types and
 // kval_sum depend on the location counts alone (select_person), and the
 // victims of unsuccessful slots are never read.
+// With counted tables e0off and e1off hold the errand buckets.
 struct SlotPlan {
     int32_t hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt;
     int wpd, h0, h1;
@@ -544,8 +539,14 @@ struct AgentArrays {
     const int32_t* hh_off;
     const int32_t* wp_off;
     const int32_t* wp_people;
+    const uint32_t* wp_of;
     const int32_t* er_off;
     const int32_t* er_people;
+    // Counted tables (er_off, er_people unused): people per bucket, and the
+    // agents' keys of the day, er_slots apart per errand.
+    const uint32_t* er_cnt;
+    const uint16_t* er_keys;
+    int64_t er_slots;
     const uint8_t* st_p;
     const uint8_t* st_s;
     const uint8_t* dy_p;
@@ -615,12 +616,39 @@ __device__ __forceinline__ Infectivity infectivity(const Model& M, const AgentAr
     return f;
 }
 
+// The same in 30 bits.
+__device__ __forceinline__ uint32_t pack_infectivity(const Infectivity& f) {
+    return (uint32_t)(f.prof_p + 1) | ((uint32_t)f.dd_p << 3) | ((uint32_t)(f.prof_s + 1) << 7) |
+           ((uint32_t)f.dd_s << 10) | ((uint32_t)f.gen_p << 14) | ((uint32_t)f.gen_s << 22);
+}
+__device__ __forceinline__ Infectivity unpack_infectivity(uint32_t w) {
+    return Infectivity{(int)(w & 7u) - 1, (int)((w >> 3) & 15u), (int)((w >> 7) & 7u) - 1, (int)((w >> 10) & 15u),
+                       (uint8_t)(w >> 14), (uint8_t)(w >> 22)};
+}
+
 // Whether the infector can infect at all today: with alpha*factor <= 0 every
 // draw y >= 0 fails y < p*kval, so contacts need not be generated.
 __device__ __forceinline__ bool can_infect(const Model& M, const Infectivity& f) {
     const bool p = f.prof_p >= 0 && M.shed[f.prof_p][f.dd_p] * M.factor[0] > 0.f;
     const bool s = f.prof_s >= 0 && M.shed[f.prof_s][f.dd_s] * M.factor[1] > 0.f;
     return p || s;
+}
+
+// The words of an infector's success draws (4 counters; the 5 weekend slots
+// reach 11 words of them): slot c uses words 2c (pandemic) and 2c + 1
+// (seasonal).
+struct SuccessDraws {
+    uint32_t u[16];
+};
+template <int C>
+__device__ __forceinline__ void success_draws(const Model& M, uint64_t M2, SuccessDraws& d) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        U4 w{};
+        if (q < (C + 1) / 2) w = draw4(M2 + (uint64_t)q, M.key0, M.key1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d.u[4 * q + j] = w.w[j];
+    }
 }
 
 // Per-contact draws and claims (device_processContacts PandemicSim.cu:3177-3231).
@@ -632,17 +660,11 @@ __device__ __forceinline__ bool can_infect(const Model& M, const Infectivity& f)
 template <int C>
 __device__ __forceinline__ void process_contacts(const Model& M, const AgentArrays& A, const Infectivity& f, int kval_sum,
                                                  int32_t (&vic)[8], const int (&typ)[8], const SlotPlan& P,
-                                                 bool resolved, int32_t idx, uint64_t M2, uint32_t pos,
+                                                 bool resolved, int32_t idx, const SuccessDraws& draws, uint32_t pos,
                                                  bool (&newp)[8], bool (&news)[8]) {
     const float prob_p = f.prof_p >= 0 ? infection_probability(M, f.prof_p, f.dd_p, 0, kval_sum) : -1.f;
     const float prob_s = f.prof_s >= 0 ? infection_probability(M, f.prof_s, f.dd_s, 1, kval_sum) : -1.f;
-    uint32_t u[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const U4 w = draw4(M2 + (uint64_t)q, M.key0, M.key1);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) u[4 * q + j] = w.w[j];
-    }
+    const uint32_t(&u)[16] = draws.u;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const float kv = typ[c] == CT_NONE ? 0.f : 1.f;
@@ -682,20 +704,37 @@ __device__ __forceinline__ void process_contacts(const Model& M, const AgentArra
     }
 }
 
-// Appends the victims this lane posted first to the claim lists (as
-// id_bias + victim).  All 64 lanes must call.
+// Appends the victims each thread posted first to the claim lists (as
+// id_bias + victim).  All threads of the block must call.  One atomic per
+// block and strain: atomics on one address pass at about 2 ns each, so one
+// per wave took longer than the contacts themselves.
 __device__ __forceinline__ void append_claims(uint32_t* n_claimed, int32_t* __restrict__ list_p,
                                               int32_t* __restrict__ list_s, int32_t id_bias,
                                               const int32_t (&vic)[8], const bool (&newp)[8], const bool (&news)[8],
                                               int lane) {
-    uint32_t np = 0, ns = 0;
+    __shared__ uint32_t s_cnt[2], s_base[2];
+    uint32_t n[2] = {0, 0};
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        np += newp[c];
-        ns += news[c];
+        n[0] += newp[c];
+        n[1] += news[c];
     }
-    uint32_t ip = wave_append(&n_claimed[0], np, lane);
-    uint32_t is = wave_append(&n_claimed[1], ns, lane);
+    if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t at[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t inc = wave_incl_scan(n[k], lane);
+        const uint32_t total = __shfl(inc, 63, 64);
+        uint32_t base = 0;
+        if (lane == 0 && total) base = atomicAdd(&s_cnt[k], total);
+        at[k] = __shfl(base, 0, 64) + inc - n[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 && s_cnt[threadIdx.x])
+        s_base[threadIdx.x] = atomicAdd(&n_claimed[threadIdx.x], s_cnt[threadIdx.x]);
+    __syncthreads();
+    uint32_t ip = s_base[0] + at[0], is = s_base[1] + at[1];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         if (newp[c]) list_p[ip++] = id_bias + vic[c];
@@ -712,166 +751,244 @@ __device__ __forceinline__ void clear_contacts(int32_t (&vic)[8], int (&typ)[8],
     }
 }
 
+// The same with a queue (counted tables): successful slots are queued, two
+// slots per round, and claimed together by the block (PickPush), so a wave
+// does not go through the look-up chain of every slot in which one of its
+// lanes succeeds.  All threads of the block must call, the idle ones with
+// active false.
+template <int C, class Queue>
+__device__ __forceinline__ void queue_contacts(const Model& M, bool active, const Infectivity& f, int kval_sum,
+                                               const int (&typ)[8], const SlotPlan& P, int32_t idx,
+                                               const SuccessDraws& draws, uint32_t pos, const Queue& queue) {
+    float prob_p = -1.f, prob_s = -1.f;
+    if (active && f.prof_p >= 0) prob_p = infection_probability(M, f.prof_p, f.dd_p, 0, kval_sum);
+    if (active && f.prof_s >= 0) prob_s = infection_probability(M, f.prof_s, f.dd_s, 1, kval_sum);
+    const uint32_t(&u)[16] = draws.u;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const float kv = typ[c] == CT_NONE ? 0.f : 1.f;
+        const bool draw_p = unit_float(u[2 * c]) < prob_p * kv;
+        const bool draw_s = unit_float(u[2 * c + 1]) < prob_s * kv;
+        if (active && (draw_p || draw_s)) {  // kv = 1: a real contact, count > 1
+            const uint32_t prof_p = infection_profile(M, u[2 * c] ^ u[(2 * c + 1) % 16]);
+            const uint32_t prof_s = infection_profile(M, u[2 * c + 1] ^ u[(2 * c + 2) % 16]);
+            const bool home = c < 3, work = !home && c < 3 + P.wpd, first = c < 3 + P.wpd + P.h0;
+            const int32_t off = home ? P.hoff : (work ? P.woff : (first ? P.e0off : P.e1off));
+            const int32_t cnt = home ? P.hcnt : (work ? P.wcnt : (first ? P.e0cnt : P.e1cnt));
+            queue.push(off, (uint32_t)cnt, P.r[c] % (uint32_t)cnt, home ? 1u : (work ? 2u : 0u), idx,
+                       pos * 8u + (uint32_t)c,
+                       f.gen_p | ((uint32_t)f.gen_s << 8) | (prof_p << 16) | (prof_s << 20) |
+                           ((draw_p ? 1u : 0u) << 24) | ((draw_s ? 1u : 0u) << 25));
+        }
+        if (c % 2 == 1 || c == C - 1) queue.round(c == C - 1);
+    }
+}
+
+// No queue: errand victims come from the sorted table.
+struct NoQueue {
+    static constexpr bool counted = false;
+};
+
+// People and table position (counted tables: the bucket) of an errand bucket.
+template <bool COUNTED>
+__device__ __forceinline__ void errand_bucket(const AgentArrays& A, uint32_t key, int32_t& off, int32_t& cnt) {
+    if (COUNTED) {
+        off = (int32_t)key;
+        cnt = (int32_t)A.er_cnt[key];
+    } else {
+        off = A.er_off[key];
+        cnt = A.er_off[key + 1] - off;
+    }
+}
+
 // D6w + D7: one infector of kernel_doWeekday (PandemicSim.cu:3236-3308) with
 // device_makeContacts_weekday (:1669-1829).  idx: the infector; pos: its
 // position in the day's infected list; cbase, eoff: the day's contact and
 // errand counters.
-__device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArrays& A, int day, uint64_t cbase,
-                                                 uint64_t eoff, uint64_t workplace_off, int32_t idx, int64_t pos,
+// With a queue every thread of the block calls, the idle ones with active
+// false.
+template <class Queue>
+__device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArrays& A, bool active,
+                                                 const Infectivity& f, int day, uint64_t cbase,
+                                                 uint64_t eoff, int32_t idx, int64_t pos,
                                                  int32_t (&vic)[8], int (&typ)[8], bool (&newp)[8],
-                                                 bool (&news)[8]) {
-    const Infectivity f = infectivity(M, A, idx, day);
-    if (!can_infect(M, f) && !A.trace_victim) return;
-    const uint64_t Mc = cbase + (uint64_t)(6 * pos);
-    const U4 ua = draw4(Mc, M.key0, M.key1);
-    const U4 ub = draw4(Mc + 1, M.key0, M.key1);
-    const uint32_t u[8] = {ua.w[0], ua.w[1], ua.w[2], ua.w[3], ub.w[0], ub.w[1], ub.w[2], ub.w[3]};
-    const uint8_t myage = A.age[idx];
-    const bool adult = myage == kAgeAdult;
-    // household
-    const int32_t hh = A.household[idx];
-    const int32_t hoff = A.hh_off[hh];
-    const int32_t hcnt = A.hh_off[hh + 1] - hoff;
-    // workplace (device_recalcWorkplace PandemicSim.cu:3872-3890)
-    const U4 uw = draw4(workplace_off + (uint64_t)(idx / 4), M.key0, M.key1);
-    uint8_t a2 = myage;
-    const int32_t wp = assign_workplace(M, word(uw, idx % 4), &a2);
-    const int32_t woff = A.wp_off[wp];
-    const int32_t wcnt = A.wp_off[wp + 1] - woff;
-    const int wpd = workplace_max_contacts(M, wp);
-    // errands (device_recalc_weekdayErrandDests_assignProfile :3667-3705)
-    const U4 ue = draw4(eoff + (uint64_t)(idx / 2), M.key0, M.key1);
-    const int rs = 2 * (idx % 2);
-    const ErrandWalk wk = pinned(M.wd_walk);
-    int32_t d1, d2;
-    weekday_dests(M, wk, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
-    const int prof = adult ? (int)((word(ue, rs) ^ word(ue, rs + 1)) % 3u) : 3;
-    const int h0 = M.wd_assign[prof][0], h1 = M.wd_assign[prof][1];
-    uint32_t k0, k1;
-    weekday_keys(M, d1, d2, k0, k1);
-    const int32_t e0off = A.er_off[k0], e0cnt = A.er_off[k0 + 1] - e0off;
-    const int32_t e1off = A.er_off[k1], e1cnt = A.er_off[k1 + 1] - e1off;
-    const int wtype = adult ? CT_WORKPLACE : CT_SCHOOL;
-    const int etype = adult ? CT_ERRAND : CT_AFTERSCHOOL;
-    const SlotPlan P{hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt, wpd, h0, h1,
-                     {u[0], u[1], u[2], u[3], u[4], u[5], u[6], u[7]}};
+                                                 bool (&news)[8], const SuccessDraws& draws, const Queue& queue) {
     const bool resolved = A.trace_victim != nullptr;
+    SlotPlan P{};
     int kval = 0;
-    int32_t where[8];  // the contact's location (trace only)
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        int t;
-        if (resolved) {
-            if (c < 3) {
-                t = select_person(idx, hoff, hcnt, u[c], CT_HOME, nullptr, vic[c]);
-                where[c] = hh;
-            } else if (c < 3 + wpd) {
-                t = select_person(idx, woff, wcnt, u[c], wtype, A.wp_people, vic[c]);
-                where[c] = wp;
-            } else {
-                const int e = c - 3 - wpd;
-                if (e < h0) {
-                    t = select_person(idx, e0off, e0cnt, u[c], etype, A.er_people, vic[c]);
-                    where[c] = d1;
-                } else if (e < h0 + h1) {
-                    t = select_person(idx, e1off, e1cnt, u[c], etype, A.er_people, vic[c]);
-                    where[c] = adult ? M.W + d2 : d2;
-                } else {
-                    vic[c] = -1;
-                    t = CT_NONE;
-                    where[c] = -1;
-                }
-            }
-        } else {
-            // select_person's type without the pick
-            const int e = c - 3 - wpd;
-            const int32_t cnt = c < 3 ? hcnt : (c < 3 + wpd ? wcnt : (e < h0 ? e0cnt : (e < h0 + h1 ? e1cnt : 0)));
-            const int ty = c < 3 ? CT_HOME : (c < 3 + wpd ? wtype : etype);
-            t = (e < h0 + h1 && cnt > 1) ? ty : CT_NONE;
+    if (active) {
+        if constexpr (!Queue::counted) {  // (queued infectors can)
+            if (!can_infect(M, f) && !A.trace_victim) return;
         }
-        typ[c] = t;
-        kval += t != CT_NONE;
-    }
-    apply_drops(M, day, false, Mc, 8, vic, typ);
-    if (A.trace_victim) {
+        const uint64_t Mc = cbase + (uint64_t)(6 * pos);
+        const U4 ua = draw4(Mc, M.key0, M.key1);
+        const U4 ub = draw4(Mc + 1, M.key0, M.key1);
+        const uint32_t u[8] = {ua.w[0], ua.w[1], ua.w[2], ua.w[3], ub.w[0], ub.w[1], ub.w[2], ub.w[3]};
+        const uint8_t myage = A.age[idx];
+        const bool adult = myage == kAgeAdult;
+        // household
+        const int32_t hh = A.household[idx];
+        const int32_t hoff = A.hh_off[hh];
+        const int32_t hcnt = A.hh_off[hh + 1] - hoff;
+        // workplace (device_recalcWorkplace PandemicSim.cu:3872-3890) and its
+        // contacts, kept per agent since the setup (PopArrays::wp_of)
+        const uint32_t pw = A.wp_of[idx];
+        const int32_t wp = (int32_t)(pw & kWorkplaceMask);
+        const int wpd = (int)(pw >> kWorkplaceBits);
+        const int32_t woff = A.wp_off[wp];
+        const int32_t wcnt = A.wp_off[wp + 1] - woff;
+        // errands (device_recalc_weekdayErrandDests_assignProfile :3667-3705)
+        const U4 ue = draw4(eoff + (uint64_t)(idx / 2), M.key0, M.key1);
+        const int rs = 2 * (idx % 2);
+        const ErrandWalk wk = pinned(M.wd_walk);
+        int32_t d1, d2;
+        weekday_dests(M, wk, word(ue, rs), word(ue, rs + 1), adult, d1, d2);
+        const int prof = adult ? (int)((word(ue, rs) ^ word(ue, rs + 1)) % 3u) : 3;
+        const int h0 = M.wd_assign[prof][0], h1 = M.wd_assign[prof][1];
+        uint32_t k0, k1;
+        weekday_keys(M, d1, d2, k0, k1);
+        int32_t e0off, e0cnt, e1off, e1cnt;
+        errand_bucket<Queue::counted>(A, k0, e0off, e0cnt);
+        errand_bucket<Queue::counted>(A, k1, e1off, e1cnt);
+        const int wtype = adult ? CT_WORKPLACE : CT_SCHOOL;
+        const int etype = adult ? CT_ERRAND : CT_AFTERSCHOOL;
+        P = SlotPlan{hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt, wpd, h0, h1,
+                         {u[0], u[1], u[2], u[3], u[4], u[5], u[6], u[7]}};
+        int32_t where[8];  // the contact's location (trace only)
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            A.trace_victim[pos * 8 + c] = vic[c];
-            A.trace_type[pos * 8 + c] = (uint8_t)typ[c];
-            A.trace_loc[pos * 8 + c] = vic[c] < 0 ? -1 : where[c];
+            int t;
+            if (resolved) {
+                if (c < 3) {
+                    t = select_person(idx, hoff, hcnt, u[c], CT_HOME, nullptr, vic[c]);
+                    where[c] = hh;
+                } else if (c < 3 + wpd) {
+                    t = select_person(idx, woff, wcnt, u[c], wtype, A.wp_people, vic[c]);
+                    where[c] = wp;
+                } else {
+                    const int e = c - 3 - wpd;
+                    if (e < h0) {
+                        t = select_person(idx, e0off, e0cnt, u[c], etype, A.er_people, vic[c]);
+                        where[c] = d1;
+                    } else if (e < h0 + h1) {
+                        t = select_person(idx, e1off, e1cnt, u[c], etype, A.er_people, vic[c]);
+                        where[c] = adult ? M.W + d2 : d2;
+                    } else {
+                        vic[c] = -1;
+                        t = CT_NONE;
+                        where[c] = -1;
+                    }
+                }
+            } else {
+                // select_person's type without the pick
+                const int e = c - 3 - wpd;
+                const int32_t cnt = c < 3 ? hcnt : (c < 3 + wpd ? wcnt : (e < h0 ? e0cnt : (e < h0 + h1 ? e1cnt : 0)));
+                const int ty = c < 3 ? CT_HOME : (c < 3 + wpd ? wtype : etype);
+                t = (e < h0 + h1 && cnt > 1) ? ty : CT_NONE;
+            }
+            typ[c] = t;
+            kval += t != CT_NONE;
+        }
+        apply_drops(M, day, false, Mc, 8, vic, typ);
+        if (A.trace_victim) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                A.trace_victim[pos * 8 + c] = vic[c];
+                A.trace_type[pos * 8 + c] = (uint8_t)typ[c];
+                A.trace_loc[pos * 8 + c] = vic[c] < 0 ? -1 : where[c];
+            }
         }
     }
     // Traced days run the draws of every infector, as the reference does: an
     // infector that cannot infect has p <= 0 (or NaN), so none of its draws
     // succeeds and it posts no claim.
-    if (can_infect(M, f) || A.trace_draw)
-        process_contacts<8>(M, A, f, kval, vic, typ, P, resolved, idx, Mc + 2, (uint32_t)pos, newp, news);
+    if constexpr (Queue::counted)
+        queue_contacts<8>(M, active, f, kval, typ, P, idx, draws, (uint32_t)pos, queue);
+    else if (can_infect(M, f) || A.trace_draw)
+        process_contacts<8>(M, A, f, kval, vic, typ, P, resolved, idx, draws, (uint32_t)pos, newp, news);
     else if (A.trace_attempt)
         for (int c = 0; c < 8; ++c) A.trace_attempt[pos * 8 + c] = 0;
 }
 
 // D6e + D7: one infector of kernel_doWeekend (PandemicSim.cu:3311-3379) with
 // device_makeContacts_weekend (:1833-1950).
-__device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArrays& A, int day, uint64_t cbase,
+template <class Queue>
+__device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArrays& A, bool active,
+                                                 const Infectivity& f, int day, uint64_t cbase,
                                                  uint64_t eoff, int32_t idx, int64_t pos, int32_t (&vic)[8],
-                                                 int (&typ)[8], bool (&newp)[8], bool (&news)[8]) {
-    const Infectivity f = infectivity(M, A, idx, day);
-    if (!can_infect(M, f) && !A.trace_victim) return;
-    const uint64_t Mc = cbase + (uint64_t)(6 * pos);
-    const U4 u = draw4(Mc, M.key0, M.key1);
-    const int32_t hh = A.household[idx];
-    const int32_t hoff = A.hh_off[hh];
-    const int32_t hcnt = A.hh_off[hh + 1] - hoff;
+                                                 int (&typ)[8], bool (&newp)[8], bool (&news)[8],
+                                                 const SuccessDraws& draws, const Queue& queue) {
     const bool resolved = A.trace_victim != nullptr;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        if (resolved)
-            typ[c] = select_person(idx, hoff, hcnt, u.w[c], CT_HOME, nullptr, vic[c]);
-        else
-            typ[c] = hcnt > 1 ? CT_HOME : CT_NONE;
-    }
-    const int prof = (int)(u.w[3] % 6u);
-    uint32_t v32[2];
-    draw2x32((uint32_t)(Mc + 1), (uint32_t)M.key0, (uint32_t)M.key1, v32);
-    const ErrandWalk wk = pinned(M.we_walk);
-    int32_t hour[3], loc[3];
-    weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
-    int32_t where[5] = {hh, hh, hh, -1, -1};  // the contact's location (trace only)
-    int32_t eo[2], ec[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const int slot = M.we_assign[prof][k];
-        const int hsel = slot == 0 ? hour[0] : (slot == 1 ? hour[1] : hour[2]);
-        const int lsel = slot == 0 ? loc[0] : (slot == 1 ? loc[1] : loc[2]);
-        const int32_t l = min(max(lsel - M.we_base, 0), M.we_E - 1);
-        const int32_t key = hsel * M.we_E + l;
-        eo[k] = A.er_off[key];
-        ec[k] = A.er_off[key + 1] - eo[k];
-        if (resolved)
-            typ[3 + k] = select_person(idx, eo[k], ec[k], v32[k], CT_ERRAND, A.er_people, vic[3 + k]);
-        else
-            typ[3 + k] = ec[k] > 1 ? CT_ERRAND : CT_NONE;
-        where[3 + k] = hsel * M.W + lsel;
-    }
-    const SlotPlan P{hoff, hcnt, 0, 0, eo[0], ec[0], eo[1], ec[1], 0, 1, 1,
-                     {u.w[0], u.w[1], u.w[2], v32[0], v32[1], 0u, 0u, 0u}};
+    SlotPlan P{};
     int kval = 0;
+    if (active) {
+        if constexpr (!Queue::counted) {
+            if (!can_infect(M, f) && !A.trace_victim) return;
+        }
+        const uint64_t Mc = cbase + (uint64_t)(6 * pos);
+        const U4 u = draw4(Mc, M.key0, M.key1);
+        const int32_t hh = A.household[idx];
+        const int32_t hoff = A.hh_off[hh];
+        const int32_t hcnt = A.hh_off[hh + 1] - hoff;
 #pragma unroll
-    for (int c = 0; c < 5; ++c) kval += typ[c] != CT_NONE;
-    apply_drops(M, day, true, Mc, 5, vic, typ);
-    if (A.trace_victim) {
+        for (int c = 0; c < 3; ++c) {
+            if (resolved)
+                typ[c] = select_person(idx, hoff, hcnt, u.w[c], CT_HOME, nullptr, vic[c]);
+            else
+                typ[c] = hcnt > 1 ? CT_HOME : CT_NONE;
+        }
+        const int prof = (int)(u.w[3] % 6u);
+        uint32_t v32[2];
+        draw2x32((uint32_t)(Mc + 1), (uint32_t)M.key0, (uint32_t)M.key1, v32);
+        int32_t where[5] = {hh, hh, hh, -1, -1};  // the contact's location (trace only)
+        int32_t eo[2], ec[2];
+        if constexpr (Queue::counted) {
+            const uint16_t* keys = A.er_keys + idx;
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            A.trace_victim[pos * 5 + c] = vic[c];
-            A.trace_type[pos * 5 + c] = (uint8_t)typ[c];
-            A.trace_loc[pos * 5 + c] = vic[c] < 0 ? -1 : where[c];
+            for (int k = 0; k < 2; ++k) {
+                errand_bucket<true>(A, keys[M.we_assign[prof][k] * A.er_slots], eo[k], ec[k]);
+                typ[3 + k] = ec[k] > 1 ? CT_ERRAND : CT_NONE;
+            }
+        } else {
+            const ErrandWalk wk = pinned(M.we_walk);
+            int32_t hour[3], loc[3];
+            weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * idx), hour, loc);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int slot = M.we_assign[prof][k];
+                const int hsel = slot == 0 ? hour[0] : (slot == 1 ? hour[1] : hour[2]);
+                const int lsel = slot == 0 ? loc[0] : (slot == 1 ? loc[1] : loc[2]);
+                const int32_t l = min(max(lsel - M.we_base, 0), M.we_E - 1);
+                const int32_t key = hsel * M.we_E + l;
+                errand_bucket<false>(A, (uint32_t)key, eo[k], ec[k]);
+                if (resolved)
+                    typ[3 + k] = select_person(idx, eo[k], ec[k], v32[k], CT_ERRAND, A.er_people, vic[3 + k]);
+                else
+                    typ[3 + k] = ec[k] > 1 ? CT_ERRAND : CT_NONE;
+                where[3 + k] = hsel * M.W + lsel;
+            }
+        }
+        P = SlotPlan{hoff, hcnt, 0, 0, eo[0], ec[0], eo[1], ec[1], 0, 1, 1,
+                         {u.w[0], u.w[1], u.w[2], v32[0], v32[1], 0u, 0u, 0u}};
+#pragma unroll
+        for (int c = 0; c < 5; ++c) kval += typ[c] != CT_NONE;
+        apply_drops(M, day, true, Mc, 5, vic, typ);
+        if (A.trace_victim) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                A.trace_victim[pos * 5 + c] = vic[c];
+                A.trace_type[pos * 5 + c] = (uint8_t)typ[c];
+                A.trace_loc[pos * 5 + c] = vic[c] < 0 ? -1 : where[c];
+            }
         }
     }
     // Traced days run the draws of every infector, as the reference does: an
     // infector that cannot infect has p <= 0 (or NaN), so none of its draws
     // succeeds and it posts no claim.
-    if (can_infect(M, f) || A.trace_draw)
-        process_contacts<5>(M, A, f, kval, vic, typ, P, resolved, idx, Mc + 2, (uint32_t)pos, newp, news);
+    if constexpr (Queue::counted)
+        queue_contacts<5>(M, active, f, kval, typ, P, idx, draws, (uint32_t)pos, queue);
+    else if (can_infect(M, f) || A.trace_draw)
+        process_contacts<5>(M, A, f, kval, vic, typ, P, resolved, idx, draws, (uint32_t)pos, newp, news);
     else if (A.trace_attempt)
         for (int c = 0; c < 5; ++c) A.trace_attempt[pos * 5 + c] = 0;
 }
@@ -881,19 +998,14 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
 // 1; the quotient only falls with kval_sum).  Needs nothing but the
 // infector's strain state and its own draws, none of the tables.
 template <int C>
-__device__ __forceinline__ bool may_infect(const Model& M, const Infectivity& f, uint64_t M2) {
+__device__ __forceinline__ bool may_infect(const Model& M, const Infectivity& f, const SuccessDraws& d) {
     const float bp = f.prof_p >= 0 ? infection_probability(M, f.prof_p, f.dd_p, 0, 1) : -1.f;
     const float bs = f.prof_s >= 0 ? infection_probability(M, f.prof_s, f.dd_s, 1, 1) : -1.f;
     bool any = false;
 #pragma unroll
-    for (int q = 0; q < (C + 1) / 2; ++q) {
-        const U4 w = draw4(M2 + (uint64_t)q, M.key0, M.key1);
-        any |= unit_float(w.w[0]) < bp;
-        any |= unit_float(w.w[1]) < bs;
-        if (2 * q + 1 < C) {
-            any |= unit_float(w.w[2]) < bp;
-            any |= unit_float(w.w[3]) < bs;
-        }
+    for (int c = 0; c < C; ++c) {
+        any |= unit_float(d.u[2 * c]) < bp;
+        any |= unit_float(d.u[2 * c + 1]) < bs;
     }
     return any;
 }
@@ -901,9 +1013,9 @@ __device__ __forceinline__ bool may_infect(const Model& M, const Infectivity& f,
 // Contacts of the day's I infectors in two phases.  Most infectors cannot
 // infect anyone today (half of the infectious days shed below 0.1%), and a
 // wave holds a random mix, so instead of branching per lane a block tests T
-// infectors at a time (test(pos, item) -> may_infect) and queues the ones
-// left in LDS; whenever T are queued it runs them together (run(active,
-// item), called by all threads).  Claims resolve by position and slot, so
+// infectors at a time (test(pos, item, draws) -> may_infect) and queues the
+// ones left, with their draws, in LDS; whenever T are queued it runs them
+// together (run(active, item, draws), called by all threads).  Claims resolve by position and slot, so
 // the order does not matter.  VALU bound (8 draws of ~145 instructions per
 // infector before, 4 plus 8 per one left now): 50M agents x 100 days,
 // contacts 41.6 -> 20.1 ms.
@@ -911,9 +1023,11 @@ struct QueuedInfector {
     int32_t idx, pos, r;
 };
 
-template <int T, class Test, class Run>
+template <int T, int C, class Test, class Run>
 __device__ __forceinline__ void filtered_contacts(int64_t I, Test test, Run run) {
+    constexpr int NW = 4 * ((C + 1) / 2);  // words drawn
     __shared__ QueuedInfector s_q[2 * T];
+    __shared__ uint32_t s_u[NW][2 * T];
     __shared__ uint32_t s_n;
     const int tid = threadIdx.x, lane = tid & 63;
     if (tid == 0) s_n = 0;
@@ -922,24 +1036,34 @@ __device__ __forceinline__ void filtered_contacts(int64_t I, Test test, Run run)
     for (int64_t b0 = (int64_t)blockIdx.x * T;; b0 += stride) {
         const bool more = b0 < I;  // the last turn only empties the queue
         QueuedInfector item{};
+        SuccessDraws draws{};
         if (more) {
             const int64_t pos = b0 + tid;
-            const bool keep = pos < I && test(pos, item);
+            const bool keep = pos < I && test(pos, item, draws);
             const uint64_t m = __ballot(keep);
             uint32_t at = 0;
             if (lane == 0 && m) at = atomicAdd(&s_n, (uint32_t)__popcll(m));
             at = __shfl(at, 0, 64);
-            if (keep) s_q[at + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = item;
+            if (keep) {
+                at += (uint32_t)__popcll(m & ((1ull << lane) - 1));
+                s_q[at] = item;
+#pragma unroll
+                for (int j = 0; j < NW; ++j) s_u[j][at] = draws.u[j];
+            }
             __syncthreads();
         }
         const uint32_t n = s_n;  // below 2T; below T on the last turn
         const uint32_t take = min(n, (uint32_t)T);
         if (take == (uint32_t)T || (!more && take)) {
             const bool active = (uint32_t)tid < take;
-            if (active) item = s_q[n - take + tid];
+            if (active) {
+                item = s_q[n - take + tid];
+#pragma unroll
+                for (int j = 0; j < NW; ++j) draws.u[j] = s_u[j][n - take + tid];
+            }
             __syncthreads();
             if (tid == 0) s_n = n - take;
-            run(active, item);
+            run(active, item, draws);
         }
         if (!more) break;
         __syncthreads();

@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "../../include/pandemic/pt_abi.h"
+#include "pt_count.h"
 #include "pt_day.h"
 #include "pt_model.h"
 #include "pt_sort.h"
@@ -139,7 +140,7 @@ __global__ void k_generate_households(const Model* __restrict__ Mp, const uint8_
 // K5: assignWorkplaceFunctor (PandemicSim.cu:3750-3778), four people per
 // counter workplace_off + g, g = 0..N/4.
 __global__ void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workplace_off, uint8_t* __restrict__ age,
-                                    uint32_t* __restrict__ wp_keys) {
+                                    uint32_t* __restrict__ wp_keys, uint32_t* __restrict__ wp_of) {
     const Model& M = *Mp;
     const int N = M.N;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -153,6 +154,7 @@ __global__ void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workp
                 const int32_t wp = assign_workplace(M, u.w[i], &a);
                 age[p] = a;
                 wp_keys[p] = (uint32_t)wp;
+                wp_of[p] = (uint32_t)wp | ((uint32_t)workplace_max_contacts(M, wp) << kWorkplaceBits);
             }
         }
     }
@@ -202,6 +204,13 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(const Model* __restrict
     const int64_t b = blockIdx.x;
     sweep_block(*Mp, N, st->day, b * kSweepTile, st_p, st_s, dy_p, dy_s, blk_counts + b * 16, blk_ninf + b,
                 staging + b * kSweepTile, 0);
+}
+
+// The day's errand and contact counters (:3030-3040, :1409-1415, :1278-1279);
+// rand_offset itself moves at the day's end.
+__device__ __forceinline__ void plan_offsets(DayState* st, bool weekend, int64_t N) {
+    st->errand_off = st->rand_offset;
+    st->contact_base = st->rand_offset + (weekend ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
 }
 
 // Day plan (one block): daily counts, the infected count and block offsets
@@ -287,11 +296,91 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DayState* __restrict__ st
             st->skip_mark = mark ? 0 : 1;
             st->skip_full = mark ? 1 : 0;
             st->skip_subset = 1;
-            st->errand_off = st->rand_offset;
-            st->rand_offset += weekend ? (uint64_t)(2 * N) : (uint64_t)(N / 2);
-            st->contact_base = st->rand_offset;
-            st->rand_offset += (uint64_t)6 * (uint64_t)I;
+            plan_offsets(st, weekend, N);
         }
+    }
+}
+
+// Counted days: the compaction also tests the infectors' success draws and
+// lists the ones left (list_infectors), and, for up to kFusedPlan sweep
+// blocks, is the day plan too (PLAN): every block sums the counts of the
+// blocks before it instead of waiting for a launch of one block.
+constexpr int kFusedPlan = 1024;
+template <bool WEEKEND, bool PLAN>
+__global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
+                                                       const int32_t* __restrict__ staging,
+                                                       const uint32_t* __restrict__ blk_ninf,
+                                                       const uint32_t* __restrict__ blk_off,
+                                                       const uint32_t* __restrict__ blk_counts, int nblk,
+                                                       int32_t* __restrict__ out_counts,
+                                                       int32_t* __restrict__ out_inf, int32_t* __restrict__ infected,
+                                                       AgentArrays A, CountTable T) {
+    if (st->done) return;
+    constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
+    const Model& M = *Mp;
+    const int tid = threadIdx.x;
+    const int day = st->day;
+    const int64_t N = M.N;
+    const uint64_t cbase = st->rand_offset + (WEEKEND ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
+    uint32_t off;
+    if constexpr (PLAN) {
+        const int lane = tid & 63, wave = tid >> 6;
+        __shared__ uint32_t s_w[16], s_off;
+        const uint32_t v = tid < nblk ? blk_ninf[tid] : 0u;
+        const uint32_t inc = wave_incl_scan(v, lane);
+        if (lane == 63) s_w[wave] = inc;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const uint32_t x = s_w[w];
+            if (w < wave) before += x;
+            total += x;
+        }
+        if (tid == (int)blockIdx.x) s_off = before + inc - v;
+        if (blockIdx.x == 0) {
+            // Daily counts: a wave per counter.
+            uint32_t c = 0;
+            for (int b = lane; b < nblk; b += 64) c += blk_counts[(int64_t)b * 16 + wave];
+            c = wave_sum(c);
+            if (lane == 0) out_counts[day * 16 + wave] = (int32_t)c;
+            if (tid == 0) {
+                st->n_infected = (int32_t)total;
+                st->days_run = day + 1;
+                out_inf[day] = (int32_t)total;
+                if (total == 0) {
+                    st->done = 1;  // nobody left to compact: other blocks may or may not see it
+                    st->skip_full = st->skip_subset = st->skip_mark = 1;
+                } else {
+                    st->skip_full = 0;  // every bucket is counted
+                    st->skip_subset = st->skip_mark = 1;
+                    plan_offsets(st, WEEKEND, N);
+                }
+            }
+        }
+        __syncthreads();
+        off = s_off;
+    } else {
+        off = blk_off[blockIdx.x];
+    }
+    const uint32_t n = blk_ninf[blockIdx.x];
+    const int32_t* src = staging + (int64_t)blockIdx.x * kSweepTile;
+    for (uint32_t i0 = 0; i0 < n; i0 += blockDim.x) {
+        const uint32_t i = i0 + tid;
+        int32_t idx = 0;
+        Infectivity f{};
+        bool keep = false;
+        if (i < n) {
+            idx = src[i];
+            infected[off + i] = idx;
+            f = infectivity(M, A, idx, day);
+            if (can_infect(M, f)) {
+                SuccessDraws draws;
+                success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
+                keep = may_infect<C>(M, f, draws);
+            }
+        }
+        list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
     }
 }
 
@@ -449,47 +538,79 @@ __global__ __launch_bounds__(256) void k_mark_weekend(const Model* __restrict__ 
 // D6w/D6e + D7 over the day's infected list (weekday_contacts,
 // weekend_contacts); claims go to the per-strain claim lists.
 // TRACE: every infector's contacts are made and recorded (A's trace arrays).
-template <bool WEEKEND, bool TRACE>
+// COUNTED: errand buckets are counted, not sorted (pt_count.h).
+template <bool WEEKEND, bool TRACE, bool COUNTED>
 __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __restrict__ Mp, DayState* __restrict__ st,
                                                               const int32_t* __restrict__ infected, AgentArrays A,
                                                               int32_t* __restrict__ list_p,
-                                                              int32_t* __restrict__ list_s, uint64_t workplace_off) {
+                                                              int32_t* __restrict__ list_s, CountTable T) {
+    static_assert(!TRACE || !COUNTED, "traced contacts look every victim up");
     if (st->done) return;
     const Model& M = *Mp;
     const int I = st->n_infected;
+    if ((int64_t)blockIdx.x * kContactThreads >= (COUNTED ? (int64_t)T.n[1] : (int64_t)I)) return;
     const int day = st->day;
     const uint64_t cbase = st->contact_base;
     const uint64_t eoff = st->errand_off;
     const int lane = threadIdx.x & 63;
     if constexpr (!TRACE) A.clear_trace();  // known to the compiler
-    auto run = [&](bool active, const QueuedInfector& q) {
-        int32_t vic[8];
-        int typ[8];
-        bool newp[8], news[8];
+    constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
+    int32_t vic[8];
+    int typ[8];
+    bool newp[8], news[8];
+    auto contacts = [&](bool active, const Infectivity& f, int32_t idx, int32_t pos, const SuccessDraws& draws,
+                        const auto& queue) {
         clear_contacts(vic, typ, newp, news);
-        if (active) {
-            if (WEEKEND)
-                weekend_contacts(M, A, day, cbase, eoff, q.idx, q.pos, vic, typ, newp, news);
-            else
-                weekday_contacts(M, A, day, cbase, eoff, workplace_off, q.idx, q.pos, vic, typ, newp, news);
-        }
-        append_claims(st->n_claimed, list_p, list_s, 0, vic, newp, news, lane);
+        if (WEEKEND)
+            weekend_contacts(M, A, active, f, day, cbase, eoff, idx, pos, vic, typ, newp, news, draws, queue);
+        else
+            weekday_contacts(M, A, active, f, day, cbase, eoff, idx, pos, vic, typ, newp, news, draws, queue);
     };
-    if constexpr (TRACE) {
-        const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-        for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x; b0 < I; b0 += stride) {
+    const int64_t stride = (int64_t)gridDim.x * kContactThreads;
+    if constexpr (COUNTED) {
+        const ClaimArrays claims = claim_arrays(A, list_p, list_s, st->n_claimed);
+        __shared__ PickQueue s_pick;
+        if (threadIdx.x == 0)  // first used behind a barrier of the first round
+            s_pick.n = s_pick.errands = s_pick.taken = s_pick.n_claim[0] = s_pick.n_claim[1] = 0;
+        __syncthreads();
+        const PickPush push{T, claims, st, &s_pick, 0};
+        const int64_t n = T.n[1];
+        for (int64_t b0 = (int64_t)blockIdx.x * kContactThreads; b0 < n; b0 += stride) {
+            const int64_t i = b0 + threadIdx.x;
+            const bool active = i < n;
+            int32_t idx = 0, pos = 0;
+            Infectivity f{};
+            SuccessDraws draws{};
+            if (active) {
+                idx = T.sv_idx[i];
+                pos = T.sv_pos[i];
+                f = unpack_infectivity(T.sv_f[i]);
+                success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)pos) + 2, draws);
+            }
+            contacts(active, f, idx, pos, draws, push);
+        }
+    } else if constexpr (TRACE) {
+        for (int64_t b0 = (int64_t)blockIdx.x * kContactThreads; b0 < I; b0 += stride) {
             const int64_t pos = b0 + threadIdx.x;
-            run(pos < I, QueuedInfector{pos < I ? infected[pos] : 0, (int32_t)pos, 0});
+            const int32_t idx = pos < I ? infected[pos] : 0;
+            SuccessDraws draws;
+            success_draws<8>(M, cbase + (uint64_t)(6 * pos) + 2, draws);
+            contacts(pos < I, infectivity(M, A, idx, day), idx, (int32_t)pos, draws, NoQueue{});
+            append_claims(st->n_claimed, list_p, list_s, 0, vic, newp, news, lane);
         }
     } else {
-        filtered_contacts<kContactThreads>(
+        filtered_contacts<kContactThreads, C>(
             I,
-            [&](int64_t pos, QueuedInfector& q) {
+            [&](int64_t pos, QueuedInfector& q, SuccessDraws& draws) {
                 q = QueuedInfector{infected[pos], (int32_t)pos, 0};
+                success_draws<C>(M, cbase + (uint64_t)(6 * pos) + 2, draws);
                 const Infectivity f = infectivity(M, A, q.idx, day);
-                return can_infect(M, f) && may_infect<WEEKEND ? 5 : 8>(M, f, cbase + (uint64_t)(6 * pos) + 2);
+                return can_infect(M, f) && may_infect<C>(M, f, draws);
             },
-            run);
+            [&](bool active, const QueuedInfector& q, const SuccessDraws& draws) {
+                contacts(active, infectivity(M, A, q.idx, day), q.idx, q.pos, draws, NoQueue{});
+                append_claims(st->n_claimed, list_p, list_s, 0, vic, newp, news, lane);
+            });
     }
 }
 
@@ -505,6 +626,7 @@ __global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t*
     tab_pairs[d] = st->skip_full == 0 ? (n_kept ? (int32_t)*n_kept : n_full)
                                       : (st->skip_subset == 0 ? (int32_t)st->n_sel : 0);
     st->day += 1;
+    st->rand_offset = st->contact_base + (uint64_t)6 * (uint64_t)st->n_infected;
     st->n_claimed[0] = 0;
     st->n_claimed[1] = 0;
     st->skip_full = 1;
@@ -635,7 +757,8 @@ int round_half_up(double d) { return (int)floor(d + 0.5); }  // roundHalfUp_toIn
 const char* kKernelNames[KC_COUNT] = {"sweep",         "plan",       "compact",   "gen_weekday",
                                       "gen_weekend",   "sort_upsweep", "sort_scan", "sort_downsweep",
                                       "offsets",       "contacts_weekday", "contacts_weekend", "apply",
-                                      "end_day",       "mark",       "select",    "subset_sort", "setup"};
+                                      "end_day",       "mark",       "select",    "subset_sort", "setup",
+                                      "count_scan",    "collect",    "resolve"};
 
 // Per-class kernel timing.  mode 0: off; -1: every class; k+1: class k only.
 // Launches are also accounted to the simulated day they belong to (day is
@@ -808,7 +931,7 @@ hipError_t build_population(const Model* d_model, int64_t N, int H, int W, const
     k_generate_households<<<grid_for(H, 256, 65535), 256, 0, st>>>(d_model, P.hh_types, P.hh_off, P.household, P.age);
     if (marks) (void)hipEventRecord(marks[1], st);
     // K5/K6: workplaces, then the workplace table (PandemicSim.cu:3812-3862).
-    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, tmp);
+    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, tmp, P.wp_of);
     e = build_table(ts, tmp, nullptr, N, nullptr, W, ID_IDENTITY, (int32_t)N, P.wp_people, P.wp_off, nullptr, st,
                     nullptr);
     if (e != hipSuccess) return e;
@@ -839,6 +962,7 @@ struct pt_sim {
     uint8_t* age = nullptr;
     uint8_t* snap = nullptr;  // 6N bytes
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
+    uint32_t* wp_of = nullptr;
     uint8_t* hh_types = nullptr;
     int32_t *infected = nullptr, *staging = nullptr;
     uint32_t* keys = nullptr;        // 3N
@@ -877,6 +1001,11 @@ struct pt_sim {
     bool trace_on = false;
     int32_t *tr_victim = nullptr, *tr_loc = nullptr;
     uint8_t *tr_type = nullptr, *tr_attempt = nullptr, *tr_action = nullptr, *tr_draw = nullptr, *tr_prof = nullptr;
+    // Counted errand tables (pt_count.h), [0] weekday, [1] weekend.
+    CountPlan count_plan[2];
+    CountScratch count_scratch;
+    CountTable count_table[2] = {};
+    bool last_counted = false;  // the last day enqueued built no table
     int cus = 128;                                   // compute units of the device
     int launch[PT_LAUNCH_KNOBS] = {8, 16, 8, 100, 75, 8, 1};  // pt_launch_knob values
 };
@@ -929,6 +1058,7 @@ void free_population(pt_sim* s) {
     dev_free(s->hh_off);
     dev_free(s->wp_off);
     dev_free(s->wp_people);
+    dev_free(s->wp_of);
     dev_free(s->hh_types);
     dev_free(s->infected);
     dev_free(s->staging);
@@ -949,8 +1079,48 @@ void free_population(pt_sim* s) {
     dev_free(s->sel_ids);
     dev_free(s->sblk_cnt);
     dev_free(s->sblk_off);
+    for (auto& p : s->count_plan) p.release();
+    s->count_scratch.release();
     table_scratch_free(s->tables);
     s->setup_done = s->seeded = s->have_snapshot = false;
+}
+
+// Counted tables where the layouts allow: buffers of the table paths that a
+// counted day does not use hold its keys, lists and picks.
+int setup_counts(pt_sim* s) {
+    const Model& m = s->model;
+    const int32_t K[2] = {m.wd_K, kWeHours * m.we_E};
+    for (int w = 0; w < 2; ++w) {
+        CountPlan& p = s->count_plan[w];
+        CountRep c{};
+        c.K = K[w];
+        p.reps.assign(1, c);
+        p.build({s->N}, w ? 3 : 2, s->cus);
+        if (p.upload(s->stream)) return PT_ENOMEM;
+    }
+    if (s->count_scratch.alloc(s->count_plan[0], s->count_plan[1])) return PT_ENOMEM;
+    for (int w = 0; w < 2; ++w) {
+        const CountPlan& p = s->count_plan[w];
+        if (!p.on) continue;
+        CountTable& t = s->count_table[w];
+        s->count_scratch.fill(t, p);
+        t.keys = reinterpret_cast<uint16_t*>(s->keys);  // 3 x 2 of its 12 bytes per agent
+        t.slots = (s->N + 7) / 8 * 8;
+        t.list = s->er_people;
+        t.pk_bucket = s->stage_keys;
+        t.pk_want = (uint32_t*)s->stage_ids;
+        t.pk_claim = s->sel_keys;
+        t.pk_payload = (uint32_t*)s->sel_ids;
+        t.pk_idx = (int32_t*)s->tables.pairs_a;  // at most 2 picks per agent, 6 words per agent here
+        t.pk_r = t.pk_idx + 3 * s->N;
+        t.pk_chunk = (int32_t*)s->tables.pairs_b;
+        t.pk_len = t.pk_chunk + 3 * s->N;
+        t.sv_idx = (int32_t*)s->stage_keys + 2 * s->N;  // past the picks
+        t.sv_pos = s->stage_ids + 2 * s->N;
+        t.sv_f = s->sel_keys + 2 * s->N;
+        HIP_TRY(set_count_lds(p));
+    }
+    return PT_OK;
 }
 
 AgentArrays agent_arrays(pt_sim* s) {
@@ -962,6 +1132,10 @@ AgentArrays agent_arrays(pt_sim* s) {
     A.wp_people = s->wp_people;
     A.er_off = s->er_off;
     A.er_people = s->er_people;
+    A.wp_of = s->wp_of;
+    A.er_cnt = nullptr;
+    A.er_keys = nullptr;
+    A.er_slots = 0;
     A.st_p = s->st_p;
     A.st_s = s->st_s;
     A.dy_p = s->dy_p;
@@ -979,38 +1153,15 @@ AgentArrays agent_arrays(pt_sim* s) {
     return A;
 }
 
-// Enqueues one loop iteration for host day index d (runToCompletion body,
-// PandemicSim.cu:882-954).  Every kernel is a no-op once the device state
-// says the loop has ended.
-int enqueue_day(pt_sim* s, int d) {
-    const bool weekend = (d % 7) >= 5;
+// The day's sorted errand table: every bucket, or the queried ones.
+int enqueue_table(pt_sim* s, bool weekend, int64_t n, int32_t K, int64_t nwords, const AgentArrays& A) {
     hipStream_t stc = s->stream;
-    s->timer.day = d;
     LaunchTimer* tm = &s->timer;
-    const int N = (int)s->N;
     DayState* st = s->d_state;
-    launch(tm, KC_SWEEP, k_sweep, dim3(s->nblk_sweep), dim3(kSweepThreads), stc, (const Model*)s->d_model, s->N, st,
-           s->st_p, s->st_s,
-           (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, s->blk_counts, s->blk_ninf, s->staging);
-    // Marking pays off while the queried share of the buckets is likely to
-    // stay below the subset threshold: I <= K * mark_limit / 100.
-    const int mpct = s->launch[PT_LAUNCH_MARK_LIMIT];
-    const int32_t lim_wd = (int32_t)std::min<int64_t>(mark_limit(s->model.wd_K, mpct), INT32_MAX);
-    const int32_t lim_we = (int32_t)std::min<int64_t>(mark_limit((int64_t)kWeHours * s->model.we_E, mpct), INT32_MAX);
-    launch(tm, KC_PLAN, k_plan, dim3(1), dim3(kPlanThreads), stc, st, s->nblk_sweep, (const uint32_t*)s->blk_counts,
-           (const uint32_t*)s->blk_ninf, s->blk_off, s->d_counts, s->d_inf, s->N, lim_wd, lim_we, s->table_mode);
-    const int64_t n = weekend ? 3 * s->N : 2 * s->N;
-    const int32_t K = weekend ? kWeHours * s->model.we_E : s->model.wd_K;
-    const IdMode mode = weekend ? ID_DIV3 : ID_HOUR_MAJOR;
-    // Which buckets will be queried today (marks cleared by the compaction),
-    // and which table path to take.
-    const int64_t nwords = ((int64_t)K + 31) / 32;
-    launch(tm, KC_COMPACT, k_compact, dim3(s->nblk_sweep), dim3(256), stc, (const DayState*)st,
-           (const int32_t*)s->staging, (const uint32_t*)s->blk_ninf, (const uint32_t*)s->blk_off, s->infected,
-           s->mark, nwords);
-    AgentArrays A = agent_arrays(s);
     const Model* M = s->d_model;
     const int32_t* infected = s->infected;
+    const int N = (int)s->N;
+    const IdMode mode = weekend ? ID_DIV3 : ID_HOUR_MAJOR;
     if (weekend)
         launch(tm, KC_MARK, k_mark_weekend, dim3(s->grid_contacts), dim3(256), stc, M, (const DayState*)st, infected, A,
                s->mark);
@@ -1052,26 +1203,87 @@ int enqueue_day(pt_sim* s, int d) {
     e = build_table(s->tables, s->keys, nullptr, n, nullptr, K, mode, N, s->er_people, s->er_off, &st->done, stc, tm,
                     weekend ? kNoDrop : (uint32_t)(K - 1), &sel);
     if (e != hipSuccess) return fail(PT_EDEVICE, "table build: %s", hipGetErrorString(e));
-    if (weekend)
-        launch(tm, KC_CONTACTS_WEEKEND, s->trace_on ? k_contacts<true, true> : k_contacts<true, false>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
-               infected, A, s->list_p, s->list_s, s->workplace_off);
-    else
-        launch(tm, KC_CONTACTS_WEEKDAY, s->trace_on ? k_contacts<false, true> : k_contacts<false, false>, dim3(s->grid_contacts), dim3(kContactThreads), stc, M, st,
-               infected, A, s->list_p, s->list_s, s->workplace_off);
+    return PT_OK;
+}
+
+// Enqueues one loop iteration for host day index d (runToCompletion body,
+// PandemicSim.cu:882-954).  Every kernel is a no-op once the device state
+// says the loop has ended.
+int enqueue_day(pt_sim* s, int d) {
+    const bool weekend = (d % 7) >= 5;
+    hipStream_t stc = s->stream;
+    s->timer.day = d;
+    LaunchTimer* tm = &s->timer;
+    DayState* st = s->d_state;
+    launch(tm, KC_SWEEP, k_sweep, dim3(s->nblk_sweep), dim3(kSweepThreads), stc, (const Model*)s->d_model, s->N, st,
+           s->st_p, s->st_s,
+           (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, s->blk_counts, s->blk_ninf, s->staging);
+    // Marking pays off while the queried share of the buckets is likely to
+    // stay below the subset threshold: I <= K * mark_limit / 100.
+    const int mpct = s->launch[PT_LAUNCH_MARK_LIMIT];
+    const int32_t lim_wd = (int32_t)std::min<int64_t>(mark_limit(s->model.wd_K, mpct), INT32_MAX);
+    const int32_t lim_we = (int32_t)std::min<int64_t>(mark_limit((int64_t)kWeHours * s->model.we_E, mpct), INT32_MAX);
+    const CountPlan& cp = s->count_plan[weekend ? 1 : 0];
+    const CountTable& ct = s->count_table[weekend ? 1 : 0];
+    const bool counted = s->table_mode == TABLES_AUTO && cp.on && !s->trace_on;
+    const bool fused_plan = counted && s->nblk_sweep <= kFusedPlan;
+    AgentArrays A = agent_arrays(s);
+    const Model* M = s->d_model;
+    if (counted) {
+        A.er_keys = ct.keys;
+        A.er_slots = ct.slots;
+        A.er_cnt = ct.pre + cp.reps[0].mbase + (int64_t)cp.reps[0].C * cp.reps[0].K;
+        enqueue_counts(cp, ct, &st->done, st, M, s->age, weekend, stc, tm);
+    }
+    // (A counted day counts every bucket: nothing to mark or decide.)
+    if (!fused_plan)
+        launch(tm, KC_PLAN, k_plan, dim3(1), dim3(kPlanThreads), stc, st, s->nblk_sweep,
+               (const uint32_t*)s->blk_counts, (const uint32_t*)s->blk_ninf, s->blk_off, s->d_counts, s->d_inf, s->N,
+               lim_wd, lim_we, counted ? (int)TABLES_FULL : s->table_mode);
+    const int64_t n = weekend ? 3 * s->N : 2 * s->N;
+    const int32_t K = weekend ? kWeHours * s->model.we_E : s->model.wd_K;
+    // Which buckets will be queried today (marks cleared by the compaction),
+    // and which table path to take.
+    const int64_t nwords = ((int64_t)K + 31) / 32;
+    if (counted) {
+        const auto k = weekend ? (fused_plan ? k_compact_test<true, true> : k_compact_test<true, false>)
+                               : (fused_plan ? k_compact_test<false, true> : k_compact_test<false, false>);
+        launch(tm, KC_COMPACT, k, dim3(s->nblk_sweep), dim3(1024), stc, M, st, (const int32_t*)s->staging,
+               (const uint32_t*)s->blk_ninf, (const uint32_t*)s->blk_off, (const uint32_t*)s->blk_counts,
+               s->nblk_sweep, s->d_counts, s->d_inf, s->infected, A, ct);
+    } else {
+        launch(tm, KC_COMPACT, k_compact, dim3(s->nblk_sweep), dim3(256), stc, (const DayState*)st,
+               (const int32_t*)s->staging, (const uint32_t*)s->blk_ninf, (const uint32_t*)s->blk_off, s->infected,
+               s->mark, nwords);
+    }
+    const int32_t* infected = s->infected;
+    const int grid = grid_for(s->N, kContactThreads, s->grid_contacts);  // no more blocks than agents can fill
+    if (!counted)
+        if (const int rc = enqueue_table(s, weekend, n, K, nwords, A)) return rc;
+    const auto contacts = weekend ? (s->trace_on ? k_contacts<true, true, false>
+                                                  : (counted ? k_contacts<true, false, true> : k_contacts<true, false, false>))
+                                  : (s->trace_on ? k_contacts<false, true, false>
+                                                  : (counted ? k_contacts<false, false, true> : k_contacts<false, false, false>));
+    launch(tm, weekend ? KC_CONTACTS_WEEKEND : KC_CONTACTS_WEEKDAY, contacts, dim3(grid),
+           dim3(kContactThreads), stc, M, st, infected, A, s->list_p, s->list_s, ct);
+    if (counted) {
+        enqueue_picks(cp, ct, claim_arrays(A, s->list_p, s->list_s, st->n_claimed), st, st, M, grid, weekend, stc, tm);
+    }
     if (s->trace_on)
         k_trace_actions<<<s->grid_contacts, 256, 0, stc>>>((const DayState*)st, weekend ? 5 : 8,
                                                             (const int32_t*)s->tr_victim,
                                                             (const uint8_t*)s->tr_attempt,
                                                             (const uint64_t*)s->claim_p,
                                                             (const uint64_t*)s->claim_s, s->tr_action);
-    launch(tm, KC_APPLY, k_apply, dim3(s->grid_contacts), dim3(256), stc, (const DayState*)st, s->claim_p, s->claim_s,
+    launch(tm, KC_APPLY, k_apply, dim3(grid), dim3(256), stc, (const DayState*)st, s->claim_p, s->claim_s,
            (const int32_t*)s->list_p, (const int32_t*)s->list_s, s->st_p, s->st_s, s->dy_p, s->dy_s, s->gn_p, s->gn_s);
     launch(tm, KC_END_DAY, k_end_day, dim3(1), dim3(1), stc, st, s->d_tab_full, s->d_tab_pairs, (int32_t)n,
-           weekend ? (const uint32_t*)nullptr : (const uint32_t*)s->tables.n_kept);
-    e = hipGetLastError();
+           weekend || counted ? (const uint32_t*)nullptr : (const uint32_t*)s->tables.n_kept);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(PT_EDEVICE, "day launch: %s", hipGetErrorString(e));
     s->last_weekend = weekend ? 1 : 0;
     s->last_table_n = n;
+    s->last_counted = counted;
     s->host_day = d + 1;
     s->timer.day = -1;
     return 0;
@@ -1096,6 +1308,34 @@ int read_state(pt_sim* s, DayState* h) {
     HIP_TRY(hipMemcpyAsync(h, s->d_state, sizeof *h, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return 0;
+}
+
+// Parity hook after a counted day: the table that day did not build, in full.
+int build_last_table(pt_sim* s) {
+    if (!s->last_counted) return PT_OK;
+    const bool weekend = s->last_weekend == 1;
+    DayState h;
+    if (read_state(s, &h)) return PT_EDEVICE;
+    h.skip_full = 0;  // the key kernels run; errand_off is still the day's
+    DayState* d = nullptr;
+    if (dev_alloc(&d, 1)) return PT_ENOMEM;
+    hipError_t e = hipMemcpy(d, &h, sizeof h, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        if (weekend)
+            k_gen_weekend<<<s->grid_gen, 256, 0, s->stream>>>(s->d_model, d, s->keys);
+        else
+            k_gen_weekday<<<s->grid_gen, 256, 0, s->stream>>>(s->d_model, d, s->age, s->keys);
+        const int32_t K = weekend ? kWeHours * s->model.we_E : s->model.wd_K;
+        e = build_table(s->tables, s->keys, nullptr, s->last_table_n, nullptr, K, weekend ? ID_DIV3 : ID_HOUR_MAJOR,
+                        (int32_t)s->N, s->er_people, s->er_off, nullptr, s->stream, nullptr,
+                        weekend ? kNoDrop : (uint32_t)(K - 1));
+        const hipError_t es = hipStreamSynchronize(s->stream);
+        if (e == hipSuccess) e = es;
+    }
+    (void)hipFree(d);
+    if (e != hipSuccess) return fail(PT_EDEVICE, "errand table: %s", hipGetErrorString(e));
+    s->last_counted = false;  // er_off and er_people hold it now
+    return PT_OK;
 }
 
 // Parity hook: the last weekday table in the reference's layout (bucket
@@ -1257,8 +1497,9 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
         dev_alloc(&s->dy_s, Npad) || dev_alloc(&s->gn_p, Npad) || dev_alloc(&s->gn_s, Npad) ||
         dev_alloc(&s->age, N) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
         dev_alloc(&s->hh_off, (int64_t)H + 1) ||
-        dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->infected, N) ||
-        dev_alloc(&s->staging, (int64_t)s->nblk_sweep * kSweepTile) || dev_alloc(&s->keys, n3) ||
+        dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->wp_of, N) ||
+        dev_alloc(&s->infected, N) ||
+        dev_alloc(&s->staging, (int64_t)s->nblk_sweep * kSweepTile) || dev_alloc(&s->keys, n3 + 16) ||
         dev_alloc(&s->er_people, n3) || dev_alloc(&s->er_off, std::max<int64_t>(kmax, (int64_t)s->W) + 1) ||
         dev_alloc(&s->claim_p, N) || dev_alloc(&s->claim_s, N) || dev_alloc(&s->list_p, N) ||
         dev_alloc(&s->list_s, N) || dev_alloc(&s->blk_counts, (int64_t)s->nblk_sweep * 16) ||
@@ -1277,6 +1518,11 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
     }
     s->tables.wide_bits = s->launch[PT_LAUNCH_SORT_WIDE_BITS];
     s->tables.max_bits = s->launch[PT_LAUNCH_SORT_MAX_BITS];
+    if (const int rc = setup_counts(s)) {
+        const std::string msg = g_err;
+        free_population(s);
+        return fail(rc, "%s", msg.c_str());
+    }
     if (s->trace_on && alloc_trace(s)) {
         free_population(s);
         return fail(PT_ENOMEM, "trace allocation failed");
@@ -1286,7 +1532,7 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
     // households is the workplace counter, PandemicSim.cu:2570-2571, :3817).
     s->workplace_off = (uint64_t)(H / 4);
     s->rand_after_setup = s->workplace_off + (uint64_t)(N / 4);
-    const PopArrays P{s->hh_types, s->hh_off, s->household, s->age, s->wp_off, s->wp_people, s->st_p, s->st_s,
+    const PopArrays P{s->hh_types, s->hh_off, s->household, s->age, s->wp_off, s->wp_people, s->wp_of, s->st_p, s->st_s,
                       s->dy_p, s->dy_s, s->gn_p, s->gn_s, s->claim_p, s->claim_s};
     hipError_t e = build_population(s->d_model, N, H, s->W, P, s->keys, s->tables, s->workplace_off, st,
                                     s->setup_ev + 2);
@@ -1501,12 +1747,14 @@ int pt_sim_copy_array(pt_sim* s, int32_t which, void* dst, int64_t bytes) {
             return PT_OK;
         }
         case PT_ERRAND_PEOPLE:
+            if (int rc = build_last_table(s)) return rc;
             if (s->last_weekend == 1) {
                 src = s->er_people;
                 break;
             }
             return expand_weekday_table(s, nullptr, (int32_t*)dst, need / 4);
         case PT_ERRAND_OFFSETS: {
+            if (int rc = build_last_table(s)) return rc;
             if (s->last_weekend == 0) return expand_weekday_table(s, (int32_t*)dst, nullptr, 0);
             // Expand the dense bucket layout to the reference's
             // hour * W + location layout (lower_bound semantics).

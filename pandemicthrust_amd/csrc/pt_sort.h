@@ -33,6 +33,9 @@ enum KernelClass : int {
     KC_SELECT,
     KC_SUBSET_SORT,  // idle: subset and full errand tables share one build (the sort classes); index kept
     KC_SETUP,
+    KC_COUNT_SCAN,
+    KC_COLLECT,
+    KC_RESOLVE,
     KC_COUNT
 };
 
@@ -47,14 +50,20 @@ struct LaunchTimer {
 };
 
 template <typename F, typename... Args>
-inline void launch(LaunchTimer* tm, int cls, F kernel, dim3 grid, dim3 block, hipStream_t stream, Args... args) {
+inline void launch_lds(LaunchTimer* tm, int cls, F kernel, dim3 grid, dim3 block, size_t lds, hipStream_t stream,
+                       Args... args) {
     if (tm && tm->want(cls)) {
         hipEvent_t a, b;
         tm->events(cls, &a, &b);
-        hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, a, b, 0, args...);
+        hipExtLaunchKernelGGL(kernel, grid, block, lds, stream, a, b, 0, args...);
     } else {
-        kernel<<<grid, block, 0, stream>>>(args...);
+        kernel<<<grid, block, lds, stream>>>(args...);
     }
+}
+
+template <typename F, typename... Args>
+inline void launch(LaunchTimer* tm, int cls, F kernel, dim3 grid, dim3 block, hipStream_t stream, Args... args) {
+    launch_lds(tm, cls, kernel, grid, block, 0, stream, args...);
 }
 
 // How a person id follows from the input position j.

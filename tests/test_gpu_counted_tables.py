@@ -1,0 +1,67 @@
+"""Counted errand tables (csrc/pt_count.h) against the sorted tables: the
+automatic mode counts every bucket and picks single people, mode 1 sorts the
+whole table.  Both must give the same days, state and generation tallies.
+
+Sizes: populations below one chunk and at odd remainders; so few buckets that
+a bucket's list in a chunk exceeds 64 ids (bisected instead of ranked); many
+nearly empty buckets (empty chunks of a bucket); bucket counts on both sides
+of the largest counted layout (40,000: weekday 2,901 per location scale,
+weekend 13,000), where only the weekday or neither layout is counted."""
+import numpy as np
+import pytest
+
+import oracle_ctypes as O
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # people, locations, days, seeds per strain
+    (0.0004, 0.0004, 14, 20),
+    (0.004, 0.0011, 9, 60),        # about 30 buckets for 9,400 agents
+    (0.1, 0.0011, 9, 3000),        # the same for 235,000: lists of hundreds of ids
+    (0.02, 0.3, 9, 300),
+    (0.05, 3.05, 9, 2000),         # weekend 39,650 buckets: both layouts counted
+    (0.05, 3.1, 9, 2000),          # weekend 40,300: sorted, weekday counted
+    (0.05, 13.75, 6, 2000),        # weekday 39,889
+    (0.05, 13.85, 6, 2000),        # weekday 40,179: sorted
+]
+
+
+@pytest.mark.parametrize("people,locations,days,seeds", CASES)
+def test_counted_equals_sorted(people, locations, days, seeds):
+    from pandemicthrust_amd import Params, PandemicSim
+    row = [str(days), "2.6", "1.9", str(seeds), str(seeds), str(people), str(locations), "0.8", "0.3"]
+    runs = []
+    for mode in (0, 1):
+        s = PandemicSim(Params.from_row(row), 17)
+        s.set_table_mode(mode)
+        s.setup_sim()
+        counts, inf = s.run()
+        runs.append([counts, inf, *s.generation_offsets(), *[s.array(w) for w in range(6)]])
+        s.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("people,locations", [(0.0007, 0.0007), (0.06, 0.0011), (0.05, 0.6)])
+def test_counted_days_equal_the_oracle(people, locations):
+    """Every day's counts and state; after a counted day the table hooks
+    return that day's whole table."""
+    from pandemicthrust_amd import Params, PandemicSim
+    from pandemicthrust_amd.api import PT_ERRAND_OFFSETS, PT_ERRAND_PEOPLE
+    row = ["9", "2.4", "1.7", "40", "40", str(people), str(locations), "0.9", "0.2"]
+    gpu = PandemicSim(Params.from_row(row), 23)
+    ref = O.OracleSim(O.params_from_row(row), 23)
+    gpu.setup_sim()
+    ref.setup()
+    for day in range(9):
+        rg, cg, ig = gpu.step()
+        rr, cr, ir = ref.step()
+        assert (rg, ig) == (rr, ir) and np.array_equal(cg, cr), day
+        for w in range(6):
+            assert np.array_equal(gpu.array(w), ref.array(w)), (day, w)
+        if rr == 1:
+            break
+        if day in (1, 5):
+            assert np.array_equal(gpu.array(PT_ERRAND_OFFSETS), ref.array(O.OR_ERRAND_OFFSETS)), day
+            assert np.array_equal(gpu.array(PT_ERRAND_PEOPLE), ref.array(O.OR_ERRAND_PEOPLE)), day
