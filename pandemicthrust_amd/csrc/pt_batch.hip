@@ -39,6 +39,7 @@
 
 #include "../../include/pandemic/pt_abi.h"
 #include "../../include/pandemic/pt_batch.h"
+#include "pt_count.h"
 #include "pt_day.h"
 #include "pt_model.h"
 #include "pt_sort.h"
@@ -211,13 +212,139 @@ __global__ __launch_bounds__(kRepThreads) void kb_plan(const DayState* __restric
             const bool mark = table_mode == TABLES_SUBSET || (table_mode == TABLES_AUTO && I <= mark_limit(K, mark_pct));
             st->skip_mark = mark ? 0 : 1;
             st->skip_full = mark ? 1 : 0;
-            const int64_t N = ri.N;
-            st->errand_off = st->rand_offset;
-            st->rand_offset += weekend ? (uint64_t)(2 * N) : (uint64_t)(N / 2);
-            st->contact_base = st->rand_offset;
-            st->rand_offset += (uint64_t)6 * (uint64_t)I;
+            plan_offsets(st, weekend, ri.N);
             rep_I[r] = I;
         }
+    }
+}
+
+// Counted days: the plan of every replicate and the draw test of its
+// infectors, as the single simulation's k_compact_test with PLAN (replicates
+// of up to kFusedPlan sweep tiles).  No infected list is kept.
+constexpr int kFusedPlan = 1024;
+template <bool WEEKEND>
+__global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restrict__ g, DayState* __restrict__ sts,
+                                                        const RepInfo* __restrict__ reps,
+                                                        const Model* __restrict__ models,
+                                                        const int32_t* __restrict__ tile_rep,
+                                                        const int32_t* __restrict__ staging,
+                                                        const uint32_t* __restrict__ blk_ninf,
+                                                        const uint32_t* __restrict__ blk_counts,
+                                                        int32_t* __restrict__ out_counts,
+                                                        int32_t* __restrict__ out_inf, int D, BatchArrays B,
+                                                        CountTable T) {
+    if (g->done) return;
+    const int64_t b = blockIdx.x;
+    const int r = tile_rep[b];
+    DayState* st = sts + r;
+    if (st->done) return;
+    constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
+    const Model& M = models[r];
+    const RepInfo ri = reps[r];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int day = st->day;
+    const int64_t N = ri.N;
+    const uint64_t cbase = st->rand_offset + (WEEKEND ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
+    __shared__ uint32_t s_w[16], s_off;
+    const uint32_t v = tid < ri.ntiles ? blk_ninf[ri.tile0 + tid] : 0u;
+    const uint32_t inc = wave_incl_scan(v, lane);
+    if (lane == 63) s_w[wave] = inc;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const uint32_t x = s_w[w];
+        if (w < wave) before += x;
+        total += x;
+    }
+    if (tid == (int)b - ri.tile0) s_off = before + inc - v;
+    if (b == ri.tile0) {
+        uint32_t c = 0;
+        for (int t = lane; t < ri.ntiles; t += 64) c += blk_counts[(int64_t)(ri.tile0 + t) * 16 + wave];
+        c = wave_sum(c);
+        if (lane == 0) out_counts[((int64_t)r * D + day) * 16 + wave] = (int32_t)c;
+        if (tid == 0) {
+            st->n_infected = (int32_t)total;
+            st->days_run = day + 1;
+            out_inf[(int64_t)r * D + day] = (int32_t)total;
+            if (total == 0)
+                st->done = 1;  // nobody left to test: the replicate's other blocks may or may not see it
+            else
+                plan_offsets(st, WEEKEND, N);
+        }
+    }
+    __syncthreads();
+    const uint32_t off = s_off, n = blk_ninf[b];
+    const int32_t* src = staging + b * kSweepTile;
+    AgentArrays A = view(B, ri, 0u);
+    for (uint32_t i0 = 0; i0 < n; i0 += blockDim.x) {
+        const uint32_t i = i0 + tid;
+        int32_t idx = 0;
+        Infectivity f{};
+        bool keep = false;
+        if (i < n) {
+            idx = src[i] - (int32_t)ri.abase;
+            f = infectivity(M, A, idx, day);
+            if (can_infect(M, f)) {
+                SuccessDraws draws;
+                success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
+                keep = may_infect<C>(M, f, draws);
+            }
+        }
+        list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), r, true);
+    }
+}
+
+// Contacts of the listed infectors (counted tables).
+template <bool WEEKEND>
+__global__ __launch_bounds__(kContactThreads) void kb_contacts_counted(DayState* __restrict__ g,
+                                                                       const DayState* __restrict__ sts,
+                                                                       const RepInfo* __restrict__ reps,
+                                                                       const Model* __restrict__ models, BatchArrays B,
+                                                                       int32_t* __restrict__ list_p,
+                                                                       int32_t* __restrict__ list_s, CountTable T) {
+    if (g->done) return;
+    const int64_t n = T.n[1];
+    if ((int64_t)blockIdx.x * kContactThreads >= n) return;
+    constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
+    __shared__ PickQueue s_pick;
+    if (threadIdx.x == 0)  // first used behind a barrier of the first round
+        s_pick.n = s_pick.errands = s_pick.taken = s_pick.n_claim[0] = s_pick.n_claim[1] = 0;
+    __syncthreads();
+    const ClaimArrays claims{B.st_p, B.st_s, B.wp_people, B.claim_p, B.claim_s, list_p, list_s, g->n_claimed};
+    const int64_t stride = (int64_t)gridDim.x * kContactThreads;
+    for (int64_t b0 = (int64_t)blockIdx.x * kContactThreads; b0 < n; b0 += stride) {
+        const int64_t i = b0 + threadIdx.x;
+        const bool active = i < n;
+        int32_t idx = 0, pos = 0, r = 0;
+        Infectivity f{};
+        SuccessDraws draws{};
+        if (active) {
+            idx = T.sv_idx[i];
+            pos = T.sv_pos[i];
+            r = T.sv_r[i];
+            f = unpack_infectivity(T.sv_f[i]);
+        }
+        const Model& M = models[r];
+        const DayState& st = sts[r];
+        if (active) success_draws<C>(M, st.contact_base + (uint64_t)(6 * (int64_t)pos) + 2, draws);
+        const RepInfo ri = reps[r];
+        AgentArrays A = view(B, ri, 0u);
+        const CountRep cr = T.reps[r];
+        A.er_cnt = count_row(T, cr, cr.C);
+        A.er_keys = T.keys + ri.abase;
+        A.er_slots = T.slots;
+        int32_t vic[8];
+        int typ[8];
+        bool newp[8], news[8];
+        clear_contacts(vic, typ, newp, news);
+        const PickPush push{T, claims, sts, &s_pick, r};
+        if (WEEKEND)
+            weekend_contacts(M, A, active, f, st.day, st.contact_base, st.errand_off, idx, pos, vic, typ, newp, news,
+                             draws, push);
+        else
+            weekday_contacts(M, A, active, f, st.day, st.contact_base, st.errand_off, idx, pos, vic, typ, newp, news,
+                             draws, push);
     }
 }
 
@@ -505,13 +632,19 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts(DayState* __restr
 
 __global__ void kb_end_day(DayState* __restrict__ g, DayState* __restrict__ sts, int R) {
     if (g->done) return;
+    bool running = false;
     for (int r = threadIdx.x; r < R; r += blockDim.x) {
         DayState* st = sts + r;
         if (st->done) continue;
         st->day += 1;
+        st->rand_offset = st->contact_base + (uint64_t)6 * (uint64_t)st->n_infected;
         if (st->day >= st->max_days) st->done = 1;
+        running = true;
     }
+    // (With sorted tables kb_start finds the end of the batch on the next day.)
+    running = __syncthreads_or(running);
     if (threadIdx.x == 0) {
+        if (!running) g->done = 1;
         g->day += 1;
         g->n_claimed[0] = 0;
         g->n_claimed[1] = 0;
@@ -571,6 +704,10 @@ struct pt_batch {
     unsigned long long* d_scratch64 = nullptr;  // max(R, 512)
     TableScratch tables;
     int grid_contacts = 2048;
+    // Counted errand tables (pt_count.h), [0] weekday, [1] weekend.
+    CountPlan count_plan[2];
+    CountScratch count_scratch;
+    CountTable count_table[2] = {};
     int cus = 256;                                   // compute units of the device
     int launch[PT_LAUNCH_KNOBS] = {8, 16, 8, 100, 75, 9, 1};  // pt_launch_knob values
     hipEvent_t run_begin = nullptr, run_end = nullptr;
@@ -633,6 +770,8 @@ void free_batch_population(pt_batch* b) {
     dev_free(b->seg_start);
     dev_free(b->seg_count);
     b->seg_tables = false;
+    for (auto& p : b->count_plan) p.release();
+    b->count_scratch.release();
     dev_free(b->d_counts);
     dev_free(b->d_inf);
     table_scratch_free(b->tables);
@@ -679,6 +818,16 @@ BatchArrays batch_arrays(pt_batch* b) {
     return B;
 }
 
+// Infections of the day, then the day counters.
+int enqueue_day_end(pt_batch* b, int grid) {
+    k_apply<<<grid, 256, 0, b->stream>>>(b->d_g, b->claim_p, b->claim_s, b->list_p, b->list_s, b->st_p, b->st_s,
+                                         b->dy_p, b->dy_s, b->gn_p, b->gn_s);
+    kb_end_day<<<1, 256, 0, b->stream>>>(b->d_g, b->d_states, b->R);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(PT_EDEVICE, "batch day launch: %s", hipGetErrorString(e));
+    return 0;
+}
+
 // One lockstep day d of every replicate.
 int enqueue_batch_day(pt_batch* b, int d) {
     const bool weekend = (d % 7) >= 5;
@@ -687,6 +836,22 @@ int enqueue_batch_day(pt_batch* b, int d) {
     const int R = b->R;
     kb_sweep<<<b->ntiles, kSweepThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep, b->st_p, b->st_s, b->dy_p,
                                                  b->dy_s, b->blk_counts, b->blk_ninf, b->staging);
+    const CountPlan& cp = b->count_plan[weekend ? 1 : 0];
+    if (b->table_mode == TABLES_AUTO && cp.on) {
+        const CountTable& ct = b->count_table[weekend ? 1 : 0];
+        const BatchArrays B = batch_arrays(b);
+        enqueue_counts(cp, ct, &g->done, b->d_states, b->d_models, b->age, weekend, s, nullptr);
+        const auto test = weekend ? kb_compact_test<true> : kb_compact_test<false>;
+        test<<<b->ntiles, 1024, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep, b->staging, b->blk_ninf,
+                                        b->blk_counts, b->d_counts, b->d_inf, b->D, B, ct);
+        const int grid = grid_for(b->n_agents, kContactThreads, b->grid_contacts);
+        const auto contacts = weekend ? kb_contacts_counted<true> : kb_contacts_counted<false>;
+        contacts<<<grid, kContactThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, B, b->list_p, b->list_s, ct);
+        const ClaimArrays claims{b->st_p, b->st_s, b->wp_people, b->claim_p, b->claim_s, b->list_p, b->list_s,
+                                 g->n_claimed};
+        enqueue_picks(cp, ct, claims, g, b->d_states, b->d_models, grid, weekend, s, nullptr);
+        return enqueue_day_end(b, grid);
+    }
     kb_plan<<<R, kRepThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->blk_counts, b->blk_ninf, b->blk_off,
                                       b->rep_I, b->d_counts, b->d_inf, b->D, b->table_mode,
                                       b->launch[PT_LAUNCH_MARK_LIMIT]);
@@ -760,12 +925,55 @@ int enqueue_batch_day(pt_batch* b, int d) {
         kb_contacts<false><<<b->grid_contacts, kContactThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models,
                                                                         b->inf_start, R, b->infected, B, b->list_p,
                                                                         b->list_s);
-    k_apply<<<b->grid_contacts, 256, 0, s>>>(g, b->claim_p, b->claim_s, b->list_p, b->list_s, b->st_p, b->st_s,
-                                             b->dy_p, b->dy_s, b->gn_p, b->gn_s);
-    kb_end_day<<<1, 256, 0, s>>>(g, b->d_states, R);
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(PT_EDEVICE, "batch day launch: %s", hipGetErrorString(e));
-    return 0;
+    return enqueue_day_end(b, b->grid_contacts);
+}
+
+// Counted tables where every replicate's layout allows; buffers of the table
+// paths that a counted day does not use hold its keys, lists and picks.
+int setup_batch_counts(pt_batch* b) {
+    int tiles = 0;
+    std::vector<int64_t> N(b->R);
+    for (int r = 0; r < b->R; ++r) {
+        N[r] = b->reps[r].N;
+        tiles = std::max(tiles, b->reps[r].ntiles);
+    }
+    if (tiles > kFusedPlan) return PT_OK;
+    for (int w = 0; w < 2; ++w) {
+        CountPlan& p = b->count_plan[w];
+        p.reps.resize(b->R);
+        for (int r = 0; r < b->R; ++r) {
+            p.reps[r] = CountRep{};
+            p.reps[r].K = w ? kWeHours * b->models[r].we_E : b->models[r].wd_K;
+            p.reps[r].abase = b->reps[r].abase;
+        }
+        p.build(N, w ? 3 : 2, b->cus);
+        if (p.upload(b->stream)) return PT_ENOMEM;
+    }
+    if (b->count_scratch.alloc(b->count_plan[0], b->count_plan[1])) return PT_ENOMEM;
+    const int64_t P = b->P;
+    for (int w = 0; w < 2; ++w) {
+        const CountPlan& p = b->count_plan[w];
+        if (!p.on) continue;
+        CountTable& t = b->count_table[w];
+        b->count_scratch.fill(t, p);
+        t.keys = reinterpret_cast<uint16_t*>(b->tables.keys_b);  // 6 of its 12 bytes per slot
+        t.slots = P;
+        t.list = b->er_people;
+        t.pk_bucket = b->stage_keys;  // at most 2 picks per agent
+        t.pk_want = (uint32_t*)b->stage_ids;
+        t.pk_claim = b->sel_keys;
+        t.pk_payload = (uint32_t*)b->sel_ids;
+        t.pk_idx = (int32_t*)b->tables.pairs_a;
+        t.pk_r = t.pk_idx + 3 * P;
+        t.pk_chunk = (int32_t*)b->tables.pairs_b;
+        t.pk_len = t.pk_chunk + 3 * P;
+        t.sv_idx = (int32_t*)b->stage_keys + 2 * P;
+        t.sv_pos = b->stage_ids + 2 * P;
+        t.sv_f = b->sel_keys + 2 * P;
+        t.sv_r = b->sel_ids + 2 * P;
+        HIP_TRY(set_count_lds(p));
+    }
+    return PT_OK;
 }
 
 void drop_day_graphs(pt_batch* b) {
@@ -955,6 +1163,11 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
     }
     b->tables.wide_bits = b->launch[PT_LAUNCH_SORT_WIDE_BITS];
     b->tables.max_bits = b->launch[PT_LAUNCH_SORT_MAX_BITS];
+    if (const int rc = setup_batch_counts(b)) {
+        const std::string msg = pt_last_error();
+        free_batch_population(b);
+        return fail(rc, "%s", msg.c_str());
+    }
     HIP_TRY(hipMemcpyAsync(b->tile_rep, trep.data(), sizeof(int32_t) * tiles, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(b->d_models, b->models.data(), sizeof(Model) * R, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(b->d_reps, b->reps.data(), sizeof(RepInfo) * R, hipMemcpyHostToDevice, st));

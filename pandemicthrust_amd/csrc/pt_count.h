@@ -641,9 +641,12 @@ struct CountPlan {
     // a simulation has too many buckets for LDS, or so few for its agents
     // (over kCountMaxLen people per bucket in the smallest chunk) that lists
     // would approach the whole table.
+    // At least about `want` chunks in all, if lists stay above one id.
     void build(const std::vector<int64_t>& N, int keys_per_agent, int64_t want) {
         kpa = keys_per_agent;
         int32_t kmax = 0;
+        int64_t total = 0;
+        for (int64_t n : N) total += n;
         on = true;
         for (size_t r = 0; r < reps.size(); ++r) {
             kmax = std::max(kmax, reps[r].K);
@@ -655,7 +658,7 @@ struct CountPlan {
         threads = 1024;
         for (size_t r = 0; r < reps.size(); ++r) {
             CountRep& c = reps[r];
-            c.A = count_chunk(N[r], c.K, kpa, want);
+            c.A = count_chunk(N[r], c.K, kpa, std::max<int64_t>(1, want * N[r] / total));
             c.C = (int32_t)((N[r] + c.A - 1) / c.A);
             c.qw = (c.K + 31) / 32;
             c.mbase = entries;

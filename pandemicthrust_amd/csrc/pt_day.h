@@ -207,6 +207,14 @@ __device__ __forceinline__ void wave_sum_bins8(uint64_t v, uint32_t (&out)[8]) {
     out[7] = w[3] >> 16;
 }
 
+// The day's errand and contact counters (PandemicSim.cu:3030-3040,
+// :1409-1415, :1278-1279, :1393-1394);
+// rand_offset itself moves at the day's end.
+__device__ __forceinline__ void plan_offsets(DayState* st, bool weekend, int64_t N) {
+    st->errand_off = st->rand_offset;
+    st->contact_base = st->rand_offset + (weekend ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
+}
+
 // ---------------- D1 + D2: sweep ----------------
 
 // One sweep block (kSweepThreads threads) over agents [t0, t0 + kSweepTile)

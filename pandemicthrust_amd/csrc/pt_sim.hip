@@ -206,13 +206,6 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep(const Model* __restrict
                 staging + b * kSweepTile, 0);
 }
 
-// The day's errand and contact counters (:3030-3040, :1409-1415, :1278-1279);
-// rand_offset itself moves at the day's end.
-__device__ __forceinline__ void plan_offsets(DayState* st, bool weekend, int64_t N) {
-    st->errand_off = st->rand_offset;
-    st->contact_base = st->rand_offset + (weekend ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
-}
-
 // Day plan (one block): daily counts, the infected count and block offsets
 // of the compaction, the stop rule (PandemicSim.cu:899-901) and the RNG
 // offsets of the day (:3030-3040 weekday, :1409-1415 weekend, :1278-1279 and

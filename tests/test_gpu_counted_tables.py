@@ -65,3 +65,40 @@ def test_counted_days_equal_the_oracle(people, locations):
         if day in (1, 5):
             assert np.array_equal(gpu.array(PT_ERRAND_OFFSETS), ref.array(O.OR_ERRAND_OFFSETS)), day
             assert np.array_equal(gpu.array(PT_ERRAND_PEOPLE), ref.array(O.OR_ERRAND_PEOPLE)), day
+
+
+def test_batch_counts_equal_sorts():
+    """A batch of unlike replicates (sizes, location scales, lengths; one
+    without infected, one that dies out early): counted days equal sorted
+    ones, and equal each replicate's single run."""
+    from pandemicthrust_amd import PandemicBatch, PandemicSim, Params
+    rows = [["16", "2.2", "1.4", "30", "30", "0.05", "0.05", "1", "0"],
+            ["9", "1.8", "1.3", "5", "0", "0.0004", "0.0004", "1", "0"],
+            ["20", "2.6", "1.9", "200", "100", "0.02", "0.2", "0.8", "0.3"],
+            ["12", "0", "0", "4", "4", "0.003", "0.003", "1", "0"],
+            ["20", "1.8", "1.3", "0", "0", "0.004", "0.004", "1", "0"],
+            ["14", "2.4", "1.7", "900", "400", "0.09", "0.0011", "1", "0"]]
+    params, seeds = [Params.from_row(r) for r in rows], [11, 12, 13, 14, 15, 16]
+    res = []
+    for mode in (0, 1):
+        b = PandemicBatch(params, seeds)
+        b.set_table_mode(mode)
+        b.setup()
+        b.snapshot()
+        first = b.run()
+        b.restore()
+        again = b.run()         # replayed graphs, from the same state
+        for x, y in zip(first, again):
+            assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+        res.append((first, [[b.array(r, w) for w in range(6)] for r in range(len(rows))]))
+        b.close()
+    for r in range(len(rows)):
+        for k in range(2):
+            assert np.array_equal(res[0][0][r][k], res[1][0][r][k]), r
+        for w in range(6):
+            assert np.array_equal(res[0][1][r][w], res[1][1][r][w]), (r, w)
+        s = PandemicSim(params[r], seeds[r])
+        s.setup_sim()
+        counts, inf = s.run()
+        s.close()
+        assert np.array_equal(res[0][0][r][0], counts) and np.array_equal(res[0][0][r][1], inf), r
