@@ -67,7 +67,7 @@ struct BatchArrays {
     const int32_t* hh_off;
     const int32_t* wp_off;
     const int32_t* wp_people;
-    const uint32_t* wp_of;
+    const AgentRecord* who;
     const int32_t* er_off;
     const int32_t* er_people;
     const uint8_t *st_p, *st_s, *dy_p, *dy_s, *gn_p, *gn_s;
@@ -84,7 +84,7 @@ __device__ __forceinline__ AgentArrays view(const BatchArrays& B, const RepInfo&
     A.wp_people = B.wp_people + ri.abase;
     A.er_off = B.er_off + kb;
     A.er_people = B.er_people;
-    A.wp_of = B.wp_of + ri.abase;
+    A.who = B.who + ri.abase;
     A.er_cnt = nullptr;
     A.er_keys = nullptr;
     A.er_slots = 0;
@@ -288,7 +288,8 @@ __global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restri
             if (can_infect(M, f)) {
                 SuccessDraws draws;
                 success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
-                keep = may_infect<C>(M, f, draws);
+                keep = may_infect<C>(M, f, draws, 1) &&
+                       may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], r, day, WEEKEND));
             }
         }
         list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), r, true);
@@ -309,7 +310,7 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts_counted(DayState*
     constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
     __shared__ PickQueue s_pick;
     if (threadIdx.x == 0)  // first used behind a barrier of the first round
-        s_pick.n = s_pick.errands = s_pick.taken = s_pick.n_claim[0] = s_pick.n_claim[1] = 0;
+        s_pick.reset();
     __syncthreads();
     const ClaimArrays claims{B.st_p, B.st_s, B.wp_people, B.claim_p, B.claim_s, list_p, list_s, g->n_claimed};
     const int64_t stride = (int64_t)gridDim.x * kContactThreads;
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts_counted(DayState*
         const RepInfo ri = reps[r];
         AgentArrays A = view(B, ri, 0u);
         const CountRep cr = T.reps[r];
-        A.er_cnt = count_row(T, cr, cr.C);
+        A.er_cnt = T.total + cr.tbase;
         A.er_keys = T.keys + ri.abase;
         A.er_slots = T.slots;
         int32_t vic[8];
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(kContactThreads) void kb_contacts(DayState* __restr
             q = QueuedInfector{infected[pos] - (int32_t)ri.abase, (int32_t)(pos - inf_start[r]), r};
             success_draws<C>(models[r], st.contact_base + (uint64_t)(6 * (int64_t)q.pos) + 2, draws);
             const Infectivity f = infectivity(models[r], A, q.idx, st.day);
-            return can_infect(models[r], f) && may_infect<C>(models[r], f, draws);
+            return can_infect(models[r], f) && may_infect<C>(models[r], f, draws, 1);
         },
         [&](bool active, const QueuedInfector& q, const SuccessDraws& draws) {
             int32_t vic[8];
@@ -681,7 +682,8 @@ struct pt_batch {
     uint8_t *st_p = nullptr, *st_s = nullptr, *dy_p = nullptr, *dy_s = nullptr, *gn_p = nullptr, *gn_s = nullptr;
     uint8_t *age = nullptr, *hh_types = nullptr, *snap = nullptr;
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
-    uint32_t* wp_of = nullptr;
+    AgentRecord* who = nullptr;
+    int32_t* wp_lone = nullptr;
     uint64_t *claim_p = nullptr, *claim_s = nullptr;
     int32_t *list_p = nullptr, *list_s = nullptr, *infected = nullptr, *staging = nullptr;
     uint32_t *blk_counts = nullptr, *blk_ninf = nullptr, *blk_off = nullptr;
@@ -741,7 +743,8 @@ void free_batch_population(pt_batch* b) {
     dev_free(b->hh_off);
     dev_free(b->wp_off);
     dev_free(b->wp_people);
-    dev_free(b->wp_of);
+    dev_free(b->who);
+    dev_free(b->wp_lone);
     dev_free(b->claim_p);
     dev_free(b->claim_s);
     dev_free(b->list_p);
@@ -804,7 +807,7 @@ BatchArrays batch_arrays(pt_batch* b) {
     B.hh_off = b->hh_off;
     B.wp_off = b->wp_off;
     B.wp_people = b->wp_people;
-    B.wp_of = b->wp_of;
+    B.who = b->who;
     B.er_off = b->er_off;
     B.er_people = b->er_people;
     B.st_p = b->st_p;
@@ -947,9 +950,15 @@ int setup_batch_counts(pt_batch* b) {
             p.reps[r].abase = b->reps[r].abase;
         }
         p.build(N, w ? 3 : 2, b->cus);
-        if (p.upload(b->stream)) return PT_ENOMEM;
     }
-    if (b->count_scratch.alloc(b->count_plan[0], b->count_plan[1])) return PT_ENOMEM;
+    if (b->count_plan[0].upload(b->stream) || b->count_plan[1].upload(b->stream) ||
+        b->count_scratch.alloc(b->count_plan[0], b->count_plan[1], 0)) {
+        // no memory for the matrices: sorted tables
+        (void)hipGetLastError();
+        for (CountPlan& p : b->count_plan) p.release();
+        b->count_scratch.release();
+        return PT_OK;
+    }
     const int64_t P = b->P;
     for (int w = 0; w < 2; ++w) {
         const CountPlan& p = b->count_plan[w];
@@ -971,6 +980,7 @@ int setup_batch_counts(pt_batch* b) {
         t.sv_pos = b->stage_ids + 2 * P;
         t.sv_f = b->sel_keys + 2 * P;
         t.sv_r = b->sel_ids + 2 * P;
+        t.wp_lone = b->wp_lone;
         HIP_TRY(set_count_lds(p));
     }
     return PT_OK;
@@ -1141,7 +1151,7 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
     if (dev_alloc(&b->tile_rep, tiles) || dev_alloc(&b->st_p, P) || dev_alloc(&b->st_s, P) ||
         dev_alloc(&b->dy_p, P) || dev_alloc(&b->dy_s, P) || dev_alloc(&b->gn_p, P) || dev_alloc(&b->gn_s, P) ||
         dev_alloc(&b->age, P) || dev_alloc(&b->snap, 6 * P) || dev_alloc(&b->household, P) ||
-        dev_alloc(&b->hh_off, HH) || dev_alloc(&b->wp_off, WW) || dev_alloc(&b->wp_people, P) || dev_alloc(&b->wp_of, P) ||
+        dev_alloc(&b->hh_off, HH) || dev_alloc(&b->wp_off, WW) || dev_alloc(&b->wp_people, P) || dev_alloc(&b->who, P) || dev_alloc(&b->wp_lone, R) ||
         dev_alloc(&b->claim_p, P) || dev_alloc(&b->claim_s, P) || dev_alloc(&b->list_p, P) ||
         dev_alloc(&b->list_s, P) || dev_alloc(&b->infected, P) || dev_alloc(&b->staging, P) ||
         dev_alloc(&b->blk_counts, (int64_t)tiles * 16) || dev_alloc(&b->blk_ninf, tiles) ||
@@ -1229,7 +1239,7 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
         const RepInfo& ri = b->reps[r];
         const int64_t a = ri.abase;
         const PopArrays Pa{b->hh_types + ri.hbase, b->hh_off + ri.hbase, b->household + a, b->age + a,
-                           b->wp_off + ri.wbase, b->wp_people + a, b->wp_of + a, b->st_p + a, b->st_s + a, b->dy_p + a, b->dy_s + a,
+                           b->wp_off + ri.wbase, b->wp_people + a, b->who + a, b->wp_lone + r, b->st_p + a, b->st_s + a, b->dy_p + a, b->dy_s + a,
                            b->gn_p + a, b->gn_s + a, b->claim_p + a, b->claim_s + a};
         hipError_t e = build_population(b->d_models + r, ri.N, ri.H, ri.W, Pa, b->sel_keys, b->tables,
                                         ri.workplace_off, st);

@@ -10,9 +10,10 @@
 //   k_count       a block per chunk of consecutive agents draws their
 //                 errands, counts them per bucket in LDS and writes the
 //                 counts (one matrix row per chunk) and the 2-byte keys
-//   k_count_scan  per bucket, the exclusive prefix over the chunks (in
-//                 place) and the total: pre[c][b] people of bucket b lie in
-//                 chunks before c
+//   k_count_scan  per bucket, the exclusive prefix over the chunks and the
+//                 total: pre[b][c] people of bucket b lie in chunks before
+//                 c.  Transposed, so that a rank's chunk is found within one
+//                 or two cache lines of its bucket
 //   test          the day's infectors whose success draws cannot all fail
 //                 (may_infect) go to a list
 //   contacts      of the listed infectors, with the totals; a successful
@@ -26,8 +27,16 @@
 // A chunk's list order does not matter (ranks are taken by value), so the
 // result is the id the sorted table holds at that position.
 //
-// Used for layouts of at most kCountMaxK buckets (32-bit counters in one
-// CU's 160 KB LDS).
+// Layouts of at most kCountMaxK buckets count in one block per chunk (32-bit
+// counters in one CU's 160 KB LDS).  Larger ones are split into column
+// groups (an hour, or kCountMaxK locations of one): k_keys_* write the keys
+// by hour first, then k_count_group counts (chunk, group) from them, and
+// k_collect_group lists; the rest is shared.
+//
+// Against the sorted tables: 2.35M agents x 100 days 20.7 -> 9.8 ms, 50M x
+// 100 days (split) 148 -> 82 ms, 24M with 10x the locations (split, few
+// infected, so only queried buckets were sorted) 35 -> 32 ms, 48 replicates
+// of 2.35M 260 -> 90 ms.
 //
 // Citations are relative to PandemicThrust/PandemicThrust/ of the reference.
 #pragma once
@@ -44,16 +53,23 @@ namespace pt {
 constexpr int kCountMaxK = 40000;       // 32-bit counters: 160,000 of the 163,840 bytes of LDS
 constexpr uint32_t kNoKey = 0xFFFFu;    // no pair (weekday hour 1 of a child)
 constexpr int kCountMinChunk = 1024;    // agents
+constexpr int kCountMaxRanges = 8;      // groups per hour: passes over its keys
+constexpr int kCountMaxHour = (1 << 20) - 1;  // locations per hour (20 bits beside 12 of the id; no pair is all ones)
 constexpr int kCountMaxLen = 64;        // people per bucket of a smallest chunk (CountPlan::build)
 constexpr int64_t kCountSmall = 1000000;  // agents up to which the lists' length does not matter
 
 // One simulation's counted table in one layout (weekday or weekend).
 struct CountRep {
     int64_t abase;  // first agent slot
-    int64_t mbase;  // first entry of its (C + 1) x K matrix (row C: totals)
+    int64_t mbase;  // first entry of its matrices: C x K counts, K x (C + 1) prefixes
+    int64_t tbase;  // first of its K totals
     int64_t qbase;  // first word of its C x qw mark words
     int32_t K, C, A, qw;  // buckets, chunks, agents per chunk, mark words per chunk
     int32_t chunk0; // first chunk (k_count block)
+    // Column groups: buckets [0, E) are the first hour's, the next E (weekday:
+    // the rest) the second's ...; `ranges` groups of W buckets per hour, G in
+    // all (1: not split).
+    int32_t E, W, ranges, G;
     int32_t pad;
 };
 
@@ -86,19 +102,24 @@ struct CountTable {
     const CountRep* reps;
     const CountBlock* chunks;
     const CountBlock* scans;
-    uint16_t* keys;        // keys per agent x slots
+    uint16_t* keys;        // keys per agent x slots (split weekday layouts: within the hour)
     int64_t slots;
-    uint32_t* pre;         // the matrices
-    uint32_t* cursor;      // same shape: list positions of marked (chunk, bucket)
+    uint32_t* keys32;      // the same for hours of over 65,535 locations, or the weekend's hour lists
+    uint16_t* tile_off;    // hour lists: where each tile's hours begin
+    uint32_t* cnt;         // the count matrices; then, per marked (chunk, bucket), its list's position
+    uint32_t* pre;         // the prefixes
+    uint32_t* total;       // people per bucket
     uint32_t* marks;       // mark words
     int64_t mark_words;
-    int32_t* chunk_day;    // day + 1 on which the chunk was last marked
+    int32_t* chunk_day;    // day + 1 on which the (chunk, group) was last marked
     int32_t* list;         // ids of the marked buckets, kpa * agents per chunk
-    uint32_t* n;           // [0] picks queued, [1] infectors listed
+    uint32_t* n;           // [0] picks queued, [1] infectors listed, [2] list entries (split layouts)
     // Listed infectors: agent, position, pack_infectivity, simulation (batch).
     int32_t *sv_idx, *sv_pos;
     uint32_t* sv_f;
     int32_t* sv_r;
+    int32_t* lone_day;       // per simulation: day + 1 on which some bucket had a single person
+    const int32_t* wp_lone;  // per simulation: some workplace has
     uint32_t *pk_bucket, *pk_want, *pk_claim, *pk_payload;  // queued picks: rank `want` of
     int32_t *pk_idx, *pk_r, *pk_chunk, *pk_len;             // the len ids of (chunk, bucket)
 };
@@ -108,38 +129,37 @@ __host__ __device__ inline ClaimArrays claim_arrays(const AgentArrays& A, int32_
     return ClaimArrays{A.st_p, A.st_s, A.wp_people, A.claim_p, A.claim_s, list_p, list_s, n_claimed};
 }
 
-// LDS queue of a contact block's successful draws.  A round of two slots
-// adds at most 2 per thread; the queue is emptied when the next round might
-// not fit, and after the last one.
-constexpr int kPickRound = 2 * kContactThreads;
-constexpr int kPickQueue = kPickRound + kContactThreads;
+// LDS queue of a contact block's successful draws: three per infector, or the
+// two a turn of two slots can add (queue_contacts).
+constexpr int kPickQueue = 3 * kContactThreads;
 struct PickQueue {
-    uint32_t n, errands, taken, base;
+    uint32_t n, errands, taken, base, sum, list, list_base;
     uint32_t n_claim[2], claim_base[2];
     Pick at[kPickQueue];
     int32_t claimed[2][kPickQueue];
+    __device__ __forceinline__ void reset() { n = errands = taken = list = n_claim[0] = n_claim[1] = 0; }
 };
 
-// A matrix row (row C: people per bucket).
-__device__ __forceinline__ uint32_t* count_row(const CountTable& T, const CountRep& c, int row) {
-    return T.pre + c.mbase + (int64_t)row * c.K;
+// Prefixes of bucket b.
+__device__ __forceinline__ const uint32_t* count_column(const CountTable& T, const CountRep& c, uint32_t b) {
+    return T.pre + c.mbase + (int64_t)b * (c.C + 1);
 }
 
 // The chunk holding rank j of bucket b: the last c with pre[c][b] <= j
 // (chunks without people of b share their successor's prefix).  People are
 // spread evenly over the chunks, so the chunk is within C / (2 sqrt(total))
-// (1 to 2) of j C / total: eight prefixes around it in one round trip nearly
-// always hold it, else the window moves on.
+// (1 to 2) of j C / total: the eight prefixes around it nearly always hold
+// it, else the window moves on.
 __device__ __forceinline__ int chunk_of(const CountTable& T, const CountRep& c, uint32_t b, uint32_t j, uint32_t total,
                                         uint32_t& before, uint32_t& len) {
     constexpr int W = 8;
-    const uint32_t* col = T.pre + c.mbase + b;
+    const uint32_t* col = count_column(T, c, b);
     int w = (int)((float)j * (float)c.C / (float)total) - W / 2 + 1;
     for (;;) {
         w = max(0, min(w, c.C - W + 1));  // rows w .. w + W - 1 of the C + 1 (row C: the total)
         uint32_t p[W];
 #pragma unroll
-        for (int i = 0; i < W; ++i) p[i] = col[(int64_t)min(w + i, c.C) * c.K];
+        for (int i = 0; i < W; ++i) p[i] = col[min(w + i, c.C)];
         if (w > 0 && j < p[0]) {
             w -= W - 1;
             continue;
@@ -165,22 +185,55 @@ __device__ __forceinline__ int chunk_of(const CountTable& T, const CountRep& c, 
     }
 }
 
-// Marks (chunk, bucket) for collection.
-__device__ __forceinline__ void mark_chunk(const CountTable& T, const CountRep& c, int chunk, uint32_t b,
+// Marks (chunk, bucket) for collection; true for its first mark of the day.
+// (Only split layouts use the answer: without it nothing waits.)
+__device__ __forceinline__ bool mark_chunk(const CountTable& T, const CountRep& c, int chunk, uint32_t b,
                                            int32_t stamp) {
-    atomicOr(T.marks + c.qbase + (int64_t)chunk * c.qw + (b >> 5), 1u << (b & 31));
-    T.chunk_day[c.chunk0 + chunk] = stamp;
+    const uint32_t bit = 1u << (b & 31);
+    uint32_t* word = T.marks + c.qbase + (int64_t)chunk * c.qw + (b >> 5);
+    bool first = false;
+    if (c.G > 1)
+        first = !(atomicOr(word, bit) & bit);
+    else
+        atomicOr(word, bit);
+    int g = 0;
+    if (c.G > 1) {
+        const uint32_t hour = c.G == 2 * c.ranges ? (b >= (uint32_t)c.E ? 1u : 0u) : b / (uint32_t)c.E;
+        g = (int)(hour * c.ranges + (b - hour * c.E) / (uint32_t)c.W);
+    }
+    // (Stores to these few lines from every CU would queue up: look first.)
+    int32_t* day = T.chunk_day + c.chunk0 + chunk * c.G + g;
+    if (*day != stamp) *day = stamp;
+    return first;
 }
+
+// Where a pick's first marks go (split layouts; n of them).
+struct NewLists {
+    int n;
+    int64_t at[2];     // entries of the count matrix
+    uint32_t len[2];
+};
 
 // A queued pick: finds and marks its chunk (and the next rank's, should the
 // infector itself sit at this rank: only possible in its own chunk) and
-// appends the pick to the day's list.
-__device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, uint32_t i, int day) {
+// stores the pick as the day's i-th.
+__device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, uint32_t i, int day, NewLists& lists) {
     const CountRep c = T.reps[p.r];
-    const uint32_t total = count_row(T, c, c.C)[p.at];
+    const uint32_t total = T.total[c.tbase + p.at];
     uint32_t before, len;
     const int chunk = chunk_of(T, c, p.at, p.rank, total, before, len);
-    mark_chunk(T, c, chunk, p.at, day + 1);
+    auto mark = [&](int k) {
+        if (!mark_chunk(T, c, k, p.at, day + 1)) return;
+        if (lists.n == 0) {
+            lists.at[0] = c.mbase + (int64_t)k * c.K + p.at;
+            lists.len[0] = len;
+        } else {
+            lists.at[1] = c.mbase + (int64_t)k * c.K + p.at;
+            lists.len[1] = len;
+        }
+        ++lists.n;
+    };
+    mark(chunk);
     T.pk_bucket[i] = p.at;
     T.pk_want[i] = p.rank - before;
     T.pk_claim[i] = p.claim;
@@ -191,10 +244,7 @@ __device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, 
     T.pk_len[i] = (int32_t)len;
     if (chunk == p.idx / c.A) {
         const uint32_t next = p.rank + 1 == total ? 0u : p.rank + 1;
-        if (next < before || next >= before + len) {
-            const int c2 = chunk_of(T, c, p.at, next, total, before, len);
-            mark_chunk(T, c, c2, p.at, day + 1);
-        }
+        if (next < before || next >= before + len) mark(chunk_of(T, c, p.at, next, total, before, len));
     }
 }
 
@@ -244,15 +294,22 @@ __device__ __forceinline__ void flush_picks(const CountTable& T, const ClaimArra
     const uint32_t n = q.n;
     if (tid == 0 && q.errands) q.base = atomicAdd(T.n, q.errands);
     __syncthreads();
-    for (uint32_t i0 = 0; i0 < n; i0 += blockDim.x) {
-        const uint32_t i = i0 + tid;
+    constexpr int kTurns = kPickQueue / kContactThreads;
+    NewLists lists[kTurns];
+    uint32_t list_at[kTurns];
+#pragma unroll
+    for (int t = 0; t < kTurns; ++t) {
+        const uint32_t i = (uint32_t)(t * kContactThreads + tid);
         bool newp = false, news = false;
         int64_t slot = 0;
+        lists[t].n = 0;
         if (i < n) {
             const Pick p = q.at[i];
             const uint32_t kind = p.payload >> 26;
             if (kind == 0) {
-                locate_pick(T, p, q.base + atomicAdd(&q.taken, 1u), sts[p.r].day);
+                locate_pick(T, p, q.base + atomicAdd(&q.taken, 1u), sts[p.r].day, lists[t]);
+                if (lists[t].n)
+                    list_at[t] = atomicAdd(&q.list, lists[t].len[0] + (lists[t].n > 1 ? lists[t].len[1] : 0u));
             } else {
                 const int64_t a = T.reps[p.r].abase;
                 int32_t v = (int32_t)p.at;
@@ -277,14 +334,23 @@ __device__ __forceinline__ void flush_picks(const CountTable& T, const ClaimArra
     }
     __syncthreads();
     if (tid < 2 && q.n_claim[tid]) q.claim_base[tid] = atomicAdd(&C.n_claimed[tid], q.n_claim[tid]);
+    if (tid == 2 && q.list) q.list_base = atomicAdd(&T.n[2], q.list);
     __syncthreads();
+#pragma unroll
+    for (int t = 0; t < kTurns; ++t) {
+        if (lists[t].n) {
+            const uint32_t start = q.list_base + list_at[t];
+            T.cnt[lists[t].at[0]] = start;
+            if (lists[t].n > 1) T.cnt[lists[t].at[1]] = start + lists[t].len[0];
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         int32_t* list = k ? C.list_s : C.list_p;
         for (uint32_t i = tid; i < q.n_claim[k]; i += blockDim.x) list[q.claim_base[k] + i] = q.claimed[k][i];
     }
     __syncthreads();
-    if (tid == 0) q.n = q.errands = q.taken = q.n_claim[0] = q.n_claim[1] = 0;
+    if (tid == 0) q.reset();
     __syncthreads();
 }
 
@@ -311,11 +377,18 @@ struct PickPush {
         }
         q->at[atomicAdd(&q->n, 1u)] = Pick{at, rank, idx, r, claim, payload | (kind << 26)};
     }
-    __device__ __forceinline__ void round(bool last) const {
+    // Whether the block's successes (mine: this thread's) fit the queue.
+    __device__ __forceinline__ bool fits(uint32_t mine) const {
+        const uint32_t sum = wave_sum(mine);
+        if (threadIdx.x == 0) q->sum = 0;
         __syncthreads();
-        const uint32_t n = q->n;
-        if (n && (last || n > (uint32_t)(kPickQueue - kPickRound))) flush_picks(T, C, *q, sts);
+        if ((threadIdx.x & 63) == 0 && sum) atomicAdd(&q->sum, sum);
         __syncthreads();
+        return q->sum <= (uint32_t)kPickQueue;
+    }
+    __device__ __forceinline__ void flush() const {
+        __syncthreads();
+        if (q->n) flush_picks(T, C, *q, sts);
     }
 };
 
@@ -336,6 +409,8 @@ __global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done
     const CountRep c = T.reps[blk.r];
     const int tid = threadIdx.x, nt = blockDim.x;
     const uint32_t K = (uint32_t)c.K;
+    __shared__ __align__(16) WalkRow s_row[kWalkRows];
+    const LdsWalk wk = load_walk(WEEKEND ? M.we_table : M.wd_table, s_row);
     for (int i = tid; i < c.K; i += nt) s_cnt[i] = 0;
     __syncthreads();
     const int64_t N = M.N;
@@ -349,7 +424,6 @@ __global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done
             bad = true;
     };
     if (WEEKEND) {
-        const ErrandWalk wk = pinned(M.we_walk);
         const int base = M.we_base, E = M.we_E;
         uint16_t* out = T.keys + c.abase;
         for (int64_t p = a0 + tid; p < a1; p += nt) {
@@ -363,7 +437,6 @@ __global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done
             }
         }
     } else {
-        const ErrandWalk wk = pinned(M.wd_walk);
         const int base = M.wd_base, base1 = M.wd_base1 - M.wd_E;  // hour-1 keys follow the wd_E hour-0 keys
         const uint8_t* age = ages + c.abase;
         uint32_t* out0 = reinterpret_cast<uint32_t*>(T.keys + c.abase);
@@ -395,38 +468,46 @@ __global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done
     }
     if (bad) st->fault = 1;
     __syncthreads();
-    uint32_t* row = T.pre + c.mbase + (int64_t)blk.at * c.K;
+    uint32_t* row = T.cnt + c.mbase + (int64_t)blk.at * c.K;
     for (int i = tid; i < c.K; i += nt) row[i] = s_cnt[i];
 }
 
-// Column prefixes of the count matrices, 64 buckets per block: 16 row groups
-// sum up to 16 rows each in registers, so 256 rows take one round trip.
-// Also clears the day's marks, picks and lists.
-constexpr int kScanCols = 64, kScanGroups = 16, kScanRows = 16;
-__global__ __launch_bounds__(kScanCols* kScanGroups) void k_count_scan(const int32_t* __restrict__ done,
+// Column prefixes of the count matrices, kScanCols buckets per block of 1024
+// threads: the row groups sum up to 8 rows each in registers, and the
+// prefixes go out through LDS as runs of consecutive chunks.  The fewer
+// chunks, the more buckets per block (CountPlan::scan_cols).  Also clears the
+// day's marks, picks and lists.
+constexpr int kCountScanThreads = 1024, kScanRows = 8;
+template <int kScanCols>
+__global__ __launch_bounds__(kCountScanThreads) void k_count_scan(const int32_t* __restrict__ done,
                                                                        const DayState* __restrict__ sts,
                                                                        CountTable T) {
     if (*done) return;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < T.mark_words;
          i += (int64_t)gridDim.x * blockDim.x)
         T.marks[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < 2) T.n[threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x < 3) T.n[threadIdx.x] = 0u;
     const CountBlock blk = T.scans[blockIdx.x];
     if (sts[blk.r].done) return;
     const CountRep c = T.reps[blk.r];
+    constexpr int kScanGroups = kCountScanThreads / kScanCols;
+    constexpr int RT = kScanGroups * kScanRows;  // rows per turn
     __shared__ uint32_t s_sum[kScanGroups][kScanCols];
+    __shared__ uint32_t s_pre[kScanCols][RT + 1];
     const int col = threadIdx.x % kScanCols, grp = threadIdx.x / kScanCols;
     const int b = blk.at + col;
-    uint32_t* m = T.pre + c.mbase + b;
+    const uint32_t* m = T.cnt + c.mbase + b;
+    uint32_t* out = T.pre + c.mbase + (int64_t)blk.at * (c.C + 1);
+    const int cols = min(kScanCols, c.K - blk.at);
     uint32_t carry = 0;
-    for (int s0 = 0; s0 < c.C; s0 += kScanGroups * kScanRows) {
-        const int rows = min(c.C - s0, kScanGroups * kScanRows);
+    for (int s0 = 0; s0 < c.C; s0 += RT) {
+        const int rows = min(c.C - s0, RT);
         const int per = (rows + kScanGroups - 1) / kScanGroups;
-        const int r0 = s0 + grp * per, r1 = min(s0 + rows, r0 + per);
+        const int r0 = grp * per, r1 = min(rows, r0 + per);
         uint32_t v[kScanRows], sum = 0;
 #pragma unroll
         for (int i = 0; i < kScanRows; ++i) {
-            v[i] = r0 + i < r1 && b < c.K ? m[(int64_t)(r0 + i) * c.K] : 0u;
+            v[i] = r0 + i < r1 && col < cols ? m[(int64_t)(s0 + r0 + i) * c.K] : 0u;
             sum += v[i];
         }
         s_sum[grp][col] = sum;
@@ -438,14 +519,36 @@ __global__ __launch_bounds__(kScanCols* kScanGroups) void k_count_scan(const int
             if (g < grp) run += x;
             carry += x;
         }
-        __syncthreads();
 #pragma unroll
         for (int i = 0; i < kScanRows; ++i) {
-            if (r0 + i < r1 && b < c.K) m[(int64_t)(r0 + i) * c.K] = run;
+            if (r0 + i < r1) s_pre[col][r0 + i] = run;
             run += v[i];
         }
+        __syncthreads();
+        const bool last = s0 + RT >= c.C;
+        if (last && grp == 0) s_pre[col][rows] = carry;
+        __syncthreads();
+        const int len = rows + (last ? 1 : 0);  // the total ends the row
+        for (int i = threadIdx.x; i < cols * len; i += kCountScanThreads) {
+            const int q = i / len, k = i % len;
+            out[(int64_t)q * (c.C + 1) + s0 + k] = s_pre[q][k];
+        }
+        __syncthreads();
     }
-    if (grp == 0 && b < c.K) m[(int64_t)c.C * c.K] = carry;
+    if (grp == 0 && col < cols) {
+        T.total[c.tbase + b] = carry;
+        if (carry == 1) T.lone_day[blk.r] = sts[blk.r].day + 1;
+    }
+}
+
+// Least contact count of an infector (may_infect): its household, its
+// workplace unless some workplace has one person only, and its two errands
+// (every errand profile has two) unless some bucket of the day has.
+__device__ __forceinline__ int least_contacts(const CountTable& T, AgentRecord a, int r, int day, bool weekend) {
+    int k = record_household_size(a) > 1 ? 3 : 0;
+    if (!weekend && !T.wp_lone[r]) k += record_workplace_contacts(a);
+    if (T.lone_day[r] != day + 1) k += 2;
+    return max(k, 1);
 }
 
 // Lists the ids of the chunk's marked buckets: reserves each bucket's part of
@@ -468,8 +571,7 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
     const int tid = threadIdx.x, nt = blockDim.x;
     const uint32_t* marks = T.marks + c.qbase + (int64_t)blk.at * c.qw;
     const int64_t a0 = (int64_t)blk.at * c.A, a1 = min((int64_t)models[blk.r].N, a0 + c.A);
-    uint32_t* start = T.cursor + c.mbase + (int64_t)blk.at * c.K;
-    const uint32_t* row = count_row(T, c, blk.at);
+    uint32_t* start = T.cnt + c.mbase + (int64_t)blk.at * c.K;  // (the prefixes hold the counts now)
     if (tid == 0) s_top = (uint32_t)(KPA * (c.abase + a0));
     for (int i = tid; i < c.K; i += nt) s_cur[i] = ~0u;
     __syncthreads();
@@ -478,7 +580,7 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
         while (w) {
             const int b = i * 32 + __ffs(w) - 1;
             w &= w - 1;
-            start[b] = s_cur[b] = atomicAdd(&s_top, row[c.K + b] - row[b]);
+            start[b] = s_cur[b] = atomicAdd(&s_top, start[b]);
         }
     }
     __syncthreads();
@@ -497,6 +599,293 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
             }
         }
     }
+}
+
+// ---- split layouts (more than kCountMaxK buckets; one simulation) ----
+
+constexpr int kTileAgents = 4096;  // weekend hour lists: agents per tile, ids within it 12 bits
+constexpr int kTileBits = 12;
+constexpr int kTileThreads = 512;
+constexpr int kTileHours = 16;     // tile_off entries per tile (11 used)
+
+// Weekday keys by hour, a pair of agents per thread and turn.  VALU bound: 50M
+// agents 160 us, of which the draws 99; the walk rows in LDS (load_walk) took
+// it from 184.
+template <class KT>
+__global__ __launch_bounds__(256) void k_keys_weekday(DayState* __restrict__ st, const Model* __restrict__ Mp,
+                                                      const uint8_t* __restrict__ age, CountTable T) {
+    if (st->done) return;
+    const Model& M = *Mp;
+    const int64_t N = M.N;
+    __shared__ __align__(16) WalkRow s_row[kWalkRows];
+    const LdsWalk wk = load_walk(M.wd_table, s_row);
+    __syncthreads();
+    const int base = M.wd_base, base1 = M.wd_base1;
+    const uint64_t eoff = st->rand_offset;
+    KT* keys = sizeof(KT) == 2 ? reinterpret_cast<KT*>(T.keys) : reinterpret_cast<KT*>(T.keys32);
+    bool bad = false;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; 2 * g < N; g += stride) {
+        const U4 u = draw4(eoff + (uint64_t)g, M.key0, M.key1);
+        KT k0[2], k1[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int64_t p = 2 * g + k;
+            const bool adult = p < N && age[p] == kAgeAdult;
+            int32_t d1, d2;
+            weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
+            bad |= (uint32_t)(d1 - base) >= (uint32_t)M.wd_E;
+            k0[k] = (KT)(d1 - base);
+            k1[k] = adult ? (KT)(d2 - base1) : (KT)~0u;
+        }
+        // (slots is a multiple of 8: the pair's store stays inside the plane)
+        struct alignas(2 * sizeof(KT)) Two {
+            KT a, b;
+        };
+        reinterpret_cast<Two*>(keys)[g] = Two{k0[0], k0[1]};
+        reinterpret_cast<Two*>(keys + T.slots)[g] = Two{k1[0], k1[1]};
+    }
+    if (bad) st->fault = 1;
+}
+
+// Weekend pairs by hour: a block draws a tile's errands and writes them
+// grouped by hour (location << kTileBits | id within the tile), staged in
+// LDS so that the stores are contiguous.  VALU bound like k_count; the rank
+// of a pair within its hour is a returning LDS add, its order is free.  50M
+// agents 545 us, of which the draws 395.
+__global__ __launch_bounds__(kTileThreads) void k_keys_weekend(DayState* __restrict__ st,
+                                                               const Model* __restrict__ Mp, CountTable T) {
+    if (st->done) return;
+    constexpr int PER = kTileAgents / kTileThreads;
+    __shared__ uint32_t s_stage[3 * kTileAgents];
+    __shared__ uint32_t s_cnt[kTileHours], s_base[kTileHours];
+    const Model& M = *Mp;
+    const int tid = threadIdx.x;
+    const int64_t t0 = (int64_t)blockIdx.x * kTileAgents;
+    __shared__ __align__(16) WalkRow s_row[kWalkRows];
+    const LdsWalk wk = load_walk(M.we_table, s_row);
+    if (tid < kTileHours) s_cnt[tid] = 0;
+    __syncthreads();
+    const uint64_t eoff = st->rand_offset;
+    uint32_t pair[3 * PER], at[3 * PER];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int id = i * kTileThreads + tid;
+        const int64_t p = t0 + id;
+        int32_t hour[3], loc[3];
+        if (p < M.N) weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            at[3 * i + e] = ~0u;
+            if (p < M.N) {
+                const uint32_t l = (uint32_t)(loc[e] - M.we_base);
+                bad |= l >= (uint32_t)M.we_E;
+                pair[3 * i + e] = (l << kTileBits) | (uint32_t)id;
+                at[3 * i + e] = ((uint32_t)hour[e] << 16) | atomicAdd(&s_cnt[hour[e]], 1u);
+            }
+        }
+    }
+    if (bad) st->fault = 1;
+    __syncthreads();
+    if (tid < kTileHours) {
+        uint32_t b = 0;
+        for (int h = 0; h < tid; ++h) b += s_cnt[h];
+        s_base[tid] = b;
+        T.tile_off[(int64_t)blockIdx.x * kTileHours + tid] = (uint16_t)b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3 * PER; ++i)
+        if (at[i] != ~0u) s_stage[s_base[at[i] >> 16] + (at[i] & 0xFFFFu)] = pair[i];
+    __syncthreads();
+    const int n = 3 * (int)min((int64_t)kTileAgents, (int64_t)M.N - t0);
+    uint32_t* out = T.keys32 + 3 * t0;
+    for (int i = tid; i < n; i += kTileThreads) out[i] = s_stage[i];
+}
+
+// Calls f(location within the hour, agent) for every pair of the (chunk,
+// group)'s hour in part `part` of `parts`; out-of-group locations included.
+template <bool WEEKEND, class KT, class F>
+__device__ __forceinline__ void group_pairs(const CountTable& T, const CountRep& c, int64_t N, int chunk, int hour,
+                                            int part, int parts, F f) {
+    const int64_t a0 = (int64_t)chunk * c.A, a1 = min(N, a0 + c.A);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    if (WEEKEND) {
+        // A wave per tile.
+        const int lane = tid & 63, waves = nt >> 6;
+        const int t1 = (int)((a1 + kTileAgents - 1) / kTileAgents);
+        for (int t = (int)(a0 / kTileAgents) + part * waves + (tid >> 6); t < t1; t += parts * waves) {
+            const uint16_t* o = T.tile_off + (int64_t)t * kTileHours + hour;
+            const int b = o[0], e = o[1];
+            const uint32_t* src = T.keys32 + (int64_t)t * 3 * kTileAgents;
+            constexpr int U = 8;
+            for (int i0 = b; i0 < e; i0 += U * 64) {
+                uint32_t v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int i = i0 + u * 64 + lane;
+                    v[u] = i < e ? src[i] : ~0u;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (v[u] != ~0u)
+                        f(v[u] >> kTileBits, t * kTileAgents + (int)(v[u] & ((1u << kTileBits) - 1u)));
+            }
+        }
+    } else {
+        constexpr int V = 16 / sizeof(KT);
+        const KT* keys = (sizeof(KT) == 2 ? reinterpret_cast<const KT*>(T.keys) : reinterpret_cast<const KT*>(T.keys32)) +
+                         hour * T.slots;
+        constexpr int U = 4;
+        for (int64_t g0 = a0 / V + (int64_t)part * U * nt + tid; g0 * V < a1; g0 += (int64_t)parts * U * nt) {
+            uint4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t g = g0 + (int64_t)u * nt;
+                v[u] = g * V < a1 ? reinterpret_cast<const uint4*>(keys)[g] : make_uint4(~0u, ~0u, ~0u, ~0u);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t p0 = (g0 + (int64_t)u * nt) * V;
+                const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int k = 0; k < V; ++k) {
+                    const uint32_t key = sizeof(KT) == 2 ? (w[k / 2] >> (16 * (k % 2))) & 0xFFFFu : w[k];
+                    if (key != (uint32_t)(KT)~0u && p0 + k < a1) f(key, (int)(p0 + k));
+                }
+            }
+        }
+    }
+}
+
+// Group g of chunk: its hour, first location there, locations, and first
+// bucket.
+struct GroupColumns {
+    int hour, lo, n, bucket;
+};
+__device__ __forceinline__ GroupColumns group_columns(const CountRep& c, int g) {
+    GroupColumns q;
+    q.hour = g / c.ranges;
+    q.lo = (g % c.ranges) * c.W;
+    q.bucket = q.hour * c.E + q.lo;
+    // an hour ends where the next begins, the last at K
+    const int end = q.hour == c.G / c.ranges - 1 ? c.K : (q.hour + 1) * c.E;
+    q.n = max(0, min(c.W, end - q.bucket));
+    return q;
+}
+
+// All groups of an hour.
+__device__ __forceinline__ GroupColumns hour_columns(const CountRep& c, int hour) {
+    const GroupColumns last = group_columns(c, hour * c.ranges + c.ranges - 1);
+    return GroupColumns{hour, 0, last.lo + last.n, hour * c.E};
+}
+
+// Counts of a (chunk, group).  Reads the hour's keys (16 bytes per lane and
+// load) once per group of the hour; LDS adds hide behind them: 50M agents, 40
+// us per weekday (5 TB/s), 163 us per weekend day (3.7 TB/s).
+template <bool WEEKEND, class KT>
+__global__ __launch_bounds__(1024) void k_count_group(const DayState* __restrict__ st, const Model* __restrict__ Mp,
+                                                      CountTable T) {
+    if (st->done) return;
+    extern __shared__ uint32_t s_cnt[];
+    const CountRep c = T.reps[0];
+    const int chunk = blockIdx.x / c.G;
+    const GroupColumns q = group_columns(c, blockIdx.x % c.G);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    for (int i = tid; i < q.n; i += nt) s_cnt[i] = 0;
+    __syncthreads();
+    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, 0, 1, [&](uint32_t l, int) {
+        const uint32_t i = l - (uint32_t)q.lo;
+        if (i < (uint32_t)q.n) atomicAdd(&s_cnt[i], 1u);
+    });
+    __syncthreads();
+    uint32_t* row = T.cnt + c.mbase + (int64_t)chunk * c.K + q.bucket;
+    for (int i = tid; i < q.n; i += nt) row[i] = s_cnt[i];
+}
+
+// Lists of a (chunk, group)'s marked buckets, reserved with their first marks
+// (the count matrix holds each list's start, and its end once collected).
+// Up to kFewMarks marks per group of an hour, kCollectParts small blocks share
+// the hour's keys and append with atomics on the matrix; above, a block per
+// group appends with LDS counters.  Both are bound by reading the hour's keys:
+// 50M agents, a weekday with few marks 29 us (7 TB/s, one block per group 109
+// us), with many 65 us; 8 parts of 256 threads: the same on weekdays, 155 us
+// instead of 98-140 on weekends of up to 96 marks.
+constexpr uint32_t kFewMarks = 96;
+constexpr int kCollectParts = 16, kCollectFewThreads = 512;
+
+// Marked buckets of the group, by the whole block; f(bucket) for each.
+template <class F>
+__device__ __forceinline__ void for_marked(const uint32_t* __restrict__ marks, const GroupColumns& q, F f) {
+    for (int i = q.bucket / 32 + threadIdx.x; i * 32 < q.bucket + q.n; i += blockDim.x) {
+        uint32_t w = marks[i];
+        while (w) {
+            const int b = i * 32 + __ffs(w) - 1;
+            w &= w - 1;
+            if (b >= q.bucket && b < q.bucket + q.n) f(b);
+        }
+    }
+}
+
+template <bool WEEKEND, class KT>
+__global__ __launch_bounds__(kCollectFewThreads) void k_collect_few(const DayState* __restrict__ st,
+                                                                    const Model* __restrict__ Mp, CountTable T) {
+    if (st->done) return;
+    const CountRep c = T.reps[0];
+    // (chunk, hour): the hour's groups share one pass over its keys
+    const int ch = blockIdx.x / kCollectParts, part = blockIdx.x % kCollectParts;
+    bool any = false;
+    for (int g = 0; g < c.ranges; ++g) any |= T.chunk_day[ch * c.ranges + g] == st->day + 1;
+    if (!any) return;
+    extern __shared__ uint32_t s_bits[];
+    __shared__ uint32_t s_n;
+    const int hours = c.G / c.ranges, chunk = ch / hours, tid = threadIdx.x;
+    const GroupColumns q = hour_columns(c, ch % hours);
+    for (int i = tid; i < (q.n + 31) / 32; i += blockDim.x) s_bits[i] = 0;
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+    for_marked(T.marks + c.qbase + (int64_t)chunk * c.qw, q, [&](int b) {
+        atomicAdd(&s_n, 1u);
+        atomicOr(&s_bits[(b - q.bucket) >> 5], 1u << ((b - q.bucket) & 31));
+    });
+    __syncthreads();
+    if (s_n > kFewMarks * (uint32_t)c.ranges) return;
+    uint32_t* cursor = T.cnt + c.mbase + (int64_t)chunk * c.K + q.bucket;
+    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, part, kCollectParts, [&](uint32_t l, int p) {
+        const uint32_t i = l - (uint32_t)q.lo;
+        if (i < (uint32_t)q.n && is_marked(s_bits, i)) T.list[atomicAdd(&cursor[i], 1u)] = p;
+    });
+}
+
+template <bool WEEKEND, class KT>
+__global__ __launch_bounds__(1024) void k_collect_group(const DayState* __restrict__ st, const Model* __restrict__ Mp,
+                                                        CountTable T) {
+    if (st->done) return;
+    const CountRep c = T.reps[0];
+    if (T.chunk_day[blockIdx.x] != st->day + 1) return;
+    extern __shared__ uint32_t s_cur[];
+    __shared__ uint32_t s_n;
+    const int chunk = blockIdx.x / c.G;
+    const GroupColumns q = group_columns(c, blockIdx.x % c.G);
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const uint32_t* marks = T.marks + c.qbase + (int64_t)chunk * c.qw;
+    uint32_t* cursor = T.cnt + c.mbase + (int64_t)chunk * c.K + q.bucket;
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+    for_marked(marks, hour_columns(c, q.hour), [&](int) { atomicAdd(&s_n, 1u); });
+    __syncthreads();
+    if (s_n <= kFewMarks * (uint32_t)c.ranges) return;
+    for (int i = tid; i < q.n; i += nt) s_cur[i] = ~0u;
+    __syncthreads();
+    for_marked(marks, q, [&](int b) { s_cur[b - q.bucket] = cursor[b - q.bucket]; });
+    __syncthreads();
+    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, 0, 1, [&](uint32_t l, int p) {
+        const uint32_t i = l - (uint32_t)q.lo;
+        if (i < (uint32_t)q.n && s_cur[i] != ~0u) T.list[atomicAdd(&s_cur[i], 1u)] = p;
+    });
+    __syncthreads();
+    for_marked(marks, q, [&](int b) { cursor[b - q.bucket] = s_cur[b - q.bucket]; });
 }
 
 // Short lists rank every id against the others, in registers;
@@ -564,11 +953,12 @@ __device__ __forceinline__ int32_t picked_person(const CountTable& T, uint32_t q
     uint32_t want = T.pk_want[q], len = (uint32_t)T.pk_len[q];
     int chunk = T.pk_chunk[q];
     for (int round = 0;; ++round) {
-        const int32_t* l = T.list + T.cursor[c.mbase + (int64_t)chunk * c.K + b];
+        // (split layouts: the entry is the list's end now)
+        const int32_t* l = T.list + (T.cnt[c.mbase + (int64_t)chunk * c.K + b] - (c.G > 1 ? len : 0u));
         const int32_t v = rank_in_list(l, len, want, chunk * c.A, c.A, sub);
         if (v != idx || round) return v;
-        const uint32_t total = count_row(T, c, c.C)[b];  // the next person instead (select_person)
-        uint32_t j = count_row(T, c, chunk)[b] + want + 1, before;
+        const uint32_t total = T.total[c.tbase + b];  // the next person instead (select_person)
+        uint32_t j = count_column(T, c, b)[chunk] + want + 1, before;
         if (j == total) j = 0;
         chunk = chunk_of(T, c, b, j, total, before, len);
         want = j - before;
@@ -629,9 +1019,10 @@ inline int32_t count_chunk(int64_t N, int64_t K, int kpa, int64_t want) {
 // The plan of one layout on the host, and its device copies.
 struct CountPlan {
     bool on = false;
-    int n_chunks = 0, n_scans = 0, threads = 0, kpa = 0;
+    bool split = false, wide = false;  // column groups; hours of over 65,535 locations
+    int n_chunks = 0, n_scans = 0, threads = 0, kpa = 0, scan_cols = 0;
     size_t lds = 0;
-    int64_t entries = 0, mark_words = 0;
+    int64_t entries = 0, mark_words = 0, buckets = 0;
     std::vector<CountRep> reps;
     std::vector<CountBlock> chunks, scans;
     CountRep* d_reps = nullptr;
@@ -654,6 +1045,7 @@ struct CountPlan {
         }
         on = on && kmax <= kCountMaxK;
         if (!on) return;
+        for (auto& c : reps) c.G = c.ranges = 1, c.E = c.W = c.K;
         lds = sizeof(uint32_t) * (size_t)kmax;
         threads = 1024;
         for (size_t r = 0; r < reps.size(); ++r) {
@@ -662,18 +1054,61 @@ struct CountPlan {
             c.C = (int32_t)((N[r] + c.A - 1) / c.A);
             c.qw = (c.K + 31) / 32;
             c.mbase = entries;
+            c.tbase = buckets;
+            buckets += c.K;
             c.qbase = mark_words;
             c.chunk0 = (int32_t)chunks.size();
             entries += (int64_t)(c.C + 1) * c.K;
             mark_words += (int64_t)c.C * c.qw;
             for (int k = 0; k < c.C; ++k) chunks.push_back({(int32_t)r, k});
-            for (int b = 0; b < c.K; b += kScanCols) scans.push_back({(int32_t)r, b});
         }
         n_chunks = (int)chunks.size();
+        plan_scans();
+    }
+    // A block's rows per turn cover the chunks of most simulations at once.
+    void plan_scans() {
+        int32_t chunks_max = 0;
+        for (const auto& c : reps) chunks_max = std::max(chunks_max, c.C);
+        scan_cols = chunks_max > 128 && buckets < 32768 ? 32 : (chunks_max > 32 ? 64 : (chunks_max > 8 ? 256 : 1024));
+        for (size_t r = 0; r < reps.size(); ++r)
+            for (int b = 0; b < reps[r].K; b += scan_cols) scans.push_back({(int32_t)r, b});
         n_scans = (int)scans.size();
+    }
+    // One simulation of more buckets: column groups, E locations in the first
+    // hour, `hours` hours.  Chunks so that the (chunk, group) blocks fill the
+    // chip once or a few times (a block may take a CU's whole LDS) with at
+    // most about 16 people per bucket and chunk.
+    void build_split(int64_t N, int keys_per_agent, int32_t E, int hours, int cus) {
+        CountRep& c = reps[0];
+        kpa = keys_per_agent;
+        c.E = E;
+        const int32_t last = c.K - (hours - 1) * E, widest = std::max(E, last);
+        c.ranges = (widest + kCountMaxK - 1) / kCountMaxK;
+        if (c.ranges > kCountMaxRanges || widest > kCountMaxHour) return;
+        c.W = (widest + c.ranges - 1) / c.ranges;
+        c.G = hours * c.ranges;
+        int64_t A = 0;
+        for (int k = 1;; ++k) {
+            const int64_t C = std::max<int64_t>(1, (int64_t)cus * k / c.G);
+            A = ((N + C - 1) / C + kTileAgents - 1) / kTileAgents * kTileAgents;
+            if (kpa * A <= 16 * (int64_t)c.K || A == kTileAgents) break;
+        }
+        on = split = true;
+        wide = widest > 0xFFFF;
+        c.A = (int32_t)A;
+        c.C = (int32_t)((N + A - 1) / A);
+        c.qw = (c.K + 31) / 32;
+        entries = (int64_t)(c.C + 1) * c.K;
+        buckets = c.K;
+        mark_words = (int64_t)c.C * c.qw;
+        lds = sizeof(uint32_t) * (size_t)c.W;
+        threads = 1024;
+        n_chunks = c.C * c.G;
+        plan_scans();
     }
     int upload(hipStream_t st) {
         if (!on) return 0;
+        chunks.resize(n_chunks);  // (a split layout numbers its blocks itself)
         if (dev_alloc(&d_reps, (int64_t)reps.size()) || dev_alloc(&d_chunks, n_chunks) || dev_alloc(&d_scans, n_scans))
             return PT_ENOMEM;
         HIP_TRY(hipMemcpyAsync(d_reps, reps.data(), sizeof(CountRep) * reps.size(), hipMemcpyHostToDevice, st));
@@ -689,44 +1124,56 @@ struct CountPlan {
     }
 };
 
-// Buffers shared by the two layouts.
+// Buffers shared by the two layouts (a: weekday, b: weekend).
 struct CountScratch {
-    uint32_t *pre = nullptr, *cursor = nullptr, *marks = nullptr, *n = nullptr;
+    uint32_t *cnt = nullptr, *pre = nullptr, *total = nullptr, *marks = nullptr, *n = nullptr;
     int32_t* chunk_day = nullptr;
-    int alloc(const CountPlan& a, const CountPlan& b) {
+    uint16_t* tile_off = nullptr;
+    int32_t* lone_day = nullptr;
+    int alloc(const CountPlan& a, const CountPlan& b, int64_t N) {
         const int64_t e = std::max(a.entries, b.entries);
         if (e == 0) return 0;
-        return dev_alloc(&pre, e) || dev_alloc(&cursor, e) || dev_alloc(&marks, std::max(a.mark_words, b.mark_words)) ||
-                       dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 2)
+        return dev_alloc(&cnt, e) || dev_alloc(&pre, e) || dev_alloc(&total, std::max(a.buckets, b.buckets)) || dev_alloc(&marks, std::max(a.mark_words, b.mark_words)) ||
+                       dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 3) || dev_alloc(&lone_day, (int64_t)std::max(a.reps.size(), b.reps.size())) ||
+                       (b.split && dev_alloc(&tile_off, (N / kTileAgents + 1) * kTileHours))
                    ? PT_ENOMEM
                    : 0;
     }
     void release() {
+        dev_free(cnt);
         dev_free(pre);
-        dev_free(cursor);
+        dev_free(total);
         dev_free(marks);
         dev_free(chunk_day);
         dev_free(n);
+        dev_free(lone_day);
+        dev_free(tile_off);
     }
     void fill(CountTable& t, const CountPlan& p) const {
         t.reps = p.d_reps;
         t.chunks = p.d_chunks;
         t.scans = p.d_scans;
+        t.cnt = cnt;
         t.pre = pre;
-        t.cursor = cursor;
+        t.total = total;
         t.marks = marks;
         t.mark_words = p.mark_words;
         t.chunk_day = chunk_day;
         t.n = n;
+        t.tile_off = tile_off;
+        t.lone_day = lone_day;
     }
 };
 
 // LDS above the default limit for the counting kernels.
 inline hipError_t set_count_lds(const CountPlan& p) {
     if (!p.on || p.lds <= 64 * 1024) return hipSuccess;
-    for (const void* k : {reinterpret_cast<const void*>(&k_count<false>), reinterpret_cast<const void*>(&k_count<true>),
-                          reinterpret_cast<const void*>(&k_collect<false>),
-                          reinterpret_cast<const void*>(&k_collect<true>)}) {
+    const auto ptr = [](auto* k) { return reinterpret_cast<const void*>(k); };
+    for (const void* k :
+         {ptr(&k_count<false>), ptr(&k_count<true>), ptr(&k_collect<false>), ptr(&k_collect<true>),
+          ptr(&k_count_group<false, uint16_t>), ptr(&k_count_group<false, uint32_t>),
+          ptr(&k_count_group<true, uint32_t>), ptr(&k_collect_group<false, uint16_t>),
+          ptr(&k_collect_group<false, uint32_t>), ptr(&k_collect_group<true, uint32_t>)}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(4 * kCountMaxK));
         if (e != hipSuccess) return e;
     }
@@ -735,18 +1182,44 @@ inline hipError_t set_count_lds(const CountPlan& p) {
 
 // Before contacts: keys, counts, prefixes.  After: lists, picks, claims.
 inline void enqueue_counts(const CountPlan& p, const CountTable& t, const int32_t* done, DayState* sts,
-                           const Model* models, const uint8_t* age, bool weekend, hipStream_t st, LaunchTimer* tm) {
-    launch_lds(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_count<true> : k_count<false>,
-               dim3(p.n_chunks), dim3(p.threads), p.lds, st, done, sts, models, age, t);
-    launch(tm, KC_COUNT_SCAN, k_count_scan, dim3(p.n_scans), dim3(kScanCols * kScanGroups), st, done,
-           (const DayState*)sts, t);
+                           const Model* models, const uint8_t* age, bool weekend, hipStream_t st, LaunchTimer* tm,
+                           int64_t models_n = 0, int grid_keys = 0) {
+    if (p.split) {
+        const int64_t N = models_n;
+        if (weekend)
+            launch(tm, KC_GEN_WEEKEND, k_keys_weekend, dim3((int)((N + kTileAgents - 1) / kTileAgents)),
+                   dim3(kTileThreads), st, sts, models, t);
+        else
+            launch(tm, KC_GEN_WEEKDAY, p.wide ? k_keys_weekday<uint32_t> : k_keys_weekday<uint16_t>,
+                   dim3(grid_for((N + 1) / 2, 256, grid_keys)), dim3(256), st, sts, models, age, t);
+        const auto k = weekend ? k_count_group<true, uint32_t>
+                               : (p.wide ? k_count_group<false, uint32_t> : k_count_group<false, uint16_t>);
+        launch_lds(tm, KC_TABLE_COUNT, k, dim3(p.n_chunks), dim3(p.threads), p.lds, st, (const DayState*)sts, models, t);
+    } else {
+        launch_lds(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_count<true> : k_count<false>,
+                   dim3(p.n_chunks), dim3(p.threads), p.lds, st, done, sts, models, age, t);
+    }
+    const auto scan = p.scan_cols == 32
+                          ? k_count_scan<32>
+                          : (p.scan_cols == 64 ? k_count_scan<64> : (p.scan_cols == 256 ? k_count_scan<256> : k_count_scan<1024>));
+    launch(tm, KC_COUNT_SCAN, scan, dim3(p.n_scans), dim3(kCountScanThreads), st, done, (const DayState*)sts, t);
 }
 
 inline void enqueue_picks(const CountPlan& p, const CountTable& t, const ClaimArrays& c, DayState* g,
                           const DayState* sts, const Model* models, int grid, bool weekend, hipStream_t st,
                           LaunchTimer* tm) {
-    launch_lds(tm, KC_COLLECT, weekend ? k_collect<true> : k_collect<false>, dim3(p.n_chunks), dim3(p.threads), p.lds,
-               st, (const int32_t*)&g->done, sts, models, t);
+    if (p.split) {
+        const auto few = weekend ? k_collect_few<true, uint32_t>
+                                 : (p.wide ? k_collect_few<false, uint32_t> : k_collect_few<false, uint16_t>);
+        launch_lds(tm, KC_COLLECT, few, dim3(p.n_chunks / p.reps[0].ranges * kCollectParts), dim3(kCollectFewThreads),
+                   sizeof(uint32_t) * (size_t)(p.reps[0].W * p.reps[0].ranges / 32 + 2), st, sts, models, t);
+        const auto k = weekend ? k_collect_group<true, uint32_t>
+                               : (p.wide ? k_collect_group<false, uint32_t> : k_collect_group<false, uint16_t>);
+        launch_lds(tm, KC_COLLECT, k, dim3(p.n_chunks), dim3(p.threads), p.lds, st, sts, models, t);
+    } else {
+        launch_lds(tm, KC_COLLECT, weekend ? k_collect<true> : k_collect<false>, dim3(p.n_chunks), dim3(p.threads),
+                   p.lds, st, (const int32_t*)&g->done, sts, models, t);
+    }
     launch(tm, KC_RESOLVE, k_resolve, dim3(grid), dim3(256), st, g, t, c);
 }
 

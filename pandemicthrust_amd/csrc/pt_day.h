@@ -82,9 +82,23 @@ int build_model(const pt_params* p, const int32_t seed_key[2], Model& m);
 // PT_EINVAL).
 int apply_interventions(const pt_interventions* iv, Model& m);
 
-// Locations number below 2^28 (location_scaling <= 1e4); 0..3 contacts a day.
-constexpr int kWorkplaceBits = 28;
-constexpr uint32_t kWorkplaceMask = (1u << kWorkplaceBits) - 1u;
+// What a contact needs of an agent, in one 8-byte record instead of five
+// gathers (age, household, its two offsets, workplace): x = first person of
+// the household | its size << 28 | adult << 31; y = workplace or school | its
+// contacts per day << 28.  Agents and locations number below 2^28
+// (pt_sim_setup; location_scaling <= 1e4), households hold at most 5 people.
+struct AgentRecord {
+    uint32_t x, y;
+};
+__device__ __forceinline__ AgentRecord make_record(int32_t hoff, int32_t hcnt, bool adult, int32_t wp, int wpd) {
+    return AgentRecord{(uint32_t)hoff | ((uint32_t)hcnt << 28) | (adult ? 0x80000000u : 0u),
+                       (uint32_t)wp | ((uint32_t)wpd << 28)};
+}
+__device__ __forceinline__ int32_t record_household(AgentRecord a) { return (int32_t)(a.x & 0x0FFFFFFFu); }
+__device__ __forceinline__ int32_t record_household_size(AgentRecord a) { return (int32_t)((a.x >> 28) & 7u); }
+__device__ __forceinline__ bool record_adult(AgentRecord a) { return (a.x >> 31) != 0; }
+__device__ __forceinline__ int32_t record_workplace(AgentRecord a) { return (int32_t)(a.y & 0x0FFFFFFFu); }
+__device__ __forceinline__ int record_workplace_contacts(AgentRecord a) { return (int)(a.y >> 28); }
 
 // Population arrays of one simulation (local numbering).
 struct PopArrays {
@@ -94,7 +108,8 @@ struct PopArrays {
     uint8_t* age;        // N
     int32_t* wp_off;     // W + 1
     int32_t* wp_people;  // N
-    uint32_t* wp_of;     // N, workplace or school | its contacts per day << kWorkplaceBits
+    AgentRecord* who;    // N
+    int32_t* wp_lone;    // 1: some workplace has a single person
     uint8_t *st_p, *st_s, *dy_p, *dy_s, *gn_p, *gn_s;  // N
     uint64_t *claim_p, *claim_s;                        // N
 };
@@ -498,21 +513,23 @@ __device__ __forceinline__ int select_person(int32_t infector, int32_t loc_off, 
 // Where the victims of an infector's contact slots come from: the household
 // (slots 0..2; its members are consecutive ids), then `wpd` workplace or
 // school slots, then h0 slots in the first errand location and h1 in the
-// second (weekend: wpd = 0, h0 = h1 = 1), with each slot's draw r.  Only a
+// second (weekend: wpd = 0, h0 = h1 = 1), with each slot's draw (SlotDraws).  Only a
 // slot whose infection draw succeeds needs its victim, so outside
 // validation mode the contact kernels look victims up then (pick) instead of
 // gathering one from a location table for every slot: the contact types and
 // kval_sum depend on the location counts alone (select_person), and the
 // victims of unsuccessful slots are never read.
 // With counted tables e0off and e1off hold the errand buckets.
+// (The draws are an array of their own: inside the struct they kept all of it
+// in scratch memory.)
 struct SlotPlan {
     int32_t hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt;
     int wpd, h0, h1;
-    uint32_t r[8];
 };
+using SlotDraws = uint32_t[8];
 
 // The victim of slot c (select_person's pick; the slot's count is > 1).
-__device__ __forceinline__ int32_t pick(const SlotPlan& P, const int32_t* __restrict__ wp_people,
+__device__ __forceinline__ int32_t pick(const SlotPlan& P, const SlotDraws& r, const int32_t* __restrict__ wp_people,
                                         const int32_t* __restrict__ er_people, int32_t infector, int c) {
     int32_t off, cnt;
     const int32_t* people;
@@ -534,7 +551,7 @@ __device__ __forceinline__ int32_t pick(const SlotPlan& P, const int32_t* __rest
         people = er_people;
     }
     int32_t v;
-    select_person(infector, off, cnt, P.r[c], people ? CT_ERRAND : CT_HOME, people, v);
+    select_person(infector, off, cnt, r[c], people ? CT_ERRAND : CT_HOME, people, v);
     return v;
 }
 
@@ -547,7 +564,7 @@ struct AgentArrays {
     const int32_t* hh_off;
     const int32_t* wp_off;
     const int32_t* wp_people;
-    const uint32_t* wp_of;
+    const AgentRecord* who;
     const int32_t* er_off;
     const int32_t* er_people;
     // Counted tables (er_off, er_people unused): people per bucket, and the
@@ -668,7 +685,7 @@ __device__ __forceinline__ void success_draws(const Model& M, uint64_t M2, Succe
 template <int C>
 __device__ __forceinline__ void process_contacts(const Model& M, const AgentArrays& A, const Infectivity& f, int kval_sum,
                                                  int32_t (&vic)[8], const int (&typ)[8], const SlotPlan& P,
-                                                 bool resolved, int32_t idx, const SuccessDraws& draws, uint32_t pos,
+                                                 const SlotDraws& slot_draws, bool resolved, int32_t idx, const SuccessDraws& draws, uint32_t pos,
                                                  bool (&newp)[8], bool (&news)[8]) {
     const float prob_p = f.prof_p >= 0 ? infection_probability(M, f.prof_p, f.dd_p, 0, kval_sum) : -1.f;
     const float prob_s = f.prof_s >= 0 ? infection_probability(M, f.prof_s, f.dd_s, 1, kval_sum) : -1.f;
@@ -681,7 +698,7 @@ __device__ __forceinline__ void process_contacts(const Model& M, const AgentArra
         const bool draw_s = unit_float(u[2 * c + 1]) < prob_s * kv;
         int32_t v = vic[c];
         if (!resolved && (draw_p || draw_s)) {  // kv = 1: a real contact, count > 1
-            v = pick(P, A.wp_people, A.er_people, idx, c);
+            v = pick(P, slot_draws, A.wp_people, A.er_people, idx, c);
             vic[c] = v;
         }
         if (A.trace_draw) {
@@ -759,36 +776,52 @@ __device__ __forceinline__ void clear_contacts(int32_t (&vic)[8], int (&typ)[8],
     }
 }
 
-// The same with a queue (counted tables): successful slots are queued, two
-// slots per round, and claimed together by the block (PickPush), so a wave
-// does not go through the look-up chain of every slot in which one of its
-// lanes succeeds.  All threads of the block must call, the idle ones with
-// active false.
+// The same with a queue (counted tables): successful slots are queued and
+// claimed together by the block (PickPush), so a wave does not go through the
+// look-up chain of every slot in which one of its lanes succeeds.  All
+// threads of the block must call, the idle ones with active false.
 template <int C, class Queue>
 __device__ __forceinline__ void queue_contacts(const Model& M, bool active, const Infectivity& f, int kval_sum,
-                                               const int (&typ)[8], const SlotPlan& P, int32_t idx,
-                                               const SuccessDraws& draws, uint32_t pos, const Queue& queue) {
+                                               const int (&typ)[8], const SlotPlan& P,
+                                               const SlotDraws& slot_draws, int32_t idx, const SuccessDraws& draws,
+                                               uint32_t pos, const Queue& queue) {
     float prob_p = -1.f, prob_s = -1.f;
     if (active && f.prof_p >= 0) prob_p = infection_probability(M, f.prof_p, f.dd_p, 0, kval_sum);
     if (active && f.prof_s >= 0) prob_s = infection_probability(M, f.prof_s, f.dd_s, 1, kval_sum);
     const uint32_t(&u)[16] = draws.u;
+    uint32_t hit_p = 0, hit_s = 0;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
         const float kv = typ[c] == CT_NONE ? 0.f : 1.f;
-        const bool draw_p = unit_float(u[2 * c]) < prob_p * kv;
-        const bool draw_s = unit_float(u[2 * c + 1]) < prob_s * kv;
-        if (active && (draw_p || draw_s)) {  // kv = 1: a real contact, count > 1
-            const uint32_t prof_p = infection_profile(M, u[2 * c] ^ u[(2 * c + 1) % 16]);
-            const uint32_t prof_s = infection_profile(M, u[2 * c + 1] ^ u[(2 * c + 2) % 16]);
-            const bool home = c < 3, work = !home && c < 3 + P.wpd, first = c < 3 + P.wpd + P.h0;
-            const int32_t off = home ? P.hoff : (work ? P.woff : (first ? P.e0off : P.e1off));
-            const int32_t cnt = home ? P.hcnt : (work ? P.wcnt : (first ? P.e0cnt : P.e1cnt));
-            queue.push(off, (uint32_t)cnt, P.r[c] % (uint32_t)cnt, home ? 1u : (work ? 2u : 0u), idx,
-                       pos * 8u + (uint32_t)c,
-                       f.gen_p | ((uint32_t)f.gen_s << 8) | (prof_p << 16) | (prof_s << 20) |
-                           ((draw_p ? 1u : 0u) << 24) | ((draw_s ? 1u : 0u) << 25));
+        hit_p |= (unit_float(u[2 * c]) < prob_p * kv ? 1u : 0u) << c;
+        hit_s |= (unit_float(u[2 * c + 1]) < prob_s * kv ? 1u : 0u) << c;
+    }
+    const uint32_t hit = active ? hit_p | hit_s : 0u;  // kv = 1: real contacts, count > 1
+    // In registers: selects between the plan's fields would become loads from
+    // scratch memory.
+    int32_t hoff = P.hoff, hcnt = P.hcnt, woff = P.woff, wcnt = P.wcnt, e0off = P.e0off, e0cnt = P.e0cnt,
+            e1off = P.e1off, e1cnt = P.e1cnt, wpd = P.wpd, h0 = P.h0;
+    asm volatile("" : "+v"(hoff), "+v"(hcnt), "+v"(woff), "+v"(wcnt), "+v"(e0off), "+v"(e0cnt), "+v"(e1off),
+                 "+v"(e1cnt), "+v"(wpd), "+v"(h0));
+    // All slots in one turn when the block's successes fit the queue, else
+    // two slots (at most 2 per thread) per turn.
+    const int step = queue.fits((uint32_t)__popc(hit)) ? C : 2;
+    for (int c0 = 0; c0 < C; c0 += step) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            if (c >= c0 && c < c0 + step && ((hit >> c) & 1u)) {
+                const uint32_t prof_p = infection_profile(M, u[2 * c] ^ u[(2 * c + 1) % 16]);
+                const uint32_t prof_s = infection_profile(M, u[2 * c + 1] ^ u[(2 * c + 2) % 16]);
+                const bool home = c < 3, work = !home && c < 3 + wpd, first = c < 3 + wpd + h0;
+                const int32_t off = home ? hoff : (work ? woff : (first ? e0off : e1off));
+                const int32_t cnt = home ? hcnt : (work ? wcnt : (first ? e0cnt : e1cnt));
+                queue.push(off, (uint32_t)cnt, slot_draws[c] % (uint32_t)cnt, home ? 1u : (work ? 2u : 0u), idx,
+                           pos * 8u + (uint32_t)c,
+                           f.gen_p | ((uint32_t)f.gen_s << 8) | (prof_p << 16) | (prof_s << 20) |
+                               (((hit_p >> c) & 1u) << 24) | (((hit_s >> c) & 1u) << 25));
+            }
         }
-        if (c % 2 == 1 || c == C - 1) queue.round(c == C - 1);
+        queue.flush();
     }
 }
 
@@ -823,6 +856,7 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
                                                  bool (&news)[8], const SuccessDraws& draws, const Queue& queue) {
     const bool resolved = A.trace_victim != nullptr;
     SlotPlan P{};
+    SlotDraws r = {};
     int kval = 0;
     if (active) {
         if constexpr (!Queue::counted) {  // (queued infectors can)
@@ -831,18 +865,18 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
         const uint64_t Mc = cbase + (uint64_t)(6 * pos);
         const U4 ua = draw4(Mc, M.key0, M.key1);
         const U4 ub = draw4(Mc + 1, M.key0, M.key1);
-        const uint32_t u[8] = {ua.w[0], ua.w[1], ua.w[2], ua.w[3], ub.w[0], ub.w[1], ub.w[2], ub.w[3]};
-        const uint8_t myage = A.age[idx];
-        const bool adult = myage == kAgeAdult;
-        // household
-        const int32_t hh = A.household[idx];
-        const int32_t hoff = A.hh_off[hh];
-        const int32_t hcnt = A.hh_off[hh + 1] - hoff;
-        // workplace (device_recalcWorkplace PandemicSim.cu:3872-3890) and its
-        // contacts, kept per agent since the setup (PopArrays::wp_of)
-        const uint32_t pw = A.wp_of[idx];
-        const int32_t wp = (int32_t)(pw & kWorkplaceMask);
-        const int wpd = (int)(pw >> kWorkplaceBits);
+        const uint32_t(&u)[8] = r;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            r[q] = ua.w[q];
+            r[4 + q] = ub.w[q];
+        }
+        const AgentRecord me = A.who[idx];
+        const bool adult = record_adult(me);
+        const int32_t hoff = record_household(me), hcnt = record_household_size(me);
+        // workplace (device_recalcWorkplace PandemicSim.cu:3872-3890)
+        const int32_t wp = record_workplace(me);
+        const int wpd = record_workplace_contacts(me);
         const int32_t woff = A.wp_off[wp];
         const int32_t wcnt = A.wp_off[wp + 1] - woff;
         // errands (device_recalc_weekdayErrandDests_assignProfile :3667-3705)
@@ -860,8 +894,7 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
         errand_bucket<Queue::counted>(A, k1, e1off, e1cnt);
         const int wtype = adult ? CT_WORKPLACE : CT_SCHOOL;
         const int etype = adult ? CT_ERRAND : CT_AFTERSCHOOL;
-        P = SlotPlan{hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt, wpd, h0, h1,
-                         {u[0], u[1], u[2], u[3], u[4], u[5], u[6], u[7]}};
+        P = SlotPlan{hoff, hcnt, woff, wcnt, e0off, e0cnt, e1off, e1cnt, wpd, h0, h1};
         int32_t where[8];  // the contact's location (trace only)
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
@@ -869,7 +902,7 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
             if (resolved) {
                 if (c < 3) {
                     t = select_person(idx, hoff, hcnt, u[c], CT_HOME, nullptr, vic[c]);
-                    where[c] = hh;
+                    where[c] = A.household[idx];
                 } else if (c < 3 + wpd) {
                     t = select_person(idx, woff, wcnt, u[c], wtype, A.wp_people, vic[c]);
                     where[c] = wp;
@@ -911,9 +944,9 @@ __device__ __forceinline__ void weekday_contacts(const Model& M, const AgentArra
     // infector that cannot infect has p <= 0 (or NaN), so none of its draws
     // succeeds and it posts no claim.
     if constexpr (Queue::counted)
-        queue_contacts<8>(M, active, f, kval, typ, P, idx, draws, (uint32_t)pos, queue);
+        queue_contacts<8>(M, active, f, kval, typ, P, r, idx, draws, (uint32_t)pos, queue);
     else if (can_infect(M, f) || A.trace_draw)
-        process_contacts<8>(M, A, f, kval, vic, typ, P, resolved, idx, draws, (uint32_t)pos, newp, news);
+        process_contacts<8>(M, A, f, kval, vic, typ, P, r, resolved, idx, draws, (uint32_t)pos, newp, news);
     else if (A.trace_attempt)
         for (int c = 0; c < 8; ++c) A.trace_attempt[pos * 8 + c] = 0;
 }
@@ -928,6 +961,7 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
                                                  const SuccessDraws& draws, const Queue& queue) {
     const bool resolved = A.trace_victim != nullptr;
     SlotPlan P{};
+    SlotDraws r = {};
     int kval = 0;
     if (active) {
         if constexpr (!Queue::counted) {
@@ -935,9 +969,8 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
         }
         const uint64_t Mc = cbase + (uint64_t)(6 * pos);
         const U4 u = draw4(Mc, M.key0, M.key1);
-        const int32_t hh = A.household[idx];
-        const int32_t hoff = A.hh_off[hh];
-        const int32_t hcnt = A.hh_off[hh + 1] - hoff;
+        const AgentRecord me = A.who[idx];
+        const int32_t hoff = record_household(me), hcnt = record_household_size(me);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             if (resolved)
@@ -948,13 +981,14 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
         const int prof = (int)(u.w[3] % 6u);
         uint32_t v32[2];
         draw2x32((uint32_t)(Mc + 1), (uint32_t)M.key0, (uint32_t)M.key1, v32);
+        const int32_t hh = resolved ? A.household[idx] : 0;
         int32_t where[5] = {hh, hh, hh, -1, -1};  // the contact's location (trace only)
         int32_t eo[2], ec[2];
-        if constexpr (Queue::counted) {
+        if (Queue::counted && A.er_keys) {
             const uint16_t* keys = A.er_keys + idx;
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                errand_bucket<true>(A, keys[M.we_assign[prof][k] * A.er_slots], eo[k], ec[k]);
+                errand_bucket<Queue::counted>(A, keys[M.we_assign[prof][k] * A.er_slots], eo[k], ec[k]);
                 typ[3 + k] = ec[k] > 1 ? CT_ERRAND : CT_NONE;
             }
         } else {
@@ -968,7 +1002,7 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
                 const int lsel = slot == 0 ? loc[0] : (slot == 1 ? loc[1] : loc[2]);
                 const int32_t l = min(max(lsel - M.we_base, 0), M.we_E - 1);
                 const int32_t key = hsel * M.we_E + l;
-                errand_bucket<false>(A, (uint32_t)key, eo[k], ec[k]);
+                errand_bucket<Queue::counted>(A, (uint32_t)key, eo[k], ec[k]);
                 if (resolved)
                     typ[3 + k] = select_person(idx, eo[k], ec[k], v32[k], CT_ERRAND, A.er_people, vic[3 + k]);
                 else
@@ -976,8 +1010,11 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
                 where[3 + k] = hsel * M.W + lsel;
             }
         }
-        P = SlotPlan{hoff, hcnt, 0, 0, eo[0], ec[0], eo[1], ec[1], 0, 1, 1,
-                         {u.w[0], u.w[1], u.w[2], v32[0], v32[1], 0u, 0u, 0u}};
+        P = SlotPlan{hoff, hcnt, 0, 0, eo[0], ec[0], eo[1], ec[1], 0, 1, 1};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[q] = u.w[q];
+        r[3] = v32[0];
+        r[4] = v32[1];
 #pragma unroll
         for (int c = 0; c < 5; ++c) kval += typ[c] != CT_NONE;
         apply_drops(M, day, true, Mc, 5, vic, typ);
@@ -994,21 +1031,21 @@ __device__ __forceinline__ void weekend_contacts(const Model& M, const AgentArra
     // infector that cannot infect has p <= 0 (or NaN), so none of its draws
     // succeeds and it posts no claim.
     if constexpr (Queue::counted)
-        queue_contacts<5>(M, active, f, kval, typ, P, idx, draws, (uint32_t)pos, queue);
+        queue_contacts<5>(M, active, f, kval, typ, P, r, idx, draws, (uint32_t)pos, queue);
     else if (can_infect(M, f) || A.trace_draw)
-        process_contacts<5>(M, A, f, kval, vic, typ, P, resolved, idx, draws, (uint32_t)pos, newp, news);
+        process_contacts<5>(M, A, f, kval, vic, typ, P, r, resolved, idx, draws, (uint32_t)pos, newp, news);
     else if (A.trace_attempt)
         for (int c = 0; c < 5; ++c) A.trace_attempt[pos * 5 + c] = 0;
 }
 
 // Whether any contact draw of an infector can succeed: y < p for one of its
-// slots' uniforms against the largest p any contact count gives (kval_sum =
-// 1; the quotient only falls with kval_sum).  Needs nothing but the
-// infector's strain state and its own draws, none of the tables.
+// slots' uniforms against the p that a contact count of at least kval gives
+// (the rounded quotient only falls with the count).  With kval = 1 it needs
+// nothing but the infector's strain state and its own draws.
 template <int C>
-__device__ __forceinline__ bool may_infect(const Model& M, const Infectivity& f, const SuccessDraws& d) {
-    const float bp = f.prof_p >= 0 ? infection_probability(M, f.prof_p, f.dd_p, 0, 1) : -1.f;
-    const float bs = f.prof_s >= 0 ? infection_probability(M, f.prof_s, f.dd_s, 1, 1) : -1.f;
+__device__ __forceinline__ bool may_infect(const Model& M, const Infectivity& f, const SuccessDraws& d, int kval) {
+    const float bp = f.prof_p >= 0 ? infection_probability(M, f.prof_p, f.dd_p, 0, kval) : -1.f;
+    const float bs = f.prof_s >= 0 ? infection_probability(M, f.prof_s, f.dd_s, 1, kval) : -1.f;
     bool any = false;
 #pragma unroll
     for (int c = 0; c < C; ++c) {

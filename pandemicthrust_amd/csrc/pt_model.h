@@ -81,10 +81,24 @@ struct ErrandWalk {
     int32_t offset[kWalkRows];
 };
 
+// The same as a table of the rows, for kernels that keep it in LDS
+// (LdsWalk): row i ends at threshold[i]; hi + lo = the pdfs before it.
+struct WalkRow {
+    float hi, lo, rcp, pdf;
+    float count;
+    uint32_t last;  // bits of the largest float below count
+    int32_t offset, pad;
+};
+struct WalkTable {
+    WalkRow row[kWalkRows];
+    float threshold[kWalkRows];
+};
+
 // The model with its prepared walks: resident in device memory, one copy per
 // simulation.
 struct Model : ModelData {
     ErrandWalk wd_walk, we_walk;
+    WalkTable wd_table, we_table;
 };
 
 // ---------------- Threefry (Salmon et al., SC'11) ----------------
@@ -285,6 +299,37 @@ __device__ __forceinline__ int32_t walk_location(const RowPick& p) {
     return location_in_row(q, p.count) + p.offset;
 }
 
+// The walk with its row constants read from LDS by row number instead of
+// selected: 15 selects and 3 subtractions less per errand, two LDS reads more
+// (weekday keys of 50M agents 176 -> 148 us, weekend keys 501 -> 457 us).
+// Thresholds: remainder > pdf exactly when y > the sum of the pdfs so far
+// (the remainders are exact), i.e. when y exceeds that sum rounded down.  The
+// remainder is y minus that sum as two exact subtractions: hi is the sum
+// rounded to a multiple of 256, which y is a multiple of behind the first row
+// (y > 2^31 there), so y - hi is exact, and the rest is the exact remainder.
+struct LdsWalk {
+    const WalkRow* row;
+    float t0, t1, t2;
+};
+// s_row: kWalkRows rows of LDS, filled by the block (barrier after it).
+__device__ __forceinline__ LdsWalk load_walk(const WalkTable& t, WalkRow* s_row) {
+    constexpr int kWords = sizeof(t.row) / 4;
+    if (threadIdx.x < kWords)
+        reinterpret_cast<uint32_t*>(s_row)[threadIdx.x] = reinterpret_cast<const uint32_t*>(t.row)[threadIdx.x];
+    return LdsWalk{s_row, t.threshold[0], t.threshold[1], t.threshold[2]};
+}
+__device__ __forceinline__ int32_t fish_errand_dest(const LdsWalk& k, uint32_t r) {
+    const float y = (float)r;
+    int i = y > k.t0 ? 1 : 0;
+    i = y > k.t1 ? 2 : i;
+    i = y > k.t2 ? 3 : i;
+    const WalkRow w = k.row[i];
+    const float frac = (y - w.hi) - w.lo;
+    const float q0 = frac * w.rcp;
+    const float q = __builtin_fmaf(__builtin_fmaf(-q0, w.pdf, frac), w.rcp, q0);
+    return (int32_t)(uint32_t)__uint_as_float(min(__float_as_uint(q * w.count), w.last)) + w.offset;
+}
+
 // An adult's weekday errand (device_fishAfterschoolOrErrandDestination_weekday,
 // PandemicSim.cu:2909-2947) or a weekend errand
 // (device_fishWeekendErrandDestination, :1017-1044); a child's weekday
@@ -299,7 +344,8 @@ __device__ __forceinline__ int32_t fish_afterschool(const Model& M, uint32_t r) 
 // Weekday errand destinations of one person from its two draws
 // (device_assignAfterschoolOrErrandDests_weekday, PandemicSim.cu:2950-2969),
 // returned as locations (hour 1's W offset is not added).
-__device__ __forceinline__ void weekday_dests(const Model& M, const ErrandWalk& k, uint32_t r1, uint32_t r2,
+template <class Walk>
+__device__ __forceinline__ void weekday_dests(const Model& M, const Walk& k, uint32_t r1, uint32_t r2,
                                               bool adult, int32_t& d1, int32_t& d2) {
     // A wave holds adults and children alike, so every lane does both and
     // selects.
@@ -385,7 +431,8 @@ __device__ __forceinline__ int next_hour(int h) { return h == kWeHours - 1 ? 0 :
 
 // device_generateWeekendErrands (PandemicSim.cu:980-1014): three distinct
 // hours and their destinations.
-__device__ __forceinline__ void weekend_errands(const Model& M, const ErrandWalk& k, uint64_t off, int32_t hour[3],
+template <class Walk>
+__device__ __forceinline__ void weekend_errands(const Model& M, const Walk& k, uint64_t off, int32_t hour[3],
                                                 int32_t loc[3]) {
     const U4 a = draw4(off, M.key0, M.key1);
     const U4 b = draw4(off + 1, M.key0, M.key1);

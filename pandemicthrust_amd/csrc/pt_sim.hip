@@ -140,8 +140,11 @@ __global__ void k_generate_households(const Model* __restrict__ Mp, const uint8_
 // K5: assignWorkplaceFunctor (PandemicSim.cu:3750-3778), four people per
 // counter workplace_off + g, g = 0..N/4.
 __global__ void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workplace_off, uint8_t* __restrict__ age,
-                                    uint32_t* __restrict__ wp_keys, uint32_t* __restrict__ wp_of) {
+                                    const int32_t* __restrict__ household, const int32_t* __restrict__ hh_off,
+                                    uint32_t* __restrict__ wp_keys, AgentRecord* __restrict__ who,
+                                    int32_t* __restrict__ wp_lone) {
     const Model& M = *Mp;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *wp_lone = 0;  // for k_lone_workplaces
     const int N = M.N;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g <= N / 4; g += stride) {
@@ -154,10 +157,20 @@ __global__ void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workp
                 const int32_t wp = assign_workplace(M, u.w[i], &a);
                 age[p] = a;
                 wp_keys[p] = (uint32_t)wp;
-                wp_of[p] = (uint32_t)wp | ((uint32_t)workplace_max_contacts(M, wp) << kWorkplaceBits);
+                const int32_t h = household[p], off = hh_off[h];
+                who[p] = make_record(off, hh_off[h + 1] - off, a == kAgeAdult, wp, workplace_max_contacts(M, wp));
             }
         }
     }
+}
+
+// Whether some workplace has a single person (such people have no workplace
+// contacts).
+__global__ void k_lone_workplaces(const Model* __restrict__ Mp, const int32_t* __restrict__ wp_off,
+                                  int32_t* __restrict__ lone) {
+    const int W = Mp->W;
+    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < W; w += gridDim.x * blockDim.x)
+        if (wp_off[w + 1] - wp_off[w] == 1) *lone = 1;
 }
 
 // K7: setup_initializeStatusArrays (PandemicSim.cu:3654-3664).  Agents
@@ -370,7 +383,8 @@ __global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__
             if (can_infect(M, f)) {
                 SuccessDraws draws;
                 success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
-                keep = may_infect<C>(M, f, draws);
+                keep = may_infect<C>(M, f, draws, 1) &&
+                       may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND));
             }
         }
         list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
@@ -564,7 +578,7 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
         const ClaimArrays claims = claim_arrays(A, list_p, list_s, st->n_claimed);
         __shared__ PickQueue s_pick;
         if (threadIdx.x == 0)  // first used behind a barrier of the first round
-            s_pick.n = s_pick.errands = s_pick.taken = s_pick.n_claim[0] = s_pick.n_claim[1] = 0;
+            s_pick.reset();
         __syncthreads();
         const PickPush push{T, claims, st, &s_pick, 0};
         const int64_t n = T.n[1];
@@ -598,7 +612,7 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
                 q = QueuedInfector{infected[pos], (int32_t)pos, 0};
                 success_draws<C>(M, cbase + (uint64_t)(6 * pos) + 2, draws);
                 const Infectivity f = infectivity(M, A, q.idx, day);
-                return can_infect(M, f) && may_infect<C>(M, f, draws);
+                return can_infect(M, f) && may_infect<C>(M, f, draws, 1);
             },
             [&](bool active, const QueuedInfector& q, const SuccessDraws& draws) {
                 contacts(active, infectivity(M, A, q.idx, day), q.idx, q.pos, draws, NoQueue{});
@@ -745,13 +759,35 @@ ErrandWalk prepare_walk(const Model& m, const float* pdf) {
     return w;
 }
 
+WalkTable walk_table(const ErrandWalk& w) {
+    WalkTable t{};
+    double sum = 0;  // exact: four floats of similar size
+    for (int r = 0; r < kWalkRows; ++r) {
+        WalkRow& q = t.row[r];
+        q.hi = (float)(256.0 * floor(sum / 256.0 + 0.5));
+        q.lo = (float)(sum - (double)q.hi);
+        q.rcp = w.rcp[r];
+        q.pdf = w.pdf[r];
+        q.count = w.count[r];
+        uint32_t bits;
+        memcpy(&bits, &w.count[r], 4);
+        q.last = bits - 1;
+        q.offset = w.offset[r];
+        sum += (double)w.pdf[r];
+        float f = (float)sum;
+        if ((double)f > sum) f = std::nextafter(f, 0.f);
+        t.threshold[r] = f;
+    }
+    return t;
+}
+
 int round_half_up(double d) { return (int)floor(d + 0.5); }  // roundHalfUp_toInt, PandemicSim.cu:1662
 
 const char* kKernelNames[KC_COUNT] = {"sweep",         "plan",       "compact",   "gen_weekday",
                                       "gen_weekend",   "sort_upsweep", "sort_scan", "sort_downsweep",
                                       "offsets",       "contacts_weekday", "contacts_weekend", "apply",
                                       "end_day",       "mark",       "select",    "subset_sort", "setup",
-                                      "count_scan",    "collect",    "resolve"};
+                                      "table_count",   "count_scan", "collect",   "resolve"};
 
 // Per-class kernel timing.  mode 0: off; -1: every class; k+1: class k only.
 // Launches are also accounted to the simulated day they belong to (day is
@@ -849,6 +885,8 @@ int build_model(const pt_params* p, const int32_t seed_key[2], Model& m) {
     }
     m.wd_walk = prepare_walk(m, m.wd_pdf);
     m.we_walk = prepare_walk(m, m.we_pdf);
+    m.wd_table = walk_table(m.wd_walk);
+    m.we_table = walk_table(m.we_walk);
     // setup_calculateInfectionData (PandemicSim.cu:2828-2840)
     for (int i = 3; i < 6; ++i)
         for (int j = 0; j < 10; ++j) m.shed[i][j] = m.shed[i][j] * p->asymp_factor;
@@ -924,10 +962,12 @@ hipError_t build_population(const Model* d_model, int64_t N, int H, int W, const
     k_generate_households<<<grid_for(H, 256, 65535), 256, 0, st>>>(d_model, P.hh_types, P.hh_off, P.household, P.age);
     if (marks) (void)hipEventRecord(marks[1], st);
     // K5/K6: workplaces, then the workplace table (PandemicSim.cu:3812-3862).
-    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, tmp, P.wp_of);
+    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, P.household,
+                                                                     P.hh_off, tmp, P.who, P.wp_lone);
     e = build_table(ts, tmp, nullptr, N, nullptr, W, ID_IDENTITY, (int32_t)N, P.wp_people, P.wp_off, nullptr, st,
                     nullptr);
     if (e != hipSuccess) return e;
+    k_lone_workplaces<<<grid_for(W, 256, 1024), 256, 0, st>>>(d_model, P.wp_off, P.wp_lone);
     if (marks) (void)hipEventRecord(marks[2], st);
     // K7: statuses; claim words start empty.
     k_init_status<<<grid_for(N, 256, 65535), 256, 0, st>>>(d_model, N, P.st_p, P.st_s, P.dy_p, P.dy_s, P.gn_p,
@@ -955,7 +995,8 @@ struct pt_sim {
     uint8_t* age = nullptr;
     uint8_t* snap = nullptr;  // 6N bytes
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
-    uint32_t* wp_of = nullptr;
+    AgentRecord* who = nullptr;
+    int32_t* wp_lone = nullptr;
     uint8_t* hh_types = nullptr;
     int32_t *infected = nullptr, *staging = nullptr;
     uint32_t* keys = nullptr;        // 3N
@@ -1051,7 +1092,8 @@ void free_population(pt_sim* s) {
     dev_free(s->hh_off);
     dev_free(s->wp_off);
     dev_free(s->wp_people);
-    dev_free(s->wp_of);
+    dev_free(s->who);
+    dev_free(s->wp_lone);
     dev_free(s->hh_types);
     dev_free(s->infected);
     dev_free(s->staging);
@@ -1089,9 +1131,16 @@ int setup_counts(pt_sim* s) {
         c.K = K[w];
         p.reps.assign(1, c);
         p.build({s->N}, w ? 3 : 2, s->cus);
-        if (p.upload(s->stream)) return PT_ENOMEM;
+        if (K[w] > kCountMaxK) p.build_split(s->N, w ? 3 : 2, w ? m.we_E : m.wd_E, w ? kWeHours : kWdHours, s->cus);
     }
-    if (s->count_scratch.alloc(s->count_plan[0], s->count_plan[1])) return PT_ENOMEM;
+    if (s->count_plan[0].upload(s->stream) || s->count_plan[1].upload(s->stream) ||
+        s->count_scratch.alloc(s->count_plan[0], s->count_plan[1], s->N)) {
+        // no memory for the matrices: sorted tables
+        (void)hipGetLastError();
+        for (CountPlan& p : s->count_plan) p.release();
+        s->count_scratch.release();
+        return PT_OK;
+    }
     for (int w = 0; w < 2; ++w) {
         const CountPlan& p = s->count_plan[w];
         if (!p.on) continue;
@@ -1099,6 +1148,7 @@ int setup_counts(pt_sim* s) {
         s->count_scratch.fill(t, p);
         t.keys = reinterpret_cast<uint16_t*>(s->keys);  // 3 x 2 of its 12 bytes per agent
         t.slots = (s->N + 7) / 8 * 8;
+        t.keys32 = s->keys;
         t.list = s->er_people;
         t.pk_bucket = s->stage_keys;
         t.pk_want = (uint32_t*)s->stage_ids;
@@ -1111,6 +1161,7 @@ int setup_counts(pt_sim* s) {
         t.sv_idx = (int32_t*)s->stage_keys + 2 * s->N;  // past the picks
         t.sv_pos = s->stage_ids + 2 * s->N;
         t.sv_f = s->sel_keys + 2 * s->N;
+        t.wp_lone = s->wp_lone;
         HIP_TRY(set_count_lds(p));
     }
     return PT_OK;
@@ -1125,7 +1176,7 @@ AgentArrays agent_arrays(pt_sim* s) {
     A.wp_people = s->wp_people;
     A.er_off = s->er_off;
     A.er_people = s->er_people;
-    A.wp_of = s->wp_of;
+    A.who = s->who;
     A.er_cnt = nullptr;
     A.er_keys = nullptr;
     A.er_slots = 0;
@@ -1223,10 +1274,10 @@ int enqueue_day(pt_sim* s, int d) {
     AgentArrays A = agent_arrays(s);
     const Model* M = s->d_model;
     if (counted) {
-        A.er_keys = ct.keys;
+        A.er_keys = cp.split ? nullptr : ct.keys;  // (weekend hour lists are not by agent)
         A.er_slots = ct.slots;
-        A.er_cnt = ct.pre + cp.reps[0].mbase + (int64_t)cp.reps[0].C * cp.reps[0].K;
-        enqueue_counts(cp, ct, &st->done, st, M, s->age, weekend, stc, tm);
+        A.er_cnt = ct.total;
+        enqueue_counts(cp, ct, &st->done, st, M, s->age, weekend, stc, tm, s->N, s->grid_gen);
     }
     // (A counted day counts every bucket: nothing to mark or decide.)
     if (!fused_plan)
@@ -1490,7 +1541,7 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
         dev_alloc(&s->dy_s, Npad) || dev_alloc(&s->gn_p, Npad) || dev_alloc(&s->gn_s, Npad) ||
         dev_alloc(&s->age, N) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
         dev_alloc(&s->hh_off, (int64_t)H + 1) ||
-        dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->wp_of, N) ||
+        dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->who, N) || dev_alloc(&s->wp_lone, 1) ||
         dev_alloc(&s->infected, N) ||
         dev_alloc(&s->staging, (int64_t)s->nblk_sweep * kSweepTile) || dev_alloc(&s->keys, n3 + 16) ||
         dev_alloc(&s->er_people, n3) || dev_alloc(&s->er_off, std::max<int64_t>(kmax, (int64_t)s->W) + 1) ||
@@ -1525,7 +1576,7 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
     // households is the workplace counter, PandemicSim.cu:2570-2571, :3817).
     s->workplace_off = (uint64_t)(H / 4);
     s->rand_after_setup = s->workplace_off + (uint64_t)(N / 4);
-    const PopArrays P{s->hh_types, s->hh_off, s->household, s->age, s->wp_off, s->wp_people, s->wp_of, s->st_p, s->st_s,
+    const PopArrays P{s->hh_types, s->hh_off, s->household, s->age, s->wp_off, s->wp_people, s->who, s->wp_lone, s->st_p, s->st_s,
                       s->dy_p, s->dy_s, s->gn_p, s->gn_s, s->claim_p, s->claim_s};
     hipError_t e = build_population(s->d_model, N, H, s->W, P, s->keys, s->tables, s->workplace_off, st,
                                     s->setup_ev + 2);

@@ -33,6 +33,7 @@ enum KernelClass : int {
     KC_SELECT,
     KC_SUBSET_SORT,  // idle: subset and full errand tables share one build (the sort classes); index kept
     KC_SETUP,
+    KC_TABLE_COUNT,
     KC_COUNT_SCAN,
     KC_COLLECT,
     KC_RESOLVE,

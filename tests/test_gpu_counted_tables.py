@@ -5,8 +5,10 @@ whole table.  Both must give the same days, state and generation tallies.
 Sizes: populations below one chunk and at odd remainders; so few buckets that
 a bucket's list in a chunk exceeds 64 ids (bisected instead of ranked); many
 nearly empty buckets (empty chunks of a bucket); bucket counts on both sides
-of the largest counted layout (40,000: weekday 2,901 per location scale,
-weekend 13,000), where only the weekday or neither layout is counted."""
+of the largest layout counted in one block (40,000: weekday 2,901 per
+location scale, weekend 13,000), of the 65,535 locations per hour up to which
+split weekday keys take 2 bytes, and of the 8 groups per hour up to which
+layouts are split at all."""
 import numpy as np
 import pytest
 
@@ -20,10 +22,16 @@ CASES = [
     (0.004, 0.0011, 9, 60),        # about 30 buckets for 9,400 agents
     (0.1, 0.0011, 9, 3000),        # the same for 235,000: lists of hundreds of ids
     (0.02, 0.3, 9, 300),
-    (0.05, 3.05, 9, 2000),         # weekend 39,650 buckets: both layouts counted
-    (0.05, 3.1, 9, 2000),          # weekend 40,300: sorted, weekday counted
+    (0.05, 3.05, 9, 2000),         # weekend 39,650 buckets: not split
+    (0.05, 3.1, 9, 2000),          # weekend 40,300: split by hour
     (0.05, 13.75, 6, 2000),        # weekday 39,889
-    (0.05, 13.85, 6, 2000),        # weekday 40,179: sorted
+    (0.05, 13.85, 6, 2000),        # weekday 40,179: split
+    (0.6, 21.24, 7, 20000),        # 1.4M agents: several chunks, one group per hour
+    (0.0004, 25.1, 7, 20),         # 943 agents; weekday hour 0 in two groups (40,160 locations)
+    (0.1, 40.9, 7, 5000),          # 65,440 locations in weekday hour 0
+    (0.1, 41.0, 7, 5000),          # 65,600: 4-byte keys
+    (0.3, 200.0, 7, 5000),         # 320,000: 8 groups
+    (0.05, 200.5, 7, 5000),        # 320,800: weekday sorted
 ]
 
 
