@@ -1,14 +1,21 @@
 // pt_mlp.hip — MLP ensemble surrogate on gfx950 MFMA (include/pandemic/pt_surrogate.h).
 //
-// All matrix products go through one tiled GEMM kernel on
-// v_mfma_f32_16x16x32_bf16: BF16 operands, FP32 accumulation.  A 256-thread
-// block computes a 64 x 64 tile of C = A * B (four waves, each 32 x 32 = 2 x 2
-// MFMA tiles), staging 64 x 64 slices of A and B in LDS per K step (16-byte
-// vector reads from global memory); operands may be read transposed, and the
-// epilogue fuses bias + GELU (forward),
-// bias (output layer), GELU backward (input gradients) or a plain FP32
-// store (weight gradients).  Every launch covers all ensemble members
-// (blockIdx.z), which train on the same batch.
+// All matrix products run on v_mfma_f32_16x16x32_bf16: BF16 operands, FP32
+// accumulation, K in ascending order.  Every launch covers all ensemble
+// members, which train on the same batch.  A training step is ten launches:
+//
+//   forward, 5   bias + GELU in the epilogue; the first layer gathers its
+//                rows of X itself, the last one goes on to the loss: output
+//                gradients, their column sums and the squared errors
+//   backward, 4  input gradients; GELU backward and the column sums in the
+//                epilogue (the first also closes the step's loss)
+//   update, 1    the weight gradients of all layers, each tile followed by
+//                its Adam step in the epilogue
+//
+// The products are small (2.7 GFLOP for 5 members at batch 1024, 1 us of the
+// chip's MFMA rate), so the loads' latency, the epilogues' traffic and the
+// launches bound a step: 5 members x 1024, 395 -> 202 us per step (19 launches
+// and the FP32 gradients' round trips before).
 //
 // MFMA lane layout (checked on the device): lane l supplies row l % 16 of A
 // and column l % 16 of B with eight K values each (K group l / 16), and
@@ -32,12 +39,14 @@ namespace {
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kDims[PT_MLP_LAYERS + 1] = {PT_MLP_IN, PT_MLP_HIDDEN, PT_MLP_HIDDEN, PT_MLP_HIDDEN, PT_MLP_HIDDEN,
                                            PT_MLP_OUT};
-constexpr int kTM = 64, kTN = 64, kTK = 64;
+constexpr int kTile = 64;      // rows and columns of a tile (the loss tiles: kColRows rows), K per step
 constexpr int kGemmThreads = 256;
+constexpr int kXcds = 8;
 constexpr int kMaxWidth = PT_MLP_OUT;  // widest layer output
 
 // Offsets of W_l and b_l in a member's parameter block.
@@ -63,221 +72,573 @@ __device__ __forceinline__ float gelu_grad(float x) {
     return cdf + x * pdf;
 }
 
-enum Epilogue : int { EPI_BIAS_GELU = 0, EPI_BIAS, EPI_GELU_GRAD, EPI_F32 };
-
-// Operands and outputs of one batched GEMM; *_z are per-member strides in
-// elements (0: shared by all members).
-struct GemmArgs {
-    const bf16* A;
-    int64_t lda, a_z;
-    const bf16* B;
-    int64_t ldb, b_z;
-    int M, N, K;
-    const float* bias;  // EPI_BIAS_GELU, EPI_BIAS
-    int64_t bias_z;
-    const float* pre;   // EPI_GELU_GRAD: pre-activations [M][N]
-    int64_t pre_z;
-    float* out_f32;     // pre-activations / outputs / input gradients / weight gradients
-    int64_t f32_z;
-    bf16* out_bf16;     // activations / input gradients
-    int64_t bf16_z;
-    int64_t ldc;
-    // EPI_GELU_GRAD (may be null): the FP32 column sums of each block's 64
-    // output rows, colpart[z][blockIdx.y][col] (N columns per row tile).
-    float* colpart;
+// One operand of a tile's product, ROWS (rows of A or columns of B) x K.
+// Stored with K contiguous (KMAJOR false: base[row * ld + k]) or with the
+// rows contiguous (base[k * ld + row]); either way 64 K values of it are runs
+// of 64 contiguous elements in memory, read by the whole block as 16-byte
+// vectors (every stride, offset and extent here is a multiple of 8) and kept
+// in LDS as they come, 128 bytes per run.  A K-contiguous fragment is one
+// 16-byte LDS read per lane; a K-major one is two transposing reads
+// (ds_read_b64_tr_b16: of 4 K rows x 16 columns, lane i of 16 receives column
+// i).  Runs are placed so that the 16 lanes of a fragment spread over all
+// banks: the 16-byte chunk index is XORed with the run's row.
+//
+// Rows past the operand's extent repeat its last one (their products are not
+// stored); K past its extent is zeroed on the way to LDS.
+template <bool KMAJOR, int ROWS>
+struct Operand {
+    static_assert(!KMAJOR || ROWS == kTile, "K-major operands come in 64-column tiles");
+    static constexpr int V = (KMAJOR ? kTile : ROWS) * 8 / kGemmThreads;  // vectors per thread and K step
+    const bf16* p;
+    int64_t ld;
+    int K;
+    int32_t at[V];  // runs of a K-contiguous operand
+    __device__ __forceinline__ Operand(const bf16* base, int64_t ld_, int extent, int row0, int K_)
+        : p(base), ld(ld_), K(K_) {
+        const int run = threadIdx.x >> 3, c = threadIdx.x & 7;
+        if (KMAJOR) {
+            p += row0 + (row0 + c * 8 < extent ? c * 8 : 0);
+        } else {
+#pragma unroll
+            for (int q = 0; q < V; ++q) at[q] = min(row0 + run + 32 * q, extent - 1);
+        }
+    }
+    __device__ __forceinline__ void load(bf16x8 (&v)[V], int k0) const {
+        const int run = threadIdx.x >> 3, c = threadIdx.x & 7;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const int k = KMAJOR ? k0 + run + 32 * q : k0 + c * 8;
+            const int kk = k < K ? k : k0;
+            v[q] = *reinterpret_cast<const bf16x8*>(KMAJOR ? p + (int64_t)kk * ld : p + (int64_t)at[q] * ld + kk);
+        }
+    }
+    __device__ __forceinline__ void store(bf16* s, const bf16x8 (&v)[V], int k0) const {
+        const int run = threadIdx.x >> 3, c = threadIdx.x & 7;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const int r = run + 32 * q;
+            bf16x8 x = v[q];
+            if (k0 + kTile > K && (KMAJOR ? k0 + r : k0 + c * 8) >= K) x = (bf16x8)(bf16)0.0f;
+            *reinterpret_cast<bf16x8*>(s + place(r, c)) = x;
+        }
+    }
+    // Element offset of chunk c of run r.
+    static __device__ __forceinline__ int place(int r, int c) {
+        if (KMAJOR) return ((r & 48) | ((r >> 3) & 1) | ((r & 7) << 1)) * kTile + (c ^ ((r & 3) << 1)) * 8;
+        return r * kTile + (c ^ ((r >> 1) & 7)) * 8;
+    }
+    // The fragment of K values k .. k + 31 of the 16 rows from row0.
+    static __device__ __forceinline__ bf16x8 fragment(const bf16* s, int row0, int k, int lane) {
+        const int g = lane >> 4, i = lane & 15;
+        if constexpr (KMAJOR) {
+            typedef __attribute__((address_space(3))) bf16x4* lds4;
+            const bf16* x = s + place(k + 8 * g + (i >> 2), row0 / 8 + ((i & 3) >> 1)) + (i & 1) * 4;
+            const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4)x);
+            const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4)(x + 8 * kTile));  // K + 4: 8 runs on
+            return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        } else {
+            return *reinterpret_cast<const bf16x8*>(s + place(row0 + i, k / 8 + g));
+        }
+    }
 };
 
-// C[M][N] = A(m, k) * B(k, n): A(m, k) = TA ? A[k lda + m] : A[m lda + k],
-// B(k, n) = TB ? B[n ldb + k] : B[k ldb + n].
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(kGemmThreads) void k_gemm(GemmArgs g) {
-    const int z = blockIdx.z;
-    const bf16* __restrict__ A = g.A + z * g.a_z;
-    const bf16* __restrict__ B = g.B + z * g.b_z;
-    const int m0 = blockIdx.y * kTM, n0 = blockIdx.x * kTN;
-    // Tiles stored [row or column][k] with rows of kTK + 8 bf16, so each
-    // lane's eight K values are one aligned 16-byte LDS read.
-    __shared__ __attribute__((aligned(16))) bf16 sA[kTM][kTK + 8];
-    __shared__ __attribute__((aligned(16))) bf16 sB[kTN][kTK + 8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    floatx4 acc[2][2];
+constexpr int kRowPad = kTile + 4;  // floats per row of an output tile in LDS
+constexpr size_t tile_lds(int TM) { return (size_t)2 * (TM + kTile) * kTile * sizeof(bf16); }
+static_assert(tile_lds(kTile) >= kTile * kRowPad * sizeof(float) && tile_lds(128) >= 128 * kRowPad * sizeof(float),
+              "an output tile fits in the operands' LDS");
+
+// acc = A * B over all of K for one TM x 64 tile; four waves, each
+// (TM / 2) x 32.  One barrier per K step of 64: operands are double buffered
+// in LDS and loaded two steps ahead into registers, so that a K of 512 pays
+// the memory latency about once (with one step ahead, two barriers and K-major
+// operands transposed in the registers of a single wave: 16-24 us per product
+// of 2.7 GFLOP, now 13, of which GELU and the stores are half).  Ends with a barrier: LDS may be reused.
+template <int TM, class OA, class OB>
+__device__ __forceinline__ void tile_product(const OA& A, const OB& B, int K, bf16* s,
+                                             floatx4 (&acc)[TM / 32][2]) {
+    constexpr int MI = TM / 32;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * 32;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 zero8 = (bf16x8)(bf16)0.0f;
-    // Global reads are 16-byte vectors of 8 consecutive elements of the
-    // contiguous dimension (every stride, offset and extent here is a
-    // multiple of 8, so a vector is wholly inside or wholly outside).  An
-    // operand stored K-major (A with TA, B without TB) is read by one wave
-    // (wave 0 for A, wave 1 for B) as 8 x 8 blocks, 8 K rows of 8
-    // consecutive M or N, transposed in registers and stored as 16-byte LDS
-    // rows of 8 K values.  The next K step's vectors are loaded before the
-    // current step's products, so their latency overlaps the MFMA work.
-    constexpr int kVec = kTM * kTK / 8 / kGemmThreads;  // vectors per thread per operand
-    static_assert(kTM == 64 && kTN == 64 && kTK == 64, "the 8 x 8 block loads assume 64 x 64 tiles");
-    bf16x8 ra[TA ? 8 : kVec], rb[TB ? kVec : 8];
-    const int bk = (lane >> 3) * 8, bmn = (lane & 7) * 8;  // this lane's 8 x 8 block: K rows, M / N columns
-    auto load = [&](int k0) {
-        if constexpr (TA) {
-            if (wave == 0) {
-                const int m = m0 + bmn;
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int k = k0 + bk + r;
-                    ra[r] = zero8;
-                    if (m < g.M && k < g.K) ra[r] = *reinterpret_cast<const bf16x8*>(A + (int64_t)k * g.lda + m);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < kVec; ++q) {
-                const int v = tid + q * kGemmThreads;
-                const int mm = v / (kTK / 8), kk = (v % (kTK / 8)) * 8;
-                const int m = m0 + mm, k = k0 + kk;
-                ra[q] = zero8;
-                if (m < g.M && k < g.K) ra[q] = *reinterpret_cast<const bf16x8*>(A + (int64_t)m * g.lda + k);
-            }
-        }
-        if constexpr (!TB) {
-            if (wave == 1) {
-                const int n = n0 + bmn;
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int k = k0 + bk + r;
-                    rb[r] = zero8;
-                    if (n < g.N && k < g.K) rb[r] = *reinterpret_cast<const bf16x8*>(B + (int64_t)k * g.ldb + n);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < kVec; ++q) {
-                const int v = tid + q * kGemmThreads;
-                const int nn = v / (kTK / 8), kk = (v % (kTK / 8)) * 8;
-                const int n = n0 + nn, k = k0 + kk;
-                rb[q] = zero8;
-                if (n < g.N && k < g.K) rb[q] = *reinterpret_cast<const bf16x8*>(B + (int64_t)n * g.ldb + k);
-            }
-        }
-    };
-    // Row c of the transposed block: element r is x[r][c].
-    auto column = [](const bf16x8 (&x)[8], int c) {
-        bf16x8 o;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) o[r] = x[r][c];
-        return o;
-    };
-    auto stage = [&]() {
-        if constexpr (TA) {
-            if (wave == 0) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) *reinterpret_cast<bf16x8*>(&sA[bmn + c][bk]) = column(ra, c);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < kVec; ++q) {
-                const int v = tid + q * kGemmThreads;
-                const int mm = v / (kTK / 8), kk = (v % (kTK / 8)) * 8;
-                *reinterpret_cast<bf16x8*>(&sA[mm][kk]) = ra[q];
-            }
-        }
-        if constexpr (!TB) {
-            if (wave == 1) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) *reinterpret_cast<bf16x8*>(&sB[bmn + c][bk]) = column(rb, c);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < kVec; ++q) {
-                const int v = tid + q * kGemmThreads;
-                const int nn = v / (kTK / 8), kk = (v % (kTK / 8)) * 8;
-                *reinterpret_cast<bf16x8*>(&sB[nn][kk]) = rb[q];
-            }
-        }
-    };
-    load(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stage();
-        __syncthreads();
-        if (k0 + kTK < g.K) load(k0 + kTK);
-#pragma unroll
-        for (int kc = 0; kc < kTK; kc += 32) {
-            const int kq = kc + 8 * (lane >> 4);
-#pragma unroll
-            for (int ti = 0; ti < 2; ++ti) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sA[wm + ti * 16 + (lane & 15)][kq]);
-#pragma unroll
-                for (int tj = 0; tj < 2; ++tj) {
-                    const bf16x8 b = *reinterpret_cast<const bf16x8*>(&sB[wn + tj * 16 + (lane & 15)][kq]);
-                    acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[ti][tj], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
+    bf16* const sa[2] = {s, s + (TM + kTile) * kTile};
+    bf16* const sb[2] = {s + TM * kTile, s + (TM + kTile + TM) * kTile};
+    bf16x8 ra[2][OA::V], rb[2][OB::V];
+    A.load(ra[0], 0);
+    B.load(rb[0], 0);
+    if (kTile < K) {
+        A.load(ra[1], kTile);
+        B.load(rb[1], kTile);
     }
-    float cs[2] = {0.f, 0.f};  // EPI_GELU_GRAD: this lane's column sums
+    A.store(sa[0], ra[0], 0);
+    B.store(sb[0], rb[0], 0);
+    if (2 * kTile < K) {
+        A.load(ra[0], 2 * kTile);
+        B.load(rb[0], 2 * kTile);
+    }
+    __syncthreads();
+    for (int k0 = 0; k0 < K; k0 += 2 * kTile) {
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti)
-#pragma unroll
-        for (int tj = 0; tj < 2; ++tj)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm + ti * 16 + 4 * (lane >> 4) + r;
-                const int col = n0 + wn + tj * 16 + (lane & 15);
-                if (row >= g.M || col >= g.N) continue;
-                const float v = acc[ti][tj][r];
-                const int64_t o = (int64_t)row * g.ldc + col;
-                if (EPI == EPI_BIAS_GELU) {
-                    const float pre = v + g.bias[z * g.bias_z + col];
-                    g.out_f32[z * g.f32_z + o] = pre;
-                    g.out_bf16[z * g.bf16_z + o] = (bf16)gelu(pre);
-                } else if (EPI == EPI_BIAS) {
-                    g.out_f32[z * g.f32_z + o] = v + g.bias[z * g.bias_z + col];
-                } else if (EPI == EPI_GELU_GRAD) {
-                    const float d = v * gelu_grad(g.pre[z * g.pre_z + o]);
-                    g.out_f32[z * g.f32_z + o] = d;
-                    g.out_bf16[z * g.bf16_z + o] = (bf16)d;
-                    cs[tj] += d;
-                } else {
-                    g.out_f32[z * g.f32_z + o] = v;
+        for (int h = 0; h < 2; ++h) {
+            const int k = k0 + h * kTile;
+            if (k >= K) break;
+            if (k + kTile < K) {
+                A.store(sa[1 - h], ra[1 - h], k + kTile);
+                B.store(sb[1 - h], rb[1 - h], k + kTile);
+                if (k + 3 * kTile < K) {
+                    A.load(ra[1 - h], k + 3 * kTile);
+                    B.load(rb[1 - h], k + 3 * kTile);
                 }
             }
-    if constexpr (EPI == EPI_GELU_GRAD) {
-        // Column sums of the tile: this lane's 8 rows, then the 4 lane
-        // groups of a 16-column slice, then the two row halves, in that
-        // fixed order.
-        if (g.colpart) {
-            __shared__ float s_cs[2][kTN];
 #pragma unroll
-            for (int tj = 0; tj < 2; ++tj) {
-                cs[tj] += __shfl_xor(cs[tj], 16, 64);
-                cs[tj] += __shfl_xor(cs[tj], 32, 64);
-                if (lane < 16) s_cs[wm / 32][wn + tj * 16 + lane] = cs[tj];
+            for (int kc = 0; kc < kTile; kc += 32) {
+                bf16x8 b[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) b[j] = OB::fragment(sb[h], wn + j * 16, kc, lane);
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const bf16x8 a = OA::fragment(sa[h], wm + i * 16, kc, lane);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
+                }
             }
             __syncthreads();
-            const int col = n0 + tid;
-            if (tid < kTN && col < g.N)
-                g.colpart[((int64_t)z * gridDim.y + blockIdx.y) * g.N + col] = s_cs[0][tid] + s_cs[1][tid];
         }
     }
 }
 
-// Batch gather: xb[b][i] = bf16(X[rows[b]][i]), yb[b][j] = Y[rows[b]][j].
-// step (may be null): [0] the step index within a training call, which
-// selects the batch's rows order + step[0] * B.
-__global__ void k_gather(const float* __restrict__ X, const float* __restrict__ Y, const int32_t* __restrict__ order,
-                         const int64_t* __restrict__ step, int B, bf16* __restrict__ xb, float* __restrict__ yb) {
-    const int32_t* rows = order + (step ? step[0] * B : 0);
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    const int64_t nx = (int64_t)B * PT_MLP_IN, ny = (int64_t)B * PT_MLP_OUT;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nx + ny; i += stride) {
-        if (i < nx) {
-            const int64_t b = i / PT_MLP_IN, c = i % PT_MLP_IN;
-            xb[i] = (bf16)X[(int64_t)rows[b] * PT_MLP_IN + c];
+// The tile in LDS, row by row, so that the epilogues read and write global
+// memory as 256-byte runs (four columns per thread, 16 rows per turn).
+template <int TM>
+__device__ __forceinline__ void tile_to_rows(const floatx4 (&acc)[TM / 32][2], float (*sc)[kRowPad]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * 32;
+#pragma unroll
+    for (int i = 0; i < TM / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[wm + i * 16 + 4 * (lane >> 4) + r][wn + j * 16 + (lane & 15)] = acc[i][j][r];
+    __syncthreads();
+}
+
+__device__ __forceinline__ floatx4 load4(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
+__device__ __forceinline__ void store4(float* p, floatx4 v) { *reinterpret_cast<floatx4*>(p) = v; }
+__device__ __forceinline__ void store4(bf16* p, floatx4 v) {
+    bf16x4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = (bf16)v[k];
+    *reinterpret_cast<bf16x4*>(p) = o;
+}
+
+// Blocks go round the XCDs, each with an L2 of its own: XCD x works through
+// the x-th eighth of the tiles, so that the tiles that share operand rows, and
+// a member's weights, share an L2.  -1: no tile.
+__device__ __forceinline__ int tile_of_block(int block, int tiles) {
+    const int per = (tiles + kXcds - 1) / kXcds, t = (block % kXcds) * per + block / kXcds;
+    return block / kXcds < per && t < tiles ? t : -1;
+}
+inline int blocks_for_tiles(int tiles) { return (tiles + kXcds - 1) / kXcds * kXcds; }
+
+// Where a training batch's rows come from: row b of the batch is row
+// rows[step * B + b] of X and Y (rows null: row b itself).
+struct Batch {
+    const float *X, *Y;
+    const int32_t* rows;
+    const int64_t* step;  // may be null: step 0
+    __device__ __forceinline__ const int32_t* first(int B) const { return rows ? rows + (step ? step[0] * B : 0) : rows; }
+};
+
+// One layer forward, C = act * W + bias over M rows.
+enum Forward : int { FWD_FIRST = 0, FWD_HIDDEN, FWD_OUT, FWD_LOSS };
+struct ForwardArgs {
+    const bf16* A;  // activations [M][K]; FWD_FIRST writes them (the batch in BF16)
+    int64_t a_z;    // per-member stride in elements (0: shared by all members)
+    const bf16* W;  // [K][N]
+    const float* bias;
+    int64_t param_z;
+    int M, N, K, members;
+    float* pre;     // FWD_FIRST, FWD_HIDDEN: pre-activations; FWD_OUT: outputs
+    int64_t pre_z;
+    bf16* act;      // FWD_FIRST, FWD_HIDDEN: activations; FWD_LOSS: output gradients
+    int64_t act_z;
+    Batch batch;    // FWD_FIRST, FWD_LOSS
+    bf16* xb;       // FWD_FIRST (may be null): the batch's inputs in BF16
+    float* part;    // FWD_LOSS: squared errors per tile [member][tile]
+    float* colpart; // FWD_LOSS: column sums [member][row chunk][N]
+};
+
+// Bias gradients: db[n] = sum over rows of dz[row][n], per member.  Partial
+// sums per row chunk come with the gradients: 64-row tiles of the hidden
+// layers, chunks of kColRows rows of the output layer (4 row groups, added in
+// a fixed order); the update adds the chunks in order.  Every order is fixed,
+// so the result does not depend on scheduling.
+constexpr int kColGroups = 4, kColRows = 128;
+
+template <int MODE>
+__global__ __launch_bounds__(kGemmThreads, MODE == FWD_LOSS ? 3 : 4) void k_forward(ForwardArgs g) {
+    constexpr int TM = MODE == FWD_LOSS ? kColRows : kTile;
+    __shared__ __attribute__((aligned(16))) bf16 s[tile_lds(TM) / sizeof(bf16)];
+    __shared__ float s_sum[kColGroups][kTile];
+    const int tn = (g.N + kTile - 1) / kTile, tm = (g.M + TM - 1) / TM;
+    const int t = tile_of_block(blockIdx.x, tn * tm * g.members);
+    if (t < 0) return;
+    const int z = t / (tn * tm), mt = t / tn % tm, m0 = mt * TM, n0 = t % tn * kTile;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const Operand<true, kTile> B(g.W + z * g.param_z, g.N, g.N, n0, g.K);
+    floatx4 acc[TM / 32][2];
+    if constexpr (MODE == FWD_FIRST) {
+        // K = 16: one MFMA per tile, its K past 16 zero; rows gathered from X
+        // by 64 x 2 threads.
+        typedef Operand<false, kTile> OA;
+        bf16x8 rb[2];
+        B.load(rb, 0);
+        const int32_t* rows = g.batch.first(g.M);
+        const int r = tid >> 2, c = tid & 3, m = min(m0 + r, g.M - 1);
+        bf16x8 x = (bf16x8)(bf16)0.0f;
+        if (c * 8 < PT_MLP_IN) {
+            const float* src = g.batch.X + (int64_t)(rows ? rows[m] : m) * PT_MLP_IN + c * 8;
+            const floatx4 lo = load4(src), hi = load4(src + 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                x[k] = (bf16)lo[k];
+                x[k + 4] = (bf16)hi[k];
+            }
+            if (g.xb && z == 0 && n0 == 0 && m0 + r < g.M)
+                *reinterpret_cast<bf16x8*>(g.xb + (int64_t)m * PT_MLP_IN + c * 8) = x;
+        }
+        *reinterpret_cast<bf16x8*>(s + OA::place(r, c)) = x;
+        bf16* sb = s + kTile * kTile;
+        B.store(sb, rb, 0);
+        __syncthreads();
+        const int wave = tid >> 6, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    OA::fragment(s, wm + i * 16, 0, lane), Operand<true, kTile>::fragment(sb, wn + j * 16, 0, lane),
+                    floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        __syncthreads();
+    } else {
+        const Operand<false, TM> A(g.A + z * g.a_z, g.K, g.M, m0, g.K);
+        tile_product<TM>(A, B, g.K, s, acc);
+    }
+    float(*sc)[kRowPad] = reinterpret_cast<float(*)[kRowPad]>(s);
+    tile_to_rows<TM>(acc, sc);
+    const int c4 = (tid & 15) * 4, col = n0 + c4;
+    const bool in = col < g.N;
+    const floatx4 bias = in ? load4(g.bias + z * g.param_z + col) : floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (MODE != FWD_LOSS) {
+#pragma unroll
+        for (int q = 0; q < TM / 16; ++q) {
+            const int r = q * 16 + (tid >> 4), row = m0 + r;
+            if (!in || row >= g.M) continue;
+            const int64_t o = (int64_t)row * g.N + col;
+            const floatx4 pre = load4(&sc[r][c4]) + bias;
+            store4(g.pre + z * g.pre_z + o, pre);
+            if (MODE != FWD_OUT) {
+                floatx4 a;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) a[k] = gelu(pre[k]);
+                store4(g.act + z * g.act_z + o, a);
+            }
+        }
+    } else {
+        // Mean-squared error: dz = 2 (pred - y) / (M * N), in BF16 for the
+        // products and in FP32 for the column sums.
+        const int32_t* rows = g.batch.first(g.M);
+        const float scale = 2.0f / (float)((int64_t)g.M * g.N);
+        float e = 0.f;
+#pragma unroll
+        for (int q = 0; q < TM / 16; ++q) {
+            const int r = q * 16 + (tid >> 4), row = m0 + r;
+            if (!in || row >= g.M) continue;
+            const floatx4 pred = load4(&sc[r][c4]) + bias;
+            const floatx4 y = load4(g.batch.Y + (int64_t)(rows ? rows[row] : row) * g.N + col);
+            floatx4 dz;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float d = pred[k] - y[k];
+                e += d * d;
+                dz[k] = d * scale;
+            }
+            store4(g.act + z * g.act_z + (int64_t)row * g.N + col, dz);
+            store4(&sc[r][c4], dz);
+        }
+#pragma unroll
+        for (int x = 32; x; x >>= 1) e += __shfl_xor(e, x, 64);
+        __shared__ float s_e[kGemmThreads / 64];
+        if (lane == 0) s_e[tid >> 6] = e;
+        __syncthreads();
+        const int c = tid % kTile, grp = tid / kTile, rn = min(TM, g.M - m0);
+        float sum = 0.f;
+        for (int r = grp; r < rn; r += kColGroups) sum += sc[r][c];
+        s_sum[grp][c] = sum;
+        __syncthreads();
+        if (tid == 0) g.part[(z * tm + mt) * tn + n0 / kTile] = s_e[0] + s_e[1] + s_e[2] + s_e[3];
+        if (grp == 0 && n0 + c < g.N) {
+            float tot = 0.f;
+#pragma unroll
+            for (int q = 0; q < kColGroups; ++q) tot += s_sum[q][c];
+            g.colpart[((int64_t)z * tm + mt) * g.N + n0 + c] = tot;
+        }
+    }
+}
+
+// The loss of every member from its tiles' squared errors, in a fixed order,
+// by one block; then the step index advances, and the bias corrections
+// 1 - beta^t of the Adam step that follows, t = Adam steps taken before this
+// one + 1, are set.
+struct StepArgs {
+    const float* part;
+    int tiles, members;  // tiles per member
+    int64_t n;           // outputs per member
+    float* loss;
+    int64_t loss_z;
+    int64_t* step;       // null: one loss per member, no Adam step; [0] step of the call, [1] Adam steps before the call
+    float* bias_corr;    // [2]
+};
+__device__ __forceinline__ void finish_loss(const StepArgs& a) {
+    const int lane = threadIdx.x & 63;
+    const int64_t at = a.step ? a.step[0] : 0;
+    for (int z = threadIdx.x >> 6; z < a.members; z += kGemmThreads / 64) {
+        float t = 0.f;
+        for (int b = lane; b < a.tiles; b += 64) t += a.part[z * a.tiles + b];
+#pragma unroll
+        for (int x = 32; x; x >>= 1) t += __shfl_xor(t, x, 64);
+        if (lane == 0) a.loss[z * a.loss_z + at] = t / (float)a.n;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && a.step) {
+        const double t = (double)(a.step[1] + at + 1);
+        a.bias_corr[0] = (float)(1.0 - pow(0.9, t));
+        a.bias_corr[1] = (float)(1.0 - pow(0.999, t));
+        a.step[0] = at + 1;
+    }
+}
+
+// Input gradients of a layer: dz_in = (dz W^T) * gelu'(pre), M rows, N = the
+// layer's inputs, K = its outputs; and their column sums per 64-row tile,
+// colpart[member][row tile][N].  finish (the first of the chain): the block
+// after the tiles closes the loss.
+struct BackwardArgs {
+    const bf16* dz;
+    int64_t dz_z;
+    const bf16* W;  // [N][K]
+    int64_t param_z;
+    int M, N, K, members;
+    const float* pre;
+    int64_t pre_z;
+    bf16* out;
+    int64_t out_z;
+    float* colpart;
+    int finish;
+    StepArgs step;
+};
+__global__ __launch_bounds__(kGemmThreads, 4) void k_backward(BackwardArgs g) {
+    __shared__ __attribute__((aligned(16))) bf16 s[tile_lds(kTile) / sizeof(bf16)];
+    __shared__ float s_cs[2][kTile];
+    const int tn = (g.N + kTile - 1) / kTile, tm = (g.M + kTile - 1) / kTile, tiles = tn * tm * g.members;
+    if (g.finish) {
+        if (blockIdx.x == gridDim.x - 1) return finish_loss(g.step);
+    }
+    const int t = tile_of_block(blockIdx.x, tiles);
+    if (t < 0) return;
+    const int z = t / (tn * tm), mt = t / tn % tm, m0 = mt * kTile, n0 = t % tn * kTile;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int c4 = (tid & 15) * 4, col = n0 + c4;
+    // (M and N are multiples of 64 here: batches and hidden layers)
+    floatx4 pre[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        pre[q] = load4(g.pre + z * g.pre_z + (int64_t)(m0 + q * 16 + (tid >> 4)) * g.N + col);
+    const Operand<false, kTile> A(g.dz + z * g.dz_z, g.K, g.M, m0, g.K), B(g.W + z * g.param_z, g.K, g.N, n0, g.K);
+    floatx4 acc[2][2];
+    tile_product<kTile>(A, B, g.K, s, acc);
+    float(*sc)[kRowPad] = reinterpret_cast<float(*)[kRowPad]>(s);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) store4(&sc[q * 16 + (tid >> 4)][c4], pre[q]);
+    __syncthreads();
+    // Column sums of the tile: this lane's 8 rows, then the 4 lane groups of
+    // a 16-column slice, then the two row halves, in that fixed order.
+    float cs[2] = {0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float* x = &sc[wm + i * 16 + 4 * (lane >> 4) + r][wn + j * 16 + (lane & 15)];
+                const float d = acc[i][j][r] * gelu_grad(*x);
+                *x = d;
+                cs[j] += d;
+            }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        cs[j] += __shfl_xor(cs[j], 16, 64);
+        cs[j] += __shfl_xor(cs[j], 32, 64);
+        if (lane < 16) s_cs[wm / 32][wn + j * 16 + lane] = cs[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = q * 16 + (tid >> 4);
+        store4(g.out + z * g.out_z + (int64_t)(m0 + r) * g.N + col, load4(&sc[r][c4]));
+    }
+    if (tid < kTile) g.colpart[((int64_t)z * tm + mt) * g.N + n0 + tid] = s_cs[0][tid] + s_cs[1][tid];
+}
+
+// Adam on one FP32 master parameter.
+__device__ __forceinline__ void adam(float& p, float& m1, float& m2, float gi, float lr, float bc1, float bc2) {
+    const float a = 0.9f * m1 + 0.1f * gi;
+    const float b = 0.999f * m2 + 0.001f * gi * gi;
+    m1 = a;
+    m2 = b;
+    const float mh = a / bc1, vh = b / bc2;
+    p = p - lr * mh / (sqrtf(vh) + 1e-8f);
+}
+
+// Weight and bias gradients of every layer, dW = act^T dz over the batch and
+// the column sums' totals: stored (ADAM false), or used at once for the Adam
+// step of the tile's parameters, which saves the gradients' round trip.  Bound
+// by the parameters' traffic (26 bytes each).  Blocks: the layers' tiles
+// member by member, then 256 biases per block.
+struct UpdateArgs {
+    const bf16* act[PT_MLP_LAYERS];
+    int64_t act_z[PT_MLP_LAYERS];
+    const bf16* dz[PT_MLP_LAYERS];
+    int64_t dz_z[PT_MLP_LAYERS];
+    const float* colpart[PT_MLP_LAYERS];  // [member][R][width]
+    int R_hidden, R_out;
+    int members, batch;
+    int64_t count;                        // parameters per member
+    float* grads;
+    float *p, *m1, *m2;
+    bf16* pb;
+    float lr;
+    const float* bias_corr;
+};
+constexpr int layer_tiles(int l) { return (kDims[l] + kTile - 1) / kTile * ((kDims[l + 1] + kTile - 1) / kTile); }
+constexpr int member_tiles() {
+    int n = 0;
+    for (int l = 0; l < PT_MLP_LAYERS; ++l) n += layer_tiles(l);
+    return n;
+}
+constexpr int member_biases() {
+    int n = 0;
+    for (int l = 0; l < PT_MLP_LAYERS; ++l) n += kDims[l + 1];
+    return n;
+}
+constexpr int kBiasBlocks = (member_biases() + kGemmThreads - 1) / kGemmThreads;
+
+template <bool ADAM>
+__global__ __launch_bounds__(kGemmThreads, 4) void k_update(UpdateArgs g) {
+    __shared__ __attribute__((aligned(16))) bf16 s[tile_lds(kTile) / sizeof(bf16)];
+    const int tid = threadIdx.x, tiles = member_tiles() * g.members;
+    float bc1 = 0.f, bc2 = 0.f;
+    if (ADAM) {
+        bc1 = g.bias_corr[0];
+        bc2 = g.bias_corr[1];
+    }
+    const int tile_blocks = (tiles + kXcds - 1) / kXcds * kXcds;
+    if ((int)blockIdx.x >= tile_blocks) {
+        const int b = blockIdx.x - tile_blocks, z = b / kBiasBlocks;
+        int j = b % kBiasBlocks * kGemmThreads + tid;
+        int64_t at = z * g.count;
+#pragma unroll
+        for (int l = 0; l < PT_MLP_LAYERS; ++l) {
+            const int n = kDims[l + 1];
+            at += (int64_t)kDims[l] * n;
+            if (j >= 0 && j < n) {
+                const int R = l == PT_MLP_LAYERS - 1 ? g.R_out : g.R_hidden;
+                const float* c = g.colpart[l] + (int64_t)z * R * n + j;
+                float sum = 0.f;
+                for (int r = 0; r < R; ++r) sum += c[(int64_t)r * n];
+                const int64_t i = at + j;
+                if (ADAM) {
+                    float p = g.p[i], m1 = g.m1[i], m2 = g.m2[i];
+                    adam(p, m1, m2, sum, g.lr, bc1, bc2);
+                    g.m1[i] = m1;
+                    g.m2[i] = m2;
+                    g.p[i] = p;
+                    g.pb[i] = (bf16)p;
+                } else {
+                    g.grads[i] = sum;
+                }
+            }
+            j -= n;
+            at += n;
+        }
+        return;
+    }
+    const int t = tile_of_block(blockIdx.x, tiles);
+    if (t < 0) return;
+    const int z = t / member_tiles();
+    int tl = t % member_tiles(), M = 0, N = 0;
+    int64_t at = z * g.count, act_z = 0, dz_z = 0;
+    const bf16 *act = nullptr, *dz = nullptr;
+    bool found = false;
+#pragma unroll
+    for (int l = 0; l < PT_MLP_LAYERS; ++l) {
+        if (found) continue;
+        M = kDims[l];
+        N = kDims[l + 1];
+        act = g.act[l];
+        act_z = g.act_z[l];
+        dz = g.dz[l];
+        dz_z = g.dz_z[l];
+        if (tl < layer_tiles(l)) {
+            found = true;
         } else {
-            const int64_t j = i - nx, b = j / PT_MLP_OUT, c = j % PT_MLP_OUT;
-            yb[j] = Y[(int64_t)rows[b] * PT_MLP_OUT + c];
+            tl -= layer_tiles(l);
+            at += (int64_t)M * N + N;
+        }
+    }
+    const int tn = (N + kTile - 1) / kTile, m0 = tl / tn * kTile, n0 = tl % tn * kTile;
+    const Operand<true, kTile> A(act + z * act_z, M, M, m0, g.batch), B(dz + z * dz_z, N, N, n0, g.batch);
+    floatx4 acc[2][2];
+    tile_product<kTile>(A, B, g.batch, s, acc);
+    const int c4 = (tid & 15) * 4, col = n0 + c4;
+    floatx4 p[4], m1[4], m2[4];
+    if (ADAM) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = m0 + q * 16 + (tid >> 4);
+            if (row >= M || col >= N) continue;
+            const int64_t i = at + (int64_t)row * N + col;
+            p[q] = load4(g.p + i);
+            m1[q] = load4(g.m1 + i);
+            m2[q] = load4(g.m2 + i);
+        }
+    }
+    float(*sc)[kRowPad] = reinterpret_cast<float(*)[kRowPad]>(s);
+    tile_to_rows<kTile>(acc, sc);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = q * 16 + (tid >> 4), row = m0 + r;
+        if (row >= M || col >= N) continue;
+        const int64_t i = at + (int64_t)row * N + col;
+        const floatx4 gi = load4(&sc[r][c4]);
+        if (ADAM) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float pk = p[q][k], m1k = m1[q][k], m2k = m2[q][k];
+                adam(pk, m1k, m2k, gi[k], g.lr, bc1, bc2);
+                p[q][k] = pk;
+                m1[q][k] = m1k;
+                m2[q][k] = m2k;
+            }
+            store4(g.m1 + i, m1[q]);
+            store4(g.m2 + i, m2[q]);
+            store4(g.p + i, p[q]);
+            store4(g.pb + i, p[q]);
+        } else {
+            store4(g.grads + i, gi);
         }
     }
 }
@@ -285,161 +646,6 @@ __global__ void k_gather(const float* __restrict__ X, const float* __restrict__ 
 __global__ void k_to_bf16(const float* __restrict__ x, int64_t n, bf16* __restrict__ y) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) y[i] = (bf16)x[i];
-}
-
-constexpr int kLossThreads = 256;
-constexpr int kLossBlocks = 64;
-
-// Mean-squared error of member blockIdx.y: dz = 2 (pred - y) / (B * 720)
-// (FP32 and BF16) and per-block partial sums of (pred - y)^2.
-__global__ __launch_bounds__(kLossThreads) void k_loss(const float* __restrict__ pred, const float* __restrict__ yb,
-                                                       int B, float* __restrict__ dz32, bf16* __restrict__ dz16,
-                                                       int64_t dz_z, float* __restrict__ part) {
-    const int z = blockIdx.y;
-    const int64_t n = (int64_t)B * PT_MLP_OUT;
-    const float* p = pred + z * n;
-    const float scale = 2.0f / (float)n;
-    float s = 0.f;
-    for (int64_t i = (int64_t)blockIdx.x * kLossThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kLossThreads) {
-        const float d = p[i] - yb[i];
-        s += d * d;
-        const float g = d * scale;
-        dz32[z * dz_z + i] = g;
-        dz16[z * dz_z + i] = (bf16)g;
-    }
-    __shared__ float s_w[kLossThreads / 64];
-    s = s + __shfl_xor(s, 32, 64);
-    s = s + __shfl_xor(s, 16, 64);
-    s = s + __shfl_xor(s, 8, 64);
-    s = s + __shfl_xor(s, 4, 64);
-    s = s + __shfl_xor(s, 2, 64);
-    s = s + __shfl_xor(s, 1, 64);
-    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int w = 0; w < kLossThreads / 64; ++w) t += s_w[w];
-        part[z * gridDim.x + blockIdx.x] = t;
-    }
-}
-
-// Loss of member threadIdx.x from the block partials, in a fixed order.
-// step (may be null): [0] the step index, the loss's column.
-__global__ void k_loss_final(const float* __restrict__ part, int nblk, int members, int64_t n,
-                             float* __restrict__ loss, int64_t loss_z, const int64_t* __restrict__ step) {
-    const int z = threadIdx.x;
-    if (z >= members) return;
-    float t = 0.f;
-    for (int b = 0; b < nblk; ++b) t += part[z * nblk + b];
-    loss[z * loss_z + (step ? step[0] : 0)] = t / (float)n;
-}
-
-// Bias gradients: db[n] = sum over rows of dz[row][n], per member.  Partial
-// sums per row chunk: for a hidden layer the input-gradient GEMM's epilogue
-// leaves them (64-row tiles); for the output layer k_colsum_part sums a
-// chunk of kColRows rows for 64 columns (4 row groups, added in a fixed
-// order) into part[z][chunk][n].  k_colsum_final adds the chunks in order.
-// Every order is fixed, so the result does not depend on scheduling.
-constexpr int kColCols = 64, kColGroups = 4, kColRows = 128;
-__global__ __launch_bounds__(kColCols * kColGroups) void k_colsum_part(const float* __restrict__ dz, int M, int N,
-                                                                      int64_t dz_z, float* __restrict__ part) {
-    const int z = blockIdx.z, chunk = blockIdx.y, R = gridDim.y;
-    const int c = threadIdx.x % kColCols, grp = threadIdx.x / kColCols;
-    const int n = blockIdx.x * kColCols + c;
-    const float* d = dz + z * dz_z;
-    const int m1 = min(M, (chunk + 1) * kColRows);
-    float s = 0.f;
-    if (n < N)
-        for (int m = chunk * kColRows + grp; m < m1; m += kColGroups) s += d[(int64_t)m * N + n];
-    __shared__ float s_p[kColGroups][kColCols];
-    s_p[grp][c] = s;
-    __syncthreads();
-    if (grp == 0 && n < N) {
-        float t = 0.f;
-#pragma unroll
-        for (int q = 0; q < kColGroups; ++q) t += s_p[q][c];
-        part[((int64_t)z * R + chunk) * N + n] = t;
-    }
-}
-
-__global__ void k_colsum_final(const float* __restrict__ part, int R, int N, int members, float* __restrict__ db,
-                               int64_t db_z) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= members * N) return;
-    const int z = i / N, n = i % N;
-    float t = 0.f;
-    for (int r = 0; r < R; ++r) t += part[((int64_t)z * R + r) * N + n];
-    db[z * db_z + n] = t;
-}
-
-// Adam on the FP32 master parameters, then their BF16 copies.
-// Adam with bias corrections 1 - beta^t for t = step[1] + 1 (the Adam
-// steps taken before this one, plus this one).
-// Bias gradients (colpart set): summed here from layer l's partial sums,
-// slice l of colpart ([member][R][width], R = r_out chunks for the output
-// layer, r_hidden tiles for the others), in chunk order, the order
-// k_colsum_final uses, instead of read from g.  Grid: x over one member's
-// count parameters, y = member.
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
-                       float* __restrict__ m2, bf16* __restrict__ pb, int64_t count, float lr,
-                       const int64_t* __restrict__ step, const float* __restrict__ colpart, int64_t slice,
-                       int r_hidden, int r_out) {
-    const double t = (double)(step[1] + 1);
-    const float bc1 = (float)(1.0 - pow(0.9, t)), bc2 = (float)(1.0 - pow(0.999, t));
-    const int z = blockIdx.y;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < count; j += stride) {
-        const int64_t i = (int64_t)z * count + j;
-        int bl = -1;
-        int64_t bj = 0, o = 0;
-#pragma unroll
-        for (int l = 0; l < PT_MLP_LAYERS; ++l) {
-            o += (int64_t)kDims[l] * kDims[l + 1];
-            if (j >= o && j < o + kDims[l + 1]) {
-                bl = l;
-                bj = j - o;
-            }
-            o += kDims[l + 1];
-        }
-        float gi;
-        if (colpart && bl >= 0) {
-            const int R = bl == PT_MLP_LAYERS - 1 ? r_out : r_hidden;
-            const int N = kDims[bl + 1];
-            const float* c = colpart + bl * slice + (int64_t)z * R * N + bj;
-            float s = 0.f;
-            for (int r = 0; r < R; ++r) s += c[(int64_t)r * N];
-            gi = s;
-        } else {
-            gi = g[i];
-        }
-        const float a = 0.9f * m1[i] + 0.1f * gi;
-        const float b = 0.999f * m2[i] + 0.001f * gi * gi;
-        m1[i] = a;
-        m2[i] = b;
-        const float mh = a / bc1, vh = b / bc2;
-        const float w = p[i] - lr * mh / (sqrtf(vh) + 1e-8f);
-        p[i] = w;
-        pb[i] = (bf16)w;
-    }
-}
-
-// Ends a training step: the next step's index and Adam count.
-// The end of a training step: k_loss_final for every member (threads
-// 0..members-1, loss column step[0]), then the step index and the Adam
-// step count advance.
-__global__ void k_loss_step(const float* __restrict__ part, int nblk, int members, int64_t n,
-                            float* __restrict__ loss, int64_t loss_z, int64_t* __restrict__ step) {
-    const int z = threadIdx.x;
-    if (z < members) {
-        float t = 0.f;
-        for (int b = 0; b < nblk; ++b) t += part[z * nblk + b];
-        loss[z * loss_z + step[0]] = t / (float)n;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        step[0] += 1;
-        step[1] += 1;
-    }
 }
 
 }  // namespace
@@ -457,13 +663,11 @@ struct pt_mlp {
     int32_t* order = nullptr;
     int64_t order_cap = 0;
     bf16* xb = nullptr;
-    float* yb = nullptr;
-    bf16* act[PT_MLP_LAYERS] = {};   // act[0] = xb; act[1..4] hidden outputs
+    bf16* act[PT_MLP_LAYERS] = {};   // act[1..4]: hidden outputs
     float* pre[PT_MLP_LAYERS - 1] = {};
     float* pred = nullptr;
-    float* dz32[2] = {};
-    bf16* dz16[2] = {};
-    float* part = nullptr;
+    bf16* dz[PT_MLP_LAYERS] = {};  // gradients of the layers' outputs before GELU
+    float* part = nullptr;         // squared errors per output tile
     float* colpart = nullptr;  // bias-gradient partial sums [layers][members][row chunks or tiles][kMaxWidth]
     float* loss = nullptr;
     int64_t loss_cap = 0;
@@ -475,130 +679,114 @@ struct pt_mlp {
     // taken.  One step is captured as a HIP graph per training call and
     // replayed (use_graphs), or enqueued kernel by kernel.
     int64_t* d_step = nullptr;
+    float* bias_corr = nullptr;  // Adam's bias corrections of the step (finish_loss)
     bool use_graphs = true;
 };
 
 namespace {
 
 int64_t act_z(const pt_mlp* m) { return (int64_t)m->batch * PT_MLP_HIDDEN; }
-int64_t dz_z(const pt_mlp* m) { return (int64_t)m->batch * kMaxWidth; }
+int64_t dz_z(const pt_mlp* m, int l) { return (int64_t)m->batch * kDims[l + 1]; }
+int out_tiles(int rows) { return (rows + kColRows - 1) / kColRows * ((PT_MLP_OUT + kTile - 1) / kTile); }
+int row_tiles(const pt_mlp* m) { return (m->batch + kTile - 1) / kTile; }
+// Floats per layer slice of colpart: members x (row tiles) x kMaxWidth.
+int64_t colpart_slice(const pt_mlp* m) { return (int64_t)m->members * row_tiles(m) * kMaxWidth; }
 
-template <bool TA, bool TB, int EPI>
-void gemm(pt_mlp* m, const GemmArgs& g) {
-    const dim3 grid((g.N + kTN - 1) / kTN, (g.M + kTM - 1) / kTM, m->members);
-    k_gemm<TA, TB, EPI><<<grid, kGemmThreads, 0, m->stream>>>(g);
-}
-
-GemmArgs args() {
-    GemmArgs g;
-    memset(&g, 0, sizeof g);
-    return g;
-}
-
-// Forward pass of every member on rows already in xb (rows <= batch).
-void forward(pt_mlp* m, int rows) {
-    const int64_t P = m->L.count;
+// Forward pass of every member on `rows` rows (at most batch) of b: outputs
+// into pred, or (training) the loss and the output gradients.
+void forward(pt_mlp* m, int rows, const Batch& b, bool training) {
     for (int l = 0; l < PT_MLP_LAYERS; ++l) {
-        GemmArgs g = args();
-        g.A = m->act[l];
-        g.lda = kDims[l];
-        g.a_z = l == 0 ? 0 : act_z(m);
-        g.B = m->wb + m->L.w[l];
-        g.ldb = kDims[l + 1];
-        g.b_z = P;
+        ForwardArgs g;
+        memset(&g, 0, sizeof g);
+        g.A = l == 0 ? nullptr : m->act[l];
+        g.a_z = act_z(m);
+        g.W = m->wb + m->L.w[l];
+        g.bias = m->params + m->L.b[l];
+        g.param_z = m->L.count;
         g.M = rows;
         g.N = kDims[l + 1];
         g.K = kDims[l];
-        g.bias = m->params + m->L.b[l];
-        g.bias_z = P;
-        g.ldc = kDims[l + 1];
-        if (l < PT_MLP_LAYERS - 1) {
-            g.out_f32 = m->pre[l];
-            g.f32_z = act_z(m);
-            g.out_bf16 = m->act[l + 1];
-            g.bf16_z = act_z(m);
-            gemm<false, false, EPI_BIAS_GELU>(m, g);
+        g.members = m->members;
+        g.batch = b;
+        const bool out = l == PT_MLP_LAYERS - 1;
+        const int tiles = (g.N + kTile - 1) / kTile * ((rows + kTile - 1) / kTile) * m->members;
+        if (!out) {
+            g.pre = m->pre[l];
+            g.pre_z = act_z(m);
+            g.act = m->act[l + 1];
+            g.act_z = act_z(m);
+            if (l == 0 && training) g.xb = m->xb;
+            (l == 0 ? k_forward<FWD_FIRST> : k_forward<FWD_HIDDEN>)<<<blocks_for_tiles(tiles), kGemmThreads, 0,
+                                                                     m->stream>>>(g);
+        } else if (!training) {
+            g.pre = m->pred;
+            g.pre_z = (int64_t)m->batch * PT_MLP_OUT;
+            k_forward<FWD_OUT><<<blocks_for_tiles(tiles), kGemmThreads, 0, m->stream>>>(g);
         } else {
-            g.out_f32 = m->pred;
-            g.f32_z = (int64_t)m->batch * PT_MLP_OUT;
-            gemm<false, false, EPI_BIAS>(m, g);
+            g.act = m->dz[l];
+            g.act_z = dz_z(m, l);
+            g.part = m->part;
+            g.colpart = m->colpart + l * colpart_slice(m);
+            k_forward<FWD_LOSS><<<blocks_for_tiles(out_tiles(rows) * m->members), kGemmThreads, 0, m->stream>>>(g);
         }
     }
 }
 
-int64_t colpart_slice(const pt_mlp* m);
-
-// Loss and gradients of every member for the batch in xb / yb.
-// step (may be null): the training step counters (the loss column).
-// bias_sums: also add the bias gradients' partial sums into grads and the
-// loss partials into loss (else the partials stay for k_adam, in colpart's
-// per-layer slices, and for k_loss_step, in part).
-void backward(pt_mlp* m, float* loss, int64_t loss_z, const int64_t* step, bool bias_sums) {
-    const int64_t P = m->L.count;
-    const int B = m->batch;
-    k_loss<<<dim3(kLossBlocks, m->members), kLossThreads, 0, m->stream>>>(m->pred, m->yb, B, m->dz32[0], m->dz16[0],
-                                                                          dz_z(m), m->part);
-    if (bias_sums)
-        k_loss_final<<<1, 64, 0, m->stream>>>(m->part, kLossBlocks, m->members, (int64_t)B * PT_MLP_OUT, loss, loss_z,
-                                              step);
-    int cur = 0;
-    for (int l = PT_MLP_LAYERS - 1; l >= 0; --l) {
-        const int nout = kDims[l + 1], nin = kDims[l];
-        // dW_l = act_l^T dz_l
-        GemmArgs g = args();
-        g.A = m->act[l];
-        g.lda = nin;
-        g.a_z = l == 0 ? 0 : act_z(m);
-        g.B = m->dz16[cur];
-        g.ldb = nout;
-        g.b_z = dz_z(m);
-        g.M = nin;
-        g.N = nout;
-        g.K = B;
-        g.out_f32 = m->grads + m->L.w[l];
-        g.f32_z = P;
-        g.ldc = nout;
-        gemm<true, false, EPI_F32>(m, g);
-        // db_l: the output layer's dz comes from the loss kernel and is summed
-        // here in 128-row chunks; a hidden layer's column sums per 64-row
-        // tile came with its dz from the input-gradient GEMM's epilogue.
-        int R = (B + kTM - 1) / kTM;
-        float* part_l = m->colpart + l * colpart_slice(m);
-        if (l == PT_MLP_LAYERS - 1) {
-            R = (B + kColRows - 1) / kColRows;
-            k_colsum_part<<<dim3((nout + kColCols - 1) / kColCols, R, m->members), kColCols * kColGroups, 0,
-                            m->stream>>>(m->dz32[cur], B, nout, dz_z(m), part_l);
-        }
-        if (bias_sums)
-            k_colsum_final<<<(m->members * nout + 255) / 256, 256, 0, m->stream>>>(part_l, R, nout, m->members,
-                                                                                  m->grads + m->L.b[l], P);
-        if (l == 0) break;
+// Gradients of every member after forward(training), and the loss.  step (may
+// be null): the training step counters.
+void backward(pt_mlp* m, float* loss, int64_t loss_z, int64_t* step) {
+    for (int l = PT_MLP_LAYERS - 1; l > 0; --l) {
         // dz_{l-1} = (dz_l W_l^T) * gelu'(pre_{l-1})
-        GemmArgs h = args();
-        h.A = m->dz16[cur];
-        h.lda = nout;
-        h.a_z = dz_z(m);
-        h.B = m->wb + m->L.w[l];
-        h.ldb = nout;
-        h.b_z = P;
-        h.M = B;
-        h.N = nin;
-        h.K = nout;
-        h.pre = m->pre[l - 1];
-        h.pre_z = act_z(m);
-        h.out_f32 = m->dz32[1 - cur];
-        h.f32_z = dz_z(m);
-        h.out_bf16 = m->dz16[1 - cur];
-        h.bf16_z = dz_z(m);
-        h.ldc = nin;
-        h.colpart = m->colpart + (l - 1) * colpart_slice(m);
-        gemm<false, true, EPI_GELU_GRAD>(m, h);
-        cur = 1 - cur;
+        BackwardArgs g;
+        memset(&g, 0, sizeof g);
+        g.dz = m->dz[l];
+        g.dz_z = dz_z(m, l);
+        g.W = m->wb + m->L.w[l];
+        g.param_z = m->L.count;
+        g.M = m->batch;
+        g.N = kDims[l];
+        g.K = kDims[l + 1];
+        g.members = m->members;
+        g.pre = m->pre[l - 1];
+        g.pre_z = act_z(m);
+        g.out = m->dz[l - 1];
+        g.out_z = dz_z(m, l - 1);
+        g.colpart = m->colpart + (l - 1) * colpart_slice(m);
+        g.finish = l == PT_MLP_LAYERS - 1;
+        g.step = StepArgs{m->part, out_tiles(m->batch), m->members, (int64_t)m->batch * PT_MLP_OUT, loss, loss_z, step,
+                          m->bias_corr};
+        const int tiles = g.N / kTile * row_tiles(m) * m->members;
+        k_backward<<<blocks_for_tiles(tiles) + g.finish, kGemmThreads, 0, m->stream>>>(g);
     }
 }
 
-// Floats per layer slice of colpart: members x (row tiles of kTM) x kMaxWidth.
-int64_t colpart_slice(const pt_mlp* m) { return (int64_t)m->members * ((m->batch + kTM - 1) / kTM) * kMaxWidth; }
+// Weight and bias gradients after backward: Adam steps, or (adam false) left
+// in grads.
+void update(pt_mlp* m, bool adam, float lr) {
+    UpdateArgs g;
+    memset(&g, 0, sizeof g);
+    for (int l = 0; l < PT_MLP_LAYERS; ++l) {
+        g.act[l] = l == 0 ? m->xb : m->act[l];
+        g.act_z[l] = l == 0 ? 0 : act_z(m);
+        g.dz[l] = m->dz[l];
+        g.dz_z[l] = dz_z(m, l);
+        g.colpart[l] = m->colpart + l * colpart_slice(m);
+    }
+    g.R_hidden = row_tiles(m);
+    g.R_out = (m->batch + kColRows - 1) / kColRows;
+    g.members = m->members;
+    g.batch = m->batch;
+    g.count = m->L.count;
+    g.grads = m->grads;
+    g.p = m->params;
+    g.m1 = m->m1;
+    g.m2 = m->m2;
+    g.pb = m->wb;
+    g.lr = lr;
+    g.bias_corr = m->bias_corr;
+    const int blocks = blocks_for_tiles(member_tiles() * m->members) + kBiasBlocks * m->members;
+    (adam ? k_update<true> : k_update<false>)<<<blocks, kGemmThreads, 0, m->stream>>>(g);
+}
 
 int upload_rows(pt_mlp* m, const int32_t* rows, int64_t n) {
     for (int64_t i = 0; i < n; ++i)
@@ -635,20 +823,17 @@ int pt_mlp_create(int32_t members, int32_t batch, int32_t device, pt_mlp** out) 
     const int64_t P = m->L.count * members;
     bool bad = dev_alloc(&m->params, P) || dev_alloc(&m->grads, P) || dev_alloc(&m->m1, P) || dev_alloc(&m->m2, P) ||
                dev_alloc(&m->wb, P) || dev_alloc(&m->xb, (int64_t)batch * PT_MLP_IN) ||
-               dev_alloc(&m->yb, (int64_t)batch * PT_MLP_OUT) ||
                dev_alloc(&m->pred, (int64_t)members * batch * PT_MLP_OUT) ||
-               dev_alloc(&m->part, (int64_t)members * kLossBlocks) ||
-               dev_alloc(&m->colpart, (int64_t)PT_MLP_LAYERS * members * ((batch + kTM - 1) / kTM) * kMaxWidth);
+               dev_alloc(&m->part, (int64_t)members * out_tiles(batch)) ||
+               dev_alloc(&m->colpart, PT_MLP_LAYERS * colpart_slice(m)) || dev_alloc(&m->bias_corr, 2);
     for (int l = 1; l < PT_MLP_LAYERS && !bad; ++l) bad = dev_alloc(&m->act[l], members * act_z(m)) != 0;
     for (int l = 0; l < PT_MLP_LAYERS - 1 && !bad; ++l) bad = dev_alloc(&m->pre[l], members * act_z(m)) != 0;
-    for (int i = 0; i < 2 && !bad; ++i)
-        bad = dev_alloc(&m->dz32[i], members * dz_z(m)) || dev_alloc(&m->dz16[i], members * dz_z(m));
+    for (int l = 0; l < PT_MLP_LAYERS && !bad; ++l) bad = dev_alloc(&m->dz[l], members * dz_z(m, l)) != 0;
     if (bad) {
         const std::string msg = pt_last_error();
         pt_mlp_destroy(m);
         return fail(PT_ENOMEM, "%s", msg.c_str());
     }
-    m->act[0] = m->xb;
     (void)hipEventCreate(&m->ev0);
     (void)hipEventCreate(&m->ev1);
     if (dev_alloc(&m->d_step, 2)) {
@@ -705,21 +890,14 @@ int pt_mlp_train(pt_mlp* m, const int32_t* order, int32_t steps, float lr, float
         if (dev_alloc(&m->loss, (int64_t)steps * m->members)) return PT_ENOMEM;
         m->loss_cap = (int64_t)steps * m->members;
     }
-    const int64_t P = m->L.count * m->members;
     // Every kernel of a step reads the step index and Adam count from
     // d_step, so one captured step serves all of them.
     const int64_t h_step[2] = {0, m->t};
     HIP_TRY(hipMemcpyAsync(m->d_step, h_step, sizeof h_step, hipMemcpyHostToDevice, m->stream));
     auto one_step = [&]() {
-        k_gather<<<grid_for((int64_t)B * (PT_MLP_IN + PT_MLP_OUT), 256, 4096), 256, 0, m->stream>>>(
-            m->X, m->Y, m->order, m->d_step, B, m->xb, m->yb);
-        forward(m, B);
-        backward(m, m->loss, steps, m->d_step, false);
-        k_adam<<<dim3(grid_for(m->L.count, 256, 2048), m->members), 256, 0, m->stream>>>(
-            m->params, m->grads, m->m1, m->m2, m->wb, m->L.count, lr, m->d_step, m->colpart, colpart_slice(m),
-            (B + kTM - 1) / kTM, (B + kColRows - 1) / kColRows);
-        k_loss_step<<<1, 64, 0, m->stream>>>(m->part, kLossBlocks, m->members, (int64_t)B * PT_MLP_OUT, m->loss,
-                                             steps, m->d_step);
+        forward(m, B, Batch{m->X, m->Y, m->order, m->d_step}, true);
+        backward(m, m->loss, steps, m->d_step);
+        update(m, true, lr);
     };
     // The instantiated step graph, released on every return.
     struct ExecGuard {
@@ -780,10 +958,9 @@ int pt_mlp_gradients(pt_mlp* m, const int32_t* rows, float* grads_out, float* lo
         if (dev_alloc(&m->loss, m->members)) return PT_ENOMEM;
         m->loss_cap = m->members;
     }
-    k_gather<<<grid_for((int64_t)B * (PT_MLP_IN + PT_MLP_OUT), 256, 4096), 256, 0, m->stream>>>(
-        m->X, m->Y, m->order, (const int64_t*)nullptr, B, m->xb, m->yb);
-    forward(m, B);
-    backward(m, m->loss, 1, nullptr, true);
+    forward(m, B, Batch{m->X, m->Y, m->order, nullptr}, true);
+    backward(m, m->loss, 1, nullptr);
+    update(m, false, 0.f);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(m->stream));
     HIP_TRY(hipMemcpy(grads_out, m->grads, sizeof(float) * m->L.count * m->members, hipMemcpyDeviceToHost));
@@ -805,9 +982,7 @@ int pt_mlp_predict(pt_mlp* m, const float* X, int64_t n, float* out) {
     std::vector<float> h((size_t)m->members * B * PT_MLP_OUT);
     for (int64_t i0 = 0; i0 < n; i0 += B) {
         const int rows = (int)std::min<int64_t>(B, n - i0);
-        k_to_bf16<<<grid_for((int64_t)rows * PT_MLP_IN, 256, 1024), 256, 0, m->stream>>>(
-            m->xin + i0 * PT_MLP_IN, (int64_t)rows * PT_MLP_IN, m->xb);
-        forward(m, rows);
+        forward(m, rows, Batch{m->xin + i0 * PT_MLP_IN, nullptr, nullptr, nullptr}, false);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpyAsync(h.data(), m->pred, sizeof(float) * h.size(), hipMemcpyDeviceToHost, m->stream));
         HIP_TRY(hipStreamSynchronize(m->stream));
@@ -839,13 +1014,10 @@ void pt_mlp_destroy(pt_mlp* m) {
     dev_free(m->Y);
     dev_free(m->order);
     dev_free(m->xb);
-    dev_free(m->yb);
     for (int l = 1; l < PT_MLP_LAYERS; ++l) dev_free(m->act[l]);
     for (int l = 0; l < PT_MLP_LAYERS - 1; ++l) dev_free(m->pre[l]);
-    for (int i = 0; i < 2; ++i) {
-        dev_free(m->dz32[i]);
-        dev_free(m->dz16[i]);
-    }
+    for (int l = 0; l < PT_MLP_LAYERS; ++l) dev_free(m->dz[l]);
+    dev_free(m->bias_corr);
     dev_free(m->pred);
     dev_free(m->part);
     dev_free(m->colpart);
