@@ -14,7 +14,7 @@
 //
 // The products are small (2.7 GFLOP for 5 members at batch 1024, 1 us of the
 // chip's MFMA rate), so the loads' latency, the epilogues' traffic and the
-// launches bound a step: 5 members x 1024, 395 -> 202 us per step (19 launches
+// launches bound a step: 5 members x 1024, 395 -> 165 us per step (19 launches
 // and the FP32 gradients' round trips before).
 //
 // MFMA lane layout (checked on the device): lane l supplies row l % 16 of A
@@ -64,10 +64,11 @@ struct Layout {
     }
 };
 
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
-
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
+// 2 Phi(x); GELU and its derivative from it.
+__device__ __forceinline__ float two_phi(float x) { return 1.0f + erff(x * 0.70710678118654752f); }
+__device__ __forceinline__ float gelu(float x, float phi2) { return 0.5f * x * phi2; }
+__device__ __forceinline__ float gelu_grad(float x, float phi2) {
+    const float cdf = 0.5f * phi2;
     const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
     return cdf + x * pdf;
 }
@@ -89,27 +90,34 @@ template <bool KMAJOR, int ROWS>
 struct Operand {
     static_assert(!KMAJOR || ROWS == kTile, "K-major operands come in 64-column tiles");
     static constexpr int V = (KMAJOR ? kTile : ROWS) * 8 / kGemmThreads;  // vectors per thread and K step
-    const bf16* p;
+    const bf16* p;     // uniform; this thread's vectors are at 32-bit offsets
     int64_t ld;
     int K;
-    int32_t at[V];  // runs of a K-contiguous operand
+    uint32_t at[V];    // vectors of K step 0
+    uint32_t back[V];  // and how far back the step's first K value is
     __device__ __forceinline__ Operand(const bf16* base, int64_t ld_, int extent, int row0, int K_)
         : p(base), ld(ld_), K(K_) {
         const int run = threadIdx.x >> 3, c = threadIdx.x & 7;
-        if (KMAJOR) {
-            p += row0 + (row0 + c * 8 < extent ? c * 8 : 0);
-        } else {
 #pragma unroll
-            for (int q = 0; q < V; ++q) at[q] = min(row0 + run + 32 * q, extent - 1);
+        for (int q = 0; q < V; ++q) {
+            const int r = run + 32 * q;
+            back[q] = KMAJOR ? (uint32_t)r * (uint32_t)ld : (uint32_t)c * 8;
+            at[q] = back[q] + (KMAJOR ? (uint32_t)(row0 + (row0 + c * 8 < extent ? c * 8 : 0))
+                                      : (uint32_t)min(row0 + r, extent - 1) * (uint32_t)ld);
         }
     }
     __device__ __forceinline__ void load(bf16x8 (&v)[V], int k0) const {
         const int run = threadIdx.x >> 3, c = threadIdx.x & 7;
+        const bf16* pk = p + (KMAJOR ? k0 * ld : (int64_t)k0);
+        if (k0 + kTile <= K) {
 #pragma unroll
-        for (int q = 0; q < V; ++q) {
-            const int k = KMAJOR ? k0 + run + 32 * q : k0 + c * 8;
-            const int kk = k < K ? k : k0;
-            v[q] = *reinterpret_cast<const bf16x8*>(KMAJOR ? p + (int64_t)kk * ld : p + (int64_t)at[q] * ld + kk);
+            for (int q = 0; q < V; ++q) v[q] = *reinterpret_cast<const bf16x8*>(pk + at[q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                const bool in = k0 + (KMAJOR ? run + 32 * q : c * 8) < K;
+                v[q] = *reinterpret_cast<const bf16x8*>(pk + (in ? at[q] : at[q] - back[q]));
+            }
         }
     }
     __device__ __forceinline__ void store(bf16* s, const bf16x8 (&v)[V], int k0) const {
@@ -118,7 +126,9 @@ struct Operand {
         for (int q = 0; q < V; ++q) {
             const int r = run + 32 * q;
             bf16x8 x = v[q];
-            if (k0 + kTile > K && (KMAJOR ? k0 + r : k0 + c * 8) >= K) x = (bf16x8)(bf16)0.0f;
+            if (k0 + kTile > K) {
+                if ((KMAJOR ? k0 + r : k0 + c * 8) >= K) x = (bf16x8)(bf16)0.0f;
+            }
             *reinterpret_cast<bf16x8*>(s + place(r, c)) = x;
         }
     }
@@ -152,7 +162,7 @@ static_assert(tile_lds(kTile) >= kTile * kRowPad * sizeof(float) && tile_lds(128
 // in LDS and loaded two steps ahead into registers, so that a K of 512 pays
 // the memory latency about once (with one step ahead, two barriers and K-major
 // operands transposed in the registers of a single wave: 16-24 us per product
-// of 2.7 GFLOP, now 13, of which GELU and the stores are half).  Ends with a barrier: LDS may be reused.
+// of 2.7 GFLOP, now 12-14, of which GELU and the stores are half).  Ends with a barrier: LDS may be reused.
 template <int TM, class OA, class OB>
 __device__ __forceinline__ void tile_product(const OA& A, const OB& B, int K, bf16* s,
                                              floatx4 (&acc)[TM / 32][2]) {
@@ -261,8 +271,8 @@ struct ForwardArgs {
     const float* bias;
     int64_t param_z;
     int M, N, K, members;
-    float* pre;     // FWD_FIRST, FWD_HIDDEN: pre-activations; FWD_OUT: outputs
-    int64_t pre_z;
+    float* out;     // FWD_FIRST, FWD_HIDDEN (null: prediction): gelu'(pre-activations); FWD_OUT: outputs
+    int64_t out_z;
     bf16* act;      // FWD_FIRST, FWD_HIDDEN: activations; FWD_LOSS: output gradients
     int64_t act_z;
     Batch batch;    // FWD_FIRST, FWD_LOSS
@@ -338,14 +348,20 @@ __global__ __launch_bounds__(kGemmThreads, MODE == FWD_LOSS ? 3 : 4) void k_forw
             const int r = q * 16 + (tid >> 4), row = m0 + r;
             if (!in || row >= g.M) continue;
             const int64_t o = (int64_t)row * g.N + col;
-            const floatx4 pre = load4(&sc[r][c4]) + bias;
-            store4(g.pre + z * g.pre_z + o, pre);
+            floatx4 pre = load4(&sc[r][c4]) + bias;
             if (MODE != FWD_OUT) {
-                floatx4 a;
+                floatx4 a, phi2;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) a[k] = gelu(pre[k]);
+                for (int k = 0; k < 4; ++k) {
+                    phi2[k] = two_phi(pre[k]);
+                    a[k] = gelu(pre[k], phi2[k]);
+                }
                 store4(g.act + z * g.act_z + o, a);
+                if (!g.out) continue;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pre[k] = gelu_grad(pre[k], phi2[k]);
             }
+            store4(g.out + z * g.out_z + o, pre);
         }
     } else {
         // Mean-squared error: dz = 2 (pred - y) / (M * N), in BF16 for the
@@ -421,7 +437,7 @@ __device__ __forceinline__ void finish_loss(const StepArgs& a) {
     }
 }
 
-// Input gradients of a layer: dz_in = (dz W^T) * gelu'(pre), M rows, N = the
+// Input gradients of a layer: dz_in = (dz W^T) * slope, M rows, N = the
 // layer's inputs, K = its outputs; and their column sums per 64-row tile,
 // colpart[member][row tile][N].  finish (the first of the chain): the block
 // after the tiles closes the loss.
@@ -431,8 +447,8 @@ struct BackwardArgs {
     const bf16* W;  // [N][K]
     int64_t param_z;
     int M, N, K, members;
-    const float* pre;
-    int64_t pre_z;
+    const float* slope;  // gelu'(pre-activations), from the forward pass (which has the erf at hand)
+    int64_t slope_z;
     bf16* out;
     int64_t out_z;
     float* colpart;
@@ -453,16 +469,16 @@ __global__ __launch_bounds__(kGemmThreads, 4) void k_backward(BackwardArgs g) {
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     const int c4 = (tid & 15) * 4, col = n0 + c4;
     // (M and N are multiples of 64 here: batches and hidden layers)
-    floatx4 pre[4];
+    floatx4 slope[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        pre[q] = load4(g.pre + z * g.pre_z + (int64_t)(m0 + q * 16 + (tid >> 4)) * g.N + col);
+        slope[q] = load4(g.slope + z * g.slope_z + (int64_t)(m0 + q * 16 + (tid >> 4)) * g.N + col);
     const Operand<false, kTile> A(g.dz + z * g.dz_z, g.K, g.M, m0, g.K), B(g.W + z * g.param_z, g.K, g.N, n0, g.K);
     floatx4 acc[2][2];
     tile_product<kTile>(A, B, g.K, s, acc);
     float(*sc)[kRowPad] = reinterpret_cast<float(*)[kRowPad]>(s);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) store4(&sc[q * 16 + (tid >> 4)][c4], pre[q]);
+    for (int q = 0; q < 4; ++q) store4(&sc[q * 16 + (tid >> 4)][c4], slope[q]);
     __syncthreads();
     // Column sums of the tile: this lane's 8 rows, then the 4 lane groups of
     // a 16-column slice, then the two row halves, in that fixed order.
@@ -474,7 +490,7 @@ __global__ __launch_bounds__(kGemmThreads, 4) void k_backward(BackwardArgs g) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float* x = &sc[wm + i * 16 + 4 * (lane >> 4) + r][wn + j * 16 + (lane & 15)];
-                const float d = acc[i][j][r] * gelu_grad(*x);
+                const float d = acc[i][j][r] * *x;
                 *x = d;
                 cs[j] += d;
             }
@@ -506,7 +522,8 @@ __device__ __forceinline__ void adam(float& p, float& m1, float& m2, float gi, f
 // Weight and bias gradients of every layer, dW = act^T dz over the batch and
 // the column sums' totals: stored (ADAM false), or used at once for the Adam
 // step of the tile's parameters, which saves the gradients' round trip.  Bound
-// by the parameters' traffic (26 bytes each).  Blocks: the layers' tiles
+// by memory: the parameters' 26 bytes each and the operands, 200 MB in 44 us
+// for 5 members at batch 1024.  Blocks: the layers' tiles
 // member by member, then 256 biases per block.
 struct UpdateArgs {
     const bf16* act[PT_MLP_LAYERS];
@@ -664,7 +681,7 @@ struct pt_mlp {
     int64_t order_cap = 0;
     bf16* xb = nullptr;
     bf16* act[PT_MLP_LAYERS] = {};   // act[1..4]: hidden outputs
-    float* pre[PT_MLP_LAYERS - 1] = {};
+    float* slope[PT_MLP_LAYERS - 1] = {};  // gelu' of the hidden layers' pre-activations
     float* pred = nullptr;
     bf16* dz[PT_MLP_LAYERS] = {};  // gradients of the layers' outputs before GELU
     float* part = nullptr;         // squared errors per output tile
@@ -676,7 +693,7 @@ struct pt_mlp {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0;
     // Training steps: [0] step index within the current call, [1] Adam steps
-    // taken.  One step is captured as a HIP graph per training call and
+    // taken.  Up to eight steps are captured as a HIP graph per training call and
     // replayed (use_graphs), or enqueued kernel by kernel.
     int64_t* d_step = nullptr;
     float* bias_corr = nullptr;  // Adam's bias corrections of the step (finish_loss)
@@ -711,16 +728,16 @@ void forward(pt_mlp* m, int rows, const Batch& b, bool training) {
         const bool out = l == PT_MLP_LAYERS - 1;
         const int tiles = (g.N + kTile - 1) / kTile * ((rows + kTile - 1) / kTile) * m->members;
         if (!out) {
-            g.pre = m->pre[l];
-            g.pre_z = act_z(m);
+            if (training) g.out = m->slope[l];
+            g.out_z = act_z(m);
             g.act = m->act[l + 1];
             g.act_z = act_z(m);
             if (l == 0 && training) g.xb = m->xb;
             (l == 0 ? k_forward<FWD_FIRST> : k_forward<FWD_HIDDEN>)<<<blocks_for_tiles(tiles), kGemmThreads, 0,
                                                                      m->stream>>>(g);
         } else if (!training) {
-            g.pre = m->pred;
-            g.pre_z = (int64_t)m->batch * PT_MLP_OUT;
+            g.out = m->pred;
+            g.out_z = (int64_t)m->batch * PT_MLP_OUT;
             k_forward<FWD_OUT><<<blocks_for_tiles(tiles), kGemmThreads, 0, m->stream>>>(g);
         } else {
             g.act = m->dz[l];
@@ -736,7 +753,7 @@ void forward(pt_mlp* m, int rows, const Batch& b, bool training) {
 // be null): the training step counters.
 void backward(pt_mlp* m, float* loss, int64_t loss_z, int64_t* step) {
     for (int l = PT_MLP_LAYERS - 1; l > 0; --l) {
-        // dz_{l-1} = (dz_l W_l^T) * gelu'(pre_{l-1})
+        // dz_{l-1} = (dz_l W_l^T) * slope_{l-1}
         BackwardArgs g;
         memset(&g, 0, sizeof g);
         g.dz = m->dz[l];
@@ -747,8 +764,8 @@ void backward(pt_mlp* m, float* loss, int64_t loss_z, int64_t* step) {
         g.N = kDims[l];
         g.K = kDims[l + 1];
         g.members = m->members;
-        g.pre = m->pre[l - 1];
-        g.pre_z = act_z(m);
+        g.slope = m->slope[l - 1];
+        g.slope_z = act_z(m);
         g.out = m->dz[l - 1];
         g.out_z = dz_z(m, l - 1);
         g.colpart = m->colpart + (l - 1) * colpart_slice(m);
@@ -827,7 +844,7 @@ int pt_mlp_create(int32_t members, int32_t batch, int32_t device, pt_mlp** out) 
                dev_alloc(&m->part, (int64_t)members * out_tiles(batch)) ||
                dev_alloc(&m->colpart, PT_MLP_LAYERS * colpart_slice(m)) || dev_alloc(&m->bias_corr, 2);
     for (int l = 1; l < PT_MLP_LAYERS && !bad; ++l) bad = dev_alloc(&m->act[l], members * act_z(m)) != 0;
-    for (int l = 0; l < PT_MLP_LAYERS - 1 && !bad; ++l) bad = dev_alloc(&m->pre[l], members * act_z(m)) != 0;
+    for (int l = 0; l < PT_MLP_LAYERS - 1 && !bad; ++l) bad = dev_alloc(&m->slope[l], members * act_z(m)) != 0;
     for (int l = 0; l < PT_MLP_LAYERS && !bad; ++l) bad = dev_alloc(&m->dz[l], members * dz_z(m, l)) != 0;
     if (bad) {
         const std::string msg = pt_last_error();
@@ -899,7 +916,10 @@ int pt_mlp_train(pt_mlp* m, const int32_t* order, int32_t steps, float lr, float
         backward(m, m->loss, steps, m->d_step);
         update(m, true, lr);
     };
-    // The instantiated step graph, released on every return.
+    // Steps per graph: 8 us pass between two graphs (100 steps of 5 x 1024, one
+    // step per graph: 0.8 ms).
+    const int per = std::min(steps, 8);
+    // The instantiated graph, released on every return.
     struct ExecGuard {
         hipGraphExec_t e = nullptr;
         ~ExecGuard() {
@@ -909,7 +929,7 @@ int pt_mlp_train(pt_mlp* m, const int32_t* order, int32_t steps, float lr, float
     if (m->use_graphs) {
         hipGraph_t graph = nullptr;
         HIP_TRY(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        one_step();
+        for (int k = 0; k < per; ++k) one_step();
         // Ends the capture whatever happened inside it; a failed launch
         // there is reported here.
         const hipError_t ce = hipStreamEndCapture(m->stream, &graph);
@@ -922,12 +942,14 @@ int pt_mlp_train(pt_mlp* m, const int32_t* order, int32_t steps, float lr, float
         if (e != hipSuccess) return fail(PT_EDEVICE, "training graph: %s", hipGetErrorString(e));
     }
     HIP_TRY(hipEventRecord(m->ev0, m->stream));
-    for (int s = 0; s < steps; ++s) {
-        if (exec.e) {
+    for (int s = 0; s < steps;) {
+        if (exec.e && s + per <= steps) {
             const hipError_t e = hipGraphLaunch(exec.e, m->stream);
             if (e != hipSuccess) return fail(PT_EDEVICE, "training graph launch: %s", hipGetErrorString(e));
+            s += per;
         } else {
             one_step();
+            ++s;
         }
     }
     m->t += steps;
@@ -1015,7 +1037,7 @@ void pt_mlp_destroy(pt_mlp* m) {
     dev_free(m->order);
     dev_free(m->xb);
     for (int l = 1; l < PT_MLP_LAYERS; ++l) dev_free(m->act[l]);
-    for (int l = 0; l < PT_MLP_LAYERS - 1; ++l) dev_free(m->pre[l]);
+    for (int l = 0; l < PT_MLP_LAYERS - 1; ++l) dev_free(m->slope[l]);
     for (int l = 0; l < PT_MLP_LAYERS; ++l) dev_free(m->dz[l]);
     dev_free(m->bias_corr);
     dev_free(m->pred);
