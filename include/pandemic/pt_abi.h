@@ -282,9 +282,12 @@ int pt_sim_get_launch(pt_sim* sim, int32_t knob);
  * ascending within a key (the stable sort's order), and
  * offsets[n_buckets + 1] with offsets[k] = number of keys below k (so
  * offsets[n_buckets] = n).  All three are device pointers on `device`;
- * stream is a hipStream_t (NULL: the default stream).  The radix scratch
- * (about 20 bytes per pair) is allocated for the call and freed before it
- * returns, so the call synchronises the stream.  n < 2^31, n_buckets >= 1.
+ * stream is a hipStream_t (NULL: the default stream).  The call
+ * synchronises the stream.  Its radix scratch (9 bytes per pair for up to
+ * 65,536 buckets, up to 20 for more) is one block; a block of up to 512 MiB
+ * per device is kept for the next call, and given back when an allocation of
+ * this library fails or a call needs less than a quarter of it.
+ * n < 2^31, n_buckets >= 1.
  * Keys are not checked on the device: a key >= n_buckets leaves the table
  * unspecified, but every write stays inside people[n] and
  * offsets[n_buckets + 1]. */

@@ -56,7 +56,7 @@ struct DeviceScope {
 template <class T>
 int dev_alloc(T** p, int64_t count) {
     if (count <= 0) count = 1;
-    if (hipMalloc((void**)p, (size_t)count * sizeof(T)) != hipSuccess) {
+    if (device_malloc((void**)p, (size_t)count * sizeof(T)) != hipSuccess) {
         *p = nullptr;
         return fail(PT_ENOMEM, "hipMalloc of %lld bytes failed", (long long)(count * (int64_t)sizeof(T)));
     }

@@ -48,6 +48,7 @@ constexpr int kTile = 64;      // rows and columns of a tile (the loss tiles: kC
 constexpr int kGemmThreads = 256;
 constexpr int kXcds = 8;
 constexpr int kMaxWidth = PT_MLP_OUT;  // widest layer output
+constexpr int64_t kSlotRows = 2048;    // result rows per pinned slot: 5.9 MB
 
 // Offsets of W_l and b_l in a member's parameter block.
 struct Layout {
@@ -690,6 +691,11 @@ struct pt_mlp {
     int64_t loss_cap = 0;
     float* xin = nullptr;  // prediction inputs
     int64_t xin_cap = 0;
+    // Prediction results on their way to the caller: pinned slots, each with
+    // an event that marks its copy's end.
+    float* slot[2] = {};
+    int64_t slot_cap = 0;  // floats
+    hipEvent_t slot_ev[2] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0;
     // Training steps: [0] step index within the current call, [1] Adam steps
@@ -1001,18 +1007,62 @@ int pt_mlp_predict(pt_mlp* m, const float* X, int64_t n, float* out) {
     }
     HIP_TRY(hipMemcpyAsync(m->xin, X, sizeof(float) * n * PT_MLP_IN, hipMemcpyHostToDevice, m->stream));
     const int B = m->batch;
-    std::vector<float> h((size_t)m->members * B * PT_MLP_OUT);
-    for (int64_t i0 = 0; i0 < n; i0 += B) {
+    // Results go through two pinned slots, so that a part's way to the
+    // caller's memory (a host copy, bound by its page faults) overlaps the
+    // next parts' products and device copies: a part is one chunk of all
+    // members, or rows of one member's chunk.
+    const int64_t rows0 = std::min<int64_t>(B, n), all = m->members * rows0;
+    const int64_t part_rows = std::min(rows0, kSlotRows);
+    const bool whole = all <= kSlotRows;
+    const int64_t want = (whole ? all : part_rows) * PT_MLP_OUT;
+    if (want > m->slot_cap) {
+        m->slot_cap = 0;
+        HIP_TRY(hipStreamSynchronize(m->stream));
+        for (int i = 0; i < 2; ++i) {
+            if (m->slot[i]) HIP_TRY(hipHostFree(m->slot[i]));
+            m->slot[i] = nullptr;
+            if (hipHostMalloc((void**)&m->slot[i], sizeof(float) * want) != hipSuccess)
+                return fail(PT_ENOMEM, "hipHostMalloc of %lld bytes failed", (long long)(sizeof(float) * want));
+        }
+        m->slot_cap = want;
+    }
+    for (hipEvent_t& e : m->slot_ev)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    struct Part {
+        int64_t at = 0;             // first row of the result
+        int rows = 0, members = 0;  // members of consecutive blocks of n rows
+    } pending[2];
+    int next = 0;
+    auto drain = [&](int i) -> int {
+        Part& q = pending[i];
+        if (q.rows == 0) return PT_OK;
+        HIP_TRY(hipEventSynchronize(m->slot_ev[i]));
+        const size_t len = (size_t)q.rows * PT_MLP_OUT;
+        for (int k = 0; k < q.members; ++k)
+            memcpy(out + (size_t)(q.at + k * n) * PT_MLP_OUT, m->slot[i] + k * len, sizeof(float) * len);
+        q.rows = 0;
+        return PT_OK;
+    };
+    int rc = PT_OK;
+    for (int64_t i0 = 0; i0 < n && !rc; i0 += B) {
         const int rows = (int)std::min<int64_t>(B, n - i0);
         forward(m, rows, Batch{m->xin + i0 * PT_MLP_IN, nullptr, nullptr, nullptr}, false);
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(h.data(), m->pred, sizeof(float) * h.size(), hipMemcpyDeviceToHost, m->stream));
-        HIP_TRY(hipStreamSynchronize(m->stream));
-        for (int k = 0; k < m->members; ++k)
-            memcpy(out + ((size_t)k * n + i0) * PT_MLP_OUT, h.data() + (size_t)k * B * PT_MLP_OUT,
-                   sizeof(float) * rows * PT_MLP_OUT);
+        for (int k = 0; k < m->members && !rc; k += whole ? m->members : 1)
+            for (int r0 = 0; r0 < rows && !rc; r0 += (int)part_rows) {
+                const int i = next, count = std::min(rows - r0, (int)part_rows);
+                if ((rc = drain(i))) break;
+                const size_t len = sizeof(float) * count * PT_MLP_OUT;
+                HIP_TRY(hipMemcpy2DAsync(m->slot[i], len, m->pred + ((int64_t)k * B + r0) * PT_MLP_OUT,
+                                         sizeof(float) * B * PT_MLP_OUT, len, whole ? m->members : 1,
+                                         hipMemcpyDeviceToHost, m->stream));
+                HIP_TRY(hipEventRecord(m->slot_ev[i], m->stream));
+                pending[i] = Part{k * n + i0 + r0, count, whole ? m->members : 1};
+                next = 1 - next;
+            }
     }
-    return PT_OK;
+    for (int i = 0; i < 2 && !rc; ++i) rc = drain((next + i) & 1);
+    return rc;
 }
 
 int pt_mlp_use_graphs(pt_mlp* m, int32_t on) {
@@ -1045,6 +1095,10 @@ void pt_mlp_destroy(pt_mlp* m) {
     dev_free(m->colpart);
     dev_free(m->loss);
     dev_free(m->xin);
+    for (int i = 0; i < 2; ++i) {
+        if (m->slot[i]) (void)hipHostFree(m->slot[i]);
+        if (m->slot_ev[i]) (void)hipEventDestroy(m->slot_ev[i]);
+    }
     if (m->ev0) (void)hipEventDestroy(m->ev0);
     if (m->ev1) (void)hipEventDestroy(m->ev1);
     dev_free(m->d_step);

@@ -97,6 +97,16 @@ struct TableScratch {
 int table_scratch_alloc(TableScratch& s, int64_t n_cap);
 void table_scratch_free(TableScratch& s);
 
+// Scratch for one build of n pairs into K buckets within a block of
+// table_scratch_bytes(n, K): only what the passes of that build touch (of 20
+// bytes per pair, 9 for 2 passes).
+size_t table_scratch_bytes(int64_t n, int32_t K);
+void table_scratch_carve(TableScratch& s, unsigned char* block, int64_t n, int32_t K);
+
+// hipMalloc; if it fails, once more after giving back the scratch block that
+// location tables keep (pt_table.hip).
+hipError_t device_malloc(void** p, size_t bytes);
+
 constexpr uint32_t kNoDrop = 0xFFFFFFFFu;
 
 // A second input for a table whose input is chosen on the device: while

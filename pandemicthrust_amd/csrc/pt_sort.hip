@@ -743,18 +743,57 @@ int table_scratch_alloc(TableScratch& s, int64_t n_cap) {
     table_scratch_free(s);
     const int64_t n = std::max<int64_t>(n_cap, 1);
     const int64_t hist_n = ((int64_t)1 << kMaxBitsSupported) * kHistBlocks + 1;
-    if (hipMalloc(&s.keys_b, n * sizeof(uint32_t)) != hipSuccess) return -1;
-    if (hipMalloc(&s.pairs_a, n * sizeof(uint2)) != hipSuccess) return -1;
-    if (hipMalloc(&s.pairs_b, n * sizeof(uint2)) != hipSuccess) return -1;
-    if (hipMalloc(&s.hist, (size_t)hist_n * sizeof(uint32_t)) != hipSuccess) return -1;
-    if (hipMalloc(&s.n_kept, sizeof(uint32_t)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.keys_b, n * sizeof(uint32_t)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.pairs_a, n * sizeof(uint2)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.pairs_b, n * sizeof(uint2)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.hist, (size_t)hist_n * sizeof(uint32_t)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.n_kept, sizeof(uint32_t)) != hipSuccess) return -1;
     // Partial sums for scans of up to max(n_cap, hist_n) values.
     const int64_t parts = (std::max<int64_t>(n, hist_n) + kScanSeg - 1) / kScanSeg + 2;
-    if (hipMalloc(&s.scan_part, (size_t)parts * sizeof(uint32_t)) != hipSuccess) return -1;
+    if (device_malloc((void**)&s.scan_part, (size_t)parts * sizeof(uint32_t)) != hipSuccess) return -1;
     s.n_cap = n_cap;
     s.wide_bits = wide_bits;
     s.max_bits = max_bits;
     return 0;
+}
+
+namespace {
+
+// Byte offsets of one build's scratch (build_table): the pairs between
+// passes, the last pass's low key bytes, the digit histograms, the scans'
+// partial sums.
+struct ScratchLayout {
+    size_t keys, pairs_a, pairs_b, hist, scan, kept, bytes;
+    ScratchLayout(int64_t n_cap, int32_t K, int max_bits) {
+        const auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        const size_t n = (size_t)std::max<int64_t>(n_cap, 1);
+        const int bits = key_bits(K), passes = radix_passes(K, max_bits);
+        const int widest = (bits + passes - 1) / passes, low = bits - bits / passes;
+        const size_t hist_n = ((size_t)1 << widest) * kHistBlocks + 1;
+        keys = 0;
+        pairs_a = up(keys + n * (low <= 8 ? 1 : (low <= 16 ? 2 : 4)) + 64);
+        pairs_b = up(pairs_a + (passes > 1 ? n * sizeof(uint2) : 0) + 64);
+        hist = up(pairs_b + (passes > 2 ? n * sizeof(uint2) : 0) + 64);
+        scan = up(hist + hist_n * sizeof(uint32_t));
+        kept = up(scan + (((std::max(n, hist_n) + kScanSeg - 1) / kScanSeg) + 2) * sizeof(uint32_t));
+        bytes = up(kept + sizeof(uint32_t));
+    }
+};
+
+}  // namespace
+
+size_t table_scratch_bytes(int64_t n, int32_t K) { return ScratchLayout(n, K, TableScratch().max_bits).bytes; }
+
+void table_scratch_carve(TableScratch& s, unsigned char* block, int64_t n, int32_t K) {
+    s = TableScratch();
+    const ScratchLayout o(n, K, s.max_bits);
+    s.keys_b = (uint32_t*)(block + o.keys);
+    s.pairs_a = (uint2*)(block + o.pairs_a);
+    s.pairs_b = (uint2*)(block + o.pairs_b);
+    s.hist = (uint32_t*)(block + o.hist);
+    s.scan_part = (uint32_t*)(block + o.scan);
+    s.n_kept = (uint32_t*)(block + o.kept);
+    s.n_cap = n;
 }
 
 void table_scratch_free(TableScratch& s) {
