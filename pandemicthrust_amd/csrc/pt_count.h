@@ -113,7 +113,7 @@ struct CountTable {
     int64_t mark_words;
     int32_t* chunk_day;    // day + 1 on which the (chunk, group) was last marked
     int32_t* list;         // ids of the marked buckets, kpa * agents per chunk
-    uint32_t* n;           // [0] picks queued, [1] infectors listed, [2] list entries (split layouts)
+    uint32_t* n;           // [0] picks queued, [1] infectors listed, [2] list entries (split layouts), [3] k_apply_end
     // Listed infectors: agent, position, pack_infectivity, simulation (batch).
     int32_t *sv_idx, *sv_pos;
     uint32_t* sv_f;
@@ -397,12 +397,10 @@ namespace {
 // Keys and counts of a chunk.  VALU bound (the errand draws); the LDS adds,
 // the 4-byte coalesced key stores and the row flush hide behind them.
 template <bool WEEKEND>
-__global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done, DayState* __restrict__ sts,
-                                                const Model* __restrict__ models, const uint8_t* __restrict__ ages,
-                                                CountTable T) {
-    if (*done) return;
+__device__ __forceinline__ void count_block(int block, DayState* __restrict__ sts, const Model* __restrict__ models,
+                                            const uint8_t* __restrict__ ages, const CountTable& T) {
     extern __shared__ uint32_t s_cnt[];
-    const CountBlock blk = T.chunks[blockIdx.x];
+    const CountBlock blk = T.chunks[block];
     DayState* st = sts + blk.r;
     if (st->done) return;
     const Model& M = models[blk.r];
@@ -472,22 +470,26 @@ __global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done
     for (int i = tid; i < c.K; i += nt) row[i] = s_cnt[i];
 }
 
+template <bool WEEKEND>
+__global__ __launch_bounds__(1024) void k_count(const int32_t* __restrict__ done, DayState* __restrict__ sts,
+                                                const Model* __restrict__ models, const uint8_t* __restrict__ ages,
+                                                CountTable T) {
+    if (*done) return;
+    count_block<WEEKEND>(blockIdx.x, sts, models, ages, T);
+}
+
 // Column prefixes of the count matrices, kScanCols buckets per block of 1024
 // threads: the row groups sum up to 8 rows each in registers, and the
 // prefixes go out through LDS as runs of consecutive chunks.  The fewer
 // chunks, the more buckets per block (CountPlan::scan_cols).  Also clears the
-// day's marks, picks and lists.
+// day's marks.
 constexpr int kCountScanThreads = 1024, kScanRows = 8;
 template <int kScanCols>
-__global__ __launch_bounds__(kCountScanThreads) void k_count_scan(const int32_t* __restrict__ done,
-                                                                       const DayState* __restrict__ sts,
-                                                                       CountTable T) {
-    if (*done) return;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < T.mark_words;
-         i += (int64_t)gridDim.x * blockDim.x)
+__device__ __forceinline__ void scan_block(int block, int blocks, const DayState* __restrict__ sts,
+                                           const CountTable& T) {
+    for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < T.mark_words; i += (int64_t)blocks * blockDim.x)
         T.marks[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < 3) T.n[threadIdx.x] = 0u;
-    const CountBlock blk = T.scans[blockIdx.x];
+    const CountBlock blk = T.scans[block];
     if (sts[blk.r].done) return;
     const CountRep c = T.reps[blk.r];
     constexpr int kScanGroups = kCountScanThreads / kScanCols;
@@ -540,14 +542,23 @@ __global__ __launch_bounds__(kCountScanThreads) void k_count_scan(const int32_t*
         if (carry == 1) T.lone_day[blk.r] = sts[blk.r].day + 1;
     }
 }
+template <int kScanCols>
+__global__ __launch_bounds__(kCountScanThreads) void k_count_scan(const int32_t* __restrict__ done,
+                                                                  const DayState* __restrict__ sts, CountTable T) {
+    if (*done) return;
+    if (blockIdx.x == 0 && threadIdx.x < 3) T.n[threadIdx.x] = 0u;  // no picks, infectors or lists yet
+    scan_block<kScanCols>(blockIdx.x, gridDim.x, sts, T);
+}
 
 // Least contact count of an infector (may_infect): its household, its
 // workplace unless some workplace has one person only, and its two errands
-// (every errand profile has two) unless some bucket of the day has.
-__device__ __forceinline__ int least_contacts(const CountTable& T, AgentRecord a, int r, int day, bool weekend) {
+// (every errand profile has two) unless some bucket of the day has, or that is
+// not known yet (counted false).
+__device__ __forceinline__ int least_contacts(const CountTable& T, AgentRecord a, int r, int day, bool weekend,
+                                              bool counted = true) {
     int k = record_household_size(a) > 1 ? 3 : 0;
     if (!weekend && !T.wp_lone[r]) k += record_workplace_contacts(a);
-    if (T.lone_day[r] != day + 1) k += 2;
+    if (counted && T.lone_day[r] != day + 1) k += 2;
     return max(k, 1);
 }
 
@@ -1134,7 +1145,7 @@ struct CountScratch {
         const int64_t e = std::max(a.entries, b.entries);
         if (e == 0) return 0;
         return dev_alloc(&cnt, e) || dev_alloc(&pre, e) || dev_alloc(&total, std::max(a.buckets, b.buckets)) || dev_alloc(&marks, std::max(a.mark_words, b.mark_words)) ||
-                       dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 3) || dev_alloc(&lone_day, (int64_t)std::max(a.reps.size(), b.reps.size())) ||
+                       dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 4) || dev_alloc(&lone_day, (int64_t)std::max(a.reps.size(), b.reps.size())) ||
                        (b.split && dev_alloc(&tile_off, (N / kTileAgents + 1) * kTileHours))
                    ? PT_ENOMEM
                    : 0;

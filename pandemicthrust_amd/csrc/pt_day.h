@@ -1192,12 +1192,11 @@ __global__ void k_compact_runs(const int32_t* __restrict__ skip, const uint32_t*
 
 // Winners write status = profile, day = current_day + 1, generation
 // (device_setInfectionStatus PandemicSim.cu:3048-3067); claim words reset.
-__global__ void k_apply(const DayState* __restrict__ st, uint64_t* __restrict__ claim_p,
+__device__ __forceinline__ void apply_claims(const DayState* st, uint64_t* __restrict__ claim_p,
                         uint64_t* __restrict__ claim_s, const int32_t* __restrict__ list_p,
                         const int32_t* __restrict__ list_s, uint8_t* __restrict__ st_p, uint8_t* __restrict__ st_s,
                         uint8_t* __restrict__ dy_p, uint8_t* __restrict__ dy_s, uint8_t* __restrict__ gn_p,
                         uint8_t* __restrict__ gn_s) {
-    if (st->done) return;
     const uint32_t np = st->n_claimed[0], ns = st->n_claimed[1];
     const uint8_t dset = (uint8_t)(st->day + 1);
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -1218,6 +1217,15 @@ __global__ void k_apply(const DayState* __restrict__ st, uint64_t* __restrict__ 
             claim_s[v] = ~0ull;
         }
     }
+}
+
+__global__ void k_apply(const DayState* __restrict__ st, uint64_t* __restrict__ claim_p,
+                        uint64_t* __restrict__ claim_s, const int32_t* __restrict__ list_p,
+                        const int32_t* __restrict__ list_s, uint8_t* __restrict__ st_p, uint8_t* __restrict__ st_s,
+                        uint8_t* __restrict__ dy_p, uint8_t* __restrict__ dy_s, uint8_t* __restrict__ gn_p,
+                        uint8_t* __restrict__ gn_s) {
+    if (st->done) return;
+    apply_claims(st, claim_p, claim_s, list_p, list_s, st_p, st_s, dy_p, dy_s, gn_p, gn_s);
 }
 
 // Plain copy of n16 16-byte words (snapshot / restore of the agent state).

@@ -312,16 +312,20 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DayState* __restrict__ st
 // blocks, is the day plan too (PLAN): every block sums the counts of the
 // blocks before it instead of waiting for a launch of one block.
 constexpr int kFusedPlan = 1024;
+constexpr int kMergedBlocks = 3;  // per CU
+struct CompactArgs {
+    const int32_t* staging;
+    const uint32_t *blk_ninf, *blk_off, *blk_counts;
+    int nblk, parts;  // sweep blocks, blocks that share the infected of each
+    int32_t *out_counts, *out_inf, *infected;
+};
 template <bool WEEKEND, bool PLAN>
-__global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
-                                                       const int32_t* __restrict__ staging,
-                                                       const uint32_t* __restrict__ blk_ninf,
-                                                       const uint32_t* __restrict__ blk_off,
-                                                       const uint32_t* __restrict__ blk_counts, int nblk,
-                                                       int32_t* __restrict__ out_counts,
-                                                       int32_t* __restrict__ out_inf, int32_t* __restrict__ infected,
-                                                       AgentArrays A, CountTable T) {
-    if (st->done) return;
+__device__ __forceinline__ void compact_test_block(int block, const Model* __restrict__ Mp, DayState* __restrict__ st,
+                                                   const CompactArgs& a, const AgentArrays& A, const CountTable& T,
+                                                   bool counted) {
+    const int32_t* __restrict__ staging = a.staging;
+    const uint32_t* __restrict__ blk_ninf = a.blk_ninf;
+    const int nblk = a.nblk, own = block / a.parts, part = block % a.parts;
     constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
     const Model& M = *Mp;
     const int tid = threadIdx.x;
@@ -343,17 +347,17 @@ __global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__
             if (w < wave) before += x;
             total += x;
         }
-        if (tid == (int)blockIdx.x) s_off = before + inc - v;
-        if (blockIdx.x == 0) {
+        if (tid == own) s_off = before + inc - v;
+        if (block == 0) {
             // Daily counts: a wave per counter.
             uint32_t c = 0;
-            for (int b = lane; b < nblk; b += 64) c += blk_counts[(int64_t)b * 16 + wave];
+            for (int b = lane; b < nblk; b += 64) c += a.blk_counts[(int64_t)b * 16 + wave];
             c = wave_sum(c);
-            if (lane == 0) out_counts[day * 16 + wave] = (int32_t)c;
+            if (lane == 0) a.out_counts[day * 16 + wave] = (int32_t)c;
             if (tid == 0) {
                 st->n_infected = (int32_t)total;
                 st->days_run = day + 1;
-                out_inf[day] = (int32_t)total;
+                a.out_inf[day] = (int32_t)total;
                 if (total == 0) {
                     st->done = 1;  // nobody left to compact: other blocks may or may not see it
                     st->skip_full = st->skip_subset = st->skip_mark = 1;
@@ -367,28 +371,70 @@ __global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__
         __syncthreads();
         off = s_off;
     } else {
-        off = blk_off[blockIdx.x];
+        off = a.blk_off[own];
     }
-    const uint32_t n = blk_ninf[blockIdx.x];
-    const int32_t* src = staging + (int64_t)blockIdx.x * kSweepTile;
-    for (uint32_t i0 = 0; i0 < n; i0 += blockDim.x) {
+    const uint32_t n = blk_ninf[own];
+    const int32_t* src = staging + (int64_t)own * kSweepTile;
+    for (uint32_t i0 = part * blockDim.x; i0 < n; i0 += a.parts * blockDim.x) {
         const uint32_t i = i0 + tid;
         int32_t idx = 0;
         Infectivity f{};
         bool keep = false;
         if (i < n) {
             idx = src[i];
-            infected[off + i] = idx;
+            a.infected[off + i] = idx;
             f = infectivity(M, A, idx, day);
             if (can_infect(M, f)) {
                 SuccessDraws draws;
                 success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
                 keep = may_infect<C>(M, f, draws, 1) &&
-                       may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND));
+                       may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND, counted));
             }
         }
         list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
     }
+}
+template <bool WEEKEND, bool PLAN>
+__global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
+                                                       CompactArgs a, AgentArrays A, CountTable T) {
+    if (st->done) return;
+    compact_test_block<WEEKEND, PLAN>(blockIdx.x, Mp, st, a, A, T, true);
+}
+
+// Small populations (merged_launches): launches of a few us each, in pairs
+// that do not depend on each other.  First the keys and counts and the sweep
+// (2.35M agents, weekday: 14 + 8 us -> 19; 100k: 4 + 7 -> 7) ...
+template <bool WEEKEND>
+__global__ __launch_bounds__(1024) void k_count_sweep(const Model* __restrict__ Mp, DayState* __restrict__ st,
+                                                      uint8_t* __restrict__ st_p, uint8_t* __restrict__ st_s,
+                                                      const uint8_t* __restrict__ dy_p,
+                                                      const uint8_t* __restrict__ dy_s,
+                                                      const uint8_t* __restrict__ age,
+                                                      uint32_t* __restrict__ blk_counts,
+                                                      uint32_t* __restrict__ blk_ninf, int32_t* __restrict__ staging,
+                                                      CountTable T, int n_chunks) {
+    if (st->done) return;
+    if ((int)blockIdx.x < n_chunks) {
+        if (blockIdx.x == 0 && threadIdx.x < 3) T.n[threadIdx.x] = 0u;  // no picks, infectors or lists yet
+        count_block<WEEKEND>(blockIdx.x, st, Mp, age, T);
+    } else if (threadIdx.x < kSweepThreads) {  // (waves that have ended do not take part in barriers)
+        const int64_t b = blockIdx.x - n_chunks;
+        sweep_block(*Mp, Mp->N, st->day, b * kSweepTile, st_p, st_s, dy_p, dy_s, blk_counts + b * 16, blk_ninf + b,
+                    staging + b * kSweepTile, 0);
+    }
+}
+
+// ... then the prefixes and the compaction, whose test does without the
+// day's lone buckets (8.5 + 13.7 us -> 17.6, and the contacts of the infectors
+// it leaves 17.7 -> 19; 100k: 5 + 10 -> 8).
+template <bool WEEKEND, int COLS>
+__global__ __launch_bounds__(1024) void k_scan_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
+                                                    CompactArgs a, AgentArrays A, CountTable T, int n_scans) {
+    if (st->done) return;
+    if ((int)blockIdx.x < n_scans)
+        scan_block<COLS>(blockIdx.x, n_scans, st, T);
+    else
+        compact_test_block<WEEKEND, true>(blockIdx.x - n_scans, Mp, st, a, A, T, false);
 }
 
 // Also clears the bucket marks when today marks (k_plan decided).
@@ -625,9 +671,8 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
 // of queried buckets (n_sel pairs).
 // tab_pairs logs the pairs of the day's table: n_kept (when set) or n_full
 // on full-table days, the selected pairs on subset days.
-__global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t* __restrict__ tab_pairs,
-                          int32_t n_full, const uint32_t* __restrict__ n_kept) {
-    if (st->done) return;
+__device__ __forceinline__ void end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t* __restrict__ tab_pairs,
+                                        int32_t n_full, const uint32_t* __restrict__ n_kept) {
     const int d = st->day;
     tab_full[d] = st->skip_full == 0 ? 1 : 0;
     tab_pairs[d] = st->skip_full == 0 ? (n_kept ? (int32_t)*n_kept : n_full)
@@ -639,6 +684,30 @@ __global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t*
     st->skip_full = 1;
     st->skip_subset = 1;
     if (st->day >= st->max_days) st->done = 1;
+}
+__global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t* __restrict__ tab_pairs,
+                          int32_t n_full, const uint32_t* __restrict__ n_kept) {
+    if (st->done) return;
+    end_day(st, tab_full, tab_pairs, n_full, n_kept);
+}
+
+// Applies the claims; the last block to finish ends the day (*ticket is 0
+// between launches).  2.35M agents: 4.4 + 3 us -> 6.1.
+__global__ __launch_bounds__(256) void k_apply_end(DayState* st, uint64_t* __restrict__ claim_p,
+                                                   uint64_t* __restrict__ claim_s, const int32_t* __restrict__ list_p,
+                                                   const int32_t* __restrict__ list_s, uint8_t* __restrict__ st_p,
+                                                   uint8_t* __restrict__ st_s, uint8_t* __restrict__ dy_p,
+                                                   uint8_t* __restrict__ dy_s, uint8_t* __restrict__ gn_p,
+                                                   uint8_t* __restrict__ gn_s, int32_t* __restrict__ tab_full,
+                                                   int32_t* __restrict__ tab_pairs, int32_t n_full,
+                                                   uint32_t* ticket) {
+    if (st->done) return;
+    apply_claims(st, claim_p, claim_s, list_p, list_s, st_p, st_s, dy_p, dy_s, gn_p, gn_s);
+    __syncthreads();  // the block is done with the day's state
+    if (threadIdx.x == 0 && atomicAdd(ticket, 1u) == gridDim.x - 1) {
+        *ticket = 0u;
+        end_day(st, tab_full, tab_pairs, n_full, nullptr);
+    }
 }
 
 // Validation trace: which successful attempts won their victim.  A claim
@@ -1163,7 +1232,12 @@ int setup_counts(pt_sim* s) {
         t.sv_f = s->sel_keys + 2 * s->N;
         t.wp_lone = s->wp_lone;
         HIP_TRY(set_count_lds(p));
+        if (p.lds > 64 * 1024 && !p.split)
+            HIP_TRY(hipFuncSetAttribute(w ? reinterpret_cast<const void*>(&k_count_sweep<true>)
+                                          : reinterpret_cast<const void*>(&k_count_sweep<false>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024));
     }
+    if (s->count_scratch.n) HIP_TRY(hipMemsetAsync(s->count_scratch.n, 0, 4 * sizeof(uint32_t), s->stream));
     return PT_OK;
 }
 
@@ -1250,6 +1324,25 @@ int enqueue_table(pt_sim* s, bool weekend, int64_t n, int32_t K, int64_t nwords,
     return PT_OK;
 }
 
+// Whether a counted day's launches go in pairs (k_count_sweep, k_scan_test,
+// k_apply_end): while the count and sweep blocks, which all ask for the
+// counters' LDS, are few enough per CU (2.35M agents, 543 blocks: 9.77 -> 9.40
+// ms per 100 days; 235k in steps 5.95 -> 4.80, 100k x 60 days 4.67 -> 4.16).
+bool merged_launches(const pt_sim* s, const CountPlan& p) {
+    return !p.split && p.lds <= (size_t)152 * 1024 && p.n_chunks + s->nblk_sweep <= kMergedBlocks * s->cus;
+}
+
+int end_enqueue(pt_sim* s, int d, bool weekend, int64_t n, bool counted) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(PT_EDEVICE, "day launch: %s", hipGetErrorString(e));
+    s->last_weekend = weekend ? 1 : 0;
+    s->last_table_n = n;
+    s->last_counted = counted;
+    s->host_day = d + 1;
+    s->timer.day = -1;
+    return 0;
+}
+
 // Enqueues one loop iteration for host day index d (runToCompletion body,
 // PandemicSim.cu:882-954).  Every kernel is a no-op once the device state
 // says the loop has ended.
@@ -1259,9 +1352,6 @@ int enqueue_day(pt_sim* s, int d) {
     s->timer.day = d;
     LaunchTimer* tm = &s->timer;
     DayState* st = s->d_state;
-    launch(tm, KC_SWEEP, k_sweep, dim3(s->nblk_sweep), dim3(kSweepThreads), stc, (const Model*)s->d_model, s->N, st,
-           s->st_p, s->st_s,
-           (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, s->blk_counts, s->blk_ninf, s->staging);
     // Marking pays off while the queried share of the buckets is likely to
     // stay below the subset threshold: I <= K * mark_limit / 100.
     const int mpct = s->launch[PT_LAUNCH_MARK_LIMIT];
@@ -1271,12 +1361,23 @@ int enqueue_day(pt_sim* s, int d) {
     const CountTable& ct = s->count_table[weekend ? 1 : 0];
     const bool counted = s->table_mode == TABLES_AUTO && cp.on && !s->trace_on;
     const bool fused_plan = counted && s->nblk_sweep <= kFusedPlan;
+    const bool merged = fused_plan && merged_launches(s, cp);
     AgentArrays A = agent_arrays(s);
     const Model* M = s->d_model;
+    if (!merged)
+        launch(tm, KC_SWEEP, k_sweep, dim3(s->nblk_sweep), dim3(kSweepThreads), stc, M, s->N, st, s->st_p, s->st_s,
+               (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, s->blk_counts, s->blk_ninf, s->staging);
     if (counted) {
         A.er_keys = cp.split ? nullptr : ct.keys;  // (weekend hour lists are not by agent)
         A.er_slots = ct.slots;
         A.er_cnt = ct.total;
+    }
+    if (merged) {
+        launch_lds(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_count_sweep<true> : k_count_sweep<false>,
+                   dim3(cp.n_chunks + s->nblk_sweep), dim3(cp.threads), cp.lds, stc, M, st, s->st_p, s->st_s,
+                   (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, (const uint8_t*)s->age, s->blk_counts,
+                   s->blk_ninf, s->staging, ct, cp.n_chunks);
+    } else if (counted) {
         enqueue_counts(cp, ct, &st->done, st, M, s->age, weekend, stc, tm, s->N, s->grid_gen);
     }
     // (A counted day counts every bucket: nothing to mark or decide.)
@@ -1290,11 +1391,26 @@ int enqueue_day(pt_sim* s, int d) {
     // and which table path to take.
     const int64_t nwords = ((int64_t)K + 31) / 32;
     if (counted) {
-        const auto k = weekend ? (fused_plan ? k_compact_test<true, true> : k_compact_test<true, false>)
-                               : (fused_plan ? k_compact_test<false, true> : k_compact_test<false, false>);
-        launch(tm, KC_COMPACT, k, dim3(s->nblk_sweep), dim3(1024), stc, M, st, (const int32_t*)s->staging,
-               (const uint32_t*)s->blk_ninf, (const uint32_t*)s->blk_off, (const uint32_t*)s->blk_counts,
-               s->nblk_sweep, s->d_counts, s->d_inf, s->infected, A, ct);
+        // A sweep block's infected, up to kSweepTile, go to several blocks
+        // while there are few sweep blocks.
+        const int parts = std::max(1, std::min(kSweepTile / 1024, 2 * s->cus / s->nblk_sweep));
+        const CompactArgs a{s->staging, s->blk_ninf, s->blk_off, s->blk_counts, s->nblk_sweep, parts,
+                            s->d_counts, s->d_inf, s->infected};
+        if (merged) {
+            const auto k = cp.scan_cols == 32
+                               ? (weekend ? k_scan_test<true, 32> : k_scan_test<false, 32>)
+                               : (cp.scan_cols == 64
+                                      ? (weekend ? k_scan_test<true, 64> : k_scan_test<false, 64>)
+                                      : (cp.scan_cols == 256
+                                             ? (weekend ? k_scan_test<true, 256> : k_scan_test<false, 256>)
+                                             : (weekend ? k_scan_test<true, 1024> : k_scan_test<false, 1024>)));
+            launch(tm, KC_COMPACT, k, dim3(cp.n_scans + s->nblk_sweep * parts), dim3(1024), stc, M, st, a, A, ct,
+                   cp.n_scans);
+        } else {
+            const auto k = weekend ? (fused_plan ? k_compact_test<true, true> : k_compact_test<true, false>)
+                                   : (fused_plan ? k_compact_test<false, true> : k_compact_test<false, false>);
+            launch(tm, KC_COMPACT, k, dim3(s->nblk_sweep * parts), dim3(1024), stc, M, st, a, A, ct);
+        }
     } else {
         launch(tm, KC_COMPACT, k_compact, dim3(s->nblk_sweep), dim3(256), stc, (const DayState*)st,
                (const int32_t*)s->staging, (const uint32_t*)s->blk_ninf, (const uint32_t*)s->blk_off, s->infected,
@@ -1319,18 +1435,17 @@ int enqueue_day(pt_sim* s, int d) {
                                                             (const uint8_t*)s->tr_attempt,
                                                             (const uint64_t*)s->claim_p,
                                                             (const uint64_t*)s->claim_s, s->tr_action);
+    if (merged) {
+        launch(tm, KC_APPLY, k_apply_end, dim3(std::min(grid, s->cus)), dim3(256), stc, st, s->claim_p, s->claim_s,
+               (const int32_t*)s->list_p, (const int32_t*)s->list_s, s->st_p, s->st_s, s->dy_p, s->dy_s, s->gn_p,
+               s->gn_s, s->d_tab_full, s->d_tab_pairs, (int32_t)n, ct.n + 3);
+        return end_enqueue(s, d, weekend, n, counted);
+    }
     launch(tm, KC_APPLY, k_apply, dim3(grid), dim3(256), stc, (const DayState*)st, s->claim_p, s->claim_s,
            (const int32_t*)s->list_p, (const int32_t*)s->list_s, s->st_p, s->st_s, s->dy_p, s->dy_s, s->gn_p, s->gn_s);
     launch(tm, KC_END_DAY, k_end_day, dim3(1), dim3(1), stc, st, s->d_tab_full, s->d_tab_pairs, (int32_t)n,
            weekend || counted ? (const uint32_t*)nullptr : (const uint32_t*)s->tables.n_kept);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(PT_EDEVICE, "day launch: %s", hipGetErrorString(e));
-    s->last_weekend = weekend ? 1 : 0;
-    s->last_table_n = n;
-    s->last_counted = counted;
-    s->host_day = d + 1;
-    s->timer.day = -1;
-    return 0;
+    return end_enqueue(s, d, weekend, n, counted);
 }
 
 int reset_day_state(pt_sim* s) {

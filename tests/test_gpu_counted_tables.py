@@ -32,6 +32,10 @@ CASES = [
     (0.1, 41.0, 7, 5000),          # 65,600: 4-byte keys
     (0.3, 200.0, 7, 5000),         # 320,000: 8 groups
     (0.05, 200.5, 7, 5000),        # 320,800: weekday sorted
+    (0.05, 2.98, 9, 2000),         # weekend 38,740 buckets: the largest counted beside the sweep
+    (1.0, 1.0, 7, 20000),          # 2.35M agents: launches in pairs
+    (2.2, 1.0, 7, 20000),          # 5.2M: single launches, the compaction plans the day
+    (3.7, 1.0, 7, 20000),          # 8.7M: a plan launch of its own
 ]
 
 
