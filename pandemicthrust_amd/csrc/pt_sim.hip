@@ -691,6 +691,21 @@ __global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t*
     end_day(st, tab_full, tab_pairs, n_full, n_kept);
 }
 
+// The loop's state and a day's row of the daily outputs, for the host to read
+// without copies: written to pinned host memory.
+struct DayReport {
+    DayState state;
+    int32_t counts[16], infected;
+    int32_t done[2];  // pt_sim_run's copies of the done flag
+};
+__global__ void k_report(const DayState* __restrict__ st, const int32_t* __restrict__ counts,
+                         const int32_t* __restrict__ infected, int day, DayReport* __restrict__ out) {
+    const int i = threadIdx.x;
+    if (i == 0) out->state = *st;
+    if (i < 16) out->counts[i] = counts[16 * day + i];
+    if (i == 16) out->infected = infected[day];
+}
+
 // Applies the claims; the last block to finish ends the day (*ticket is 0
 // between launches).  2.35M agents: 4.4 + 3 us -> 6.1.
 __global__ __launch_bounds__(256) void k_apply_end(DayState* st, uint64_t* __restrict__ claim_p,
@@ -1095,6 +1110,9 @@ struct pt_sim {
     // pt_sim_run's early stop: the loop's `done` flag copied back after each
     // group of days (pinned, two slots) and the groups' completion events.
     int32_t* h_done = nullptr;
+    // pt_sim_step's report (pinned), and whether its state is the device's.
+    DayReport* report = nullptr;
+    bool report_valid = false;
     hipEvent_t group_ev[2] = {nullptr, nullptr};
     hipEvent_t setup_ev[6] = {};               // population size (2), build_population marks (4)
     double setup_ms[PT_SETUP_PHASES] = {0};
@@ -1335,6 +1353,7 @@ bool merged_launches(const pt_sim* s, const CountPlan& p) {
 int end_enqueue(pt_sim* s, int d, bool weekend, int64_t n, bool counted) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(PT_EDEVICE, "day launch: %s", hipGetErrorString(e));
+    s->report_valid = false;
     s->last_weekend = weekend ? 1 : 0;
     s->last_table_n = n;
     s->last_counted = counted;
@@ -1456,6 +1475,7 @@ int reset_day_state(pt_sim* s) {
     h.max_days = s->params.max_days;
     h.skip_full = 1;
     h.skip_subset = 1;
+    s->report_valid = false;
     HIP_TRY(hipMemcpyAsync(s->d_state, &h, sizeof h, hipMemcpyHostToDevice, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     s->host_day = 0;
@@ -1609,11 +1629,12 @@ int pt_sim_create(const pt_params* p, const int32_t seed_key[2], int32_t device,
     (void)hipEventCreate(&s->run_end);
     for (auto& e : s->setup_ev) (void)hipEventCreate(&e);
     for (auto& e : s->group_ev) (void)hipEventCreateWithFlags(&e, hipEventDisableTiming);
-    if (hipHostMalloc((void**)&s->h_done, 2 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
-        s->h_done = nullptr;
+    if (hipHostMalloc((void**)&s->report, sizeof(DayReport), hipHostMallocDefault) != hipSuccess) {
+        s->report = nullptr;
         pt_sim_destroy(s);
         return fail(PT_ENOMEM, "pinned host allocation failed");
     }
+    s->h_done = s->report->done;
     s->setup_ms[PT_SETUP_PUSH] = ms_between(t1, std::chrono::steady_clock::now());
     *out = s;
     return PT_OK;
@@ -1744,17 +1765,24 @@ int pt_sim_step(pt_sim* s, int32_t counts16_out[16], int32_t* infected_out) {
     if (!s) return fail(PT_EINVAL, "null handle");
     if (!s->setup_done) return fail(PT_ESTATE, "step before setup");
     HIP_TRY(hipSetDevice(s->device));
-    DayState h;
-    if (read_state(s, &h)) return PT_EDEVICE;
-    if (h.done) return 1;
-    const int day = h.day;
+    auto report = [&](int day) -> int {
+        k_report<<<1, 64, 0, s->stream>>>((const DayState*)s->d_state, (const int32_t*)s->d_counts,
+                                          (const int32_t*)s->d_inf, day, s->report);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        s->report_valid = true;
+        return PT_OK;
+    };
+    if (!s->report_valid)
+        if (const int rc = report(0)) return rc;
+    if (s->report->state.done) return 1;
+    const int day = s->report->state.day;
     if (enqueue_day(s, day)) return PT_EDEVICE;
-    if (read_state(s, &h)) return PT_EDEVICE;
+    if (const int rc = report(day)) return rc;
     s->timer.collect();
-    if (h.fault) return fail(PT_EINVAL, "a kernel saw an errand destination outside the model's range");
-    int32_t c[16], inf = 0;
-    HIP_TRY(hipMemcpy(c, s->d_counts + 16 * day, sizeof c, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(&inf, s->d_inf + day, sizeof inf, hipMemcpyDeviceToHost));
+    if (s->report->state.fault) return fail(PT_EINVAL, "a kernel saw an errand destination outside the model's range");
+    const int32_t inf = s->report->infected;
+    const int32_t(&c)[16] = s->report->counts;
     if (counts16_out) memcpy(counts16_out, c, sizeof c);
     if (infected_out) *infected_out = inf;
     return inf == 0 ? 1 : 0;
@@ -2112,6 +2140,7 @@ int pt_sim_checkpoint_load(pt_sim* s, const void* buf, int64_t bytes) {
         return fail(PT_EINVAL, "checkpoint day state out of range");
     HIP_TRY(hipSetDevice(s->device));
     HIP_TRY(hipStreamSynchronize(s->stream));
+    s->report_valid = false;
     HIP_TRY(hipMemcpy(s->d_state, &st, sizeof st, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(s->d_counts, p, 4 * kCkptRows * 16, hipMemcpyHostToDevice));
     p += 4 * kCkptRows * 16;
@@ -2331,7 +2360,7 @@ void pt_sim_destroy(pt_sim* s) {
         if (e) (void)hipEventDestroy(e);
     for (auto e : s->group_ev)
         if (e) (void)hipEventDestroy(e);
-    if (s->h_done) (void)hipHostFree(s->h_done);
+    if (s->report) (void)hipHostFree(s->report);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
