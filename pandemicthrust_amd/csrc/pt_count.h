@@ -30,8 +30,8 @@
 // Layouts of at most kCountMaxK buckets count in one block per chunk (32-bit
 // counters in one CU's 160 KB LDS).  Larger ones are split into column
 // groups (an hour, or kCountMaxK locations of one): k_keys_* write the keys
-// by hour first, then k_count_group counts (chunk, group) from them, and
-// k_collect_group lists; the rest is shared.
+// by hour or group first, then k_count_group counts (chunk, group) from them,
+// and k_collect_group lists; the rest is shared.
 //
 // Against the sorted tables: 2.35M agents x 100 days 20.7 -> 9.8 ms, 50M x
 // 100 days (split) 148 -> 82 ms, 24M with 10x the locations (split, few
@@ -70,7 +70,7 @@ struct CountRep {
     // the rest) the second's ...; `ranges` groups of W buckets per hour, G in
     // all (1: not split).
     int32_t E, W, ranges, G;
-    int32_t pad;
+    int32_t toff;  // tile_off entries per tile (group lists): G + 1 and some
 };
 
 struct CountBlock {
@@ -104,8 +104,8 @@ struct CountTable {
     const CountBlock* scans;
     uint16_t* keys;        // keys per agent x slots (split weekday layouts: within the hour)
     int64_t slots;
-    uint32_t* keys32;      // the same for hours of over 65,535 locations, or the weekend's hour lists
-    uint16_t* tile_off;    // hour lists: where each tile's hours begin
+    uint32_t* keys32;      // or the pairs by tile and group
+    uint16_t* tile_off;    // where each tile's groups begin
     uint32_t* cnt;         // the count matrices; then, per marked (chunk, bucket), its list's position
     uint32_t* pre;         // the prefixes
     uint32_t* total;       // people per bucket
@@ -614,15 +614,14 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
 
 // ---- split layouts (more than kCountMaxK buckets; one simulation) ----
 
-constexpr int kTileAgents = 4096;  // weekend hour lists: agents per tile, ids within it 12 bits
+constexpr int kTileAgents = 4096;  // group lists: agents per tile, ids within it 12 bits
 constexpr int kTileBits = 12;
 constexpr int kTileThreads = 512;
-constexpr int kTileHours = 16;     // tile_off entries per tile (11 used)
+constexpr int kTileGroups = 96;    // at most 10 hours x kCountMaxRanges, and the end
 
-// Weekday keys by hour, a pair of agents per thread and turn.  VALU bound: 50M
-// agents 160 us, of which the draws 99; the walk rows in LDS (load_walk) took
-// it from 184.
-template <class KT>
+// Weekday keys by hour, a pair of agents per thread and turn (one group per
+// hour).  VALU bound: 50M agents 160 us, of which the draws 99; the walk rows
+// in LDS (load_walk) took it from 184.
 __global__ __launch_bounds__(256) void k_keys_weekday(DayState* __restrict__ st, const Model* __restrict__ Mp,
                                                       const uint8_t* __restrict__ age, CountTable T) {
     if (st->done) return;
@@ -633,12 +632,13 @@ __global__ __launch_bounds__(256) void k_keys_weekday(DayState* __restrict__ st,
     __syncthreads();
     const int base = M.wd_base, base1 = M.wd_base1;
     const uint64_t eoff = st->rand_offset;
-    KT* keys = sizeof(KT) == 2 ? reinterpret_cast<KT*>(T.keys) : reinterpret_cast<KT*>(T.keys32);
+    uint32_t* const keys0 = reinterpret_cast<uint32_t*>(T.keys);
+    uint32_t* const keys1 = reinterpret_cast<uint32_t*>(T.keys + T.slots);
     bool bad = false;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; 2 * g < N; g += stride) {
         const U4 u = draw4(eoff + (uint64_t)g, M.key0, M.key1);
-        KT k0[2], k1[2];
+        uint32_t w0 = 0, w1 = 0;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int64_t p = 2 * g + k;
@@ -646,90 +646,126 @@ __global__ __launch_bounds__(256) void k_keys_weekday(DayState* __restrict__ st,
             int32_t d1, d2;
             weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
             bad |= (uint32_t)(d1 - base) >= (uint32_t)M.wd_E;
-            k0[k] = (KT)(d1 - base);
-            k1[k] = adult ? (KT)(d2 - base1) : (KT)~0u;
+            w0 |= ((uint32_t)(d1 - base) & 0xFFFFu) << (16 * k);
+            w1 |= (adult ? (uint32_t)(d2 - base1) & 0xFFFFu : kNoKey) << (16 * k);
         }
         // (slots is a multiple of 8: the pair's store stays inside the plane)
-        struct alignas(2 * sizeof(KT)) Two {
-            KT a, b;
-        };
-        reinterpret_cast<Two*>(keys)[g] = Two{k0[0], k0[1]};
-        reinterpret_cast<Two*>(keys + T.slots)[g] = Two{k1[0], k1[1]};
+        keys0[g] = w0;
+        keys1[g] = w1;
     }
     if (bad) st->fault = 1;
 }
 
-// Weekend pairs by hour: a block draws a tile's errands and writes them
-// grouped by hour (location << kTileBits | id within the tile), staged in
-// LDS so that the stores are contiguous.  VALU bound like k_count; the rank
-// of a pair within its hour is a returning LDS add, its order is free.  50M
-// agents 545 us, of which the draws 395.
-__global__ __launch_bounds__(kTileThreads) void k_keys_weekend(DayState* __restrict__ st,
-                                                               const Model* __restrict__ Mp, CountTable T) {
+// Pairs by group: a block draws a tile's errands and writes them grouped
+// (location within the hour << kTileBits | id within the tile), staged in LDS
+// so that the stores are contiguous.  VALU bound like k_count; the rank of a
+// pair within its group is a returning LDS add, its order is free.  50M agents,
+// weekend 545 us, of which the draws 395.
+//
+// Grouping by range and not by hour alone: each block of k_count_group reads
+// its own pairs instead of its hour's (24M agents with 10 times the locations,
+// weekend: counts 205 -> 112 us).
+template <bool WEEKEND>
+__global__ __launch_bounds__(kTileThreads) void k_keys_lists(DayState* __restrict__ st, const Model* __restrict__ Mp,
+                                                             const uint8_t* __restrict__ age, CountTable T) {
     if (st->done) return;
-    constexpr int PER = kTileAgents / kTileThreads;
-    __shared__ uint32_t s_stage[3 * kTileAgents];
-    __shared__ uint32_t s_cnt[kTileHours], s_base[kTileHours];
+    constexpr int KPA = WEEKEND ? 3 : 2, PER = kTileAgents / kTileThreads;
+    __shared__ uint32_t s_stage[KPA * kTileAgents];
+    __shared__ uint32_t s_cnt[kTileGroups], s_base[kTileGroups];
     const Model& M = *Mp;
     const int tid = threadIdx.x;
     const int64_t t0 = (int64_t)blockIdx.x * kTileAgents;
     __shared__ __align__(16) WalkRow s_row[kWalkRows];
-    const LdsWalk wk = load_walk(M.we_table, s_row);
-    if (tid < kTileHours) s_cnt[tid] = 0;
+    const LdsWalk wk = load_walk(WEEKEND ? M.we_table : M.wd_table, s_row);
+    if (tid < kTileGroups) s_cnt[tid] = 0;
+    const int ranges = T.reps[0].ranges, W = T.reps[0].W, G = T.reps[0].G;
     __syncthreads();
     const uint64_t eoff = st->rand_offset;
-    uint32_t pair[3 * PER], at[3 * PER];
+    uint32_t pair[KPA * PER], at[KPA * PER];
     bool bad = false;
+    auto add = [&](int slot, int hour, uint32_t l, int id) {
+        int g = hour * ranges;
+        for (int r = 1; r < ranges; ++r) g += l >= (uint32_t)(r * W);
+        pair[slot] = (l << kTileBits) | (uint32_t)id;
+        at[slot] = ((uint32_t)g << 16) | atomicAdd(&s_cnt[g], 1u);
+    };
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int id = i * kTileThreads + tid;
-        const int64_t p = t0 + id;
-        int32_t hour[3], loc[3];
-        if (p < M.N) weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
+    for (int i = 0; i < KPA * PER; ++i) at[i] = ~0u;
+    if constexpr (WEEKEND) {
 #pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            at[3 * i + e] = ~0u;
+        for (int i = 0; i < PER; ++i) {
+            const int id = i * kTileThreads + tid;
+            const int64_t p = t0 + id;
+            int32_t hour[3], loc[3];
             if (p < M.N) {
-                const uint32_t l = (uint32_t)(loc[e] - M.we_base);
-                bad |= l >= (uint32_t)M.we_E;
-                pair[3 * i + e] = (l << kTileBits) | (uint32_t)id;
-                at[3 * i + e] = ((uint32_t)hour[e] << 16) | atomicAdd(&s_cnt[hour[e]], 1u);
+                weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * (int32_t)p), hour, loc);
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    uint32_t l = (uint32_t)(loc[e] - M.we_base);
+                    if (l >= (uint32_t)M.we_E) bad = true, l = 0;
+                    add(3 * i + e, hour[e], l, id);
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER / 2; ++i) {
+            const int64_t g = t0 / 2 + i * kTileThreads + tid;
+            if (2 * g >= M.N) continue;
+            const U4 u = draw4(eoff + (uint64_t)g, M.key0, M.key1);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int64_t p = 2 * g + k;
+                const int id = (int)(p - t0);
+                if (p >= M.N) continue;
+                const bool adult = age[p] == kAgeAdult;
+                int32_t d1, d2;
+                weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
+                uint32_t l = (uint32_t)(d1 - M.wd_base);
+                if (l >= (uint32_t)M.wd_E) bad = true, l = 0;
+                add(4 * i + 2 * k, 0, l, id);
+                if (adult) {
+                    l = (uint32_t)(d2 - M.wd_base1);
+                    if (l >= (uint32_t)M.wd_E1) bad = true, l = 0;
+                    add(4 * i + 2 * k + 1, 1, l, id);
+                }
             }
         }
     }
     if (bad) st->fault = 1;
     __syncthreads();
-    if (tid < kTileHours) {
+    if (tid <= G) {
         uint32_t b = 0;
         for (int h = 0; h < tid; ++h) b += s_cnt[h];
         s_base[tid] = b;
-        T.tile_off[(int64_t)blockIdx.x * kTileHours + tid] = (uint16_t)b;
+        T.tile_off[(int64_t)blockIdx.x * T.reps[0].toff + tid] = (uint16_t)b;
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 3 * PER; ++i)
+    for (int i = 0; i < KPA * PER; ++i)
         if (at[i] != ~0u) s_stage[s_base[at[i] >> 16] + (at[i] & 0xFFFFu)] = pair[i];
     __syncthreads();
-    const int n = 3 * (int)min((int64_t)kTileAgents, (int64_t)M.N - t0);
-    uint32_t* out = T.keys32 + 3 * t0;
+    const int n = (int)s_base[G];
+    uint32_t* out = T.keys32 + KPA * t0;
     for (int i = tid; i < n; i += kTileThreads) out[i] = s_stage[i];
 }
 
-// Calls f(location within the hour, agent) for every pair of the (chunk,
-// group)'s hour in part `part` of `parts`; out-of-group locations included.
-template <bool WEEKEND, class KT, class F>
-__device__ __forceinline__ void group_pairs(const CountTable& T, const CountRep& c, int64_t N, int chunk, int hour,
+// Calls f(location within the hour, agent) for the pairs of the chunk's groups
+// [g0, g1) in part `part` of `parts`.  L: keys per agent of the group lists,
+// or 0: 2-byte keys by hour.
+template <int L, class F>
+__device__ __forceinline__ void group_pairs(const CountTable& T, const CountRep& c, int64_t N, int chunk, int g0, int g1,
                                             int part, int parts, F f) {
     const int64_t a0 = (int64_t)chunk * c.A, a1 = min(N, a0 + c.A);
     const int tid = threadIdx.x, nt = blockDim.x;
-    if (WEEKEND) {
+    if constexpr (L > 0) {
         // A wave per tile.
         const int lane = tid & 63, waves = nt >> 6;
         const int t1 = (int)((a1 + kTileAgents - 1) / kTileAgents);
         for (int t = (int)(a0 / kTileAgents) + part * waves + (tid >> 6); t < t1; t += parts * waves) {
-            const uint16_t* o = T.tile_off + (int64_t)t * kTileHours + hour;
-            const int b = o[0], e = o[1];
-            const uint32_t* src = T.keys32 + (int64_t)t * 3 * kTileAgents;
+            const uint16_t* o = T.tile_off + (int64_t)t * c.toff;
+            const int b = o[g0], e = o[g1];
+            const uint32_t* src = T.keys32 + (int64_t)t * L * kTileAgents;
             constexpr int U = 8;
             for (int i0 = b; i0 < e; i0 += U * 64) {
                 uint32_t v[U];
@@ -745,25 +781,23 @@ __device__ __forceinline__ void group_pairs(const CountTable& T, const CountRep&
             }
         }
     } else {
-        constexpr int V = 16 / sizeof(KT);
-        const KT* keys = (sizeof(KT) == 2 ? reinterpret_cast<const KT*>(T.keys) : reinterpret_cast<const KT*>(T.keys32)) +
-                         hour * T.slots;
+        const uint16_t* keys = T.keys + g0 * T.slots;
         constexpr int U = 4;
-        for (int64_t g0 = a0 / V + (int64_t)part * U * nt + tid; g0 * V < a1; g0 += (int64_t)parts * U * nt) {
+        for (int64_t w0 = a0 / 8 + (int64_t)part * U * nt + tid; w0 * 8 < a1; w0 += (int64_t)parts * U * nt) {
             uint4 v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int64_t g = g0 + (int64_t)u * nt;
-                v[u] = g * V < a1 ? reinterpret_cast<const uint4*>(keys)[g] : make_uint4(~0u, ~0u, ~0u, ~0u);
+                const int64_t w = w0 + (int64_t)u * nt;
+                v[u] = w * 8 < a1 ? reinterpret_cast<const uint4*>(keys)[w] : make_uint4(~0u, ~0u, ~0u, ~0u);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int64_t p0 = (g0 + (int64_t)u * nt) * V;
+                const int64_t p0 = (w0 + (int64_t)u * nt) * 8;
                 const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
-                for (int k = 0; k < V; ++k) {
-                    const uint32_t key = sizeof(KT) == 2 ? (w[k / 2] >> (16 * (k % 2))) & 0xFFFFu : w[k];
-                    if (key != (uint32_t)(KT)~0u && p0 + k < a1) f(key, (int)(p0 + k));
+                for (int k = 0; k < 8; ++k) {
+                    const uint32_t key = (w[k / 2] >> (16 * (k % 2))) & 0xFFFFu;
+                    if (key != kNoKey && p0 + k < a1) f(key, (int)(p0 + k));
                 }
             }
         }
@@ -792,21 +826,21 @@ __device__ __forceinline__ GroupColumns hour_columns(const CountRep& c, int hour
     return GroupColumns{hour, 0, last.lo + last.n, hour * c.E};
 }
 
-// Counts of a (chunk, group).  Reads the hour's keys (16 bytes per lane and
-// load) once per group of the hour; LDS adds hide behind them: 50M agents, 40
-// us per weekday (5 TB/s), 163 us per weekend day (3.7 TB/s).
-template <bool WEEKEND, class KT>
+// Counts of a (chunk, group).  Bound by reading its keys (16 bytes per lane
+// and load) or pairs; LDS adds hide behind them: 50M agents, 40 us per weekday
+// (5 TB/s), 163 us per weekend day (3.7 TB/s).
+template <int L>
 __global__ __launch_bounds__(1024) void k_count_group(const DayState* __restrict__ st, const Model* __restrict__ Mp,
                                                       CountTable T) {
     if (st->done) return;
     extern __shared__ uint32_t s_cnt[];
     const CountRep c = T.reps[0];
-    const int chunk = blockIdx.x / c.G;
-    const GroupColumns q = group_columns(c, blockIdx.x % c.G);
+    const int chunk = blockIdx.x / c.G, g = blockIdx.x % c.G;
+    const GroupColumns q = group_columns(c, g);
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int i = tid; i < q.n; i += nt) s_cnt[i] = 0;
     __syncthreads();
-    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, 0, 1, [&](uint32_t l, int) {
+    group_pairs<L>(T, c, Mp->N, chunk, g, g + 1, 0, 1, [&](uint32_t l, int) {
         const uint32_t i = l - (uint32_t)q.lo;
         if (i < (uint32_t)q.n) atomicAdd(&s_cnt[i], 1u);
     });
@@ -839,7 +873,7 @@ __device__ __forceinline__ void for_marked(const uint32_t* __restrict__ marks, c
     }
 }
 
-template <bool WEEKEND, class KT>
+template <int L>
 __global__ __launch_bounds__(kCollectFewThreads) void k_collect_few(const DayState* __restrict__ st,
                                                                     const Model* __restrict__ Mp, CountTable T) {
     if (st->done) return;
@@ -863,13 +897,14 @@ __global__ __launch_bounds__(kCollectFewThreads) void k_collect_few(const DaySta
     __syncthreads();
     if (s_n > kFewMarks * (uint32_t)c.ranges) return;
     uint32_t* cursor = T.cnt + c.mbase + (int64_t)chunk * c.K + q.bucket;
-    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, part, kCollectParts, [&](uint32_t l, int p) {
-        const uint32_t i = l - (uint32_t)q.lo;
-        if (i < (uint32_t)q.n && is_marked(s_bits, i)) T.list[atomicAdd(&cursor[i], 1u)] = p;
-    });
+    group_pairs<L>(T, c, Mp->N, chunk, q.hour * c.ranges, (q.hour + 1) * c.ranges, part, kCollectParts,
+                   [&](uint32_t l, int p) {
+                       const uint32_t i = l - (uint32_t)q.lo;
+                       if (i < (uint32_t)q.n && is_marked(s_bits, i)) T.list[atomicAdd(&cursor[i], 1u)] = p;
+                   });
 }
 
-template <bool WEEKEND, class KT>
+template <int L>
 __global__ __launch_bounds__(1024) void k_collect_group(const DayState* __restrict__ st, const Model* __restrict__ Mp,
                                                         CountTable T) {
     if (st->done) return;
@@ -877,8 +912,8 @@ __global__ __launch_bounds__(1024) void k_collect_group(const DayState* __restri
     if (T.chunk_day[blockIdx.x] != st->day + 1) return;
     extern __shared__ uint32_t s_cur[];
     __shared__ uint32_t s_n;
-    const int chunk = blockIdx.x / c.G;
-    const GroupColumns q = group_columns(c, blockIdx.x % c.G);
+    const int chunk = blockIdx.x / c.G, g = blockIdx.x % c.G;
+    const GroupColumns q = group_columns(c, g);
     const int tid = threadIdx.x, nt = blockDim.x;
     const uint32_t* marks = T.marks + c.qbase + (int64_t)chunk * c.qw;
     uint32_t* cursor = T.cnt + c.mbase + (int64_t)chunk * c.K + q.bucket;
@@ -891,7 +926,7 @@ __global__ __launch_bounds__(1024) void k_collect_group(const DayState* __restri
     __syncthreads();
     for_marked(marks, q, [&](int b) { s_cur[b - q.bucket] = cursor[b - q.bucket]; });
     __syncthreads();
-    group_pairs<WEEKEND, KT>(T, c, Mp->N, chunk, q.hour, 0, 1, [&](uint32_t l, int p) {
+    group_pairs<L>(T, c, Mp->N, chunk, g, g + 1, 0, 1, [&](uint32_t l, int p) {
         const uint32_t i = l - (uint32_t)q.lo;
         if (i < (uint32_t)q.n && s_cur[i] != ~0u) T.list[atomicAdd(&s_cur[i], 1u)] = p;
     });
@@ -1030,7 +1065,7 @@ inline int32_t count_chunk(int64_t N, int64_t K, int kpa, int64_t want) {
 // The plan of one layout on the host, and its device copies.
 struct CountPlan {
     bool on = false;
-    bool split = false, wide = false;  // column groups; hours of over 65,535 locations
+    bool split = false, lists = false;  // column groups; pairs in group lists
     int n_chunks = 0, n_scans = 0, threads = 0, kpa = 0, scan_cols = 0;
     size_t lds = 0;
     int64_t entries = 0, mark_words = 0, buckets = 0;
@@ -1105,7 +1140,11 @@ struct CountPlan {
             if (kpa * A <= 16 * (int64_t)c.K || A == kTileAgents) break;
         }
         on = split = true;
-        wide = widest > 0xFFFF;
+        // Weekend hours are not in the order of the slots; a weekday hour in
+        // several groups would be read by each (24M agents, 4-byte keys:
+        // 84 us for them and 111 for the counts, instead of 114 and 53).
+        lists = kpa == 3 || c.ranges > 1;
+        c.toff = (c.G + 16) / 16 * 16;
         c.A = (int32_t)A;
         c.C = (int32_t)((N + A - 1) / A);
         c.qw = (c.K + 31) / 32;
@@ -1146,7 +1185,8 @@ struct CountScratch {
         if (e == 0) return 0;
         return dev_alloc(&cnt, e) || dev_alloc(&pre, e) || dev_alloc(&total, std::max(a.buckets, b.buckets)) || dev_alloc(&marks, std::max(a.mark_words, b.mark_words)) ||
                        dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 4) || dev_alloc(&lone_day, (int64_t)std::max(a.reps.size(), b.reps.size())) ||
-                       (b.split && dev_alloc(&tile_off, (N / kTileAgents + 1) * kTileHours))
+                       ((a.lists || b.lists) &&
+                        dev_alloc(&tile_off, (N / kTileAgents + 1) * std::max(a.lists ? a.reps[0].toff : 0, b.lists ? b.reps[0].toff : 0)))
                    ? PT_ENOMEM
                    : 0;
     }
@@ -1182,9 +1222,8 @@ inline hipError_t set_count_lds(const CountPlan& p) {
     const auto ptr = [](auto* k) { return reinterpret_cast<const void*>(k); };
     for (const void* k :
          {ptr(&k_count<false>), ptr(&k_count<true>), ptr(&k_collect<false>), ptr(&k_collect<true>),
-          ptr(&k_count_group<false, uint16_t>), ptr(&k_count_group<false, uint32_t>),
-          ptr(&k_count_group<true, uint32_t>), ptr(&k_collect_group<false, uint16_t>),
-          ptr(&k_collect_group<false, uint32_t>), ptr(&k_collect_group<true, uint32_t>)}) {
+          ptr(&k_count_group<0>), ptr(&k_count_group<2>), ptr(&k_count_group<3>), ptr(&k_collect_group<0>),
+          ptr(&k_collect_group<2>), ptr(&k_collect_group<3>)}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(4 * kCountMaxK));
         if (e != hipSuccess) return e;
     }
@@ -1197,14 +1236,13 @@ inline void enqueue_counts(const CountPlan& p, const CountTable& t, const int32_
                            int64_t models_n = 0, int grid_keys = 0) {
     if (p.split) {
         const int64_t N = models_n;
-        if (weekend)
-            launch(tm, KC_GEN_WEEKEND, k_keys_weekend, dim3((int)((N + kTileAgents - 1) / kTileAgents)),
-                   dim3(kTileThreads), st, sts, models, t);
+        if (p.lists)
+            launch(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_keys_lists<true> : k_keys_lists<false>,
+                   dim3((int)((N + kTileAgents - 1) / kTileAgents)), dim3(kTileThreads), st, sts, models, age, t);
         else
-            launch(tm, KC_GEN_WEEKDAY, p.wide ? k_keys_weekday<uint32_t> : k_keys_weekday<uint16_t>,
-                   dim3(grid_for((N + 1) / 2, 256, grid_keys)), dim3(256), st, sts, models, age, t);
-        const auto k = weekend ? k_count_group<true, uint32_t>
-                               : (p.wide ? k_count_group<false, uint32_t> : k_count_group<false, uint16_t>);
+            launch(tm, KC_GEN_WEEKDAY, k_keys_weekday, dim3(grid_for((N + 1) / 2, 256, grid_keys)), dim3(256), st, sts,
+                   models, age, t);
+        const auto k = weekend ? k_count_group<3> : (p.lists ? k_count_group<2> : k_count_group<0>);
         launch_lds(tm, KC_TABLE_COUNT, k, dim3(p.n_chunks), dim3(p.threads), p.lds, st, (const DayState*)sts, models, t);
     } else {
         launch_lds(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_count<true> : k_count<false>,
@@ -1220,12 +1258,10 @@ inline void enqueue_picks(const CountPlan& p, const CountTable& t, const ClaimAr
                           const DayState* sts, const Model* models, int grid, bool weekend, hipStream_t st,
                           LaunchTimer* tm) {
     if (p.split) {
-        const auto few = weekend ? k_collect_few<true, uint32_t>
-                                 : (p.wide ? k_collect_few<false, uint32_t> : k_collect_few<false, uint16_t>);
+        const auto few = weekend ? k_collect_few<3> : (p.lists ? k_collect_few<2> : k_collect_few<0>);
         launch_lds(tm, KC_COLLECT, few, dim3(p.n_chunks / p.reps[0].ranges * kCollectParts), dim3(kCollectFewThreads),
                    sizeof(uint32_t) * (size_t)(p.reps[0].W * p.reps[0].ranges / 32 + 2), st, sts, models, t);
-        const auto k = weekend ? k_collect_group<true, uint32_t>
-                               : (p.wide ? k_collect_group<false, uint32_t> : k_collect_group<false, uint16_t>);
+        const auto k = weekend ? k_collect_group<3> : (p.lists ? k_collect_group<2> : k_collect_group<0>);
         launch_lds(tm, KC_COLLECT, k, dim3(p.n_chunks), dim3(p.threads), p.lds, st, sts, models, t);
     } else {
         launch_lds(tm, KC_COLLECT, weekend ? k_collect<true> : k_collect<false>, dim3(p.n_chunks), dim3(p.threads),

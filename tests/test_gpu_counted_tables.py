@@ -29,7 +29,7 @@ CASES = [
     (0.6, 21.24, 7, 20000),        # 1.4M agents: several chunks, one group per hour
     (0.0004, 25.1, 7, 20),         # 943 agents; weekday hour 0 in two groups (40,160 locations)
     (0.1, 40.9, 7, 5000),          # 65,440 locations in weekday hour 0
-    (0.1, 41.0, 7, 5000),          # 65,600: 4-byte keys
+    (0.1, 41.0, 7, 5000),          # 65,600
     (0.3, 200.0, 7, 5000),         # 320,000: 8 groups
     (0.05, 200.5, 7, 5000),        # 320,800: weekday sorted
     (0.05, 2.98, 9, 2000),         # weekend 38,740 buckets: the largest counted beside the sweep
