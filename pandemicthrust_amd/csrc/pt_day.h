@@ -194,23 +194,33 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     return v;
 }
 
-// Sums over the 64 lanes of eight byte counters packed in v (bin b in byte
-// b; at most 16 per lane): three butterfly steps on the packed words (a byte
-// reaches at most 128), then three on 16-bit fields.  out[b] = the total of
-// bin b, in every lane.
-__device__ __forceinline__ void wave_sum_bins8(uint64_t v, uint32_t (&out)[8]) {
-    uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-#pragma unroll
-    for (int d = 1; d < 8; d <<= 1) {
-        lo += __shfl_xor(lo, d, 64);
-        hi += __shfl_xor(hi, d, 64);
-    }
+// v plus the value of the lane that the DPP control names (0 where there is
+// none, or in rows that ROWS leaves out).
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) {
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+// Inclusive scan over the lanes of a wave that is wholly active: within rows
+// of 16 lanes, then lane 15 to the next row, lane 31 to the upper half.
+__device__ __forceinline__ uint32_t full_wave_scan(uint32_t v) {
+    v = dpp_add<0x111>(v);  // row_shr:1
+    v = dpp_add<0x112>(v);
+    v = dpp_add<0x114>(v);
+    v = dpp_add<0x118>(v);
+    v = dpp_add<0x142, 0xA>(v);  // row_bcast:15
+    return dpp_add<0x143, 0xC>(v);  // row_bcast:31
+}
+
+// Sums over the 64 lanes (all active) of eight byte counters, four to a word
+// (bin b in byte b; at most 16 per lane): a scan over 8 lanes on the packed
+// words (a byte reaches at most 128), the rest on 16-bit fields.  out[b] = the
+// total of bin b, in lane 63.
+__device__ __forceinline__ void wave_sum_bins8(uint32_t lo, uint32_t hi, uint32_t (&out)[8]) {
+    lo = dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(lo)));
+    hi = dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(hi)));
     uint32_t w[4] = {lo & 0x00FF00FFu, (lo >> 8) & 0x00FF00FFu, hi & 0x00FF00FFu, (hi >> 8) & 0x00FF00FFu};
 #pragma unroll
-    for (int d = 8; d < 64; d <<= 1) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] += __shfl_xor(w[j], d, 64);
-    }
+    for (int j = 0; j < 4; ++j) w[j] = dpp_add<0x143, 0xC>(dpp_add<0x142, 0xA>(dpp_add<0x118>(w[j])));
     // w[0]: bins 0 and 2, w[1]: 1 and 3, w[2]: 4 and 6, w[3]: 5 and 7
     out[0] = w[0] & 0xFFFFu;
     out[2] = w[0] >> 16;
@@ -232,141 +242,141 @@ __device__ __forceinline__ void plan_offsets(DayState* st, bool weekend, int64_t
 
 // ---------------- D1 + D2: sweep ----------------
 
+// Bytewise on four agents per word (bit 7 of each byte of the result): x != 0
+// but for its lowest bit; x <= y.
+__device__ __forceinline__ uint32_t bytes_infected(uint32_t x) {
+    const uint32_t t = x & 0xFEFEFEFEu;
+    return (((t & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | t) & 0x80808080u;
+}
+__device__ __forceinline__ uint32_t bytes_at_most(uint32_t x, uint32_t y) {
+    const uint32_t z = (y | 0x80808080u) - (x & 0x7F7F7F7Fu);
+    return ((y & ~x) | (~(x ^ y) & z)) & 0x80808080u;
+}
+// Codes 0..7 of 16 agents in w (byte j of word d: agent 4 d + j), those in
+// valid (bit 8 j + d), counted in byte counters.
+__device__ __forceinline__ void count_codes(const uint32_t (&w)[4], uint32_t valid, uint32_t& lo, uint32_t& hi) {
+    uint32_t p[3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        p[b] = 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) p[b] |= (d >= b ? w[d] << (d - b) : w[d] >> (b - d)) & (0x01010101u << d);
+    }
+    const uint32_t q0 = ~p[0], a = ~(p[1] | p[2]) & valid, c = p[1] & ~p[2] & valid, e = p[2] & ~p[1] & valid,
+                   f = p[1] & p[2] & valid;
+    lo = __popc(a & q0) | (__popc(a & p[0]) << 8) | (__popc(c & q0) << 16) | (__popc(c & p[0]) << 24);
+    hi = __popc(e & q0) | (__popc(e & p[0]) << 8) | (__popc(f & q0) << 16) | (__popc(f & p[0]) << 24);
+}
+
 // One sweep block (kSweepThreads threads) over agents [t0, t0 + kSweepTile)
 // of a population of N: recover (infection day <= current_day - (latent +
 // infectious days), the reference's current_day - 10), count the 8 status
 // codes per strain and stage the ids (+ id_bias) of infected agents.
 // (kernel_countInfectedStatusAndRecover PandemicSim.cu:2097-2192,
 //  daily_buildInfectedArray_global :2207-2224.)  The status arrays hold
-// whole uint4 words past N.
+// whole uint4 words past N.  Four agents per 32-bit operation: agent by agent
+// the vector instructions, not memory, set its time (50M agents 47 us, now 35:
+// 2.9 TB/s).
 __device__ __forceinline__ void sweep_block(const Model& M, int64_t N, int day, int64_t t0, uint8_t* __restrict__ st_p,
                                             uint8_t* __restrict__ st_s, const uint8_t* __restrict__ dy_p,
                                             const uint8_t* __restrict__ dy_s, uint32_t* __restrict__ counts16,
                                             uint32_t* __restrict__ ninf_out, int32_t* __restrict__ stage,
                                             int32_t id_bias) {
-    const int dtr_p = day - (M.lat[0] + M.dur[0]);
-    const int dtr_s = day - (M.lat[1] + M.dur[1]);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t a0 = t0 + (int64_t)tid * kSweepPer;
-    uint8_t sp[kSweepPer], ss[kSweepPer];
+    static_assert(kSweepPer == 16, "four words of four agents");
     const bool full = a0 + kSweepPer <= N;
-    if (full) {
-        const uint4 vp = *reinterpret_cast<const uint4*>(st_p + a0);
-        const uint4 vs = *reinterpret_cast<const uint4*>(st_s + a0);
-        memcpy(sp, &vp, 16);
-        memcpy(ss, &vs, 16);
-    } else {
+    uint32_t valid = 0x0F0F0F0Fu;
+    if (!full) {
+        valid = 0;
 #pragma unroll
-        for (int i = 0; i < kSweepPer; ++i) {
-            sp[i] = (a0 + i < N) ? st_p[a0 + i] : kSusceptible;
-            ss[i] = (a0 + i < N) ? st_s[a0 + i] : kSusceptible;
-        }
+        for (int i = 0; i < kSweepPer; ++i) valid |= (a0 + i < N ? 1u : 0u) << (8 * (i % 4) + i / 4);
     }
-    if (dtr_p >= 0 || dtr_s >= 0) {
-        bool anyp = false, anys = false;
+    auto load = [&](const uint8_t* src, uint32_t (&w)[4]) {
+        if (full) {
+            const uint4 v = *reinterpret_cast<const uint4*>(src + a0);
+            w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
+        } else {
 #pragma unroll
-        for (int i = 0; i < kSweepPer; ++i) {
-            anyp |= sp[i] >= kInfected;
-            anys |= ss[i] >= kInfected;
-        }
-        if (anyp && dtr_p >= 0) {
-            uint8_t dp[kSweepPer];
-            if (full) {
-                const uint4 v = *reinterpret_cast<const uint4*>(dy_p + a0);
-                memcpy(dp, &v, 16);
-            } else {
-#pragma unroll
-                for (int i = 0; i < kSweepPer; ++i) dp[i] = (a0 + i < N) ? dy_p[a0 + i] : kDayNone;
-            }
-            bool dirty = false;
+            for (int d = 0; d < 4; ++d) w[d] = 0;
 #pragma unroll
             for (int i = 0; i < kSweepPer; ++i)
-                if (sp[i] >= kInfected && (int)dp[i] <= dtr_p) {
-                    sp[i] = kRecovered;
-                    dirty = true;
-                }
-            if (dirty) {
+                if (a0 + i < N) w[i / 4] |= (uint32_t)src[a0 + i] << (8 * (i % 4));
+        }
+    };
+    uint8_t* const st[2] = {st_p, st_s};
+    const uint8_t* const dy[2] = {dy_p, dy_s};
+    uint32_t w[2][4], inf = 0, lo[2], hi[2];
+    load(st_p, w[0]);
+    load(st_s, w[1]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        uint32_t x[4], any = 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) any |= x[d] = bytes_infected(w[k][d]);
+        const int due = day - (M.lat[k] + M.dur[k]);
+        if (due >= 0 && any) {
+            uint32_t v[4], rec = 0;
+            load(dy[k], v);
+            const uint32_t due4 = (uint32_t)min(due, 255) * 0x01010101u;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const uint32_t m = x[d] & bytes_at_most(v[d], due4);
+                rec |= m;
+                w[k][d] &= ~(m | (m - (m >> 7)));
+                x[d] &= ~m;
+            }
+            static_assert(kRecovered == 0, "recovered by clearing");
+            if (rec) {
                 if (full) {
-                    uint4 v;
-                    memcpy(&v, sp, 16);
-                    *reinterpret_cast<uint4*>(st_p + a0) = v;
+                    *reinterpret_cast<uint4*>(st[k] + a0) = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
                 } else {
                     for (int i = 0; i < kSweepPer; ++i)
-                        if (a0 + i < N) st_p[a0 + i] = sp[i];
+                        if (a0 + i < N) st[k][a0 + i] = (uint8_t)(w[k][i / 4] >> (8 * (i % 4)));
                 }
             }
         }
-        if (anys && dtr_s >= 0) {
-            uint8_t ds[kSweepPer];
-            if (full) {
-                const uint4 v = *reinterpret_cast<const uint4*>(dy_s + a0);
-                memcpy(ds, &v, 16);
-            } else {
 #pragma unroll
-                for (int i = 0; i < kSweepPer; ++i) ds[i] = (a0 + i < N) ? dy_s[a0 + i] : kDayNone;
-            }
-            bool dirty = false;
-#pragma unroll
-            for (int i = 0; i < kSweepPer; ++i)
-                if (ss[i] >= kInfected && (int)ds[i] <= dtr_s) {
-                    ss[i] = kRecovered;
-                    dirty = true;
-                }
-            if (dirty) {
-                if (full) {
-                    uint4 v;
-                    memcpy(&v, ss, 16);
-                    *reinterpret_cast<uint4*>(st_s + a0) = v;
-                } else {
-                    for (int i = 0; i < kSweepPer; ++i)
-                        if (a0 + i < N) st_s[a0 + i] = ss[i];
-                }
-            }
-        }
-    }
-    // Counts: 8 bins per strain packed as bytes (at most 16 per thread).
-    uint64_t cp = 0, cs = 0;
-    uint32_t inf_mask = 0;
-#pragma unroll
-    for (int i = 0; i < kSweepPer; ++i) {
-        if (a0 + i < N) {
-            cp += 1ull << (8 * (sp[i] & 7));
-            cs += 1ull << (8 * (ss[i] & 7));
-            if (sp[i] >= kInfected || ss[i] >= kInfected) inf_mask |= 1u << i;
-        }
+        for (int d = 0; d < 4; ++d) inf |= x[d] >> (7 - d);
+        count_codes(w[k], valid, lo[k], hi[k]);
     }
     __shared__ uint32_t s_cnt[kSweepThreads / 64][16];
     __shared__ uint32_t s_inf[kSweepThreads / 64];
-    {
-        uint32_t vp[8], vs[8];
-        wave_sum_bins8(cp, vp);
-        wave_sum_bins8(cs, vs);
-        if (lane == 0) {
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                s_cnt[wave][b] = vp[b];
-                s_cnt[wave][8 + b] = vs[b];
-            }
+    for (int k = 0; k < 2; ++k) {
+        uint32_t v[8];
+        wave_sum_bins8(lo[k], hi[k], v);
+        if (lane == 63) {
+#pragma unroll
+            for (int b = 0; b < 8; ++b) s_cnt[wave][8 * k + b] = v[b];
         }
     }
-    const uint32_t ninf = (uint32_t)__popc(inf_mask);
-    const uint32_t inc = wave_incl_scan(ninf, lane);
+    const uint32_t ninf = (uint32_t)__popc(inf);
+    const uint32_t inc = full_wave_scan(ninf);
     if (lane == 63) s_inf[wave] = inc;
     __syncthreads();
     uint32_t wbase = 0, total = 0;
 #pragma unroll
-    for (int w = 0; w < kSweepThreads / 64; ++w) {
-        if (w < wave) wbase += s_inf[w];
-        total += s_inf[w];
+    for (int i = 0; i < kSweepThreads / 64; ++i) {
+        if (i < wave) wbase += s_inf[i];
+        total += s_inf[i];
     }
     uint32_t pos = wbase + inc - ninf;
-#pragma unroll
-    for (int i = 0; i < kSweepPer; ++i)
-        if (inf_mask & (1u << i)) stage[pos++] = id_bias + (int32_t)(a0 + i);
+    // Bit 8 j + d -> 4 j + d -> 4 d + j: the agents in order.
+    uint32_t m = (inf & 0xFu) | ((inf >> 4) & 0xF0u) | ((inf >> 8) & 0xF00u) | ((inf >> 12) & 0xF000u);
+    uint32_t t = (m ^ (m >> 3)) & 0x0A0Au;
+    m ^= t ^ (t << 3);
+    t = (m ^ (m >> 6)) & 0x00CCu;
+    m ^= t ^ (t << 6);
+    const int32_t id0 = id_bias + (int32_t)a0;
+    while (m) {
+        stage[pos++] = id0 + __ffs(m) - 1;
+        m &= m - 1;
+    }
     if (tid < 16) {
         uint32_t s = 0;
 #pragma unroll
-        for (int w = 0; w < kSweepThreads / 64; ++w) s += s_cnt[w][tid];
+        for (int i = 0; i < kSweepThreads / 64; ++i) s += s_cnt[i][tid];
         counts16[tid] = s;
     }
     if (tid == 0) *ninf_out = total;
