@@ -572,6 +572,8 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
                                                   const DayState* __restrict__ sts,
                                                   const Model* __restrict__ models, CountTable T) {
     constexpr int KPA = WEEKEND ? 3 : 2;
+    load_arguments<5>();
+    load_together(*done, T.chunks[blockIdx.x].r, T.chunk_day[blockIdx.x], T.reps[0].K);
     if (*done) return;
     extern __shared__ uint32_t s_cur[];
     __shared__ uint32_t s_top;
@@ -1012,6 +1014,8 @@ __device__ __forceinline__ int32_t picked_person(const CountTable& T, uint32_t q
 }
 
 __global__ __launch_bounds__(256) void k_resolve(DayState* __restrict__ g, CountTable T, ClaimArrays C) {
+    load_arguments<5>();
+    load_together(g->done, T.n[0], T.reps[0].K, g->day);
     if (g->done) return;
     const uint32_t n = *T.n;
     const int sub = threadIdx.x % kPickLanes, lane = threadIdx.x & 63;

@@ -179,6 +179,36 @@ __host__ __device__ __forceinline__ int64_t mark_limit(int64_t K, int pct) { ret
 
 // ---------------- wave helpers ----------------
 
+// Scalar loads in one batch.  Left to themselves the loads of a kernel's
+// arguments, the day's state and the model come one by one as the code reaches
+// them, each a miss of the scalar cache, which starts cold: some ten in a row
+// before a kernel's first vector load, 1 to 3 us of launches that take 6 to 20.
+// First the 64-byte lines of the arguments (all inside them) ...
+template <int LINES>
+__device__ __forceinline__ void load_arguments() {
+    static_assert(LINES == 2 || LINES == 5 || LINES == 8, "lines");
+    const auto k = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    if constexpr (LINES == 2)
+        asm volatile("" ::"s"(k[0]), "s"(k[16]));
+    else if constexpr (LINES == 5)
+        asm volatile("" ::"s"(k[0]), "s"(k[16]), "s"(k[32]), "s"(k[48]), "s"(k[64]));
+    else
+        asm volatile("" ::"s"(k[0]), "s"(k[16]), "s"(k[32]), "s"(k[48]), "s"(k[64]), "s"(k[80]), "s"(k[96]), "s"(k[112]));
+}
+// ... then what they point to: values, and the lines of the state and model.
+template <class A, class B, class C, class D>
+__device__ __forceinline__ void load_together(A a, B b, C c, D d) {
+    asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
+}
+__device__ __forceinline__ void load_state_and_model(const DayState* st, const Model* M, uint32_t more) {
+    static_assert(sizeof(Model) >= 21 * 64 && sizeof(DayState) >= 68, "the lines below");
+    const uint32_t* d = reinterpret_cast<const uint32_t*>(st);
+    const uint32_t* m = reinterpret_cast<const uint32_t*>(M);
+    asm volatile("" ::"s"(more), "s"(d[1]), "s"(d[16]), "s"(m[0]), "s"(m[16]), "s"(m[32]), "s"(m[48]), "s"(m[64]), "s"(m[80]), "s"(m[96]),
+                 "s"(m[112]), "s"(m[128]), "s"(m[144]), "s"(m[160]), "s"(m[176]), "s"(m[192]), "s"(m[208]), "s"(m[224]),
+                 "s"(m[240]), "s"(m[256]), "s"(m[272]), "s"(m[288]), "s"(m[304]), "s"(m[320]));
+}
+
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -293,16 +323,9 @@ __device__ __forceinline__ void sweep_block(const Model& M, int64_t N, int day, 
         for (int i = 0; i < kSweepPer; ++i) valid |= (a0 + i < N ? 1u : 0u) << (8 * (i % 4) + i / 4);
     }
     auto load = [&](const uint8_t* src, uint32_t (&w)[4]) {
-        if (full) {
-            const uint4 v = *reinterpret_cast<const uint4*>(src + a0);
-            w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
-        } else {
-#pragma unroll
-            for (int d = 0; d < 4; ++d) w[d] = 0;
-#pragma unroll
-            for (int i = 0; i < kSweepPer; ++i)
-                if (a0 + i < N) w[i / 4] |= (uint32_t)src[a0 + i] << (8 * (i % 4));
-        }
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (a0 < N) v = *reinterpret_cast<const uint4*>(src + a0);
+        w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
     };
     uint8_t* const st[2] = {st_p, st_s};
     const uint8_t* const dy[2] = {dy_p, dy_s};
@@ -313,7 +336,7 @@ __device__ __forceinline__ void sweep_block(const Model& M, int64_t N, int day, 
     for (int k = 0; k < 2; ++k) {
         uint32_t x[4], any = 0;
 #pragma unroll
-        for (int d = 0; d < 4; ++d) any |= x[d] = bytes_infected(w[k][d]);
+        for (int d = 0; d < 4; ++d) any |= x[d] = bytes_infected(w[k][d]) & (valid << (7 - d));
         const int due = day - (M.lat[k] + M.dur[k]);
         if (due >= 0 && any) {
             uint32_t v[4], rec = 0;

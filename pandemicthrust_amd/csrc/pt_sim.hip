@@ -413,6 +413,8 @@ __global__ __launch_bounds__(1024) void k_count_sweep(const Model* __restrict__ 
                                                       uint32_t* __restrict__ blk_counts,
                                                       uint32_t* __restrict__ blk_ninf, int32_t* __restrict__ staging,
                                                       CountTable T, int n_chunks) {
+    load_arguments<5>();
+    load_state_and_model(st, Mp, (uint32_t)T.reps[0].K);
     if (st->done) return;
     if ((int)blockIdx.x < n_chunks) {
         if (blockIdx.x == 0 && threadIdx.x < 3) T.n[threadIdx.x] = 0u;  // no picks, infectors or lists yet
@@ -430,6 +432,8 @@ __global__ __launch_bounds__(1024) void k_count_sweep(const Model* __restrict__ 
 template <bool WEEKEND, int COLS>
 __global__ __launch_bounds__(1024) void k_scan_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
                                                     CompactArgs a, AgentArrays A, CountTable T, int n_scans) {
+    load_arguments<8>();
+    load_state_and_model(st, Mp, (uint32_t)T.reps[0].K);
     if (st->done) return;
     if ((int)blockIdx.x < n_scans)
         scan_block<COLS>(blockIdx.x, n_scans, st, T);
@@ -598,6 +602,10 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
                                                               int32_t* __restrict__ list_p,
                                                               int32_t* __restrict__ list_s, CountTable T) {
     static_assert(!TRACE || !COUNTED, "traced contacts look every victim up");
+    if constexpr (COUNTED) {
+        load_arguments<8>();
+        load_state_and_model(st, Mp, T.n[1]);
+    }
     if (st->done) return;
     const Model& M = *Mp;
     const int I = st->n_infected;
@@ -716,6 +724,8 @@ __global__ __launch_bounds__(256) void k_apply_end(DayState* st, uint64_t* __res
                                                    uint8_t* __restrict__ gn_s, int32_t* __restrict__ tab_full,
                                                    int32_t* __restrict__ tab_pairs, int32_t n_full,
                                                    uint32_t* ticket) {
+    load_arguments<2>();
+    load_together(st->done, st->day, st->n_claimed[0], st->max_days);
     if (st->done) return;
     apply_claims(st, claim_p, claim_s, list_p, list_s, st_p, st_s, dy_p, dy_s, gn_p, gn_s);
     __syncthreads();  // the block is done with the day's state
