@@ -309,35 +309,46 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DayState* __restrict__ st
 
 // Counted days: the compaction also tests the infectors' success draws and
 // lists the ones left (list_infectors), and, for up to kFusedPlan sweep
-// blocks, is the day plan too (PLAN): every block sums the counts of the
-// blocks before it instead of waiting for a launch of one block.
-constexpr int kFusedPlan = 1024;
-constexpr int kMergedBlocks = 3;  // per CU
+// blocks (67M agents), is the day plan too (PLAN): every block sums the counts
+// of the blocks before its own instead of waiting for a launch of one block
+// (50M agents: 18 us per day).  A block takes every gridDim-th sweep block, so
+// that it does this once.  PLAN: sweep blocks per thread of the plan, 1 or
+// kPlanPer (or 0).
+constexpr int kPlanPer = 8;
+constexpr int kFusedPlan = 1024 * kPlanPer;
+constexpr int kMergedBlocks = 3, kCompactBlocks = 2;  // per CU
 struct CompactArgs {
     const int32_t* staging;
     const uint32_t *blk_ninf, *blk_off, *blk_counts;
-    int nblk, parts;  // sweep blocks, blocks that share the infected of each
+    int nblk, parts;  // sweep blocks; blocks that share the infected of each, if there are more of those
     int32_t *out_counts, *out_inf, *infected;
 };
-template <bool WEEKEND, bool PLAN>
-__device__ __forceinline__ void compact_test_block(int block, const Model* __restrict__ Mp, DayState* __restrict__ st,
-                                                   const CompactArgs& a, const AgentArrays& A, const CountTable& T,
-                                                   bool counted) {
-    const int32_t* __restrict__ staging = a.staging;
+template <bool WEEKEND, int PLAN>
+__device__ __forceinline__ void compact_test_block(int block, int blocks, const Model* __restrict__ Mp,
+                                                   DayState* __restrict__ st, const CompactArgs& a,
+                                                   const AgentArrays& A, const CountTable& T, bool counted) {
     const uint32_t* __restrict__ blk_ninf = a.blk_ninf;
-    const int nblk = a.nblk, own = block / a.parts, part = block % a.parts;
+    const int nblk = a.nblk, first = block / a.parts, part = block % a.parts, step = blocks / a.parts;
     constexpr int C = WEEKEND ? kContactsWe : kContactsWd;
     const Model& M = *Mp;
     const int tid = threadIdx.x;
     const int day = st->day;
     const int64_t N = M.N;
     const uint64_t cbase = st->rand_offset + (WEEKEND ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
-    uint32_t off;
-    if constexpr (PLAN) {
+    constexpr int kMaxOwn = kFusedPlan / 256;
+    __shared__ uint32_t s_off[kMaxOwn];
+    if constexpr (PLAN > 0) {
         const int lane = tid & 63, wave = tid >> 6;
-        __shared__ uint32_t s_w[16], s_off;
-        const uint32_t v = tid < nblk ? blk_ninf[tid] : 0u;
-        const uint32_t inc = wave_incl_scan(v, lane);
+        __shared__ uint32_t s_w[16];
+        const int per = PLAN == 1 ? 1 : (nblk + 1023) / 1024;  // consecutive sweep blocks of this thread
+        uint32_t v[PLAN], sum = 0;
+#pragma unroll
+        for (int k = 0; k < PLAN; ++k) {
+            const int b = tid * per + k;
+            v[k] = k < per && b < nblk ? blk_ninf[b] : 0u;
+            sum += v[k];
+        }
+        const uint32_t inc = full_wave_scan(sum);
         if (lane == 63) s_w[wave] = inc;
         __syncthreads();
         uint32_t before = 0, total = 0;
@@ -347,58 +358,79 @@ __device__ __forceinline__ void compact_test_block(int block, const Model* __res
             if (w < wave) before += x;
             total += x;
         }
-        if (tid == own) s_off = before + inc - v;
-        if (block == 0) {
-            // Daily counts: a wave per counter.
+        before += inc - sum;
+        if (step >= nblk) {
+            if (PLAN == 1 && tid == first) s_off[0] = before;
+        } else {
+#pragma unroll
+            for (int k = 0; k < PLAN; ++k) {
+                const int b = tid * per + k;
+                if (k < per && b < nblk && b % step == first) s_off[b / step] = before;
+                before += v[k];
+            }
+        }
+        // Daily counts: a block per counter, or one for all, a wave each.
+        if (PLAN > 1 && block < 16) {
+            uint32_t c = 0;
+            for (int b = tid; b < nblk; b += 1024) c += a.blk_counts[(int64_t)b * 16 + block];
+            c = full_wave_scan(c);
+            __shared__ uint32_t s_c[16];
+            if (lane == 63) s_c[wave] = c;
+            __syncthreads();
+            if (tid == 0) {
+                for (int w = 1; w < 16; ++w) c = (w == 1 ? s_c[0] : c) + s_c[w];
+                a.out_counts[day * 16 + block] = (int32_t)c;
+            }
+        } else if (PLAN == 1 && block == 0) {
             uint32_t c = 0;
             for (int b = lane; b < nblk; b += 64) c += a.blk_counts[(int64_t)b * 16 + wave];
-            c = wave_sum(c);
-            if (lane == 0) a.out_counts[day * 16 + wave] = (int32_t)c;
-            if (tid == 0) {
-                st->n_infected = (int32_t)total;
-                st->days_run = day + 1;
-                a.out_inf[day] = (int32_t)total;
-                if (total == 0) {
-                    st->done = 1;  // nobody left to compact: other blocks may or may not see it
-                    st->skip_full = st->skip_subset = st->skip_mark = 1;
-                } else {
-                    st->skip_full = 0;  // every bucket is counted
-                    st->skip_subset = st->skip_mark = 1;
-                    plan_offsets(st, WEEKEND, N);
-                }
+            c = full_wave_scan(c);
+            if (lane == 63) a.out_counts[day * 16 + wave] = (int32_t)c;
+        }
+        if (block == 0 && tid == 0) {
+            st->n_infected = (int32_t)total;
+            st->days_run = day + 1;
+            a.out_inf[day] = (int32_t)total;
+            if (total == 0) {
+                st->done = 1;  // nobody left to compact: other blocks may or may not see it
+                st->skip_full = st->skip_subset = st->skip_mark = 1;
+            } else {
+                st->skip_full = 0;  // every bucket is counted
+                st->skip_subset = st->skip_mark = 1;
+                plan_offsets(st, WEEKEND, N);
             }
         }
         __syncthreads();
-        off = s_off;
-    } else {
-        off = a.blk_off[own];
     }
-    const uint32_t n = blk_ninf[own];
-    const int32_t* src = staging + (int64_t)own * kSweepTile;
-    for (uint32_t i0 = part * blockDim.x; i0 < n; i0 += a.parts * blockDim.x) {
-        const uint32_t i = i0 + tid;
-        int32_t idx = 0;
-        Infectivity f{};
-        bool keep = false;
-        if (i < n) {
-            idx = src[i];
-            a.infected[off + i] = idx;
-            f = infectivity(M, A, idx, day);
-            if (can_infect(M, f)) {
-                SuccessDraws draws;
-                success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
-                keep = may_infect<C>(M, f, draws, 1) &&
-                       may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND, counted));
+    for (int own = first; own < nblk; own += step) {
+        const uint32_t off = PLAN ? s_off[own / step] : a.blk_off[own];
+        const uint32_t n = blk_ninf[own];
+        const int32_t* src = a.staging + (int64_t)own * kSweepTile;
+        for (uint32_t i0 = part * blockDim.x; i0 < n; i0 += a.parts * blockDim.x) {
+            const uint32_t i = i0 + tid;
+            int32_t idx = 0;
+            Infectivity f{};
+            bool keep = false;
+            if (i < n) {
+                idx = src[i];
+                a.infected[off + i] = idx;
+                f = infectivity(M, A, idx, day);
+                if (can_infect(M, f)) {
+                    SuccessDraws draws;
+                    success_draws<C>(M, cbase + (uint64_t)(6 * (int64_t)(off + i)) + 2, draws);
+                    keep = may_infect<C>(M, f, draws, 1) &&
+                           may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND, counted));
+                }
             }
+            list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
         }
-        list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
     }
 }
-template <bool WEEKEND, bool PLAN>
+template <bool WEEKEND, int PLAN>
 __global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
                                                        CompactArgs a, AgentArrays A, CountTable T) {
     if (st->done) return;
-    compact_test_block<WEEKEND, PLAN>(blockIdx.x, Mp, st, a, A, T, true);
+    compact_test_block<WEEKEND, PLAN>(blockIdx.x, gridDim.x, Mp, st, a, A, T, true);
 }
 
 // Small populations (merged_launches): launches of a few us each, in pairs
@@ -438,7 +470,7 @@ __global__ __launch_bounds__(1024) void k_scan_test(const Model* __restrict__ Mp
     if ((int)blockIdx.x < n_scans)
         scan_block<COLS>(blockIdx.x, n_scans, st, T);
     else
-        compact_test_block<WEEKEND, true>(blockIdx.x - n_scans, Mp, st, a, A, T, false);
+        compact_test_block<WEEKEND, 1>(blockIdx.x - n_scans, gridDim.x - n_scans, Mp, st, a, A, T, false);
 }
 
 // Also clears the bucket marks when today marks (k_plan decided).
@@ -679,24 +711,24 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
 // of queried buckets (n_sel pairs).
 // tab_pairs logs the pairs of the day's table: n_kept (when set) or n_full
 // on full-table days, the selected pairs on subset days.
-__device__ __forceinline__ void end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t* __restrict__ tab_pairs,
-                                        int32_t n_full, const uint32_t* __restrict__ n_kept) {
-    const int d = st->day;
-    tab_full[d] = st->skip_full == 0 ? 1 : 0;
-    tab_pairs[d] = st->skip_full == 0 ? (n_kept ? (int32_t)*n_kept : n_full)
-                                      : (st->skip_subset == 0 ? (int32_t)st->n_sel : 0);
-    st->day += 1;
-    st->rand_offset = st->contact_base + (uint64_t)6 * (uint64_t)st->n_infected;
+__device__ __forceinline__ void end_day(const DayState& d, DayState* st, int32_t* __restrict__ tab_full,
+                                        int32_t* __restrict__ tab_pairs, int32_t n_full,
+                                        const uint32_t* __restrict__ n_kept) {
+    tab_full[d.day] = d.skip_full == 0 ? 1 : 0;
+    tab_pairs[d.day] = d.skip_full == 0 ? (n_kept ? (int32_t)*n_kept : n_full)
+                                        : (d.skip_subset == 0 ? (int32_t)d.n_sel : 0);
+    st->day = d.day + 1;
+    st->rand_offset = d.contact_base + (uint64_t)6 * (uint64_t)d.n_infected;
     st->n_claimed[0] = 0;
     st->n_claimed[1] = 0;
     st->skip_full = 1;
     st->skip_subset = 1;
-    if (st->day >= st->max_days) st->done = 1;
+    if (d.day + 1 >= d.max_days) st->done = 1;
 }
 __global__ void k_end_day(DayState* st, int32_t* __restrict__ tab_full, int32_t* __restrict__ tab_pairs,
                           int32_t n_full, const uint32_t* __restrict__ n_kept) {
-    if (st->done) return;
-    end_day(st, tab_full, tab_pairs, n_full, n_kept);
+    const DayState d = *st;
+    if (!d.done) end_day(d, st, tab_full, tab_pairs, n_full, n_kept);
 }
 
 // The loop's state and a day's row of the daily outputs, for the host to read
@@ -725,13 +757,15 @@ __global__ __launch_bounds__(256) void k_apply_end(DayState* st, uint64_t* __res
                                                    int32_t* __restrict__ tab_pairs, int32_t n_full,
                                                    uint32_t* ticket) {
     load_arguments<2>();
-    load_together(st->done, st->day, st->n_claimed[0], st->max_days);
-    if (st->done) return;
-    apply_claims(st, claim_p, claim_s, list_p, list_s, st_p, st_s, dy_p, dy_s, gn_p, gn_s);
+    const DayState d = *st;  // (only the last block changes it)
+    load_together(d.done, d.day, d.n_claimed[0], d.n_claimed[1]);
+    load_together(d.skip_full, d.max_days, d.n_infected, d.contact_base);
+    if (d.done) return;
+    apply_claims(&d, claim_p, claim_s, list_p, list_s, st_p, st_s, dy_p, dy_s, gn_p, gn_s);
     __syncthreads();  // the block is done with the day's state
     if (threadIdx.x == 0 && atomicAdd(ticket, 1u) == gridDim.x - 1) {
         *ticket = 0u;
-        end_day(st, tab_full, tab_pairs, n_full, nullptr);
+        end_day(d, st, tab_full, tab_pairs, n_full, nullptr);
     }
 }
 
@@ -1390,7 +1424,7 @@ int enqueue_day(pt_sim* s, int d) {
     const CountTable& ct = s->count_table[weekend ? 1 : 0];
     const bool counted = s->table_mode == TABLES_AUTO && cp.on && !s->trace_on;
     const bool fused_plan = counted && s->nblk_sweep <= kFusedPlan;
-    const bool merged = fused_plan && merged_launches(s, cp);
+    const bool merged = counted && s->nblk_sweep <= 1024 && merged_launches(s, cp);
     AgentArrays A = agent_arrays(s);
     const Model* M = s->d_model;
     if (!merged)
@@ -1436,9 +1470,15 @@ int enqueue_day(pt_sim* s, int d) {
             launch(tm, KC_COMPACT, k, dim3(cp.n_scans + s->nblk_sweep * parts), dim3(1024), stc, M, st, a, A, ct,
                    cp.n_scans);
         } else {
-            const auto k = weekend ? (fused_plan ? k_compact_test<true, true> : k_compact_test<true, false>)
-                                   : (fused_plan ? k_compact_test<false, true> : k_compact_test<false, false>);
-            launch(tm, KC_COMPACT, k, dim3(s->nblk_sweep * parts), dim3(1024), stc, M, st, a, A, ct);
+            const int plan = !fused_plan ? 0 : (s->nblk_sweep <= 1024 ? 1 : kPlanPer);
+            const auto k = weekend ? (plan == 0 ? k_compact_test<true, 0>
+                                                : (plan == 1 ? k_compact_test<true, 1> : k_compact_test<true, kPlanPer>))
+                                   : (plan == 0 ? k_compact_test<false, 0>
+                                                : (plan == 1 ? k_compact_test<false, 1> : k_compact_test<false, kPlanPer>));
+            // (a planning block takes at most kFusedPlan / 256 sweep blocks)
+            const int blocks = s->nblk_sweep * parts;
+            launch(tm, KC_COMPACT, k, dim3(fused_plan ? std::min(blocks, std::max(256, kCompactBlocks * s->cus)) : blocks),
+                   dim3(1024), stc, M, st, a, A, ct);
         }
     } else {
         launch(tm, KC_COMPACT, k_compact, dim3(s->nblk_sweep), dim3(256), stc, (const DayState*)st,

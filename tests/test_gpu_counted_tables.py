@@ -35,7 +35,8 @@ CASES = [
     (0.05, 2.98, 9, 2000),         # weekend 38,740 buckets: the largest counted beside the sweep
     (1.0, 1.0, 7, 20000),          # 2.35M agents: launches in pairs
     (2.2, 1.0, 7, 20000),          # 5.2M: single launches, the compaction plans the day
-    (3.7, 1.0, 7, 20000),          # 8.7M: a plan launch of its own
+    (3.7, 1.0, 7, 20000),          # 8.7M: several sweep blocks per thread of the plan
+    (29.0, 1.0, 4, 20000),         # 68M: a plan launch of its own
 ]
 
 
