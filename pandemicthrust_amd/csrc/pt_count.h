@@ -24,6 +24,9 @@
 //   k_resolve     16 lanes per pick find the id with the pick's rank within
 //                 its list and post the infection claim
 //
+// While chunks are small (a simulation of up to a million agents), k_resolve
+// looks through the chunk's keys itself, and nothing is marked or listed.
+//
 // A chunk's list order does not matter (ranks are taken by value), so the
 // result is the id the sorted table holds at that position.
 //
@@ -104,6 +107,9 @@ struct CountTable {
     const CountBlock* scans;
     uint16_t* keys;        // keys per agent x slots (split weekday layouts: within the hour)
     int64_t slots;
+    int32_t direct;        // picks are found in the keys (planes of keys per agent), without lists
+    int32_t n_agents;      // direct: the simulation's agents, and its weekday buckets of hour 0
+    uint32_t hour1;
     uint32_t* keys32;      // or the pairs by tile and group
     uint16_t* tile_off;    // where each tile's groups begin
     uint32_t* cnt;         // the count matrices; then, per marked (chunk, bucket), its list's position
@@ -233,7 +239,7 @@ __device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, 
         }
         ++lists.n;
     };
-    mark(chunk);
+    if (!T.direct) mark(chunk);
     T.pk_bucket[i] = p.at;
     T.pk_want[i] = p.rank - before;
     T.pk_claim[i] = p.claim;
@@ -242,7 +248,7 @@ __device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, 
     T.pk_r[i] = p.r;
     T.pk_chunk[i] = chunk;
     T.pk_len[i] = (int32_t)len;
-    if (chunk == p.idx / c.A) {
+    if (!T.direct && chunk == p.idx / c.A) {
         const uint32_t next = p.rank + 1 == total ? 0u : p.rank + 1;
         if (next < before || next >= before + len) mark(chunk_of(T, c, p.at, next, total, before, len));
     }
@@ -990,6 +996,55 @@ __device__ __forceinline__ int32_t rank_in_list(const int32_t* __restrict__ l, u
     return lo;
 }
 
+// 16 lanes: the agent with `want` agents of bucket b before it in the chunk,
+// from the chunk's keys, 1,024 agents at a time, 64 consecutive ones per lane.
+constexpr int kDirectChunk = 4096;
+__device__ __forceinline__ int32_t rank_in_keys(const CountTable& T, const CountRep& c, int chunk, uint32_t b,
+                                                uint32_t want, int sub) {
+    constexpr int kLaneAgents = 64;
+    for (int p0 = chunk * c.A + sub * kLaneAgents;; p0 += kPickLanes * kLaneAgents) {
+        uint64_t m = 0;
+        // (a weekday bucket's hour is its plane; weekend hours come in any order)
+        const int e0 = T.direct == 2 && b >= T.hour1 ? 1 : 0, e1 = T.direct == 2 ? e0 + 1 : T.direct;
+        for (int e = e0; e < e1; ++e) {
+            const uint4* keys = reinterpret_cast<const uint4*>(T.keys + e * T.slots + c.abase + p0);
+            uint4 v[kLaneAgents / 8];
+#pragma unroll
+            for (int i = 0; i < kLaneAgents / 8; ++i)
+                v[i] = p0 + 8 * i < T.n_agents ? keys[i] : make_uint4(~0u, ~0u, ~0u, ~0u);
+#pragma unroll
+            for (int i = 0; i < kLaneAgents / 8; ++i) {
+                const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+                uint32_t bits = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    bits |= ((w[k] & 0xFFFFu) == b ? 1u : 0u) << (2 * k);
+                    bits |= ((w[k] >> 16) == b ? 2u : 0u) << (2 * k);
+                }
+                m |= (uint64_t)bits << (8 * i);
+            }
+        }
+        const int left = T.n_agents - p0;  // keys past the last agent are left from other days
+        if (left < kLaneAgents) m &= left <= 0 ? 0ull : (1ull << left) - 1ull;
+        const uint32_t n = (uint32_t)__popcll(m);
+        uint32_t inc = n;  // a row of 16 lanes
+        inc = dpp_add<0x111>(inc);
+        inc = dpp_add<0x112>(inc);
+        inc = dpp_add<0x114>(inc);
+        inc = dpp_add<0x118>(inc);
+        int32_t found = -1;
+        if (inc > want && inc - n <= want) {
+            for (uint32_t t = want - (inc - n); t; --t) m &= m - 1;
+            found = p0 + __ffsll((unsigned long long)m) - 1;
+        }
+#pragma unroll
+        for (int o = kPickLanes / 2; o > 0; o >>= 1) found = max(found, __shfl_xor(found, o, kPickLanes));
+        const uint32_t all = __shfl(inc, kPickLanes - 1, kPickLanes);
+        if (found >= 0 || p0 - sub * kLaneAgents + kPickLanes * kLaneAgents >= (chunk + 1) * c.A) return found;
+        want -= all;
+    }
+}
+
 // The picked person of every queued pick and its claims (process_contacts).
 constexpr uint32_t kPicksPerClaim = 64;
 
@@ -1001,9 +1056,14 @@ __device__ __forceinline__ int32_t picked_person(const CountTable& T, uint32_t q
     uint32_t want = T.pk_want[q], len = (uint32_t)T.pk_len[q];
     int chunk = T.pk_chunk[q];
     for (int round = 0;; ++round) {
-        // (split layouts: the entry is the list's end now)
-        const int32_t* l = T.list + (T.cnt[c.mbase + (int64_t)chunk * c.K + b] - (c.G > 1 ? len : 0u));
-        const int32_t v = rank_in_list(l, len, want, chunk * c.A, c.A, sub);
+        int32_t v;
+        if (T.direct) {
+            v = rank_in_keys(T, c, chunk, b, want, sub);
+        } else {
+            // (split layouts: the entry is the list's end now)
+            const int32_t* l = T.list + (T.cnt[c.mbase + (int64_t)chunk * c.K + b] - (c.G > 1 ? len : 0u));
+            v = rank_in_list(l, len, want, chunk * c.A, c.A, sub);
+        }
         if (v != idx || round) return v;
         const uint32_t total = T.total[c.tbase + b];  // the next person instead (select_person)
         uint32_t j = count_column(T, c, b)[chunk] + want + 1, before;
@@ -1267,7 +1327,7 @@ inline void enqueue_picks(const CountPlan& p, const CountTable& t, const ClaimAr
                    sizeof(uint32_t) * (size_t)(p.reps[0].W * p.reps[0].ranges / 32 + 2), st, sts, models, t);
         const auto k = weekend ? k_collect_group<3> : (p.lists ? k_collect_group<2> : k_collect_group<0>);
         launch_lds(tm, KC_COLLECT, k, dim3(p.n_chunks), dim3(p.threads), p.lds, st, sts, models, t);
-    } else {
+    } else if (!t.direct) {
         launch_lds(tm, KC_COLLECT, weekend ? k_collect<true> : k_collect<false>, dim3(p.n_chunks), dim3(p.threads),
                    p.lds, st, (const int32_t*)&g->done, sts, models, t);
     }

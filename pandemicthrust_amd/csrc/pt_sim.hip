@@ -1293,6 +1293,17 @@ int setup_counts(pt_sim* s) {
         t.sv_pos = s->stage_ids + 2 * s->N;
         t.sv_f = s->sel_keys + 2 * s->N;
         t.wp_lone = s->wp_lone;
+        // Small chunks: k_resolve reads about half a chunk's keys per pick (4 to
+        // 12 KB of L2), which costs less than the launch that lists the marked
+        // buckets (100k agents: 6.5 + 6.5 us -> 7.6, 235k: 6.1 + 8.0 -> 9.6; at
+        // 2.35M, chunks of 9,216, listing costs 10 of 23 us for 10,000 picks).
+        t.direct = 0;
+        if (!p.split && p.reps[0].A <= kDirectChunk) {
+            t.direct = w ? 3 : 2;
+            t.n_agents = (int32_t)s->N;
+            t.hour1 = (uint32_t)m.wd_E;
+            t.mark_words = 0;
+        }
         HIP_TRY(set_count_lds(p));
         if (p.lds > 64 * 1024 && !p.split)
             HIP_TRY(hipFuncSetAttribute(w ? reinterpret_cast<const void*>(&k_count_sweep<true>)

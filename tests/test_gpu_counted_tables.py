@@ -33,6 +33,9 @@ CASES = [
     (0.3, 200.0, 7, 5000),         # 320,000: 8 groups
     (0.05, 200.5, 7, 5000),        # 320,800: weekday sorted
     (0.05, 2.98, 9, 2000),         # weekend 38,740 buckets: the largest counted beside the sweep
+    (0.28, 0.28, 9, 3000),         # 658,000 agents: chunks of 3,072, picks found in the keys
+    (0.4, 0.1, 9, 3000),           # 940,000, odd chunk and agent counts
+    (0.45, 0.45, 9, 3000),         # 1.06M: chunks above 4,096, picks from lists
     (1.0, 1.0, 7, 20000),          # 2.35M agents: launches in pairs
     (2.2, 1.0, 7, 20000),          # 5.2M: single launches, the compaction plans the day
     (3.7, 1.0, 7, 20000),          # 8.7M: several sweep blocks per thread of the plan
