@@ -10,9 +10,10 @@ before each step; setup itself is input preparation and not timed).
 value = person-days per second over the timed steps
       = steps * N * days_simulated / wall seconds of those steps.
 
-roofline: the dominant kernel class by HIP-event time (the radix downsweep
-of the errand tables).  Its algorithmic bytes follow the loop model's
-table term: an ideal single-pass table build reads the (key, id) pairs once
+roofline: the dominant kernel class by HIP-event time.  On counted days that
+is the weekend's errand keys (bound by their random draws on the vector units;
+the byte model counts what they write).  A radix class's algorithmic bytes
+follow the loop model's table term: an ideal single-pass table build reads the (key, id) pairs once
 (8 bytes each) and writes the sorted ids once (4 bytes), 12 bytes per pair
 of each day's table: E*N pairs (E = 2 on weekdays and 3 on weekends) on the
 days that build the full table, the selected pairs on the days that build
@@ -82,7 +83,7 @@ CONSTANTS_HEADER = ("constants,max_days,reproduction_number_pandemic,reproductio
                     "location_scaling_factor,percent_symptomatic,asymp_factor")
 
 
-def algorithmic_bytes(N, W, lay, inf, counts, full, pairs):
+def algorithmic_bytes(N, W, lay, inf, counts, full, pairs, counted=None):
     """Algorithmic bytes per kernel class for one loop, and the loop total of
     the per-day model B_wd = 43N + 89I + 3X + 8W + 4, B_we = 62N + 62I + 3X +
     40W + 4 (terminal I = 0 day: 2N).
@@ -96,7 +97,11 @@ def algorithmic_bytes(N, W, lay, inf, counts, full, pairs):
     id) pairs (8 B); the first downsweep reads n keys and writes key and id
     of the kept pairs (4n + 8k; selected pairs: 8m read, 8m written), middle
     ones read and write key and id (16k), the last reads pairs and writes the
-    id plus the key's low bits in kw bytes (8k + 4k + kw k)."""
+    id plus the key's low bits in kw bytes (8k + 4k + kw k).
+
+    counted: errand tables are counted, not sorted: "groups" writes the keys
+    (weekday 2 bytes, weekend pairs of 4) and reads them for the counts and
+    for the lists, "blocks" counts them as they are written (2 bytes each)."""
     per = {}
 
     def add(k, b):
@@ -138,7 +143,14 @@ def algorithmic_bytes(N, W, lay, inf, counts, full, pairs):
         else:
             add("contacts_weekday", 83 * I)
             loop += 43 * N + 89 * I + 3 * X + 8 * W + 4
-        if d < len(full) and full[d]:
+        if counted:
+            n = 3 * N if weekend else 2 * N
+            b = (4 if counted == "groups" and weekend else 2) * n
+            add("gen_weekend" if weekend else "gen_weekday", b + (0 if weekend else N))
+            if counted == "groups":
+                add("table_count", b)
+            add("collect", b)
+        elif d < len(full) and full[d]:
             n = 3 * N if weekend else 2 * N
             add("table_model", 12 * n)
             # pairs kept: the weekday table leaves out the never-queried
@@ -560,7 +572,11 @@ def main():
     days_per_step = days_total / max(args.steps, 1)
     value = N * days_total / wall
     full, pairs = sim.table_log()
-    per_loop, loop_bytes = algorithmic_bytes(N, W, lay, inf, counts, full, pairs)
+    seen = profile or kt
+    counted = None
+    if seen.get("resolve", (0, 0))[1]:
+        counted = "groups" if seen.get("table_count", (0, 0))[1] else "blocks"
+    per_loop, loop_bytes = algorithmic_bytes(N, W, lay, inf, counts, full, pairs, counted)
 
     # Per-kernel table from the profiled warmup loop (one loop's worth).
     table = {}

@@ -1448,7 +1448,7 @@ int enqueue_day(pt_sim* s, int d) {
     }
     if (merged) {
         launch_lds(tm, weekend ? KC_GEN_WEEKEND : KC_GEN_WEEKDAY, weekend ? k_count_sweep<true> : k_count_sweep<false>,
-                   dim3(cp.n_chunks + s->nblk_sweep), dim3(cp.threads), cp.lds, stc, M, st, s->st_p, s->st_s,
+                   dim3(cp.n_chunks + s->nblk_sweep), dim3(std::max(cp.threads, kSweepThreads)), cp.lds, stc, M, st, s->st_p, s->st_s,
                    (const uint8_t*)s->dy_p, (const uint8_t*)s->dy_s, (const uint8_t*)s->age, s->blk_counts,
                    s->blk_ninf, s->staging, ct, cp.n_chunks);
     } else if (counted) {

@@ -10,7 +10,8 @@ pt_sim_kernel_name by walking each run's dispatch order: kernels before the
 first sweep are setup; within a day, the scans between the selection kernel
 and the run compaction belong to the selection, and the radix-sort kernels
 after the compaction build the day's table (full or subset: the same
-launches).  The counters are calibrated with the
+launches).  Counted days have classes of their own; a launch that two classes
+share counts for the first.  The counters are calibrated with the
 snapshot-restore copy kernel (k_copy16), which reads and writes COPY_BYTES
 bytes per launch.
 """
@@ -20,6 +21,8 @@ import os
 import sys
 
 SORT = ("k_upsweep", "k_downsweep", "k_scan_reduce", "k_scan_parts", "k_scan_down", "k_offsets")
+COUNTED = {"k_count_group": "table_count", "k_count_scan": "count_scan", "k_collect": "collect",
+           "k_collect_few": "collect", "k_collect_group": "collect", "k_resolve": "resolve"}
 
 
 def short(name):
@@ -33,7 +36,7 @@ def label(seq):
     section = "setup"
     for n in seq:
         base = n.split("<")[0]
-        if base == "k_sweep":
+        if base in ("k_sweep", "k_count_sweep"):
             section = "day"
         if section == "setup":
             cls = "restore" if base in ("k_copy16", "k_fill_u64") else "setup"
@@ -43,8 +46,14 @@ def label(seq):
             cls = "sweep"
         elif base == "k_plan":
             cls = "plan"
-        elif base == "k_compact":
+        elif base in ("k_compact", "k_compact_test", "k_scan_test"):
             cls = "compact"
+        elif base in ("k_count", "k_count_sweep", "k_keys_lists"):
+            cls = "gen_weekend" if "<true" in n else "gen_weekday"
+        elif base == "k_keys_weekday":
+            cls = "gen_weekday"
+        elif base in COUNTED:
+            cls = COUNTED[base]
         elif base in ("k_mark_weekday", "k_mark_weekend", "k_decide"):
             cls = "mark"
         elif base in ("k_gen_weekday", "k_gen_weekend"):
@@ -63,8 +72,8 @@ def label(seq):
                 cls = {"k_upsweep": "sort_upsweep", "k_downsweep": "sort_downsweep", "k_offsets": "offsets"}.get(
                     base, "sort_scan")
         elif base == "k_contacts":
-            cls = "contacts_weekend" if "<true>" in n else "contacts_weekday"
-        elif base == "k_apply":
+            cls = "contacts_weekend" if "<true" in n else "contacts_weekday"
+        elif base in ("k_apply", "k_apply_end"):
             cls = "apply"
         elif base == "k_end_day":
             cls = "end_day"
@@ -125,11 +134,11 @@ def main(d, copy_bytes):
     print("Loop kernels (classes other than setup and restore): %.1f ms." % (loop_us / 1e3))
     print("Calibration: k_copy16 reads and writes %d bytes per launch; FETCH_SIZE x %.4f, WRITE_SIZE x %.4f "
           "(bytes = KiB x 1024 x factor)." % (copy_bytes, kf, kw))
-    s = agg.get("sort_downsweep")
-    if s and s["nf"] and s["nw"]:
-        per = s["rd"] / s["nf"] + s["wr"] / s["nw"]
-        print()
-        print("traffic_per_launch sort_downsweep: %.0f bytes over %d launches (avg %.2f us)" % (per, s["n"], s["us"] / s["n"]))
+    print()
+    for c, a in agg.items():
+        if a["nf"] and a["nw"] and c not in ("setup", "restore", "other"):
+            print("traffic_per_launch %s: %.0f bytes over %d launches (avg %.2f us)"
+                  % (c, a["rd"] / a["nf"] + a["wr"] / a["nw"], a["n"], a["us"] / a["n"]))
 
 
 def kernel_table(stats_csv, runs=1):
