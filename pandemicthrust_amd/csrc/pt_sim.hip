@@ -1736,7 +1736,7 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
     const int64_t stage_n = std::max<int64_t>((N / kSelAgentsWd + 1) * kSelStageWd, (N / kSelAgentsWe + 1) * kSelStageWe);
     if (dev_alloc(&s->st_p, Npad) || dev_alloc(&s->st_s, Npad) || dev_alloc(&s->dy_p, Npad) ||
         dev_alloc(&s->dy_s, Npad) || dev_alloc(&s->gn_p, Npad) || dev_alloc(&s->gn_s, Npad) ||
-        dev_alloc(&s->age, N) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
+        dev_alloc(&s->age, Npad) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
         dev_alloc(&s->hh_off, (int64_t)H + 1) ||
         dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->who, N) || dev_alloc(&s->wp_lone, 1) ||
         dev_alloc(&s->infected, N) ||
