@@ -951,8 +951,7 @@ int setup_batch_counts(pt_batch* b) {
         }
         p.build(N, w ? 3 : 2, b->cus);
     }
-    if (b->count_plan[0].upload(b->stream) || b->count_plan[1].upload(b->stream) ||
-        b->count_scratch.alloc(b->count_plan[0], b->count_plan[1], 0)) {
+    if (b->count_scratch.alloc(b->count_plan, 0, b->stream)) {
         // no memory for the matrices: sorted tables
         (void)hipGetLastError();
         for (CountPlan& p : b->count_plan) p.release();

@@ -1255,49 +1255,74 @@ struct CountPlan {
         n_chunks = c.C * c.G;
         plan_scans();
     }
-    int upload(hipStream_t st) {
-        if (!on) return 0;
-        chunks.resize(n_chunks);  // (a split layout numbers its blocks itself)
-        if (dev_alloc(&d_reps, (int64_t)reps.size()) || dev_alloc(&d_chunks, n_chunks) || dev_alloc(&d_scans, n_scans))
-            return PT_ENOMEM;
-        HIP_TRY(hipMemcpyAsync(d_reps, reps.data(), sizeof(CountRep) * reps.size(), hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_chunks, chunks.data(), sizeof(CountBlock) * n_chunks, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipMemcpyAsync(d_scans, scans.data(), sizeof(CountBlock) * n_scans, hipMemcpyHostToDevice, st));
-        return 0;
-    }
-    void release() {
-        dev_free(d_reps);
-        dev_free(d_chunks);
-        dev_free(d_scans);
-        *this = CountPlan();
-    }
+    // (the device copies belong to CountScratch's block)
+    void release() { *this = CountPlan(); }
 };
 
-// Buffers shared by the two layouts (a: weekday, b: weekend).
+// Buffers shared by the two layouts (weekday, weekend) and the device copies of
+// their plans, in one allocation: the plans, then cleared counters, all sent in
+// one copy, then the rest.
 struct CountScratch {
+    unsigned char* block = nullptr;
+    std::vector<unsigned char> image;  // what is sent, kept until it has been
     uint32_t *cnt = nullptr, *pre = nullptr, *total = nullptr, *marks = nullptr, *n = nullptr;
     int32_t* chunk_day = nullptr;
     uint16_t* tile_off = nullptr;
     int32_t* lone_day = nullptr;
-    int alloc(const CountPlan& a, const CountPlan& b, int64_t N) {
+    int alloc(CountPlan (&plan)[2], int64_t N, hipStream_t st) {
+        const CountPlan &a = plan[0], &b = plan[1];
         const int64_t e = std::max(a.entries, b.entries);
         if (e == 0) return 0;
-        return dev_alloc(&cnt, e) || dev_alloc(&pre, e) || dev_alloc(&total, std::max(a.buckets, b.buckets)) || dev_alloc(&marks, std::max(a.mark_words, b.mark_words)) ||
-                       dev_alloc(&chunk_day, std::max(a.n_chunks, b.n_chunks)) || dev_alloc(&n, 4) || dev_alloc(&lone_day, (int64_t)std::max(a.reps.size(), b.reps.size())) ||
-                       ((a.lists || b.lists) &&
-                        dev_alloc(&tile_off, (N / kTileAgents + 1) * std::max(a.lists ? a.reps[0].toff : 0, b.lists ? b.reps[0].toff : 0)))
-                   ? PT_ENOMEM
-                   : 0;
+        size_t bytes = 0;
+        const auto take = [&](size_t count, size_t size) {
+            const size_t at = bytes;
+            bytes += (std::max<size_t>(count, 1) * size + 255) / 256 * 256;
+            return at;
+        };
+        size_t at_plan[2][3] = {};
+        for (int w = 0; w < 2; ++w) {
+            CountPlan& p = plan[w];
+            if (!p.on) continue;
+            p.chunks.resize(p.n_chunks);  // (a split layout numbers its blocks itself)
+            at_plan[w][0] = take(p.reps.size(), sizeof(CountRep));
+            at_plan[w][1] = take(p.chunks.size(), sizeof(CountBlock));
+            at_plan[w][2] = take(p.scans.size(), sizeof(CountBlock));
+        }
+        const size_t at_n = take(4, sizeof(uint32_t)), sent = bytes;
+        const size_t at_lone = take(std::max(a.reps.size(), b.reps.size()), sizeof(int32_t));
+        const size_t at_day = take(std::max(a.n_chunks, b.n_chunks), sizeof(int32_t));
+        const size_t at_total = take(std::max(a.buckets, b.buckets), sizeof(uint32_t));
+        const size_t at_marks = take(std::max(a.mark_words, b.mark_words), sizeof(uint32_t));
+        const size_t at_tile = take(a.lists || b.lists ? (N / kTileAgents + 1) *
+                                        std::max(a.lists ? a.reps[0].toff : 0, b.lists ? b.reps[0].toff : 0) : 0,
+                                    sizeof(uint16_t));
+        const size_t at_cnt = take(e, sizeof(uint32_t)), at_pre = take(e, sizeof(uint32_t));
+        if (dev_alloc(&block, (int64_t)bytes)) return PT_ENOMEM;
+        image.assign(sent, 0);
+        for (int w = 0; w < 2; ++w) {
+            CountPlan& p = plan[w];
+            if (!p.on) continue;
+            memcpy(image.data() + at_plan[w][0], p.reps.data(), sizeof(CountRep) * p.reps.size());
+            memcpy(image.data() + at_plan[w][1], p.chunks.data(), sizeof(CountBlock) * p.chunks.size());
+            memcpy(image.data() + at_plan[w][2], p.scans.data(), sizeof(CountBlock) * p.scans.size());
+            p.d_reps = (CountRep*)(block + at_plan[w][0]);
+            p.d_chunks = (CountBlock*)(block + at_plan[w][1]);
+            p.d_scans = (CountBlock*)(block + at_plan[w][2]);
+        }
+        HIP_TRY(hipMemcpyAsync(block, image.data(), sent, hipMemcpyHostToDevice, st));
+        n = (uint32_t*)(block + at_n);
+        lone_day = (int32_t*)(block + at_lone);
+        chunk_day = (int32_t*)(block + at_day);
+        total = (uint32_t*)(block + at_total);
+        marks = (uint32_t*)(block + at_marks);
+        tile_off = (uint16_t*)(block + at_tile);
+        cnt = (uint32_t*)(block + at_cnt);
+        pre = (uint32_t*)(block + at_pre);
+        return 0;
     }
     void release() {
-        dev_free(cnt);
-        dev_free(pre);
-        dev_free(total);
-        dev_free(marks);
-        dev_free(chunk_day);
-        dev_free(n);
-        dev_free(lone_day);
-        dev_free(tile_off);
+        dev_free(block);
+        *this = CountScratch();
     }
     void fill(CountTable& t, const CountPlan& p) const {
         t.reps = p.d_reps;

@@ -1264,8 +1264,7 @@ int setup_counts(pt_sim* s) {
         p.build({s->N}, w ? 3 : 2, s->cus);
         if (K[w] > kCountMaxK) p.build_split(s->N, w ? 3 : 2, w ? m.we_E : m.wd_E, w ? kWeHours : kWdHours, s->cus);
     }
-    if (s->count_plan[0].upload(s->stream) || s->count_plan[1].upload(s->stream) ||
-        s->count_scratch.alloc(s->count_plan[0], s->count_plan[1], s->N)) {
+    if (s->count_scratch.alloc(s->count_plan, s->N, s->stream)) {
         // no memory for the matrices: sorted tables
         (void)hipGetLastError();
         for (CountPlan& p : s->count_plan) p.release();
@@ -1310,7 +1309,6 @@ int setup_counts(pt_sim* s) {
                                           : reinterpret_cast<const void*>(&k_count_sweep<false>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 152 * 1024));
     }
-    if (s->count_scratch.n) HIP_TRY(hipMemsetAsync(s->count_scratch.n, 0, 4 * sizeof(uint32_t), s->stream));
     return PT_OK;
 }
 
