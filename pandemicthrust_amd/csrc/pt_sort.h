@@ -137,6 +137,13 @@ hipError_t build_table(TableScratch& s, uint32_t* keys, const int32_t* vals, int
                        const int32_t* done, hipStream_t stream, LaunchTimer* tm, uint32_t drop_key = kNoDrop,
                        const AltInput* alt = nullptr);
 
+// A table of at most kSmallPairs host-counted pairs (ids = positions) and
+// kSmallBuckets buckets in one launch without scratch.
+constexpr int64_t kSmallPairs = 131072;
+constexpr int32_t kSmallBuckets = 8000;
+hipError_t build_small_table(const uint32_t* keys, int64_t n, int32_t K, int32_t* people_out, int32_t* offsets_out,
+                             hipStream_t stream);
+
 // Segmented tables: the tables of R independent simulations built by one
 // sort whose passes cover only the bits of the largest local key.  Segment r
 // holds its pairs at [seg_start[r], seg_start[r] + seg_count[r]) with keys

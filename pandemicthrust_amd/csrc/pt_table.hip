@@ -87,6 +87,12 @@ extern "C" int pt_location_table(const uint32_t* keys, int64_t n, int32_t n_buck
     DeviceScope ds(device);
     HIP_TRY(ds.err);
     hipStream_t st = (hipStream_t)stream;
+    if (n > 0 && n <= kSmallPairs && n_buckets <= kSmallBuckets) {
+        hipError_t e = build_small_table(keys, n, n_buckets, people, offsets, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) return fail(PT_EDEVICE, "location table: %s", hipGetErrorString(e));
+        return PT_OK;
+    }
     const size_t need = table_scratch_bytes(n, n_buckets);
     Block block = take_block(device);
     if (block.bytes < need || block.bytes / 4 > need) {
