@@ -47,6 +47,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "pt_day.h"
@@ -401,8 +402,8 @@ struct PickPush {
 namespace {
 
 // Keys and counts of a chunk.  VALU bound (per agent 125 instructions on weekdays,
-// 381 on weekends, of which the draws 71 and 284: 32M agents in 48 replicates 118
-// and 386 us; agent by agent with a check per key 129 weekdays); the LDS adds,
+// 381 on weekends, of which the draws 71 and 284: 32M agents in 48 replicates 102
+// and 291 us; agent by agent with a check per key 10% more); the LDS adds,
 // the 4-byte coalesced key stores and the row flush hide behind them.
 template <bool WEEKEND>
 __device__ __forceinline__ void count_block(int block, DayState* __restrict__ sts, const Model* __restrict__ models,
@@ -1196,6 +1197,12 @@ struct CountPlan {
             for (int k = 0; k < c.C; ++k) chunks.push_back({(int32_t)r, k});
         }
         n_chunks = (int)chunks.size();
+        // The largest first: a large block started last would run alone (48
+        // replicates of 50k to 2M agents: 118 -> 102 us per weekday, 386 -> 291
+        // per weekend day).
+        std::stable_sort(chunks.begin(), chunks.end(), [this](const CountBlock& x, const CountBlock& y) {
+            return reps[x.r].A > reps[y.r].A;
+        });
         // More chunks than CUs: the smallest blocks that still fill a CU's 2,048
         // threads beside the counters, so that one's start (counters cleared,
         // marks read) and end overlap the others' work.  48 replicates of 0.7M
