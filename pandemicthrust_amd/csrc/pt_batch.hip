@@ -222,8 +222,14 @@ __global__ __launch_bounds__(kRepThreads) void kb_plan(const DayState* __restric
 // infectors, as the single simulation's k_compact_test with PLAN (replicates
 // of up to kFusedPlan sweep tiles).  No infected list is kept.
 constexpr int kFusedPlan = 1024;
+// Blocks of a tile: small ones, since most tiles hold few infected and a
+// block's chain of loads sets its time (136M agents in 256 replicates, weekday:
+// 345 us with 1,024 threads, 249 with 256);
+// what is kept leaves through LDS, one list atomic per block or kTestQueue.
+constexpr int kTestThreads = 256;
+constexpr uint32_t kTestQueue = 1024;
 template <bool WEEKEND>
-__global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restrict__ g, DayState* __restrict__ sts,
+__global__ __launch_bounds__(kTestThreads) void kb_compact_test(const DayState* __restrict__ g, DayState* __restrict__ sts,
                                                         const RepInfo* __restrict__ reps,
                                                         const Model* __restrict__ models,
                                                         const int32_t* __restrict__ tile_rep,
@@ -245,24 +251,39 @@ __global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restri
     const int day = st->day;
     const int64_t N = ri.N;
     const uint64_t cbase = st->rand_offset + (WEEKEND ? (uint64_t)(2 * N) : (uint64_t)(N / 2));
-    __shared__ uint32_t s_w[16], s_off;
-    const uint32_t v = tid < ri.ntiles ? blk_ninf[ri.tile0 + tid] : 0u;
-    const uint32_t inc = wave_incl_scan(v, lane);
+    constexpr int NW = kTestThreads / 64, PER = kFusedPlan / kTestThreads;
+    __shared__ uint32_t s_w[NW], s_off, s_n, s_base;
+    if (tid == 0) s_n = 0;
+    const int per = (ri.ntiles + kTestThreads - 1) / kTestThreads;  // consecutive tiles of this thread
+    uint32_t v[PER], sum = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int t = tid * per + k;
+        v[k] = k < per && t < ri.ntiles ? blk_ninf[ri.tile0 + t] : 0u;
+        sum += v[k];
+    }
+    const uint32_t inc = full_wave_scan(sum);
     if (lane == 63) s_w[wave] = inc;
     __syncthreads();
-    uint32_t before = 0, total = 0;
+    uint32_t before = inc - sum, total = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
+    for (int w = 0; w < NW; ++w) {
         const uint32_t x = s_w[w];
         if (w < wave) before += x;
         total += x;
     }
-    if (tid == (int)b - ri.tile0) s_off = before + inc - v;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        if (k < per && tid * per + k == (int)b - ri.tile0) s_off = before;
+        before += v[k];
+    }
     if (b == ri.tile0) {
-        uint32_t c = 0;
-        for (int t = lane; t < ri.ntiles; t += 64) c += blk_counts[(int64_t)(ri.tile0 + t) * 16 + wave];
-        c = wave_sum(c);
-        if (lane == 0) out_counts[((int64_t)r * D + day) * 16 + wave] = (int32_t)c;
+        for (int q = wave; q < 16; q += NW) {
+            uint32_t c = 0;
+            for (int t = lane; t < ri.ntiles; t += 64) c += blk_counts[(int64_t)(ri.tile0 + t) * 16 + q];
+            c = full_wave_scan(c);
+            if (lane == 63) out_counts[((int64_t)r * D + day) * 16 + q] = (int32_t)c;
+        }
         if (tid == 0) {
             st->n_infected = (int32_t)total;
             st->days_run = day + 1;
@@ -277,7 +298,9 @@ __global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restri
     const uint32_t off = s_off, n = blk_ninf[b];
     const int32_t* src = staging + b * kSweepTile;
     AgentArrays A = view(B, ri, 0u);
-    for (uint32_t i0 = 0; i0 < n; i0 += blockDim.x) {
+    __shared__ int32_t s_idx[kTestQueue], s_pos[kTestQueue];
+    __shared__ uint32_t s_f[kTestQueue];
+    for (uint32_t i0 = 0; i0 < n; i0 += kTestThreads) {
         const uint32_t i = i0 + tid;
         int32_t idx = 0;
         Infectivity f{};
@@ -292,7 +315,31 @@ __global__ __launch_bounds__(1024) void kb_compact_test(const DayState* __restri
                        may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], r, day, WEEKEND));
             }
         }
-        list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), r, true);
+        const uint64_t m = __ballot(keep);
+        uint32_t at = 0;
+        if (lane == 0 && m) at = atomicAdd(&s_n, (uint32_t)__popcll(m));
+        at = __shfl(at, 0, 64) + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+        if (keep) {
+            s_idx[at] = idx;
+            s_pos[at] = (int32_t)(off + i);
+            s_f[at] = pack_infectivity(f);
+        }
+        __syncthreads();
+        const uint32_t queued = s_n;
+        __syncthreads();  // every thread has the same answer
+        if (queued > kTestQueue - kTestThreads || i0 + kTestThreads >= n) {
+            if (tid == 0 && queued) s_base = atomicAdd(&T.n[1], queued);
+            if (tid == 0) s_n = 0;
+            __syncthreads();
+            for (uint32_t k = tid; k < queued; k += kTestThreads) {
+                const uint32_t to = s_base + k;
+                T.sv_idx[to] = s_idx[k];
+                T.sv_pos[to] = s_pos[k];
+                T.sv_f[to] = s_f[k];
+                T.sv_r[to] = r;
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -845,7 +892,7 @@ int enqueue_batch_day(pt_batch* b, int d) {
         const BatchArrays B = batch_arrays(b);
         enqueue_counts(cp, ct, &g->done, b->d_states, b->d_models, b->age, weekend, s, nullptr);
         const auto test = weekend ? kb_compact_test<true> : kb_compact_test<false>;
-        test<<<b->ntiles, 1024, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep, b->staging, b->blk_ninf,
+        test<<<b->ntiles, kTestThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep, b->staging, b->blk_ninf,
                                         b->blk_counts, b->d_counts, b->d_inf, b->D, B, ct);
         const int grid = grid_for(b->n_agents, kContactThreads, b->grid_contacts);
         const auto contacts = weekend ? kb_contacts_counted<true> : kb_contacts_counted<false>;
