@@ -255,29 +255,6 @@ __device__ __forceinline__ void locate_pick(const CountTable& T, const Pick& p, 
     }
 }
 
-// Lists the infectors of a block's turn that are kept (all threads call).
-__device__ __forceinline__ void list_infectors(const CountTable& T, bool keep, int32_t idx, int32_t pos, uint32_t f,
-                                               int32_t r, bool with_r) {
-    __shared__ uint32_t s_n, s_base;
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-    const uint64_t m = __ballot(keep);
-    uint32_t at = 0;
-    if (lane == 0 && m) at = atomicAdd(&s_n, (uint32_t)__popcll(m));
-    at = __shfl(at, 0, 64) + (uint32_t)__popcll(m & ((1ull << lane) - 1));
-    __syncthreads();
-    if (threadIdx.x == 0 && s_n) s_base = atomicAdd(&T.n[1], s_n);
-    __syncthreads();
-    if (keep) {
-        const uint32_t i = s_base + at;
-        T.sv_idx[i] = idx;
-        T.sv_pos[i] = pos;
-        T.sv_f[i] = f;
-        if (with_r) T.sv_r[i] = r;
-    }
-}
-
 // Posts a successful draw's claims on the person at `slot` (process_contacts);
 // newp / news: first to claim that strain today.
 __device__ __forceinline__ void post_claims(const ClaimArrays& C, int64_t slot, uint32_t claim, uint32_t payload,

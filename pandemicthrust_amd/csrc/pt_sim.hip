@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DayState* __restrict__ st
 }
 
 // Counted days: the compaction also tests the infectors' success draws and
-// lists the ones left (list_infectors), and, for up to kFusedPlan sweep
+// lists the ones left, and, for up to kFusedPlan sweep
 // blocks (67M agents), is the day plan too (PLAN): every block sums the counts
 // of the blocks before its own instead of waiting for a launch of one block
 // (50M agents: 18 us per day).  A block takes every gridDim-th sweep block, so
@@ -402,12 +402,32 @@ __device__ __forceinline__ void compact_test_block(int block, int blocks, const 
         }
         __syncthreads();
     }
+    // The waves share out the infected of the block's sweep blocks 64 at a time,
+    // without barriers: most sweep blocks hold a few hundred, and a turn of
+    // the whole block per sweep block cost some 6 us however few.  50M agents,
+    // weekdays: 40-85 -> 26-38 us while under a million are infected, 330 -> 370
+    // at the peak (weekend days 250 -> 210); 9.8 -> 8.0 ms in 100 days.  A wave
+    // queues what it keeps.
+    // (full queues append by themselves: large ones, since appends from all
+    // over the chip queue up at one address)
+    constexpr uint32_t Q = PLAN == 1 ? 192 : 384;
+    __shared__ int32_t s_idx[16][Q], s_pos[16][Q];
+    __shared__ uint32_t s_f[16][Q], s_kept[16], s_base;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t kept = 0, turn = 0;  // of the wave; slices so far, of all
+    auto give = [&](uint32_t base) {
+        for (uint32_t k = lane; k < kept; k += 64) {
+            T.sv_idx[base + k] = s_idx[wave][k];
+            T.sv_pos[base + k] = s_pos[wave][k];
+            T.sv_f[base + k] = s_f[wave][k];
+        }
+    };
     for (int own = first; own < nblk; own += step) {
         const uint32_t off = PLAN ? s_off[own / step] : a.blk_off[own];
-        const uint32_t n = blk_ninf[own];
+        const uint32_t n = blk_ninf[own], slices = (n + 63) / 64;
         const int32_t* src = a.staging + (int64_t)own * kSweepTile;
-        for (uint32_t i0 = part * blockDim.x; i0 < n; i0 += a.parts * blockDim.x) {
-            const uint32_t i = i0 + tid;
+        for (uint32_t sl = part * 16 + (((uint32_t)wave - turn) & 15u); sl < slices; sl += 16 * a.parts) {
+            const uint32_t i = sl * 64 + lane;
             int32_t idx = 0;
             Infectivity f{};
             bool keep = false;
@@ -422,9 +442,37 @@ __device__ __forceinline__ void compact_test_block(int block, int blocks, const 
                            may_infect<C>(M, f, draws, least_contacts(T, A.who[idx], 0, day, WEEKEND, counted));
                 }
             }
-            list_infectors(T, keep, idx, (int32_t)(off + i), pack_infectivity(f), 0, false);
+            const uint64_t m = __ballot(keep);
+            if (keep) {
+                const uint32_t at = kept + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+                s_idx[wave][at] = idx;
+                s_pos[wave][at] = (int32_t)(off + i);
+                s_f[wave][at] = pack_infectivity(f);
+            }
+            kept += (uint32_t)__popcll(m);
+            if (kept > Q - 64) {
+                uint32_t base = 0;
+                if (lane == 0) base = atomicAdd(&T.n[1], kept);
+                give(__shfl(base, 0, 64));
+                kept = 0;
+            }
         }
+        turn += slices;
     }
+    // The rest, one list append for the block.
+    if (lane == 0) s_kept[wave] = kept;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        const uint32_t x = s_kept[w];
+        if (w < wave) before += x;
+        all += x;
+    }
+    if (all == 0) return;
+    if (tid == 0) s_base = atomicAdd(&T.n[1], all);
+    __syncthreads();
+    give(s_base + before);
 }
 template <bool WEEKEND, int PLAN>
 __global__ __launch_bounds__(1024) void k_compact_test(const Model* __restrict__ Mp, DayState* __restrict__ st,
