@@ -36,10 +36,10 @@
 // by hour or group first, then k_count_group counts (chunk, group) from them,
 // and k_collect_group lists; the rest is shared.
 //
-// Against the sorted tables: 2.35M agents x 100 days 20.7 -> 9.8 ms, 50M x
-// 100 days (split) 148 -> 82 ms, 24M with 10x the locations (split, few
-// infected, so only queried buckets were sorted) 35 -> 32 ms, 48 replicates
-// of 2.35M 260 -> 90 ms.
+// Whole workloads, sorted tables before: 2.35M agents x 100 days 20.7 -> 8.9
+// ms, 50M x 100 days (split) 161-175 -> 76-82 ms, 24M with 10x the locations
+// (split, few infected, so only queried buckets were sorted) 35 -> 24 ms, 48
+// replicates of 50k to 2M 259 -> 74 ms.
 //
 // Citations are relative to PandemicThrust/PandemicThrust/ of the reference.
 #pragma once
