@@ -138,9 +138,19 @@ hipError_t build_table(TableScratch& s, uint32_t* keys, const int32_t* vals, int
                        const AltInput* alt = nullptr);
 
 // A table of at most kSmallPairs host-counted pairs (ids = positions) and
-// kSmallBuckets buckets in one launch without scratch.
+// kSmallBuckets buckets in one launch without scratch.  Its blocks read the
+// keys while others write, so the outputs must lie apart from them; the radix
+// build reads the keys in its first pass only, and a caller may give up their
+// memory for the ids wherever that pass is not the last (over 256 buckets).
 constexpr int64_t kSmallPairs = 131072;
 constexpr int32_t kSmallBuckets = 8000;
+inline bool is_small_table(const uint32_t* keys, int64_t n, int32_t K, const int32_t* people, const int32_t* offsets) {
+    if (n < 1 || n > kSmallPairs || K < 1 || K > kSmallBuckets) return false;
+    const auto apart = [&](const int32_t* out, int64_t count) {
+        return (uintptr_t)(out + count) <= (uintptr_t)keys || (uintptr_t)(keys + n) <= (uintptr_t)out;
+    };
+    return apart(people, n) && apart(offsets, (int64_t)K + 1);
+}
 hipError_t build_small_table(const uint32_t* keys, int64_t n, int32_t K, int32_t* people_out, int32_t* offsets_out,
                              hipStream_t stream);
 

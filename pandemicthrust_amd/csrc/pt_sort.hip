@@ -973,7 +973,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_table(const uint32_t* _
 
 hipError_t build_small_table(const uint32_t* keys, int64_t n, int32_t K, int32_t* people_out, int32_t* offsets_out,
                              hipStream_t stream) {
-    if (n < 1 || n > kSmallPairs || K < 1 || K > kSmallBuckets) return hipErrorInvalidValue;
+    if (!is_small_table(keys, n, K, people_out, offsets_out)) return hipErrorInvalidValue;
     static_assert(2 * kSmallBuckets * sizeof(uint32_t) <= 64 * 1024, "LDS that needs no function attribute");
     k_small_table<<<(int)((n + kSmallThreads - 1) / kSmallThreads), kSmallThreads, 2 * sizeof(uint32_t) * K, stream>>>(
         keys, (int)n, K, key_bits(K), people_out, offsets_out);

@@ -87,7 +87,7 @@ extern "C" int pt_location_table(const uint32_t* keys, int64_t n, int32_t n_buck
     DeviceScope ds(device);
     HIP_TRY(ds.err);
     hipStream_t st = (hipStream_t)stream;
-    if (n > 0 && n <= kSmallPairs && n_buckets <= kSmallBuckets) {
+    if (is_small_table(keys, n, n_buckets, people, offsets)) {
         hipError_t e = build_small_table(keys, n, n_buckets, people, offsets, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) return fail(PT_EDEVICE, "location table: %s", hipGetErrorString(e));

@@ -76,7 +76,7 @@ extern "C" int pt_location_table_noalloc(const uint32_t* keys, int64_t n, int32_
                     (long long)kNoAllocMaxPairs);
     DeviceScope ds(device);
     HIP_TRY(ds.err);
-    if (n > 0 && n <= kSmallPairs && n_buckets <= kSmallBuckets) {
+    if (is_small_table(keys, n, n_buckets, people, offsets)) {
         const hipError_t e = build_small_table(keys, n, n_buckets, people, offsets, (hipStream_t)stream);
         if (e != hipSuccess) return fail(PT_EDEVICE, "location table: %s", hipGetErrorString(e));
         return PT_OK;
