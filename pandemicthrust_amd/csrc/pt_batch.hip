@@ -288,10 +288,9 @@ __global__ __launch_bounds__(kTestThreads) void kb_compact_test(const DayState* 
             st->n_infected = (int32_t)total;
             st->days_run = day + 1;
             out_inf[(int64_t)r * D + day] = (int32_t)total;
-            if (total == 0)
-                st->done = 1;  // nobody left to test: the replicate's other blocks may or may not see it
-            else
-                plan_offsets(st, WEEKEND, N);
+            // (the day's end sets done when nobody is infected: other blocks of
+            // this launch test it)
+            if (total) plan_offsets(st, WEEKEND, N);
         }
     }
     __syncthreads();
@@ -684,6 +683,10 @@ __global__ void kb_end_day(DayState* __restrict__ g, DayState* __restrict__ sts,
     for (int r = threadIdx.x; r < R; r += blockDim.x) {
         DayState* st = sts + r;
         if (st->done) continue;
+        if (st->n_infected == 0) {  // a counted day without infected (kb_compact_test)
+            st->done = 1;
+            continue;
+        }
         st->day += 1;
         st->rand_offset = st->contact_base + (uint64_t)6 * (uint64_t)st->n_infected;
         if (st->day >= st->max_days) st->done = 1;

@@ -391,14 +391,12 @@ __device__ __forceinline__ void compact_test_block(int block, int blocks, const 
             st->n_infected = (int32_t)total;
             st->days_run = day + 1;
             a.out_inf[day] = (int32_t)total;
-            if (total == 0) {
-                st->done = 1;  // nobody left to compact: other blocks may or may not see it
-                st->skip_full = st->skip_subset = st->skip_mark = 1;
-            } else {
-                st->skip_full = 0;  // every bucket is counted
-                st->skip_subset = st->skip_mark = 1;
-                plan_offsets(st, WEEKEND, N);
-            }
+            // (Nobody infected ends the loop, but not here: other blocks of
+            // this launch may not have started, and would skip their counter.
+            // The day's end sets the flag; until then its lists are empty.)
+            st->skip_full = total == 0;  // 0: every bucket is counted
+            st->skip_subset = st->skip_mark = 1;
+            if (total) plan_offsets(st, WEEKEND, N);
         }
         __syncthreads();
     }
@@ -762,6 +760,10 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(const Model* __res
 __device__ __forceinline__ void end_day(const DayState& d, DayState* st, int32_t* __restrict__ tab_full,
                                         int32_t* __restrict__ tab_pairs, int32_t n_full,
                                         const uint32_t* __restrict__ n_kept) {
+    if (d.n_infected == 0) {  // the loop's last day, only counted (compact_test_block)
+        st->done = 1;
+        return;
+    }
     tab_full[d.day] = d.skip_full == 0 ? 1 : 0;
     tab_pairs[d.day] = d.skip_full == 0 ? (n_kept ? (int32_t)*n_kept : n_full)
                                         : (d.skip_subset == 0 ? (int32_t)d.n_sel : 0);
