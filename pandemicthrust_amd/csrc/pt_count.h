@@ -46,6 +46,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <algorithm>
 #include <vector>
@@ -58,7 +59,6 @@ constexpr int kCountMaxK = 40000;       // 32-bit counters: 160,000 of the 163,8
 constexpr uint32_t kNoKey = 0xFFFFu;    // no pair (weekday hour 1 of a child)
 constexpr int kCountMinChunk = 1024;    // agents
 constexpr int kCountMaxRanges = 8;      // groups per hour: passes over its keys
-constexpr int kCountMaxHour = (1 << 20) - 1;  // locations per hour (20 bits beside 12 of the id; no pair is all ones)
 constexpr int kCountMaxLen = 64;        // people per bucket of a smallest chunk (CountPlan::build)
 constexpr int64_t kCountSmall = 1000000;  // agents up to which the lists' length does not matter
 
@@ -625,6 +625,7 @@ __global__ __launch_bounds__(1024) void k_collect(const int32_t* __restrict__ do
 
 constexpr int kTileAgents = 4096;  // group lists: agents per tile, ids within it 12 bits
 constexpr int kTileBits = 12;
+static_assert(kCountMaxRanges * kCountMaxK < (1 << (32 - kTileBits)), "a pair holds any location, and none is all ones");
 constexpr int kTileThreads = 512;
 constexpr int kTileGroups = 96;    // at most 10 hours x kCountMaxRanges, and the end
 
@@ -814,25 +815,34 @@ __device__ __forceinline__ void group_pairs(const CountTable& T, const CountRep&
 }
 
 // Group g of chunk: its hour, first location there, locations, and first
-// bucket.
+// bucket.  (A narrow hour leaves its last groups empty: the groups of all hours
+// are as wide as the widest's need.)
 struct GroupColumns {
     int hour, lo, n, bucket;
 };
-__device__ __forceinline__ GroupColumns group_columns(const CountRep& c, int g) {
+// An hour ends where the next begins, the last at K.
+__host__ __device__ inline int hour_end(const CountRep& c, int hour) {
+    return hour == c.G / c.ranges - 1 ? c.K : (hour + 1) * c.E;
+}
+__host__ __device__ inline GroupColumns group_columns(const CountRep& c, int g) {
     GroupColumns q;
     q.hour = g / c.ranges;
     q.lo = (g % c.ranges) * c.W;
     q.bucket = q.hour * c.E + q.lo;
-    // an hour ends where the next begins, the last at K
-    const int end = q.hour == c.G / c.ranges - 1 ? c.K : (q.hour + 1) * c.E;
-    q.n = max(0, min(c.W, end - q.bucket));
+    const int left = hour_end(c, q.hour) - q.bucket;
+    q.n = left < 0 ? 0 : (left < c.W ? left : c.W);
     return q;
 }
 
 // All groups of an hour.
-__device__ __forceinline__ GroupColumns hour_columns(const CountRep& c, int hour) {
-    const GroupColumns last = group_columns(c, hour * c.ranges + c.ranges - 1);
-    return GroupColumns{hour, 0, last.lo + last.n, hour * c.E};
+__host__ __device__ inline GroupColumns hour_columns(const CountRep& c, int hour) {
+    return GroupColumns{hour, 0, hour_end(c, hour) - hour * c.E, hour * c.E};
+}
+
+// The mark words that hold q's buckets: [first, end), none if it has none.
+__host__ __device__ inline int first_mark_word(const GroupColumns& q) { return q.bucket / 32; }
+__host__ __device__ inline int end_mark_word(const GroupColumns& q) {
+    return q.n > 0 ? (q.bucket + q.n + 31) / 32 : first_mark_word(q);
 }
 
 // Counts of a (chunk, group).  Bound by reading its keys (16 bytes per lane
@@ -872,7 +882,7 @@ constexpr int kCollectParts = 16, kCollectFewThreads = 512;
 // Marked buckets of the group, by the whole block; f(bucket) for each.
 template <class F>
 __device__ __forceinline__ void for_marked(const uint32_t* __restrict__ marks, const GroupColumns& q, F f) {
-    for (int i = q.bucket / 32 + threadIdx.x; i * 32 < q.bucket + q.n; i += blockDim.x) {
+    for (int i = first_mark_word(q) + threadIdx.x; i < end_mark_word(q); i += blockDim.x) {
         uint32_t w = marks[i];
         while (w) {
             const int b = i * 32 + __ffs(w) - 1;
@@ -1213,7 +1223,7 @@ struct CountPlan {
         c.E = E;
         const int32_t last = c.K - (hours - 1) * E, widest = std::max(E, last);
         c.ranges = (widest + kCountMaxK - 1) / kCountMaxK;
-        if (c.ranges > kCountMaxRanges || widest > kCountMaxHour) return;
+        if (c.ranges > kCountMaxRanges) return;
         c.W = (widest + c.ranges - 1) / c.ranges;
         c.G = hours * c.ranges;
         int64_t A = 0;
