@@ -378,6 +378,46 @@ struct PickPush {
 
 namespace {
 
+// Counting keys of two neighbouring agents (the second only if `two`) from
+// their destinations; false if one lies outside its hour, which no model
+// allows.  (A key below K is not enough: past its hour's end a destination has
+// a bucket of the next hour.)
+struct WeekdayHours {
+    int32_t base0, base1;  // first location of each hour
+    uint32_t E0, E1;       // locations; hour 1's buckets follow hour 0's
+};
+__host__ __device__ inline bool weekday_pair_keys(const WeekdayHours& H, const int32_t (&d1)[2], const int32_t (&d2)[2],
+                                                  const bool (&adult)[2], bool two, uint32_t (&k0)[2],
+                                                  uint32_t (&k1)[2]) {
+    uint32_t top0 = 0, top1 = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const bool there = i == 0 || two;
+        const uint32_t l0 = (uint32_t)(d1[i] - H.base0), l1 = (uint32_t)(d2[i] - H.base1);
+        const uint32_t c0 = there ? l0 : 0u, c1 = adult[i] ? l1 : 0u;
+        top0 = c0 > top0 ? c0 : top0;
+        top1 = c1 > top1 ? c1 : top1;
+        k0[i] = there ? l0 : kNoKey;
+        k1[i] = adult[i] ? H.E0 + l1 : kNoKey;
+    }
+    return (top0 < H.E0) & (top1 < H.E1);
+}
+__host__ __device__ inline bool weekend_pair_keys(int32_t base, uint32_t E, const int32_t (&hour)[2][3],
+                                                  const int32_t (&loc)[2][3], bool two, uint32_t (&k)[2][3]) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            const uint32_t l = (uint32_t)(loc[i][e] - base), c = i == 0 || two ? l : 0u;
+            top = c > top ? c : top;
+            // (hours below 10, E below 2^24: a 24-bit product)
+            k[i][e] = (((uint32_t)hour[i][e] & 0xFFFFFFu) * (E & 0xFFFFFFu)) + l;
+        }
+    }
+    return top < E;
+}
+
 // Keys and counts of a chunk.  VALU bound (per agent 125 instructions on weekdays,
 // 381 on weekends, of which the draws 71 and 284: 32M agents in 48 replicates 102
 // and 291 us; agent by agent with a check per key 10% more); the LDS adds,
@@ -392,7 +432,6 @@ __device__ __forceinline__ void count_block(int block, DayState* __restrict__ st
     const Model& M = models[blk.r];
     const CountRep c = T.reps[blk.r];
     const int tid = threadIdx.x, nt = blockDim.x;
-    const uint32_t K = (uint32_t)c.K;
     __shared__ __align__(16) WalkRow s_row[kWalkRows];
     const LdsWalk wk = load_walk(WEEKEND ? M.we_table : M.wd_table, s_row);
     for (int i = tid; i < c.K; i += nt) s_cnt[i] = 0;
@@ -400,8 +439,8 @@ __device__ __forceinline__ void count_block(int block, DayState* __restrict__ st
     const int64_t N = M.N;
     const int64_t a0 = (int64_t)blk.at * c.A, a1 = min(N, a0 + c.A);  // even a0
     const uint64_t eoff = st->rand_offset;  // the day's errand offset: it moves at the day's end
-    // Two agents per thread and turn; the keys, all below K unless the model is
-    // at fault, are checked together.
+    // Two agents per thread and turn; their keys, all in range unless the model
+    // is at fault, are checked together.
     bool bad = false;
     auto add = [&](bool there, uint32_t k) {
         if (there) atomicAdd(&s_cnt[k], 1u);
@@ -412,21 +451,16 @@ __device__ __forceinline__ void count_block(int block, DayState* __restrict__ st
         uint32_t* out = reinterpret_cast<uint32_t*>(T.keys + c.abase);
         for (int64_t g = a0 / 2 + tid; 2 * g < a1; g += nt) {
             const bool two = 2 * g + 1 < a1;
-            uint32_t k[2][3], top = 0;
+            uint32_t k[2][3];
+            int32_t hour[2][3], loc[2][3];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                int32_t hour[3], loc[3];
-                weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * ((int32_t)(2 * g) + i)), hour, loc);
-#pragma unroll
-                for (int e = 0; e < 3; ++e) {
-                    k[i][e] = __umul24((uint32_t)hour[e], E) + (uint32_t)(loc[e] - base);
-                    top = max(top, i == 0 || two ? k[i][e] : 0u);
-                }
-            }
+            for (int i = 0; i < 2; ++i)
+                weekend_errands(M, wk, eoff + (uint64_t)(int64_t)(2 * ((int32_t)(2 * g) + i)), hour[i], loc[i]);
+            const bool ok = weekend_pair_keys(base, E, hour, loc, two, k);
 #pragma unroll
             for (int e = 0; e < 3; ++e)
                 out[e * (T.slots / 2) + g] = (k[0][e] & 0xFFFFu) | (two ? k[1][e] << 16 : kNoKey << 16);
-            if (top < K) {
+            if (ok) {
 #pragma unroll
                 for (int e = 0; e < 3; ++e) {
                     add(true, k[0][e]);
@@ -437,7 +471,7 @@ __device__ __forceinline__ void count_block(int block, DayState* __restrict__ st
             }
         }
     } else {
-        const int base = M.wd_base, base1 = M.wd_base1 - M.wd_E;  // hour-1 keys follow the wd_E hour-0 keys
+        const WeekdayHours hours{M.wd_base, M.wd_base1, (uint32_t)M.wd_E, (uint32_t)M.wd_E1};
         const uint8_t* age = ages + c.abase;
         uint32_t* out0 = reinterpret_cast<uint32_t*>(T.keys + c.abase);
         uint32_t* out1 = reinterpret_cast<uint32_t*>(T.keys + T.slots + c.abase);
@@ -446,22 +480,18 @@ __device__ __forceinline__ void count_block(int block, DayState* __restrict__ st
             // (ages are padded to whole pairs)
             const uint32_t age2 = *reinterpret_cast<const uint16_t*>(age + 2 * g);
             const U4 u = draw4(eoff + (uint64_t)g, M.key0, M.key1);
-            uint32_t k0[2], k1[2], top = 0;
+            uint32_t k0[2], k1[2];
+            int32_t d1[2], d2[2];
             bool adult[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const bool there = i == 0 || two;
-                adult[i] = there && ((age2 >> (8 * i)) & 0xFFu) == kAgeAdult;
-                int32_t d1, d2;
-                weekday_dests(M, wk, u.w[2 * i], u.w[2 * i + 1], adult[i], d1, d2);
-                k0[i] = there ? (uint32_t)(d1 - base) : kNoKey;
-                k1[i] = adult[i] ? (uint32_t)(d2 - base1) : kNoKey;
-                top = max(top, there ? k0[i] : 0u);
-                top = max(top, adult[i] ? k1[i] : 0u);
+                adult[i] = (i == 0 || two) && ((age2 >> (8 * i)) & 0xFFu) == kAgeAdult;
+                weekday_dests(M, wk, u.w[2 * i], u.w[2 * i + 1], adult[i], d1[i], d2[i]);
             }
+            const bool ok = weekday_pair_keys(hours, d1, d2, adult, two, k0, k1);
             out0[g] = (k0[0] & 0xFFFFu) | (k0[1] << 16);
             out1[g] = (k1[0] & 0xFFFFu) | (k1[1] << 16);
-            if (top < K) {
+            if (ok) {
                 add(true, k0[0]);
                 add(two, k0[1]);
                 add(adult[0], k1[0]);
@@ -655,7 +685,7 @@ __global__ __launch_bounds__(256) void k_keys_weekday(DayState* __restrict__ st,
             const bool adult = p < N && age[p] == kAgeAdult;
             int32_t d1, d2;
             weekday_dests(M, wk, u.w[2 * k], u.w[2 * k + 1], adult, d1, d2);
-            bad |= (uint32_t)(d1 - base) >= (uint32_t)M.wd_E;
+            bad |= ((uint32_t)(d1 - base) >= (uint32_t)M.wd_E) | (adult & ((uint32_t)(d2 - base1) >= (uint32_t)M.wd_E1));
             w0 |= ((uint32_t)(d1 - base) & 0xFFFFu) << (16 * k);
             w1 |= (adult ? (uint32_t)(d2 - base1) & 0xFFFFu : kNoKey) << (16 * k);
         }

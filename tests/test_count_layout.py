@@ -1,5 +1,6 @@
 """Host code of the counted tables' headers, compiled for the CPU and run:
-count_layout_host.cpp checks the column groups of split layouts."""
+count_layout_host.cpp checks the column groups of split layouts,
+count_keys_host.cpp the keys of agent pairs and their check."""
 import os
 import shutil
 import subprocess
@@ -24,3 +25,7 @@ def run_host(source, tmp_path):
 
 def test_column_groups(tmp_path):
     assert ", 0 wrong" in run_host("count_layout_host.cpp", tmp_path)
+
+
+def test_pair_keys(tmp_path):
+    assert ", 0 wrong" in run_host("count_keys_host.cpp", tmp_path)
