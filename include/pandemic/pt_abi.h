@@ -303,8 +303,8 @@ int pt_location_table(const uint32_t* keys, int64_t n, int32_t n_buckets, int32_
  * stream and returns; results are identical to pt_location_table's.  Every
  * call on one device shares that device's array, so calls that overlap on
  * one device (other streams or threads) race: serialise them.  (Tables of at
- * most 131,072 pairs and 8,000 buckets whose outputs do not overlap the keys
- * are one launch and do not use it.) */
+ * most 131,072 pairs and 5,000 buckets, or 65,536 and 8,000, whose outputs do
+ * not overlap the keys are one launch and do not use it.) */
 #define PT_LOCATION_TABLE_NOALLOC_MAX_PAIRS 4194304
 int pt_location_table_noalloc(const uint32_t* keys, int64_t n, int32_t n_buckets, int32_t* people,
                               int32_t* offsets, int32_t device, void* stream);

@@ -144,8 +144,23 @@ hipError_t build_table(TableScratch& s, uint32_t* keys, const int32_t* vals, int
 // memory for the ids wherever that pass is not the last (over 256 buckets).
 constexpr int64_t kSmallPairs = 131072;
 constexpr int32_t kSmallBuckets = 8000;
+constexpr int kSmallWords = 40000;  // of LDS
+// Copies of its counters (log2), up to 64 as far as LDS holds them, one per so
+// many pairs that a table of a single crowded bucket is no slower than the
+// radix build (figures at k_small_table): that one takes 18 us for up to 32
+// buckets, 23-32 us (one pass) for 256, 40-50 us beyond.  A table that would
+// need more copies than fit (over 5,000 buckets and 65,536 pairs) takes the
+// radix build.
+inline int64_t small_table_pairs_per_copy(int32_t K) { return K <= 32 ? 2048 : (K <= 256 ? 8192 : 32768); }
+inline int small_table_copy_bits(int64_t n, int32_t K) {
+    const int64_t per = small_table_pairs_per_copy(K);
+    int bits = 0;
+    while (bits < 6 && n > per << bits && (4 * (int64_t)K << bits) <= kSmallWords) ++bits;
+    return bits;
+}
 inline bool is_small_table(const uint32_t* keys, int64_t n, int32_t K, const int32_t* people, const int32_t* offsets) {
     if (n < 1 || n > kSmallPairs || K < 1 || K > kSmallBuckets) return false;
+    if (n > small_table_pairs_per_copy(K) << small_table_copy_bits(n, K)) return false;
     const auto apart = [&](const int32_t* out, int64_t count) {
         return (uintptr_t)(out + count) <= (uintptr_t)keys || (uintptr_t)(keys + n) <= (uintptr_t)out;
     };

@@ -900,23 +900,36 @@ hipError_t build_table(TableScratch& s, uint32_t* keys, const int32_t* vals, int
 
 namespace {
 
-// Small tables.  The radix build is nine launches that wait for each other
-// whatever the size.  Here every block of 1,024 threads counts all keys itself
-// in LDS, apart those before its own 1,024, so that it knows where its keys
-// go: no second launch, no scratch.  Its 16 waves place their keys in turn.
-// Bound by latency and the LDS adds (n / 64 wave instructions per block).  One
-// table, 545 buckets: 29,919 pairs 36 -> 7.4 us; at the limit of 131,072 pairs
-// 16.4 us, 20.8 with 8,000 buckets, where the radix build takes 39 and 44.
+// Small tables.  The radix build is three launches per digit that wait for each
+// other whatever the size.  Here every block of 1,024 threads counts all keys
+// itself in LDS, apart those before its own 1,024, so that it knows where its
+// keys go: no second launch, no scratch.  Its 16 waves place their keys in turn.
+// Bound by latency and the LDS adds (n / 64 wave instructions per block), which
+// take turns where lanes hold one key: up to 1.8 clocks per lane, 0.8 us per
+// 1,024 pairs of one bucket.  So the counters come in copies, a lane's by its
+// number (small_table_copy_bits).  Times in us, radix build / this:
+//
+//   buckets   pairs     keys spread       9 of 10 in one bucket    all in one
+//   1         131,072   20.0 / 17.7                                (114 without copies)
+//   29        131,072   18.9 / 18.2       21.1 / 18.1              21.3 / 17.8
+//   256       131,072   27.7 / 18.1       32.3 / 17.6              32.7 / 17.4
+//   545       131,072   39.5 / 17.8       44.5 / 34.3              43.7 / 34.6
+//   5,000     131,072   45.3 / 22.7       50.3 / 39.1              50.2 / 39.4
+//   8,000     65,536    40.7 / 15.4       45.7 / 35.4              45.8 / 36.8
+//   545       29,919    36.5 / 7.7        42.6 / 27.7              43.2 / 30.1
 constexpr int kSmallThreads = 1024;
+template <bool COPIES>
 __global__ __launch_bounds__(kSmallThreads) void k_small_table(const uint32_t* __restrict__ keys, int n, int K,
-                                                               int bits, int32_t* __restrict__ people,
+                                                               int bits, int copy_bits, int32_t* __restrict__ people,
                                                                int32_t* __restrict__ offsets) {
+    if constexpr (!COPIES) copy_bits = 0;
     extern __shared__ uint32_t s_count[];  // keys before this block's own (then: where its next one goes); the others
     __shared__ uint32_t s_w[kSmallThreads / 64];
     uint32_t* const before = s_count;
-    uint32_t* const after = s_count + K;
+    uint32_t* const after = s_count + (K << copy_bits);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < 2 * K; i += kSmallThreads) s_count[i] = 0;
+    const uint32_t mask = (1u << copy_bits) - 1u, copy = lane & mask;
+    for (int i = tid; i < 2 * K << copy_bits; i += kSmallThreads) s_count[i] = 0;
     const int own0 = blockIdx.x * kSmallThreads, own = own0 + tid;
     const uint32_t key = own < n ? keys[own] : ~0u;
     __syncthreads();
@@ -930,22 +943,40 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_table(const uint32_t* _
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (k[u] < (uint32_t)K) atomicAdd((i0 + u * kSmallThreads < own0 ? before : after) + k[u], 1u);
+            if (k[u] < (uint32_t)K)
+                atomicAdd((i0 + u * kSmallThreads < own0 ? before : after) + ((k[u] << copy_bits) | copy), 1u);
     }
     __syncthreads();
-    // Exclusive prefix over the buckets, a run of consecutive ones per thread.
-    const int per = (K + kSmallThreads - 1) / kSmallThreads, b0 = min(K, tid * per), b1 = min(K, b0 + per);
+    // A bucket's sums go to its first copies (lanes begin with different
+    // copies: other banks).
+    if constexpr (COPIES) {
+        for (int b = tid; b < K; b += kSmallThreads) {
+            uint32_t tb = 0, ta = 0;
+            for (uint32_t r = 0; r <= mask; ++r) {
+                const uint32_t at = ((uint32_t)b << copy_bits) + ((r + tid) & mask);
+                tb += before[at];
+                ta += after[at];
+            }
+            before[b << copy_bits] = tb;
+            after[b << copy_bits] = ta;
+        }
+        __syncthreads();
+    }
+    // Exclusive prefix over the buckets, a run of consecutive ones per thread
+    // (an odd number: other banks).
+    const int per = (K + kSmallThreads - 1) / kSmallThreads | 1, b0 = min(K, tid * per), b1 = min(K, b0 + per);
     uint32_t sum = 0;
-    for (int b = b0; b < b1; ++b) sum += before[b] + after[b];
+    for (int b = b0; b < b1; ++b) sum += before[b << copy_bits] + after[b << copy_bits];
     const uint32_t inc = wave_incl_scan(sum, lane);
     if (lane == 63) s_w[wave] = inc;
     __syncthreads();
     uint32_t at = inc - sum;
     for (int w = 0; w < wave; ++w) at += s_w[w];
     for (int b = b0; b < b1; ++b) {
-        const uint32_t total = before[b] + after[b];
+        const uint32_t tb = before[b << copy_bits];
+        const uint32_t total = tb + after[b << copy_bits];
         if (blockIdx.x == 0) offsets[b] = (int32_t)at;
-        before[b] += at;
+        before[b << copy_bits] = tb + at;
         at += total;
     }
     if (blockIdx.x == 0 && tid == kSmallThreads - 1) offsets[K] = (int32_t)at;
@@ -961,9 +992,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_table(const uint32_t* _
     __syncthreads();
     for (int w = 0; w < kSmallThreads / 64; ++w) {
         if (w == wave && there) {
-            const uint32_t pos = before[key];
+            const uint32_t pos = before[key << copy_bits];
             people[pos + rank] = own;
-            if (rank == 0) before[key] = pos + (uint32_t)__popcll(same);
+            if (rank == 0) before[key << copy_bits] = pos + (uint32_t)__popcll(same);
         }
         __syncthreads();
     }
@@ -974,9 +1005,16 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_table(const uint32_t* _
 hipError_t build_small_table(const uint32_t* keys, int64_t n, int32_t K, int32_t* people_out, int32_t* offsets_out,
                              hipStream_t stream) {
     if (!is_small_table(keys, n, K, people_out, offsets_out)) return hipErrorInvalidValue;
-    static_assert(2 * kSmallBuckets * sizeof(uint32_t) <= 64 * 1024, "LDS that needs no function attribute");
-    k_small_table<<<(int)((n + kSmallThreads - 1) / kSmallThreads), kSmallThreads, 2 * sizeof(uint32_t) * K, stream>>>(
-        keys, (int)n, K, key_bits(K), people_out, offsets_out);
+    const int copy_bits = small_table_copy_bits(n, K);
+    const size_t lds = (2 * sizeof(uint32_t) * K) << copy_bits;
+    const auto kernel = copy_bits ? k_small_table<true> : k_small_table<false>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kSmallWords * 4);
+        if (e != hipSuccess) return e;
+    }
+    kernel<<<(int)((n + kSmallThreads - 1) / kSmallThreads), kSmallThreads, lds, stream>>>(
+        keys, (int)n, K, key_bits(K), copy_bits, people_out, offsets_out);
     return hipGetLastError();
 }
 
