@@ -692,9 +692,10 @@ struct pt_mlp {
     float* xin = nullptr;  // prediction inputs
     int64_t xin_cap = 0;
     // Prediction results on their way to the caller: pinned slots, each with
-    // an event that marks its copy's end.
+    // an event that marks its copy's end (the second slot and the events when a
+    // result first needs them).
     float* slot[2] = {};
-    int64_t slot_cap = 0;  // floats
+    int64_t slot_cap[2] = {};  // floats
     hipEvent_t slot_ev[2] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double last_ms = 0;
@@ -1010,24 +1011,27 @@ int pt_mlp_predict(pt_mlp* m, const float* X, int64_t n, float* out) {
     // Results go through two pinned slots, so that a part's way to the
     // caller's memory (a host copy, bound by its page faults) overlaps the
     // next parts' products and device copies: a part is one chunk of all
-    // members, or rows of one member's chunk.
+    // members, or rows of one member's chunk.  A result of one part takes one
+    // slot and waits for the stream: nothing else to overlap, and a handle that
+    // is asked once pays for one pinned allocation and no event (first call on
+    // a new handle, 2 x 7: 123 us with both slots and events, 99 without; later
+    // calls 60 and 54).
     const int64_t rows0 = std::min<int64_t>(B, n), all = m->members * rows0;
     const int64_t part_rows = std::min(rows0, kSlotRows);
-    const bool whole = all <= kSlotRows;
+    const bool whole = all <= kSlotRows, single = whole && n <= B;
     const int64_t want = (whole ? all : part_rows) * PT_MLP_OUT;
-    if (want > m->slot_cap) {
-        m->slot_cap = 0;
-        HIP_TRY(hipStreamSynchronize(m->stream));
-        for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < (single ? 1 : 2); ++i) {
+        if (want > m->slot_cap[i]) {
+            m->slot_cap[i] = 0;
+            HIP_TRY(hipStreamSynchronize(m->stream));
             if (m->slot[i]) HIP_TRY(hipHostFree(m->slot[i]));
             m->slot[i] = nullptr;
             if (hipHostMalloc((void**)&m->slot[i], sizeof(float) * want) != hipSuccess)
                 return fail(PT_ENOMEM, "hipHostMalloc of %lld bytes failed", (long long)(sizeof(float) * want));
+            m->slot_cap[i] = want;
         }
-        m->slot_cap = want;
+        if (!single && !m->slot_ev[i]) HIP_TRY(hipEventCreateWithFlags(&m->slot_ev[i], hipEventDisableTiming));
     }
-    for (hipEvent_t& e : m->slot_ev)
-        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     struct Part {
         int64_t at = 0;             // first row of the result
         int rows = 0, members = 0;  // members of consecutive blocks of n rows
@@ -1036,7 +1040,7 @@ int pt_mlp_predict(pt_mlp* m, const float* X, int64_t n, float* out) {
     auto drain = [&](int i) -> int {
         Part& q = pending[i];
         if (q.rows == 0) return PT_OK;
-        HIP_TRY(hipEventSynchronize(m->slot_ev[i]));
+        HIP_TRY(single ? hipStreamSynchronize(m->stream) : hipEventSynchronize(m->slot_ev[i]));
         const size_t len = (size_t)q.rows * PT_MLP_OUT;
         for (int k = 0; k < q.members; ++k)
             memcpy(out + (size_t)(q.at + k * n) * PT_MLP_OUT, m->slot[i] + k * len, sizeof(float) * len);
@@ -1056,7 +1060,7 @@ int pt_mlp_predict(pt_mlp* m, const float* X, int64_t n, float* out) {
                 HIP_TRY(hipMemcpy2DAsync(m->slot[i], len, m->pred + ((int64_t)k * B + r0) * PT_MLP_OUT,
                                          sizeof(float) * B * PT_MLP_OUT, len, whole ? m->members : 1,
                                          hipMemcpyDeviceToHost, m->stream));
-                HIP_TRY(hipEventRecord(m->slot_ev[i], m->stream));
+                if (!single) HIP_TRY(hipEventRecord(m->slot_ev[i], m->stream));
                 pending[i] = Part{k * n + i0 + r0, count, whole ? m->members : 1};
                 next = 1 - next;
             }
