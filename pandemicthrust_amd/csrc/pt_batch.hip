@@ -731,6 +731,7 @@ struct pt_batch {
     int32_t* tile_rep = nullptr;
     uint8_t *st_p = nullptr, *st_s = nullptr, *dy_p = nullptr, *dy_s = nullptr, *gn_p = nullptr, *gn_s = nullptr;
     uint8_t *age = nullptr, *hh_types = nullptr, *snap = nullptr;
+    bool one_block = false;  // st_p to age in one allocation (alloc_agent_bytes)
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
     AgentRecord* who = nullptr;
     int32_t* wp_lone = nullptr;
@@ -739,8 +740,7 @@ struct pt_batch {
     uint32_t *blk_counts = nullptr, *blk_ninf = nullptr, *blk_off = nullptr;
     int32_t *rep_I = nullptr, *inf_start = nullptr;
     uint32_t* mark = nullptr;
-    uint32_t *stage_keys = nullptr, *sel_keys = nullptr;
-    int32_t *stage_ids = nullptr, *sel_ids = nullptr;
+    SelectionBuffers selection;
     uint32_t *sblk_cnt = nullptr, *sblk_off = nullptr;
     int32_t *er_people = nullptr, *er_off = nullptr;
     // Segmented day tables (R <= kSegBlocks): each replicate's pairs sorted
@@ -780,13 +780,7 @@ namespace {
 
 void free_batch_population(pt_batch* b) {
     dev_free(b->tile_rep);
-    dev_free(b->st_p);
-    dev_free(b->st_s);
-    dev_free(b->dy_p);
-    dev_free(b->dy_s);
-    dev_free(b->gn_p);
-    dev_free(b->gn_s);
-    dev_free(b->age);
+    free_agent_bytes(*b);
     dev_free(b->hh_types);
     dev_free(b->snap);
     dev_free(b->household);
@@ -805,10 +799,7 @@ void free_batch_population(pt_batch* b) {
     dev_free(b->blk_ninf);
     dev_free(b->blk_off);
     dev_free(b->mark);
-    dev_free(b->stage_keys);
-    dev_free(b->stage_ids);
-    dev_free(b->sel_keys);
-    dev_free(b->sel_ids);
+    free_selection(b->selection);
     dev_free(b->sblk_cnt);
     dev_free(b->sblk_off);
     dev_free(b->er_people);
@@ -926,11 +917,11 @@ int enqueue_batch_day(pt_batch* b, int d) {
     const int nb = (int)(b->P / (weekend ? kSelAgentsWe : kSelAgentsWd));
     if (weekend)
         kb_select<kSelPerWe, true><<<nb, kSelThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep,
-                                                               b->age, b->mark, b->stage_keys, b->stage_ids,
+                                                               b->age, b->mark, b->selection.stage_keys, b->selection.stage_ids,
                                                                b->sblk_cnt);
     else
         kb_select<kSelPerWd, false><<<nb, kSelThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep,
-                                                                b->age, b->mark, b->stage_keys, b->stage_ids,
+                                                                b->age, b->mark, b->selection.stage_keys, b->selection.stage_ids,
                                                                 b->sblk_cnt);
     hipError_t e = exclusive_scan_u32(b->sblk_cnt, b->sblk_off, nb, b->tables.scan_part, &g->done, s);
     if (e != hipSuccess) return fail(PT_EDEVICE, "selection scan: %s", hipGetErrorString(e));
@@ -946,12 +937,12 @@ int enqueue_batch_day(pt_batch* b, int d) {
                                                            b->seg_count);
     if (weekend)
         kb_emit<kSelPerWe, true><<<nb, kSelThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep, b->age,
-                                                             b->mark, b->stage_keys, b->stage_ids, b->sblk_cnt, b->sblk_off,
-                                                             b->sel_keys, b->sel_ids, seg_start);
+                                                             b->mark, b->selection.stage_keys, b->selection.stage_ids, b->sblk_cnt, b->sblk_off,
+                                                             b->selection.sel_keys, b->selection.sel_ids, seg_start);
     else
         kb_emit<kSelPerWd, false><<<nb, kSelThreads, 0, s>>>(g, b->d_states, b->d_reps, b->d_models, b->tile_rep,
-                                                              b->age, b->mark, b->stage_keys, b->stage_ids, b->sblk_cnt,
-                                                              b->sblk_off, b->sel_keys, b->sel_ids, seg_start);
+                                                              b->age, b->mark, b->selection.stage_keys, b->selection.stage_ids, b->sblk_cnt,
+                                                              b->sblk_off, b->selection.sel_keys, b->selection.sel_ids, seg_start);
     const int64_t n_cap = (weekend ? 3 : 2) * b->P + 4 * (int64_t)R;
     if (seg) {
         SegLayout sl;
@@ -963,10 +954,10 @@ int enqueue_batch_day(pt_batch* b, int d) {
         sl.seg_kbase = weekend ? b->seg_kb_we : b->seg_kb_wd;
         sl.seg_K = weekend ? b->seg_K_we : b->seg_K_wd;
         sl.R = R;
-        e = build_table_segmented(b->tables, b->sel_keys, b->sel_ids, n_cap, weekend ? b->K_local_we : b->K_local_wd,
+        e = build_table_segmented(b->tables, b->selection.sel_keys, b->selection.sel_ids, n_cap, weekend ? b->K_local_we : b->K_local_wd,
                                   (int32_t)K, sl, b->er_people, b->er_off, &g->done, s, nullptr);
     } else {
-        e = build_table(b->tables, b->sel_keys, b->sel_ids, n_cap, &g->n_sel, (int32_t)K, ID_IDENTITY, 0,
+        e = build_table(b->tables, b->selection.sel_keys, b->selection.sel_ids, n_cap, &g->n_sel, (int32_t)K, ID_IDENTITY, 0,
                         b->er_people, b->er_off, &g->done, s, nullptr);
     }
     if (e != hipSuccess) return fail(PT_EDEVICE, "batch table build: %s", hipGetErrorString(e));
@@ -1001,7 +992,9 @@ int setup_batch_counts(pt_batch* b) {
         }
         p.build(N, w ? 3 : 2, b->cus);
     }
-    if (b->count_scratch.alloc(b->count_plan, 0, b->stream)) {
+    // (the keys take 6 of the 12 bytes per slot there)
+    if (b->count_scratch.alloc(b->count_plan, 0, b->stream, b->tables, (unsigned char*)b->tables.keys_b + 6 * b->P,
+                               6 * b->P)) {
         // no memory for the matrices: sorted tables
         (void)hipGetLastError();
         for (CountPlan& p : b->count_plan) p.release();
@@ -1014,21 +1007,21 @@ int setup_batch_counts(pt_batch* b) {
         if (!p.on) continue;
         CountTable& t = b->count_table[w];
         b->count_scratch.fill(t, p);
-        t.keys = reinterpret_cast<uint16_t*>(b->tables.keys_b);  // 6 of its 12 bytes per slot
+        t.keys = reinterpret_cast<uint16_t*>(b->tables.keys_b);
         t.slots = P;
         t.list = b->er_people;
-        t.pk_bucket = b->stage_keys;  // at most 2 picks per agent
-        t.pk_want = (uint32_t*)b->stage_ids;
-        t.pk_claim = b->sel_keys;
-        t.pk_payload = (uint32_t*)b->sel_ids;
+        t.pk_bucket = b->selection.stage_keys;  // at most 2 picks per agent
+        t.pk_want = (uint32_t*)b->selection.stage_ids;
+        t.pk_claim = b->selection.sel_keys;
+        t.pk_payload = (uint32_t*)b->selection.sel_ids;
         t.pk_idx = (int32_t*)b->tables.pairs_a;
         t.pk_r = t.pk_idx + 3 * P;
         t.pk_chunk = (int32_t*)b->tables.pairs_b;
         t.pk_len = t.pk_chunk + 3 * P;
-        t.sv_idx = (int32_t*)b->stage_keys + 2 * P;
-        t.sv_pos = b->stage_ids + 2 * P;
-        t.sv_f = b->sel_keys + 2 * P;
-        t.sv_r = b->sel_ids + 2 * P;
+        t.sv_idx = (int32_t*)b->selection.stage_keys + 2 * P;
+        t.sv_pos = b->selection.stage_ids + 2 * P;
+        t.sv_f = b->selection.sel_keys + 2 * P;
+        t.sv_r = b->selection.sel_ids + 2 * P;
         t.wp_lone = b->wp_lone;
         HIP_TRY(set_count_lds(p));
     }
@@ -1197,15 +1190,13 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
     const int64_t kmax = std::max<int64_t>(kwd, kwe);
     const int64_t n3 = 3 * P + 4 * (int64_t)R;  // segment starts are rounded up to multiples of 4
     const int64_t nsel = P / kSelAgentsWe + 1;
-    if (dev_alloc(&b->tile_rep, tiles) || dev_alloc(&b->st_p, P) || dev_alloc(&b->st_s, P) ||
-        dev_alloc(&b->dy_p, P) || dev_alloc(&b->dy_s, P) || dev_alloc(&b->gn_p, P) || dev_alloc(&b->gn_s, P) ||
-        dev_alloc(&b->age, P) || dev_alloc(&b->snap, 6 * P) || dev_alloc(&b->household, P) ||
+    if (dev_alloc(&b->tile_rep, tiles) || alloc_agent_bytes(*b, P) || dev_alloc(&b->snap, 6 * P) || dev_alloc(&b->household, P) ||
         dev_alloc(&b->hh_off, HH) || dev_alloc(&b->wp_off, WW) || dev_alloc(&b->wp_people, P) || dev_alloc(&b->who, P) || dev_alloc(&b->wp_lone, R) ||
         dev_alloc(&b->claim_p, P) || dev_alloc(&b->claim_s, P) || dev_alloc(&b->list_p, P) ||
         dev_alloc(&b->list_s, P) || dev_alloc(&b->infected, P) || dev_alloc(&b->staging, P) ||
         dev_alloc(&b->blk_counts, (int64_t)tiles * 16) || dev_alloc(&b->blk_ninf, tiles) ||
-        dev_alloc(&b->blk_off, tiles) || dev_alloc(&b->mark, kmax / 32 + 1) || dev_alloc(&b->stage_keys, n3) ||
-        dev_alloc(&b->stage_ids, n3) || dev_alloc(&b->sel_keys, n3) || dev_alloc(&b->sel_ids, n3) ||
+        dev_alloc(&b->blk_off, tiles) || dev_alloc(&b->mark, kmax / 32 + 1) || alloc_selection(b->selection, n3, n3) ||
+       
         dev_alloc(&b->sblk_cnt, nsel) || dev_alloc(&b->sblk_off, nsel) || dev_alloc(&b->er_people, n3) ||
         dev_alloc(&b->er_off, kmax + 1) || dev_alloc(&b->d_counts, (int64_t)R * b->D * 16) ||
         dev_alloc(&b->d_inf, (int64_t)R * b->D) || dev_alloc(&b->seg_blk, kSegBlocks) ||
@@ -1290,7 +1281,7 @@ int pt_batch_setup(pt_batch* b, int64_t* n_people_out) {
         const PopArrays Pa{b->hh_types + ri.hbase, b->hh_off + ri.hbase, b->household + a, b->age + a,
                            b->wp_off + ri.wbase, b->wp_people + a, b->who + a, b->wp_lone + r, b->st_p + a, b->st_s + a, b->dy_p + a, b->dy_s + a,
                            b->gn_p + a, b->gn_s + a, b->claim_p + a, b->claim_s + a};
-        hipError_t e = build_population(b->d_models + r, ri.N, ri.H, ri.W, Pa, b->sel_keys, b->tables,
+        hipError_t e = build_population(b->d_models + r, ri.N, ri.H, ri.W, Pa, b->selection.sel_keys, b->tables,
                                         ri.workplace_off, st);
         if (e != hipSuccess) return fail(PT_EDEVICE, "replicate %d setup: %s", r, hipGetErrorString(e));
     }

@@ -105,7 +105,7 @@ struct ClaimArrays {
 struct CountTable {
     const CountRep* reps;
     const CountBlock* chunks;
-    const CountBlock* scans;
+    const CountBlock* scans;  // (null: one simulation, blocks in order)
     uint16_t* keys;        // keys per agent x slots (split weekday layouts: within the hour)
     int64_t slots;
     int32_t direct;        // picks are found in the keys (planes of keys per agent), without lists
@@ -526,7 +526,7 @@ __device__ __forceinline__ void scan_block(int block, int blocks, const DayState
                                            const CountTable& T) {
     for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < T.mark_words; i += (int64_t)blocks * blockDim.x)
         T.marks[i] = 0u;
-    const CountBlock blk = T.scans[block];
+    const CountBlock blk = T.scans ? T.scans[block] : CountBlock{0, block * kScanCols};
     if (sts[blk.r].done) return;
     const CountRep c = T.reps[blk.r];
     constexpr int kScanGroups = kCountScanThreads / kScanCols;
@@ -1208,18 +1208,20 @@ struct CountPlan {
             c.tbase = buckets;
             buckets += c.K;
             c.qbase = mark_words;
-            c.chunk0 = (int32_t)chunks.size();
+            c.chunk0 = n_chunks;
+            n_chunks += c.C;
             entries += (int64_t)(c.C + 1) * c.K;
             mark_words += (int64_t)c.C * c.qw;
-            for (int k = 0; k < c.C; ++k) chunks.push_back({(int32_t)r, k});
         }
-        n_chunks = (int)chunks.size();
         // The largest first: a large block started last would run alone (48
         // replicates of 50k to 2M agents: 118 -> 102 us per weekday, 386 -> 291
         // per weekend day).
-        std::stable_sort(chunks.begin(), chunks.end(), [this](const CountBlock& x, const CountBlock& y) {
-            return reps[x.r].A > reps[y.r].A;
-        });
+        std::vector<int32_t> order(reps.size());
+        for (size_t r = 0; r < reps.size(); ++r) order[r] = (int32_t)r;
+        std::stable_sort(order.begin(), order.end(), [this](int32_t x, int32_t y) { return reps[x].A > reps[y].A; });
+        chunks.reserve(n_chunks);
+        for (int32_t r : order)
+            for (int k = 0; k < reps[r].C; ++k) chunks.push_back({r, k});
         // More chunks than CUs: the smallest blocks that still fill a CU's 2,048
         // threads beside the counters, so that one's start (counters cleared,
         // marks read) and end overlap the others' work.  48 replicates of 0.7M
@@ -1239,6 +1241,12 @@ struct CountPlan {
         int32_t chunks_max = 0;
         for (const auto& c : reps) chunks_max = std::max(chunks_max, c.C);
         scan_cols = chunks_max > 128 && buckets < 32768 ? 32 : (chunks_max > 32 ? 64 : (chunks_max > 8 ? 256 : 1024));
+        // One simulation's blocks need no list: at 50M agents it would be most of
+        // what set-up sends (70 KB, 0.4 ms through pageable memory).
+        if (reps.size() == 1) {
+            n_scans = (reps[0].K + scan_cols - 1) / scan_cols;
+            return;
+        }
         for (size_t r = 0; r < reps.size(); ++r)
             for (int b = 0; b < reps[r].K; b += scan_cols) scans.push_back({(int32_t)r, b});
         n_scans = (int)scans.size();
@@ -1285,7 +1293,9 @@ struct CountPlan {
 
 // Buffers shared by the two layouts (weekday, weekend) and the device copies of
 // their plans, in one allocation: the plans, then cleared counters, all sent in
-// one copy, then the rest.
+// one copy, then the rest.  The two matrices go to one of the caller's buffers
+// that is idle on counted days, if they fit: the sorted tables' digit counts, or
+// `spare`.
 struct CountScratch {
     unsigned char* block = nullptr;
     std::vector<unsigned char> image;  // what is sent, kept until it has been
@@ -1293,7 +1303,7 @@ struct CountScratch {
     int32_t* chunk_day = nullptr;
     uint16_t* tile_off = nullptr;
     int32_t* lone_day = nullptr;
-    int alloc(CountPlan (&plan)[2], int64_t N, hipStream_t st) {
+    int alloc(CountPlan (&plan)[2], int64_t N, hipStream_t st, const TableScratch& ts, void* spare, int64_t spare_bytes) {
         const CountPlan &a = plan[0], &b = plan[1];
         const int64_t e = std::max(a.entries, b.entries);
         if (e == 0) return 0;
@@ -1307,7 +1317,6 @@ struct CountScratch {
         for (int w = 0; w < 2; ++w) {
             CountPlan& p = plan[w];
             if (!p.on) continue;
-            p.chunks.resize(p.n_chunks);  // (a split layout numbers its blocks itself)
             at_plan[w][0] = take(p.reps.size(), sizeof(CountRep));
             at_plan[w][1] = take(p.chunks.size(), sizeof(CountBlock));
             at_plan[w][2] = take(p.scans.size(), sizeof(CountBlock));
@@ -1320,7 +1329,10 @@ struct CountScratch {
         const size_t at_tile = take(a.lists || b.lists ? (N / kTileAgents + 1) *
                                         std::max(a.lists ? a.reps[0].toff : 0, b.lists ? b.reps[0].toff : 0) : 0,
                                     sizeof(uint16_t));
-        const size_t at_cnt = take(e, sizeof(uint32_t)), at_pre = take(e, sizeof(uint32_t));
+        const int64_t matrix = (e + 63) / 64 * 64;
+        const int64_t both = 2 * matrix * (int64_t)sizeof(uint32_t);
+        void* const idle = both <= ts.hist_bytes ? ts.hist : (both <= spare_bytes ? spare : nullptr);
+        const size_t at_matrices = take(idle ? 0 : 2 * matrix, sizeof(uint32_t));
         if (dev_alloc(&block, (int64_t)bytes)) return PT_ENOMEM;
         image.assign(sent, 0);
         for (int w = 0; w < 2; ++w) {
@@ -1331,7 +1343,7 @@ struct CountScratch {
             memcpy(image.data() + at_plan[w][2], p.scans.data(), sizeof(CountBlock) * p.scans.size());
             p.d_reps = (CountRep*)(block + at_plan[w][0]);
             p.d_chunks = (CountBlock*)(block + at_plan[w][1]);
-            p.d_scans = (CountBlock*)(block + at_plan[w][2]);
+            p.d_scans = p.scans.empty() ? nullptr : (CountBlock*)(block + at_plan[w][2]);
         }
         HIP_TRY(hipMemcpyAsync(block, image.data(), sent, hipMemcpyHostToDevice, st));
         n = (uint32_t*)(block + at_n);
@@ -1340,8 +1352,8 @@ struct CountScratch {
         total = (uint32_t*)(block + at_total);
         marks = (uint32_t*)(block + at_marks);
         tile_off = (uint16_t*)(block + at_tile);
-        cnt = (uint32_t*)(block + at_cnt);
-        pre = (uint32_t*)(block + at_pre);
+        cnt = idle ? (uint32_t*)idle : (uint32_t*)(block + at_matrices);
+        pre = cnt + matrix;
         return 0;
     }
     void release() {

@@ -82,6 +82,66 @@ int build_model(const pt_params* p, const int32_t seed_key[2], Model& m);
 // PT_EINVAL).
 int apply_interventions(const pt_interventions* iv, Model& m);
 
+// Pairs of the queried buckets: staged by block, then compacted (counted days
+// keep their lists and picks here).  One allocation while it is small: one of
+// 2 MB or more costs about 25 us to make and free again (2.35M agents, set-up
+// 1.20 -> 1.15 ms), but the time of a large one grows with it (1.5 GB 270 us,
+// in four 4 x 36).
+struct SelectionBuffers {
+    uint32_t* stage_keys = nullptr;
+    int32_t* stage_ids = nullptr;
+    uint32_t* sel_keys = nullptr;
+    int32_t* sel_ids = nullptr;
+    bool one = false;
+};
+inline int alloc_selection(SelectionBuffers& b, int64_t staged, int64_t selected) {
+    const int64_t a = (staged + 63) / 64 * 64, c = (selected + 63) / 64 * 64;
+    b.one = 2 * (a + c) * (int64_t)sizeof(uint32_t) <= ((int64_t)256 << 20);
+    if (!b.one)
+        return dev_alloc(&b.stage_keys, staged) || dev_alloc(&b.stage_ids, staged) ||
+               dev_alloc(&b.sel_keys, selected) || dev_alloc(&b.sel_ids, selected);
+    if (dev_alloc(&b.stage_keys, 2 * (a + c))) return PT_ENOMEM;
+    b.stage_ids = (int32_t*)(b.stage_keys + a);
+    b.sel_keys = b.stage_keys + 2 * a;
+    b.sel_ids = (int32_t*)(b.sel_keys + c);
+    return PT_OK;
+}
+inline void free_selection(SelectionBuffers& b) {
+    dev_free(b.stage_keys);
+    if (!b.one) {
+        dev_free(b.stage_ids);
+        dev_free(b.sel_keys);
+        dev_free(b.sel_ids);
+    }
+    b = SelectionBuffers();
+}
+
+// The byte arrays of `count` agents, from 1 MB each in one allocation (seven of
+// 50 MB take 210 us to make, one of 350 MB 38 us; smaller ones cost below 1 us
+// each, as parts of the runtime's blocks).
+template <class Owner>
+int alloc_agent_bytes(Owner& o, int64_t count) {
+    uint8_t** const rest[6] = {&o.st_s, &o.dy_p, &o.dy_s, &o.gn_p, &o.gn_s, &o.age};
+    const int64_t stride = (count + 255) / 256 * 256;
+    o.one_block = stride >= ((int64_t)1 << 20);
+    if (dev_alloc(&o.st_p, o.one_block ? 7 * stride : count)) return PT_ENOMEM;
+    for (int k = 0; k < 6; ++k) {
+        if (o.one_block)
+            *rest[k] = o.st_p + (k + 1) * stride;
+        else if (dev_alloc(rest[k], count))
+            return PT_ENOMEM;
+    }
+    return PT_OK;
+}
+template <class Owner>
+void free_agent_bytes(Owner& o) {
+    dev_free(o.st_p);
+    for (uint8_t** p : {&o.st_s, &o.dy_p, &o.dy_s, &o.gn_p, &o.gn_s, &o.age}) {
+        if (!o.one_block) dev_free(*p);
+        *p = nullptr;
+    }
+}
+
 // What a contact needs of an agent, in one 8-byte record instead of five
 // gathers (age, household, its two offsets, workplace): x = first person of
 // the household | its size << 28 | adult << 31; y = workplace or school | its

@@ -183,7 +183,7 @@ __device__ __forceinline__ void draw2x32(uint32_t c, uint32_t k0, uint32_t k1, u
 
 // (float)u / UNSIGNED_MAX: the divisor converts to 2^32 in float, so this
 // is an exact scaling of the round-to-nearest conversion.
-__device__ __forceinline__ float unit_float(uint32_t u) { return (float)u / 4294967296.0f; }
+__host__ __device__ __forceinline__ float unit_float(uint32_t u) { return (float)u / 4294967296.0f; }
 
 // ---------------- setup draws ----------------
 // device_setup_fishHouseholdType (PandemicSim.cu:2360-2371)
@@ -195,12 +195,18 @@ __device__ __forceinline__ int fish_household(const Model& M, uint32_t r) {
 }
 
 // device_setup_fishWorkplace (PandemicSim.cu:2374-2399)
-__device__ __forceinline__ int32_t fish_workplace(const Model& M, uint32_t r) {
+// row: the type of the workplace.  The reference's loop, while (pdf[row] < y)
+// y -= pdf[row++], over every row with selects: the rows are read as scalars.
+__host__ __device__ __forceinline__ int32_t fish_workplace(const ModelData& M, uint32_t r, int& row) {
     float y = unit_float(r);
-    int row = 0;
-    while (M.wp_pdf[row] < y && row < kTypes - 1) {
-        y -= M.wp_pdf[row];
-        row++;
+    row = 0;
+    bool go = true;
+#pragma unroll
+    for (int t = 0; t < kTypes - 1; ++t) {
+        go = go & (M.wp_pdf[t] < y);
+        const float rest = y - M.wp_pdf[t];
+        y = go ? rest : y;
+        row = go ? t + 1 : row;
     }
     const float frac = y / M.wp_pdf[row];
     const int type_count = M.wp_count[row];
@@ -210,11 +216,12 @@ __device__ __forceinline__ int32_t fish_workplace(const Model& M, uint32_t r) {
 }
 
 // device_setup_fishSchoolAndAge (PandemicSim.cu:2402-2442)
-__device__ __forceinline__ int32_t fish_school_and_age(const Model& M, uint32_t r, uint8_t* age) {
+__host__ __device__ __forceinline__ int32_t fish_school_and_age(const ModelData& M, uint32_t r, uint8_t& age, int& type) {
     const float y = unit_float(r);
     int row = 0;
-    while (row < kChildRows - 1 && y > M.child_cdf[row]) row++;
-    const int wp_type = row + kTypePreschool;
+#pragma unroll
+    for (int t = 0; t < kChildRows - 1; ++t) row += y > M.child_cdf[t];  // (the cdf ascends)
+    type = row + kTypePreschool;
     float frac;
     if (row == 0) {
         frac = y / M.child_cdf[0];
@@ -223,17 +230,30 @@ __device__ __forceinline__ int32_t fish_school_and_age(const Model& M, uint32_t 
         const float y_here = y - M.child_cdf[row - 1];
         frac = y_here / pdf_here;
     }
-    const int type_count = M.wp_count[wp_type];
+    const int type_count = M.wp_count[type];
     int bn = (int)(frac * (float)type_count);
     if (bn >= type_count) bn = type_count - 1;
-    *age = (uint8_t)row;
-    return bn + M.wp_offset[wp_type];
+    age = (uint8_t)row;
+    return bn + M.wp_offset[type];
 }
 
-// device_setup_assignWorkplaceOrSchool (PandemicSim.cu:2445-2457)
-__device__ __forceinline__ int32_t assign_workplace(const Model& M, uint32_t r, uint8_t* age) {
-    if (*age == kAgeAdult) return fish_workplace(M, r);
-    return fish_school_and_age(M, r, age);
+// device_setup_assignWorkplaceOrSchool (PandemicSim.cu:2445-2457): the
+// workplace or school, its contacts per day (workplace_max_contacts, from the
+// type at hand instead of a search), and the age.
+__host__ __device__ __forceinline__ int32_t assign_workplace(const ModelData& M, uint32_t r, bool adult, uint8_t& age,
+                                                             int& contacts) {
+    int type;
+    int32_t wp;
+    if (adult) {
+        wp = fish_workplace(M, r, type);
+        age = kAgeAdult;
+    } else {
+        wp = fish_school_and_age(M, r, age, type);
+    }
+    // A walk that ends on a type without workplaces gives the one before its
+    // offset, the last of the type before.
+    contacts = M.wp_max[M.wp_count[type] > 0 ? type : type - 1];
+    return wp;
 }
 
 // ---------------- errand draws ----------------
@@ -453,7 +473,7 @@ __device__ __forceinline__ void weekend_errands(const Model& M, const Walk& k, u
 }
 
 // device_getWorkplaceMaxContacts (PandemicSim.cu:3492-3511)
-__device__ __forceinline__ int workplace_max_contacts(const Model& M, int32_t loc) {
+__host__ __device__ __forceinline__ int workplace_max_contacts(const ModelData& M, int32_t loc) {
     const int id = loc % M.W;
     int t = 0, off, cnt, mx;
     do {

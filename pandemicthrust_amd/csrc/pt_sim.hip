@@ -117,6 +117,8 @@ __global__ void k_household_sizes(const Model* __restrict__ Mp, const uint8_t* _
 }
 
 // K4: kernel_generateHouseholds (PandemicSim.cu:2490-2531): adults first.
+// Until workplaces are assigned an agent's age byte says where it lives:
+// its place in the household | the household's size << 3 | adult << 6.
 __global__ void k_generate_households(const Model* __restrict__ Mp, const uint8_t* __restrict__ types,
                                       const int32_t* __restrict__ hh_off, int32_t* __restrict__ household,
                                       uint8_t* __restrict__ age) {
@@ -125,60 +127,77 @@ __global__ void k_generate_households(const Model* __restrict__ Mp, const uint8_
     for (int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; h < M.H; h += stride) {
         const int t = types[h];
         const int off = hh_off[h];
-        const int na = M.hh_adults[t], nc = M.hh_children[t];
-        for (int a = 0; a < na; ++a) {
+        const int na = M.hh_adults[t], n = na + M.hh_children[t];
+        for (int a = 0; a < n; ++a) {
             household[off + a] = (int32_t)h;
-            age[off + a] = kAgeAdult;
-        }
-        for (int c = 0; c < nc; ++c) {
-            household[off + na + c] = (int32_t)h;
-            age[off + na + c] = 0;
+            age[off + a] = (uint8_t)(a | (n << 3) | (a < na ? 64 : 0));
         }
     }
 }
 
 // K5: assignWorkplaceFunctor (PandemicSim.cu:3750-3778), four people per
-// counter workplace_off + g, g = 0..N/4.
-__global__ void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workplace_off, uint8_t* __restrict__ age,
-                                    const int32_t* __restrict__ household, const int32_t* __restrict__ hh_off,
-                                    uint32_t* __restrict__ wp_keys, AgentRecord* __restrict__ who,
-                                    int32_t* __restrict__ wp_lone) {
+// counter workplace_off + g, g = 0..N/4, and the agents' records.  Bound by
+// the draws, the type walks and 17 bytes per agent.  The record's household
+// comes with the age byte and its contacts from the walk's type: gathered from
+// the household's offsets and searched by location they doubled the kernel
+// (50M agents 281 us without records, 672 with those, 275 now).
+__global__ __launch_bounds__(256) void k_assign_workplaces(const Model* __restrict__ Mp, uint64_t workplace_off,
+                                                           uint8_t* __restrict__ age, uint32_t* __restrict__ wp_keys,
+                                                           AgentRecord* __restrict__ who, int32_t* __restrict__ wp_lone) {
     const Model& M = *Mp;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *wp_lone = 0;  // for k_lone_workplaces
+    if (blockIdx.x == 0 && threadIdx.x == 0) *wp_lone = 0;  // for k_init_status
     const int N = M.N;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g <= N / 4; g += stride) {
         const U4 u = draw4(workplace_off + (uint64_t)g, M.key0, M.key1);
+        const bool full = 4 * g + 4 <= N;
+        uint32_t at = 0;  // four age bytes
+        if (full)
+            at = reinterpret_cast<const uint32_t*>(age)[g];
+        else
+            for (int i = 0; 4 * g + i < N; ++i) at |= (uint32_t)age[4 * g + i] << (8 * i);
+        uint32_t ages = 0, wp[4];
+        AgentRecord rec[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int64_t p = 4 * g + i;
-            if (p < N) {
-                uint8_t a = age[p];
-                const int32_t wp = assign_workplace(M, u.w[i], &a);
-                age[p] = a;
-                wp_keys[p] = (uint32_t)wp;
-                const int32_t h = household[p], off = hh_off[h];
-                who[p] = make_record(off, hh_off[h + 1] - off, a == kAgeAdult, wp, workplace_max_contacts(M, wp));
+            const uint32_t code = (at >> (8 * i)) & 0xFFu;
+            const bool adult = (code & 64u) != 0;
+            uint8_t a;
+            int contacts;
+            wp[i] = (uint32_t)assign_workplace(M, u.w[i], adult, a, contacts);
+            ages |= (uint32_t)a << (8 * i);
+            rec[i] = make_record((int32_t)(4 * g + i) - (int32_t)(code & 7u), (int32_t)((code >> 3) & 7u), adult,
+                                 (int32_t)wp[i], contacts);
+        }
+        if (full) {
+            reinterpret_cast<uint32_t*>(age)[g] = ages;
+            reinterpret_cast<uint4*>(wp_keys)[g] = make_uint4(wp[0], wp[1], wp[2], wp[3]);
+            uint4* w = reinterpret_cast<uint4*>(who) + 2 * g;
+            w[0] = make_uint4(rec[0].x, rec[0].y, rec[1].x, rec[1].y);
+            w[1] = make_uint4(rec[2].x, rec[2].y, rec[3].x, rec[3].y);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (4 * g + i >= N) break;
+                age[4 * g + i] = (uint8_t)(ages >> (8 * i));
+                wp_keys[4 * g + i] = wp[i];
+                who[4 * g + i] = rec[i];
             }
         }
     }
 }
 
-// Whether some workplace has a single person (such people have no workplace
-// contacts).
-__global__ void k_lone_workplaces(const Model* __restrict__ Mp, const int32_t* __restrict__ wp_off,
-                                  int32_t* __restrict__ lone) {
-    const int W = Mp->W;
-    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < W; w += gridDim.x * blockDim.x)
-        if (wp_off[w + 1] - wp_off[w] == 1) *lone = 1;
-}
-
 // K7: setup_initializeStatusArrays (PandemicSim.cu:3654-3664).  Agents
 // vaccinated against a strain (intervention stream draw below the coverage;
 // coverage 0 in the reference) start recovered for it.
+// Also notes whether some workplace has a single person (such people have no
+// workplace contacts).
 __global__ void k_init_status(const Model* __restrict__ Mp, int64_t N, uint8_t* st_p, uint8_t* st_s, uint8_t* dy_p,
-                              uint8_t* dy_s, uint8_t* gn_p, uint8_t* gn_s) {
+                              uint8_t* dy_s, uint8_t* gn_p, uint8_t* gn_s, const int32_t* __restrict__ wp_off,
+                              int32_t* __restrict__ wp_lone) {
     const Model& M = *Mp;
+    for (int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; w < M.W; w += (int64_t)gridDim.x * blockDim.x)
+        if (wp_off[w + 1] - wp_off[w] == 1) *wp_lone = 1;
     const bool vacc = M.vacc[0] > 0.f || M.vacc[1] > 0.f;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += stride) {
@@ -845,8 +864,9 @@ __global__ void k_workplace_of(const Model* __restrict__ Mp, uint64_t workplace_
     const Model& M = *Mp;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (int64_t)gridDim.x * blockDim.x) {
         const U4 u = draw4(workplace_off + (uint64_t)(i / 4), M.key0, M.key1);
-        uint8_t a = age[i];
-        out[i] = assign_workplace(M, word(u, (int)(i % 4)), &a);
+        uint8_t a;
+        int contacts;
+        out[i] = assign_workplace(M, word(u, (int)(i % 4)), age[i] == kAgeAdult, a, contacts);
     }
 }
 
@@ -1140,16 +1160,15 @@ hipError_t build_population(const Model* d_model, int64_t N, int H, int W, const
     k_generate_households<<<grid_for(H, 256, 65535), 256, 0, st>>>(d_model, P.hh_types, P.hh_off, P.household, P.age);
     if (marks) (void)hipEventRecord(marks[1], st);
     // K5/K6: workplaces, then the workplace table (PandemicSim.cu:3812-3862).
-    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, P.household,
-                                                                     P.hh_off, tmp, P.who, P.wp_lone);
+    k_assign_workplaces<<<grid_for(N / 4 + 1, 256, 65535), 256, 0, st>>>(d_model, workplace_off, P.age, tmp, P.who,
+                                                                     P.wp_lone);
     e = build_table(ts, tmp, nullptr, N, nullptr, W, ID_IDENTITY, (int32_t)N, P.wp_people, P.wp_off, nullptr, st,
                     nullptr);
     if (e != hipSuccess) return e;
-    k_lone_workplaces<<<grid_for(W, 256, 1024), 256, 0, st>>>(d_model, P.wp_off, P.wp_lone);
     if (marks) (void)hipEventRecord(marks[2], st);
     // K7: statuses; claim words start empty.
     k_init_status<<<grid_for(N, 256, 65535), 256, 0, st>>>(d_model, N, P.st_p, P.st_s, P.dy_p, P.dy_s, P.gn_p,
-                                                           P.gn_s);
+                                                           P.gn_s, P.wp_off, P.wp_lone);
     k_fill_u64<<<grid_for(N, 256, 65535), 256, 0, st>>>(P.claim_p, N, ~0ull);
     k_fill_u64<<<grid_for(N, 256, 65535), 256, 0, st>>>(P.claim_s, N, ~0ull);
     if (marks) (void)hipEventRecord(marks[3], st);
@@ -1171,6 +1190,7 @@ struct pt_sim {
     // agent arrays
     uint8_t *st_p = nullptr, *st_s = nullptr, *dy_p = nullptr, *dy_s = nullptr, *gn_p = nullptr, *gn_s = nullptr;
     uint8_t* age = nullptr;
+    bool one_block = false;  // st_p to age in one allocation (alloc_agent_bytes)
     uint8_t* snap = nullptr;  // 6N bytes
     int32_t *household = nullptr, *hh_off = nullptr, *wp_off = nullptr, *wp_people = nullptr;
     AgentRecord* who = nullptr;
@@ -1184,10 +1204,7 @@ struct pt_sim {
     int32_t *list_p = nullptr, *list_s = nullptr;
     uint32_t *blk_counts = nullptr, *blk_ninf = nullptr, *blk_off = nullptr;
     uint32_t* mark = nullptr;                                // queried-bucket bitmap
-    uint32_t* stage_keys = nullptr;                          // selection staging (per-block runs)
-    int32_t* stage_ids = nullptr;
-    uint32_t* sel_keys = nullptr;                            // 3N, compacted selection
-    int32_t* sel_ids = nullptr;                              // 3N
+    SelectionBuffers selection;      // 3N each
     uint32_t *sblk_cnt = nullptr, *sblk_off = nullptr;       // per selection block
     int table_mode = TABLES_AUTO;
     int nblk_sweep = 0;
@@ -1261,13 +1278,7 @@ int alloc_trace(pt_sim* s) {
 
 void free_population(pt_sim* s) {
     free_trace(s);
-    dev_free(s->st_p);
-    dev_free(s->st_s);
-    dev_free(s->dy_p);
-    dev_free(s->dy_s);
-    dev_free(s->gn_p);
-    dev_free(s->gn_s);
-    dev_free(s->age);
+    free_agent_bytes(*s);
     dev_free(s->snap);
     dev_free(s->household);
     dev_free(s->hh_off);
@@ -1289,10 +1300,7 @@ void free_population(pt_sim* s) {
     dev_free(s->blk_ninf);
     dev_free(s->blk_off);
     dev_free(s->mark);
-    dev_free(s->stage_keys);
-    dev_free(s->stage_ids);
-    dev_free(s->sel_keys);
-    dev_free(s->sel_ids);
+    free_selection(s->selection);
     dev_free(s->sblk_cnt);
     dev_free(s->sblk_off);
     for (auto& p : s->count_plan) p.release();
@@ -1314,7 +1322,7 @@ int setup_counts(pt_sim* s) {
         p.build({s->N}, w ? 3 : 2, s->cus);
         if (K[w] > kCountMaxK) p.build_split(s->N, w ? 3 : 2, w ? m.we_E : m.wd_E, w ? kWeHours : kWdHours, s->cus);
     }
-    if (s->count_scratch.alloc(s->count_plan, s->N, s->stream)) {
+    if (s->count_scratch.alloc(s->count_plan, s->N, s->stream, s->tables, s->tables.keys_b, 12 * s->N)) {
         // no memory for the matrices: sorted tables
         (void)hipGetLastError();
         for (CountPlan& p : s->count_plan) p.release();
@@ -1330,17 +1338,17 @@ int setup_counts(pt_sim* s) {
         t.slots = (s->N + 7) / 8 * 8;
         t.keys32 = s->keys;
         t.list = s->er_people;
-        t.pk_bucket = s->stage_keys;
-        t.pk_want = (uint32_t*)s->stage_ids;
-        t.pk_claim = s->sel_keys;
-        t.pk_payload = (uint32_t*)s->sel_ids;
+        t.pk_bucket = s->selection.stage_keys;
+        t.pk_want = (uint32_t*)s->selection.stage_ids;
+        t.pk_claim = s->selection.sel_keys;
+        t.pk_payload = (uint32_t*)s->selection.sel_ids;
         t.pk_idx = (int32_t*)s->tables.pairs_a;  // at most 2 picks per agent, 6 words per agent here
         t.pk_r = t.pk_idx + 3 * s->N;
         t.pk_chunk = (int32_t*)s->tables.pairs_b;
         t.pk_len = t.pk_chunk + 3 * s->N;
-        t.sv_idx = (int32_t*)s->stage_keys + 2 * s->N;  // past the picks
-        t.sv_pos = s->stage_ids + 2 * s->N;
-        t.sv_f = s->sel_keys + 2 * s->N;
+        t.sv_idx = (int32_t*)s->selection.stage_keys + 2 * s->N;  // past the picks
+        t.sv_pos = s->selection.stage_ids + 2 * s->N;
+        t.sv_f = s->selection.sel_keys + 2 * s->N;
         t.wp_lone = s->wp_lone;
         // Small chunks: k_resolve reads about half a chunk's keys per pick (4 to
         // 12 KB of L2), which costs less than the launch that lists the marked
@@ -1419,16 +1427,16 @@ int enqueue_table(pt_sim* s, bool weekend, int64_t n, int32_t K, int64_t nwords,
     const int nb = (int)((s->N + (weekend ? kSelAgentsWe : kSelAgentsWd) - 1) / (weekend ? kSelAgentsWe : kSelAgentsWd));
     if (weekend)
         launch(tm, KC_SELECT, k_select_weekend, dim3(nb), dim3(kSelThreads), stc, M, st, (const uint32_t*)s->mark,
-               s->stage_keys, s->stage_ids, s->sblk_cnt);
+               s->selection.stage_keys, s->selection.stage_ids, s->sblk_cnt);
     else
         launch(tm, KC_SELECT, k_select_weekday, dim3(nb), dim3(kSelThreads), stc, M, st, (const uint8_t*)s->age,
-               (const uint32_t*)s->mark, s->stage_keys, s->stage_ids, s->sblk_cnt);
+               (const uint32_t*)s->mark, s->selection.stage_keys, s->selection.stage_ids, s->sblk_cnt);
     hipError_t e =
         exclusive_scan_u32(s->sblk_cnt, s->sblk_off, nb, s->tables.scan_part, &st->skip_subset, stc, tm, KC_SELECT);
     if (e != hipSuccess) return fail(PT_EDEVICE, "selection scan: %s", hipGetErrorString(e));
     launch(tm, KC_SELECT, k_compact_runs, dim3(nb), dim3(256), stc, (const int32_t*)&st->skip_subset,
-           (const uint32_t*)s->stage_keys, (const int32_t*)s->stage_ids, (const uint32_t*)s->sblk_cnt,
-           (const uint32_t*)s->sblk_off, s->sel_keys, s->sel_ids, weekend ? kSelStageWe : kSelStageWd, &st->n_sel, nb);
+           (const uint32_t*)s->selection.stage_keys, (const int32_t*)s->selection.stage_ids, (const uint32_t*)s->sblk_cnt,
+           (const uint32_t*)s->sblk_off, s->selection.sel_keys, s->selection.sel_ids, weekend ? kSelStageWe : kSelStageWd, &st->n_sel, nb);
     // One table build serves both paths: its first pass reads the selected
     // pairs on subset days (skip_full set) and every agent's keys otherwise.
     // Weekday: the last bucket collects the hour-1 keys nobody queries
@@ -1436,8 +1444,8 @@ int enqueue_table(pt_sim* s, bool weekend, int64_t n, int32_t K, int64_t nwords,
     // (the selection never holds it).
     AltInput sel;
     sel.flag = &st->skip_full;
-    sel.keys = s->sel_keys;
-    sel.vals = s->sel_ids;
+    sel.keys = s->selection.sel_keys;
+    sel.vals = s->selection.sel_ids;
     sel.n_dev = &st->n_sel;
     e = build_table(s->tables, s->keys, nullptr, n, nullptr, K, mode, N, s->er_people, s->er_off, &st->done, stc, tm,
                     weekend ? kNoDrop : (uint32_t)(K - 1), &sel);
@@ -1782,9 +1790,7 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
     const int64_t n3 = 3 * N;
     const int64_t Npad = ((N + 15) / 16) * 16;  // the sweep reads whole uint4 words
     const int64_t stage_n = std::max<int64_t>((N / kSelAgentsWd + 1) * kSelStageWd, (N / kSelAgentsWe + 1) * kSelStageWe);
-    if (dev_alloc(&s->st_p, Npad) || dev_alloc(&s->st_s, Npad) || dev_alloc(&s->dy_p, Npad) ||
-        dev_alloc(&s->dy_s, Npad) || dev_alloc(&s->gn_p, Npad) || dev_alloc(&s->gn_s, Npad) ||
-        dev_alloc(&s->age, Npad) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
+    if (alloc_agent_bytes(*s, Npad) || dev_alloc(&s->snap, 6 * Npad) || dev_alloc(&s->household, N) ||
         dev_alloc(&s->hh_off, (int64_t)H + 1) ||
         dev_alloc(&s->wp_off, (int64_t)s->W + 1) || dev_alloc(&s->wp_people, N) || dev_alloc(&s->who, N) || dev_alloc(&s->wp_lone, 1) ||
         dev_alloc(&s->infected, N) ||
@@ -1793,9 +1799,8 @@ int pt_sim_setup(pt_sim* s, int64_t* n_people_out) {
         dev_alloc(&s->claim_p, N) || dev_alloc(&s->claim_s, N) || dev_alloc(&s->list_p, N) ||
         dev_alloc(&s->list_s, N) || dev_alloc(&s->blk_counts, (int64_t)s->nblk_sweep * 16) ||
         dev_alloc(&s->blk_ninf, s->nblk_sweep) || dev_alloc(&s->blk_off, s->nblk_sweep) ||
-        dev_alloc(&s->mark, (kmax + 31) / 32 + 1) || dev_alloc(&s->stage_keys, stage_n) ||
-        dev_alloc(&s->stage_ids, stage_n) ||
-        dev_alloc(&s->sel_keys, n3) || dev_alloc(&s->sel_ids, n3) || dev_alloc(&s->sblk_cnt, N / kSelAgentsWe + 2) ||
+        dev_alloc(&s->mark, (kmax + 31) / 32 + 1) || alloc_selection(s->selection, stage_n, n3) ||
+        dev_alloc(&s->sblk_cnt, N / kSelAgentsWe + 2) ||
         dev_alloc(&s->sblk_off, N / kSelAgentsWe + 2)) {
         const std::string msg = g_err;
         free_population(s);

@@ -78,7 +78,8 @@ struct TableScratch {
     uint32_t* keys_b = nullptr;  // n_cap: the sorted keys of the last pass
     uint2* pairs_a = nullptr;    // n_cap (key, id) pairs between passes
     uint2* pairs_b = nullptr;    // n_cap
-    uint32_t* hist = nullptr;    // 256 * kMaxSortBlocks
+    uint32_t* hist = nullptr;    // digit counts: 8.4 MB with table_scratch_alloc
+    int64_t hist_bytes = 0;      // (of table_scratch_alloc's)
     uint32_t* scan_part = nullptr;
     uint32_t* n_kept = nullptr;  // pairs kept by a first pass that dropped a key (device)
     int64_t n_cap = 0;

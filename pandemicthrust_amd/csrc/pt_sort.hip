@@ -752,6 +752,7 @@ int table_scratch_alloc(TableScratch& s, int64_t n_cap) {
     const int64_t parts = (std::max<int64_t>(n, hist_n) + kScanSeg - 1) / kScanSeg + 2;
     if (device_malloc((void**)&s.scan_part, (size_t)parts * sizeof(uint32_t)) != hipSuccess) return -1;
     s.n_cap = n_cap;
+    s.hist_bytes = hist_n * (int64_t)sizeof(uint32_t);
     s.wide_bits = wide_bits;
     s.max_bits = max_bits;
     return 0;

@@ -16,7 +16,7 @@ def run_host(source, tmp_path):
     if not (os.path.exists(HIPCC) or shutil.which(HIPCC)):
         pytest.skip("no hipcc")
     exe = str(tmp_path / "host")
-    subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-Wno-unused-function", "-I", CSRC,
+    subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-ffp-contract=off", "-Wno-unused-function", "-I", CSRC,
                     os.path.join(HERE, source), "-o", exe], check=True)
     r = subprocess.run([exe], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0, r.stdout
@@ -29,3 +29,7 @@ def test_column_groups(tmp_path):
 
 def test_pair_keys(tmp_path):
     assert ", 0 wrong" in run_host("count_keys_host.cpp", tmp_path)
+
+
+def test_contacts_by_workplace_type(tmp_path):
+    assert ", 0 wrong" in run_host("workplace_contacts_host.cpp", tmp_path)
