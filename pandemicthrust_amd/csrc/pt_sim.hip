@@ -1264,16 +1264,27 @@ void free_trace(pt_sim* s) {
     dev_free(s->tr_prof);
 }
 
+void release_counts(pt_sim* s) {
+    for (CountPlan& p : s->count_plan) p.release();
+    s->count_scratch.release();
+}
+
+// Traced days sort: the counted tables give up their buffers where there is no
+// room for both (sorted tables from then on, same results).
 int alloc_trace(pt_sim* s) {
-    free_trace(s);
     const int64_t n = 8 * s->N;
-    if (dev_alloc(&s->tr_victim, n) || dev_alloc(&s->tr_type, n) || dev_alloc(&s->tr_loc, n) ||
-        dev_alloc(&s->tr_attempt, n) || dev_alloc(&s->tr_action, n) || dev_alloc(&s->tr_draw, n) ||
-        dev_alloc(&s->tr_prof, n)) {
+    for (;;) {
         free_trace(s);
-        return PT_ENOMEM;
+        if (!(dev_alloc(&s->tr_victim, n) || dev_alloc(&s->tr_type, n) || dev_alloc(&s->tr_loc, n) ||
+              dev_alloc(&s->tr_attempt, n) || dev_alloc(&s->tr_action, n) || dev_alloc(&s->tr_draw, n) ||
+              dev_alloc(&s->tr_prof, n)))
+            return 0;
+        (void)hipGetLastError();  // (the next launch check would report it)
+        if (!s->count_scratch.block) break;
+        release_counts(s);
     }
-    return 0;
+    free_trace(s);
+    return PT_ENOMEM;
 }
 
 void free_population(pt_sim* s) {
@@ -1303,8 +1314,7 @@ void free_population(pt_sim* s) {
     free_selection(s->selection);
     dev_free(s->sblk_cnt);
     dev_free(s->sblk_off);
-    for (auto& p : s->count_plan) p.release();
-    s->count_scratch.release();
+    release_counts(s);
     table_scratch_free(s->tables);
     s->setup_done = s->seeded = s->have_snapshot = false;
 }
@@ -1325,8 +1335,7 @@ int setup_counts(pt_sim* s) {
     if (s->count_scratch.alloc(s->count_plan, s->N, s->stream, s->tables, s->tables.keys_b, 12 * s->N)) {
         // no memory for the matrices: sorted tables
         (void)hipGetLastError();
-        for (CountPlan& p : s->count_plan) p.release();
-        s->count_scratch.release();
+        release_counts(s);
         return PT_OK;
     }
     for (int w = 0; w < 2; ++w) {
