@@ -286,13 +286,18 @@ int pt_sim_get_launch(pt_sim* sim, int32_t knob);
  * synchronises the stream.  Its radix scratch (9 bytes per pair for up to
  * 65,536 buckets, up to 20 for more) is one block; a block of up to 512 MiB
  * per device is kept for the next call, and given back when an allocation of
- * this library fails or a call needs less than a quarter of it.
+ * this library fails, a call needs less than a quarter of it, or by
+ * pt_location_table_release.
  * n < 2^31, n_buckets >= 1.
  * Keys are not checked on the device: a key >= n_buckets leaves the table
  * unspecified, but every write stays inside people[n] and
  * offsets[n_buckets + 1]. */
 int pt_location_table(const uint32_t* keys, int64_t n, int32_t n_buckets, int32_t* people, int32_t* offsets,
                       int32_t device, void* stream);
+
+/* Frees the scratch block kept for pt_location_table on `device` (nothing to
+ * free is no error): for callers whose other allocators need the memory. */
+int pt_location_table_release(int32_t device);
 
 /* The same table, allocating nothing.  No counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph

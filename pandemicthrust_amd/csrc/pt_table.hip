@@ -37,8 +37,9 @@ namespace {
 // One idle scratch block per device, of at most kKeepBytes.  A call takes the
 // block out (calls that overlap allocate their own), waits for its stream, and
 // puts its block back in place of a smaller one.  A block more than four times
-// what a call needs is freed instead of used, and every block is freed when an
-// allocation of the library fails.
+// what a call needs is freed instead of used, every block is freed when an
+// allocation of the library fails, and a caller may free it
+// (pt_location_table_release).
 constexpr size_t kKeepBytes = (size_t)512 << 20;
 constexpr int kMaxDevices = 64;
 struct Block {
@@ -111,5 +112,14 @@ extern "C" int pt_location_table(const uint32_t* keys, int64_t n, int32_t n_buck
         return fail(PT_EDEVICE, "location table: %s", hipGetErrorString(e));
     }
     put_block(device, block);
+    return PT_OK;
+}
+
+extern "C" int pt_location_table_release(int32_t device) {
+    if (device < 0 || device >= kMaxDevices) return fail(PT_EINVAL, "device %d outside [0, %d)", device, kMaxDevices);
+    DeviceScope ds(device);
+    HIP_TRY(ds.err);
+    const Block block = take_block(device);
+    if (block.p) HIP_TRY(hipFree(block.p));
     return PT_OK;
 }
