@@ -1236,11 +1236,24 @@ struct CountPlan {
         }
         plan_scans();
     }
-    // A block's rows per turn cover the chunks of most simulations at once.
+    // Buckets per block of k_count_scan: the fewer, the more rows (chunks) a turn
+    // covers and the shorter the runs of the matrix that it reads.  64 unless a
+    // block would have few rows to do (32 chunks or less: 256, 8 or less: 1,024)
+    // or there would be few blocks with many (up to 128 blocks and over 128
+    // chunks: 32).  us with 32 / 64 / 256 / 1,024 buckets (* taken), and where:
+    //   657 chunks    870 buckets  *11 /  18 /   60 / 220  2.4M agents, location scale 0.3, weekday
+    //   253         6,381           *7 /   9 /   25 /  95  5.2M, 2.2, weekday
+    //   256        14,501           13 / *11 /   26 /  95  12M, 5, weekday
+    //   253        28,600           24 / *16 /   27 /  95  5.2M, 2.2, weekend
+    //   128        61,596           33 / *18 /   21 /  51  50M, 21.24, weekday
+    //    58       116,001           46 / *19 /   15 /  27  235k, 40, weekday
+    //    51       276,110          103 / *39 /   32 /  60  50M, 21.24, weekend
+    //    32       290,001           98 /  32 /  *19 /  36  24M, 100, weekday
+    //     6     1,300,000          387 /  99 /   32 / *19  24M, 100, weekend
     void plan_scans() {
         int32_t chunks_max = 0;
         for (const auto& c : reps) chunks_max = std::max(chunks_max, c.C);
-        scan_cols = chunks_max > 128 && buckets < 32768 ? 32 : (chunks_max > 32 ? 64 : (chunks_max > 8 ? 256 : 1024));
+        scan_cols = chunks_max > 128 && buckets <= 128 * 64 ? 32 : (chunks_max > 32 ? 64 : (chunks_max > 8 ? 256 : 1024));
         // One simulation's blocks need no list: at 50M agents it would be most of
         // what set-up sends (70 KB, 0.4 ms through pageable memory).
         if (reps.size() == 1) {
