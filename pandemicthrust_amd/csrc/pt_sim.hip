@@ -1473,7 +1473,6 @@ bool merged_launches(const pt_sim* s, const CountPlan& p) {
 int end_enqueue(pt_sim* s, int d, bool weekend, int64_t n, bool counted) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(PT_EDEVICE, "day launch: %s", hipGetErrorString(e));
-    s->report_valid = false;
     s->last_weekend = weekend ? 1 : 0;
     s->last_table_n = n;
     s->last_counted = counted;
@@ -1488,6 +1487,7 @@ int end_enqueue(pt_sim* s, int d, bool weekend, int64_t n, bool counted) {
 int enqueue_day(pt_sim* s, int d) {
     const bool weekend = (d % 7) >= 5;
     hipStream_t stc = s->stream;
+    s->report_valid = false;  // also if a launch fails: the day may have run
     s->timer.day = d;
     LaunchTimer* tm = &s->timer;
     DayState* st = s->d_state;
