@@ -1,14 +1,15 @@
 """A trace that fits only without the counted tables' buffers: enabling it
 succeeds, as before there were any, and the simulation goes on with sorted
 tables.  2.35M agents over 200 times the locations: 245 MB of trace arrays, 80
-MB and more of counted tables.  All but 200 MB of the free device memory is
-taken by the test."""
+MB and more of counted tables.  All but 200 MB of the device's free memory is
+taken by the test (no kernel runs while all of it is)."""
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
 
-from hip_mem import DeviceArray
+from hip_mem import DeviceArray, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -18,7 +19,7 @@ LEAVE = 204 << 20
 
 def test_trace_when_memory_is_short():
     from pandemicthrust_amd import Params, PandemicSim
-    from pandemicthrust_amd.api import device_memory
+    from pandemicthrust_amd.api import lib
     want = PandemicSim(Params.from_row(ROW), 7)
     want.setup_sim()
     counts, inf = want.run()
@@ -27,20 +28,28 @@ def test_trace_when_memory_is_short():
     s = PandemicSim(Params.from_row(ROW), 7)
     s.setup_sim()
     first = s.step()
+    assert lib().pt_location_table_release(0) == 0      # (else it is given up first)
+    gap = DeviceArray(LEAVE, np.uint8)
     hog = []
     try:
-        # In pieces of at most 16 GB; what was freed before comes back bit by bit.
-        for _ in range(60):
-            rest = device_memory()[0] - LEAVE
-            if rest > 4 << 20:
-                hog.append(DeviceArray(min(rest, 16 << 30), np.uint8))
-            else:
-                time.sleep(0.05)
-        print("left: %d MB" % (device_memory()[0] >> 20), flush=True)
+        quiet = 0
+        while quiet < 5:        # what was freed before comes back bit by bit
+            had, size = len(hog), 16 << 30
+            while size >= 4 << 20:
+                p = C.c_void_p()
+                if hip().hipMalloc(C.byref(p), size) == 0:
+                    hog.append(p)
+                else:
+                    size //= 2
+            hip().hipGetLastError()
+            quiet = quiet + 1 if len(hog) == had else 0
+            time.sleep(0.1)
+        gap.free()
+        time.sleep(0.5)
         s.enable_trace(True)
     finally:
-        for h in hog:
-            h.free()
+        for p in hog:
+            hip().hipFree(p)
     rows = [first] + [s.step() for _ in range(3)]
     s.enable_trace(False)
     rows += [s.step() for _ in range(2)]
