@@ -250,12 +250,16 @@ int pt_sim_trace_draws(pt_sim* sim, uint8_t* draw, uint8_t* profile, int64_t n);
 /* Launch shapes and table-strategy thresholds.  They change only speed:
  * results are identical for every accepted value (the kernels stride over
  * their work, the radix sort is stable at any tile size, and a table of the
- * queried buckets answers every query a full table does).
+ * queried buckets answers every query a full table does).  The radix and
+ * table-strategy settings (all but the blocks per compute unit) act on sorted
+ * tables: the workplace table, table modes 1 and 2, traced days and layouts
+ * that the automatic mode does not count.
  * pandemicthrust_amd/autotune.py picks them by measurement. */
 enum pt_launch_knob {
     PT_LAUNCH_CONTACT_BLOCKS_PER_CU = 0, /* blocks per compute unit of the mark, contact and apply kernels
                                             (1..64, default 8) */
-    PT_LAUNCH_GEN_BLOCKS_PER_CU,         /* blocks per compute unit of the errand-key kernels (1..64, default 16) */
+    PT_LAUNCH_GEN_BLOCKS_PER_CU,         /* blocks per compute unit of the errand-key kernels (1..64, default 16); on
+                                            counted days of the weekday keys of split layouts alone */
     PT_LAUNCH_SORT_WIDE_BITS,            /* radix passes of at least this many bits (at most 8) run 1024-thread
                                             blocks on 8192-pair tiles, narrower ones 512 on 4096 (1..9,
                                             default 8; 9 = never) */

@@ -14,6 +14,11 @@ from the same snapshot (coordinate descent: one setting at a time, the
 others at their best so far) and keeps the fastest by the engine's own
 loop timer (HIP events around the enqueued days).
 
+On days whose errand tables are counted, which is what the automatic table
+mode does on all but extreme layouts, the radix and table-strategy settings
+have no effect (their trials differ by noise, below MIN_GAIN, so the defaults
+stay); the contact blocks act, and the key blocks on split layouts.
+
     python -m pandemicthrust_amd.autotune --rows 64 --out tuning.json
 """
 import argparse
